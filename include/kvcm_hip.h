@@ -81,6 +81,15 @@ int32_t kvcm_hip_hash_tokens_i32(const int32_t *d_tokens, const int64_t *d_token
                                  const int64_t *d_key_offsets, kvcm_stream_t stream);
 
 /*
+ * The same for R requests of one length, laid out one behind the other ([R][tokens_per_request], token_bytes = 4 or 8):
+ * no offset arrays are read. d_key_offsets may be NULL (request r's keys start at r * (tokens_per_request / block_size));
+ * d_key_offsets_out, when not NULL, receives those R + 1 offsets. tokens_per_request must be at least block_size.
+ */
+int32_t kvcm_hip_hash_tokens_2d(const void *d_tokens, int32_t token_bytes, int32_t R, int64_t tokens_per_request,
+                                int32_t block_size, int64_t seed, int64_t *d_keys, const int64_t *d_key_offsets,
+                                int64_t *d_key_offsets_out, kvcm_stream_t stream);
+
+/*
  * Prefix-chained keys from per-block digests: keys[i] = fold of digests[0..i].
  * Replaces: ApplyPrefixHash  kv_cache_manager/optimizer/trace_converter/trace_util.cc:47-56.
  * Sequence r owns d_digests[d_offsets[r] .. d_offsets[r+1]) and writes the same index range of d_keys.

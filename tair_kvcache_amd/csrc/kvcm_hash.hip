@@ -537,6 +537,16 @@ __device__ __forceinline__ void read_row(ulonglong2 (&a)[kRowVecs], const uint64
     }
 }
 
+// R requests of the same length, one behind the other (the kernel's token_offsets is NULL): nothing has to be read before
+// the first tokens, and the key offsets, which follow from the sizes, are written on the side where the caller wants them
+// -- one launch instead of eight (the offsets were computed by seven small launches in front of this one: 42 us of host
+// time for a launch that lasts 9).
+struct Uniform {
+    int64_t tokens;            // tokens per request
+    int64_t keys;              // tokens / block size
+    int64_t *key_offsets_out;  // [R + 1], or NULL
+};
+
 // CHUNK = steps between two looks at the block boundary: 8 when block_size % 8 == 0 (a lane is then
 // active for whole chunks or not at all), otherwise 1. BS = block size when it is 1, 8, 16, 32, 64 or 128, otherwise 0.
 // KS != kKeysDirect ("keys staged", block sizes 1 to 64; chosen by the host for batches of many requests, where the launch
@@ -549,7 +559,7 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
                                                               int32_t block_size, uint64_t seed,
                                                               int64_t *__restrict__ keys,
                                                               const int64_t *__restrict__ key_offsets,
-                                                              int32_t force_global_loads) {
+                                                              const Uniform uni, int32_t force_global_loads) {
     __shared__ __attribute__((aligned(16))) uint64_t s_tile[kRing][kReqs][kTT + kPad];
     __shared__ int64_t s_start[kReqs];
     __shared__ int64_t s_ntok[kReqs];
@@ -571,13 +581,24 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
     int64_t my_ntok = 0, key_pos = 0;
     LoaderCtx<TokT> ctx;
     bool buffer_loads = false;
+    const int64_t r_first = static_cast<int64_t>(blockIdx.x) * kReqs;
     if (wave == 0) {
-        int64_t start = token_offsets[static_cast<int64_t>(blockIdx.x) * kReqs];  // rows past R idle at the first row
-        if (r < R) {
-            start = token_offsets[r];
-            const int64_t n = token_offsets[r + 1] - start;
-            my_ntok = (n / block_size) * block_size;  // a trailing partial block yields no key
-            key_pos = key_offsets ? key_offsets[r] : r * ((token_offsets[1] - token_offsets[0]) / block_size);
+        int64_t start;
+        if (token_offsets) {
+            start = token_offsets[r_first];  // rows past R idle at the first row
+            if (r < R) {
+                start = token_offsets[r];
+                const int64_t n = token_offsets[r + 1] - start;
+                my_ntok = (n / block_size) * block_size;  // a trailing partial block yields no key
+                key_pos = key_offsets ? key_offsets[r] : r * ((token_offsets[1] - token_offsets[0]) / block_size);
+            }
+        } else {
+            start = r_first * uni.tokens;
+            if (r < R) {
+                start = r * uni.tokens;
+                my_ntok = uni.keys * block_size;
+                key_pos = key_offsets ? key_offsets[r] : r * uni.keys;
+            }
         }
         s_start[lane] = start;
         s_ntok[lane] = my_ntok;
@@ -587,15 +608,23 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
     } else {
         ctx.tokens = tokens;
         ctx.s_start = s_start;
-        const int64_t total = token_offsets[R];
-        ctx.last_token = total - 1;  // >= 0 whenever a tile is loaded: some request has a full block then
-        const int64_t r_first = static_cast<int64_t>(blockIdx.x) * kReqs;
         const int64_t r_end = r_first + kReqs < R ? r_first + kReqs : R;
-        ctx.wg_first_token = token_offsets[r_first];
+        const int64_t total = token_offsets ? token_offsets[R] : R * uni.tokens;
+        const int64_t end_token = token_offsets ? token_offsets[r_end] : r_end * uni.tokens;
+        ctx.last_token = total - 1;  // >= 0 whenever a tile is loaded: some request has a full block then
+        ctx.wg_first_token = token_offsets ? token_offsets[r_first] : r_first * uni.tokens;
         const uint64_t to_end = static_cast<uint64_t>(total - ctx.wg_first_token) * sizeof(TokT);
         ctx.wg_bytes = to_end > 0xFFFFFFFFull ? 0xFFFFFFFFu : static_cast<uint32_t>(to_end);
-        const uint64_t wg_span = static_cast<uint64_t>(token_offsets[r_end] - ctx.wg_first_token) * sizeof(TokT);
+        const uint64_t wg_span = static_cast<uint64_t>(end_token - ctx.wg_first_token) * sizeof(TokT);
         buffer_loads = !force_global_loads && wg_span < 0xFFF00000ull;
+        if (uni.key_offsets_out && wave == kLoaders) {  // the last loader: its first tile is the one needed last
+            if (r < R) {
+                uni.key_offsets_out[r] = r * uni.keys;
+            }
+            if (r_end == R && lane == 0) {
+                uni.key_offsets_out[R] = R * uni.keys;
+            }
+        }
     }
     __syncthreads();
 
@@ -870,27 +899,28 @@ constexpr int32_t burst_from(int32_t block_size, bool tokens_8_byte) {
 
 template <typename TokT>
 int32_t launch_hash(const TokT *d_tokens, const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t seed,
-                    int64_t *d_keys, const int64_t *d_key_offsets, hipStream_t stream) {
+                    int64_t *d_keys, const int64_t *d_key_offsets, hipStream_t stream,
+                    const Uniform &uni = Uniform{0, 0, nullptr}) {
     if (R < 0 || block_size <= 0) {
         return KVCM_ERR_INVALID_ARG;
     }
     if (R == 0) {
         return KVCM_OK;
     }
-    if (!d_tokens || !d_token_offsets || !d_keys) {
+    if (!d_tokens || (!d_token_offsets && uni.keys <= 0) || !d_keys) {
         return KVCM_ERR_INVALID_ARG;
     }
     const dim3 grid(static_cast<uint32_t>((static_cast<int64_t>(R) + kReqs - 1) / kReqs));
     const int32_t force_global = kForceGeneralLoader;
 #define KVCM_LAUNCH_HASH(CHUNK, BS)                                                                                  \
     hipLaunchKernelGGL((hash_tokens_kernel<TokT, CHUNK, BS>), grid, dim3(kThreads), 0, stream, d_tokens,            \
-                       d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, force_global)
+                       d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, force_global)
     constexpr bool k8 = sizeof(TokT) == 8;
     const bool burst = R >= static_cast<int64_t>(burst_from(block_size, k8)) * KVCM_HASH_BURST_SCALE;
     const bool spread = block_size == 16 && k8 && !burst && R >= KVCM_HASH_SPREAD_FROM_8;
 #define KVCM_LAUNCH_HASH_STAGED(CHUNK, BS, KS)                                                                       \
     hipLaunchKernelGGL((hash_tokens_kernel<TokT, CHUNK, BS, KS>), grid, dim3(kThreads), 0, stream, d_tokens,        \
-                       d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, force_global)
+                       d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, force_global)
     // 4-byte tokens from as many requests as take the burst form: tiles of 128 raw tokens (512-byte pieces of the
     // token stream per request and load instruction instead of 256-byte ones). Cold timings, 16-token blocks, requests
     // of 4096 tokens, 64-token tiles of pre-added terms / raw tiles: 64 requests 56.8 / 57.3 us, 8192 58.1 / 60.2,
@@ -899,7 +929,7 @@ int32_t launch_hash(const TokT *d_tokens, const int64_t *d_token_offsets, int32_
                                       block_size == 128);
 #define KVCM_LAUNCH_HASH_RAW(BS)                                                                                      \
     hipLaunchKernelGGL((hash_tokens_kernel<TokT, 8, BS, kKeysBurst, true>), grid, dim3(kThreads), 0, stream, d_tokens, \
-                       d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, force_global)
+                       d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, force_global)
     if (raw) {
         if constexpr (!k8) {
             switch (block_size) {
@@ -987,6 +1017,21 @@ int32_t kvcm_hip_hash_tokens_i32(const int32_t *d_tokens, const int64_t *d_token
                                  kvcm_stream_t stream) {
     return kvcm::launch_hash<int32_t>(d_tokens, d_token_offsets, R, block_size, seed, d_keys, d_key_offsets,
                                       static_cast<hipStream_t>(stream));
+}
+
+int32_t kvcm_hip_hash_tokens_2d(const void *d_tokens, int32_t token_bytes, int32_t R, int64_t tokens_per_request,
+                                int32_t block_size, int64_t seed, int64_t *d_keys, const int64_t *d_key_offsets,
+                                int64_t *d_key_offsets_out, kvcm_stream_t stream) {
+    if ((token_bytes != 4 && token_bytes != 8) || R < 0 || block_size <= 0 || tokens_per_request < block_size) {
+        return KVCM_ERR_INVALID_ARG;
+    }
+    const kvcm::Uniform uni{tokens_per_request, tokens_per_request / block_size, d_key_offsets_out};
+    if (token_bytes == 8) {
+        return kvcm::launch_hash<int64_t>(static_cast<const int64_t *>(d_tokens), nullptr, R, block_size, seed, d_keys,
+                                          d_key_offsets, static_cast<hipStream_t>(stream), uni);
+    }
+    return kvcm::launch_hash<int32_t>(static_cast<const int32_t *>(d_tokens), nullptr, R, block_size, seed, d_keys,
+                                      d_key_offsets, static_cast<hipStream_t>(stream), uni);
 }
 
 int32_t kvcm_hip_prefix_chain(const int64_t *d_digests, const int64_t *d_offsets, int32_t R, int64_t *d_keys,

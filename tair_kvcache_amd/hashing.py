@@ -17,17 +17,6 @@ from . import _lib
 from ._torch_util import lib, ptr, require_cuda, stream_handle
 
 
-def _offsets_for(tokens, token_offsets):
-    if token_offsets is None:
-        if tokens.dim() != 2:
-            raise ValueError("tokens must be [R, L] when token_offsets is not given")
-        R, L = tokens.shape
-        off = torch.arange(R + 1, dtype=torch.int64, device=tokens.device) * L
-        return off, R
-    _require_offsets(token_offsets, "token_offsets", tokens.device)
-    return token_offsets.contiguous(), token_offsets.numel() - 1
-
-
 def _require_offsets(t, name, device, entries=None):
     """Offsets are read by the kernel as they are: int64, 1-D, on the tokens' device, R+1 entries."""
     require_cuda(t, name)
@@ -56,7 +45,16 @@ def hash_tokens(tokens: torch.Tensor, block_size: int, token_offsets: Optional[t
     if int(block_size) <= 0:
         raise ValueError("block_size must be positive")
     tokens = tokens.contiguous()
-    off, R = _offsets_for(tokens, token_offsets)
+    block_size = int(block_size)
+    if token_offsets is None:
+        if tokens.dim() != 2:
+            raise ValueError("tokens must be [R, L] when token_offsets is not given")
+        R = tokens.shape[0]
+        total = R * (tokens.shape[1] // block_size)
+    else:
+        _require_offsets(token_offsets, "token_offsets", tokens.device)
+        off = token_offsets.contiguous()
+        R, total = off.numel() - 1, None
     if key_offsets is not None:
         _require_offsets(key_offsets, "key_offsets", tokens.device, R + 1)
         key_offsets = key_offsets.contiguous()
@@ -64,24 +62,32 @@ def hash_tokens(tokens: torch.Tensor, block_size: int, token_offsets: Optional[t
         require_cuda(keys, "keys")
         if keys.dtype != torch.int64 or keys.device != tokens.device or not keys.is_contiguous():
             raise ValueError("keys must be a contiguous int64 tensor on the tokens' device")
-        if token_offsets is None and keys.numel() < R * (tokens.shape[1] // int(block_size)):
-            raise ValueError(f"keys holds {keys.numel()} entries, the batch yields "
-                             f"{R * (tokens.shape[1] // int(block_size))}")
+        if total is not None and keys.numel() < total:
+            raise ValueError(f"keys holds {keys.numel()} entries, the batch yields {total}")
+    if token_offsets is None:  # equally long requests: one launch, which also writes the key offsets
+        new_offsets = None
+        if keys is None:
+            keys = torch.empty(total, dtype=torch.int64, device=tokens.device)
+        if total == 0:  # no request holds a full block: nothing to launch (GenKeyVector returns an empty vector)
+            return keys, (torch.zeros(R + 1, dtype=torch.int64, device=tokens.device) if key_offsets is None
+                          else key_offsets)
+        if key_offsets is None:
+            new_offsets = torch.empty(R + 1, dtype=torch.int64, device=tokens.device)
+        rc = lib().kvcm_hip_hash_tokens_2d(ptr(tokens), tokens.element_size(), R, tokens.shape[1], block_size, int(seed),
+                                           ptr(keys), ptr(key_offsets), ptr(new_offsets), stream_handle(tokens.device))
+        _lib.check(rc, "kvcm_hip_hash_tokens_2d")
+        return keys, (new_offsets if key_offsets is None else key_offsets)
     if key_offsets is None:
-        counts = (off[1:] - off[:-1]) // int(block_size)
+        counts = (off[1:] - off[:-1]) // block_size
         key_offsets = torch.zeros(R + 1, dtype=torch.int64, device=tokens.device)
         torch.cumsum(counts, 0, out=key_offsets[1:])
     if keys is None:
-        if token_offsets is None:
-            total = R * (tokens.shape[1] // int(block_size))
-        else:
-            total = int(key_offsets[-1].item())
+        total = int(key_offsets[-1].item())
         keys = torch.empty(total, dtype=torch.int64, device=tokens.device)
-        if total == 0:  # no request holds a full block: nothing to launch (GenKeyVector returns an empty vector)
+        if total == 0:
             return keys, key_offsets
     fn = lib().kvcm_hip_hash_tokens if tokens.dtype == torch.int64 else lib().kvcm_hip_hash_tokens_i32
-    rc = fn(ptr(tokens), ptr(off), R, int(block_size), int(seed), ptr(keys), ptr(key_offsets),
-            stream_handle(tokens.device))
+    rc = fn(ptr(tokens), ptr(off), R, block_size, int(seed), ptr(keys), ptr(key_offsets), stream_handle(tokens.device))
     _lib.check(rc, "kvcm_hip_hash_tokens")
     return keys, key_offsets
 

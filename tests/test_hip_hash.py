@@ -304,3 +304,23 @@ def test_raw_tiles_of_4_byte_tokens(oracle, force_general_hash_loader, bs, gener
     got = host(got, np.int64)
     assert (got[:len(want)] == want).all()
     assert (got[len(want):] == -7).all()
+
+
+@pytest.mark.parametrize("R,L,bs", [(1, 16, 16), (63, 17, 16), (64, 130, 64), (65, 47, 24), (128, 128, 128), (129, 10, 3)])
+def test_equally_long_requests_need_no_offset_arrays(oracle, R, L, bs):
+    """[R, L] tokens in one launch: lengths with and without a trailing partial block, request counts around a workgroup's
+    64, both token widths, key offsets written by the launch or given by the caller (with gaps between the requests)."""
+    rng = np.random.default_rng(R * 131 + L)
+    tok = rng.integers(-2**31, 2**31 - 1, size=(R, L), dtype=np.int64)
+    want, woff = oracle.hash_tokens(tok, bs, seed=9)
+    per = L // bs
+    gaps = np.arange(R + 1, dtype=np.int64) * (per + 1)
+    for dtype in (np.int64, np.int32):
+        keys, off = _h().hash_tokens(dev(tok.astype(dtype)), bs, seed=9)
+        spread = torch.full((R * (per + 1),), -7, dtype=torch.int64, device="cuda")
+        _, same = _h().hash_tokens(dev(tok.astype(dtype)), bs, seed=9, keys=spread, key_offsets=dev(gaps))
+        sync()
+        assert (host(keys, np.int64) == want).all() and (host(off, np.int64) == woff).all()
+        assert (host(same, np.int64) == gaps).all()
+        got = host(spread, np.int64).reshape(R, per + 1)
+        assert (got[:, :per] == want.reshape(R, per)).all() and (got[:, per] == -7).all()
