@@ -68,7 +68,7 @@ const char *kvcm_hip_error_string(int32_t code);
  * `seed` (the reference uses 0), after folding tokens [0, (i+1)*block_size) with
  *   h <- h XOR (v + 0x9e3779b97f4a7c15 + (h << 12) + (h >> 32))   (int64, arithmetic >>, mod 2^64).
  * d_key_offsets may be NULL when every request has the same length L = token_offsets[1]-[0]; keys of
- * request r then start at r * (L / block_size).
+ * request r then start at r * (L / block_size). A request whose key offset is negative is left out.
  */
 int32_t kvcm_hip_hash_tokens(const int64_t *d_tokens, const int64_t *d_token_offsets, int32_t R,
                              int32_t block_size, int64_t seed, int64_t *d_keys,
@@ -88,6 +88,22 @@ int32_t kvcm_hip_hash_tokens_i32(const int32_t *d_tokens, const int64_t *d_token
 int32_t kvcm_hip_hash_tokens_2d(const void *d_tokens, int32_t token_bytes, int32_t R, int64_t tokens_per_request,
                                 int32_t block_size, int64_t seed, int64_t *d_keys, const int64_t *d_key_offsets,
                                 int64_t *d_key_offsets_out, kvcm_stream_t stream);
+
+/*
+ * Key offsets of R > 0 requests: d_key_offsets[0..R] = exclusive prefix sums of len_r / block_size. A request whose keys
+ * would end beyond `limit` gets the offset -1 (kvcm_hip_hash_tokens leaves it out). h_total, when not NULL, is PINNED
+ * host memory: the call sets it to KVCM_PENDING and the kernel to d_key_offsets[R]; kvcm_wait_value() waits for that
+ * without waiting for anything launched later.
+ */
+#define KVCM_PENDING (-INT64_C(0x4000000000000000))
+int32_t kvcm_hip_key_offsets(const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t limit,
+                             int64_t *d_key_offsets, int64_t *h_total, kvcm_stream_t stream);
+
+/*
+ * Blocks the calling thread until *h_value (pinned host memory that work on `stream` writes) is no longer KVCM_PENDING.
+ * Ends with an error instead when the stream has failed, or has drained without writing it.
+ */
+int32_t kvcm_wait_value(const int64_t *h_value, kvcm_stream_t stream);
 
 /*
  * Prefix-chained keys from per-block digests: keys[i] = fold of digests[0..i].

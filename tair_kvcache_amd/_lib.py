@@ -55,6 +55,8 @@ SIGNATURES = {
     "kvcm_hip_hash_tokens": (i32, [vp, vp, i32, i32, i64, vp, vp, vp]),
     "kvcm_hip_hash_tokens_i32": (i32, [vp, vp, i32, i32, i64, vp, vp, vp]),
     "kvcm_hip_hash_tokens_2d": (i32, [vp, i32, i32, i64, i32, i64, vp, vp, vp, vp]),
+    "kvcm_hip_key_offsets": (i32, [vp, i32, i32, i64, vp, vp, vp]),
+    "kvcm_wait_value": (i32, [vp, vp]),
     "kvcm_hip_prefix_chain": (i32, [vp, vp, i32, vp, vp]),
     "kvcm_hip_sha256_first8_be": (i32, [vp, vp, i32, vp, vp]),
     "kvcm_hip_batch_gather": (i32, [vp, i32, vp, i64, vp, vp, i32, i32, i64, i32, vp]),

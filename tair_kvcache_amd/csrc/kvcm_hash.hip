@@ -23,6 +23,9 @@
 // dependent-instruction latency of the chain wave, which no amount of bandwidth removes.
 #include "kvcm_internal.h"
 
+#include <sched.h>
+#include <time.h>
+
 #include <climits>
 
 namespace kvcm {
@@ -592,6 +595,7 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
                 my_ntok = (n / block_size) * block_size;  // a trailing partial block yields no key
                 key_pos = key_offsets ? key_offsets[r] : r * ((token_offsets[1] - token_offsets[0]) / block_size);
             }
+            my_ntok = key_pos < 0 ? 0 : my_ntok;
         } else {
             start = r_first * uni.tokens;
             if (r < R) {
@@ -599,6 +603,7 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
                 my_ntok = uni.keys * block_size;
                 key_pos = key_offsets ? key_offsets[r] : r * uni.keys;
             }
+            my_ntok = key_pos < 0 ? 0 : my_ntok;  // a negative key offset: no keys are wanted for this request
         }
         s_start[lane] = start;
         s_ntok[lane] = my_ntok;
@@ -713,6 +718,79 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
                                       key_pos);
         }
         lds_barrier();
+    }
+}
+
+// ------------------------------------------------------------------------------------------- key offsets
+
+// Where every request's keys go: exclusive prefix sums of len / block_size, and the total -- the latter straight into host
+// memory, so that a caller who has to size something by it waits for THIS kernel (a few us) and not for the hash kernel
+// behind it. Bound by latency: a workgroup scans kOffsetsPerWg requests, eight per thread (their nine offsets are in flight
+// together), and adds up everything in front of its range itself instead of waiting for a pass of partial sums: one launch,
+// no workspace. 160 requests 3.2 us against 7.5 us on the device (and 3.6 against 22 on the host) for five launches of a
+// general prefix sum; 8192 requests 8.5 against 12.5, 16 384 10.1 against 12.8, then the re-reading shows: 65 536 20 / 13.
+constexpr int kOffsetsThreads = 1024;
+constexpr int kOffsetsPerThread = 8;
+constexpr int64_t kOffsetsPerWg = kOffsetsThreads * kOffsetsPerThread;
+
+__device__ __forceinline__ int64_t keys_of(int64_t len, int32_t block_size) {
+    if (static_cast<uint64_t>(len) >> 32 == 0) {  // 32-bit division: a fifth of the instructions
+        return static_cast<uint32_t>(len) / static_cast<uint32_t>(block_size);
+    }
+    return len > 0 ? len / block_size : 0;
+}
+
+__global__ __launch_bounds__(kOffsetsThreads) void key_offsets_kernel(const int64_t *__restrict__ token_offsets, int32_t R,
+                                                                      int32_t block_size, int64_t limit,
+                                                                      int64_t *__restrict__ key_offsets, int64_t *h_total) {
+    __shared__ int64_t s_wave[2][kOffsetsThreads / 64];
+    const int32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    const int64_t base = blockIdx.x * kOffsetsPerWg;
+    int64_t before = 0;
+    for (int64_t i = threadIdx.x; i < base; i += blockDim.x) {
+        before += keys_of(token_offsets[i + 1] - token_offsets[i], block_size);
+    }
+    const int64_t first = base + static_cast<int64_t>(threadIdx.x) * kOffsetsPerThread;
+    int64_t off[kOffsetsPerThread + 1];
+#pragma unroll
+    for (int j = 0; j <= kOffsetsPerThread; ++j) {
+        off[j] = token_offsets[first + j < R ? first + j : R];
+    }
+    int64_t count[kOffsetsPerThread], sum = 0;
+#pragma unroll
+    for (int j = 0; j < kOffsetsPerThread; ++j) {
+        count[j] = keys_of(off[j + 1] - off[j], block_size);
+        sum += count[j];
+    }
+    int64_t incl = sum;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int64_t up = __shfl_up(incl, d, 64);
+        incl += lane >= d ? up : 0;
+        before += __shfl_xor(before, d, 64);
+    }
+    if (lane == 63) {
+        s_wave[0][wave] = incl;
+        s_wave[1][wave] = before;
+    }
+    __syncthreads();
+    int64_t pos = incl - sum;
+    for (int w = 0; w < waves; ++w) {
+        pos += (w < wave ? s_wave[0][w] : 0) + s_wave[1][w];
+    }
+#pragma unroll
+    for (int j = 0; j < kOffsetsPerThread; ++j) {
+        if (first + j < R) {
+            const int64_t end = pos + count[j];
+            // beyond the room the caller has: marked, and the hash kernel leaves the request out
+            key_offsets[first + j] = end <= limit ? pos : -1;
+            pos = end;
+            if (first + j == R - 1) {
+                key_offsets[R] = pos;
+                if (h_total) {
+                    __hip_atomic_store(h_total, pos, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+                }
+            }
+        }
     }
 }
 
@@ -1032,6 +1110,52 @@ int32_t kvcm_hip_hash_tokens_2d(const void *d_tokens, int32_t token_bytes, int32
     }
     return kvcm::launch_hash<int32_t>(static_cast<const int32_t *>(d_tokens), nullptr, R, block_size, seed, d_keys,
                                       d_key_offsets, static_cast<hipStream_t>(stream), uni);
+}
+
+// The value arrives a few microseconds after the kernel that writes it has started, so the thread looks for it without
+// sleeping at first (sleeping and being woken costs more than the wait), gives its core away between looks after a
+// while, and only then starts to ask the stream whether anything will still come.
+int32_t kvcm_wait_value(const int64_t *h_value, kvcm_stream_t stream) {
+    if (!h_value) {
+        return KVCM_ERR_INVALID_ARG;
+    }
+    const auto arrived = [h_value] { return __atomic_load_n(h_value, __ATOMIC_ACQUIRE) != KVCM_PENDING; };
+    for (int i = 0; i < 4096; ++i) {
+        if (arrived()) {
+            return KVCM_OK;
+        }
+        if (i >= 1024) {
+            sched_yield();
+        } else {
+            __builtin_ia32_pause();
+        }
+    }
+    for (;;) {
+        const hipError_t e = hipStreamQuery(static_cast<hipStream_t>(stream));
+        if (arrived()) {
+            return KVCM_OK;
+        }
+        if (e != hipErrorNotReady) {
+            return e == hipSuccess ? static_cast<int32_t>(hipErrorUnknown) : static_cast<int32_t>(e);
+        }
+        const struct timespec nap = {0, 20000};
+        nanosleep(&nap, nullptr);
+    }
+}
+
+int32_t kvcm_hip_key_offsets(const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t limit,
+                             int64_t *d_key_offsets, int64_t *h_total, kvcm_stream_t stream) {
+    if (R <= 0 || block_size <= 0 || !d_token_offsets || !d_key_offsets) {
+        return KVCM_ERR_INVALID_ARG;
+    }
+    if (h_total) {
+        *h_total = KVCM_PENDING;
+    }
+    const int64_t groups = (R + kvcm::kOffsetsPerWg - 1) / kvcm::kOffsetsPerWg;
+    const int64_t threads = groups > 1 ? kvcm::kOffsetsThreads : ((R + kvcm::kOffsetsPerThread - 1) / kvcm::kOffsetsPerThread + 63) / 64 * 64;
+    hipLaunchKernelGGL(kvcm::key_offsets_kernel, dim3(static_cast<uint32_t>(groups)), dim3(static_cast<uint32_t>(threads)), 0,
+                       static_cast<hipStream_t>(stream), d_token_offsets, R, block_size, limit, d_key_offsets, h_total);
+    return kvcm::launch_status();
 }
 
 int32_t kvcm_hip_prefix_chain(const int64_t *d_digests, const int64_t *d_offsets, int32_t R, int64_t *d_keys,

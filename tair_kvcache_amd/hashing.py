@@ -17,6 +17,13 @@ from . import _lib
 from ._torch_util import lib, ptr, require_cuda, stream_handle
 
 
+# Requests up to which one launch computes the key offsets: it re-reads what lies in front of every 8192 requests, torch's
+# five launches do not. Microseconds on the device, one launch / torch: 160 requests 3.2 / 7.5, 8192 8.5 / 12.5, 16 384
+# 10.1 / 12.8, 65 536 20 / 13, 131 072 33 / 13 (and 25 of host time for torch's, always).
+_NATIVE_OFFSETS_UP_TO = 32768
+_NO_LIMIT = 2**62
+
+
 def _require_offsets(t, name, device, entries=None):
     """Offsets are read by the kernel as they are: int64, 1-D, on the tokens' device, R+1 entries."""
     require_cuda(t, name)
@@ -36,8 +43,8 @@ def hash_tokens(tokens: torch.Tensor, block_size: int, token_offsets: Optional[t
     tokens: int64 or int32 device tensor, [R, L] (uniform lengths) or flat with token_offsets [R+1].
     Returns (keys, key_offsets): request r owns keys[key_offsets[r]:key_offsets[r+1]], len_r // block_size of
     them (a trailing partial block yields no key, cache_manager.cc:78). Asynchronous on the current stream when
-    `keys` and `key_offsets` are passed in (or the batch is a 2-D tensor); otherwise the key offsets are computed with
-    torch and the total is read back to size `keys`, which costs a synchronisation (about 30 us on an idle MI355X).
+    `keys` and `key_offsets` are passed in (or the batch is a 2-D tensor); otherwise the call returns once the number of
+    keys is known on the host, which does not wait for the keys themselves.
     """
     require_cuda(tokens, "tokens")
     if tokens.dtype not in (torch.int64, torch.int32):
@@ -77,18 +84,39 @@ def hash_tokens(tokens: torch.Tensor, block_size: int, token_offsets: Optional[t
                                            ptr(keys), ptr(key_offsets), ptr(new_offsets), stream_handle(tokens.device))
         _lib.check(rc, "kvcm_hip_hash_tokens_2d")
         return keys, (new_offsets if key_offsets is None else key_offsets)
+    stream = stream_handle(tokens.device)
+    pending = None
     if key_offsets is None:
-        counts = (off[1:] - off[:-1]) // block_size
-        key_offsets = torch.zeros(R + 1, dtype=torch.int64, device=tokens.device)
-        torch.cumsum(counts, 0, out=key_offsets[1:])
+        if R == 0 or R > _NATIVE_OFFSETS_UP_TO:
+            counts = (off[1:] - off[:-1]) // block_size
+            key_offsets = torch.zeros(R + 1, dtype=torch.int64, device=tokens.device)
+            torch.cumsum(counts, 0, out=key_offsets[1:])
+        else:
+            # The total is on its way to the host while the keys are being computed into a buffer of the size that the
+            # token count bounds: nobody waits for the hash kernel, and the hash kernel waits for nobody.
+            key_offsets = torch.empty(R + 1, dtype=torch.int64, device=tokens.device)
+            most = _NO_LIMIT
+            if keys is None:
+                most = tokens.numel() // block_size
+                keys = torch.empty(most, dtype=torch.int64, device=tokens.device)
+                pending = torch.empty(1, dtype=torch.int64, pin_memory=True)
+            rc = lib().kvcm_hip_key_offsets(ptr(off), R, block_size, most, ptr(key_offsets), ptr(pending), stream)
+            _lib.check(rc, "kvcm_hip_key_offsets")
     if keys is None:
         total = int(key_offsets[-1].item())
         keys = torch.empty(total, dtype=torch.int64, device=tokens.device)
         if total == 0:
             return keys, key_offsets
-    fn = lib().kvcm_hip_hash_tokens if tokens.dtype == torch.int64 else lib().kvcm_hip_hash_tokens_i32
-    rc = fn(ptr(tokens), ptr(off), R, block_size, int(seed), ptr(keys), ptr(key_offsets), stream_handle(tokens.device))
-    _lib.check(rc, "kvcm_hip_hash_tokens")
+    if keys.numel() or pending is None:
+        fn = lib().kvcm_hip_hash_tokens if tokens.dtype == torch.int64 else lib().kvcm_hip_hash_tokens_i32
+        rc = fn(ptr(tokens), ptr(off), R, block_size, int(seed), ptr(keys), ptr(key_offsets), stream)
+        _lib.check(rc, "kvcm_hip_hash_tokens")
+    if pending is not None:
+        _lib.check(lib().kvcm_wait_value(ptr(pending), stream), "kvcm_wait_value")
+        total = pending.item()
+        if total > keys.numel():
+            raise ValueError(f"token_offsets name {total} blocks of {block_size} tokens, tokens holds {tokens.numel()}")
+        keys = keys[:total]
     return keys, key_offsets
 
 

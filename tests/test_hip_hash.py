@@ -324,3 +324,27 @@ def test_equally_long_requests_need_no_offset_arrays(oracle, R, L, bs):
         assert (host(same, np.int64) == gaps).all()
         got = host(spread, np.int64).reshape(R, per + 1)
         assert (got[:, :per] == want.reshape(R, per)).all() and (got[:, per] == -7).all()
+
+
+@pytest.mark.parametrize("R", [1, 8, 9, 513, 8192, 8193, 32768, 32769])
+def test_key_offsets_of_ragged_batches(oracle, R):
+    """Offsets and keys when the caller passes neither, at the edges of the prefix-sum kernel (eight requests per thread,
+    8192 per workgroup) and beyond the request count it is used for; some requests empty or shorter than a block."""
+    rng = np.random.default_rng(R)
+    lens = rng.integers(0, 70, size=R)
+    toff = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    flat = rng.integers(0, 152064, size=max(int(toff[-1]), 1), dtype=np.int64)
+    want, woff = oracle.hash_tokens(flat, 16, token_offsets=toff, threads=8)
+    keys, off = _h().hash_tokens(dev(flat), 16, token_offsets=dev(toff))
+    sync()
+    assert (host(off, np.int64) == woff).all() and (host(keys, np.int64) == want).all()
+
+
+def test_offsets_beyond_the_tokens_are_refused():
+    """Offsets that name more blocks than the tokens can hold: nothing is written past the keys, and the call says so.
+    (The tokens are the front of a larger array, so what the launch reads is its own.)"""
+    flat = torch.zeros(4096, dtype=torch.int64, device="cuda")
+    off = torch.arange(0, 4097, 512, dtype=torch.int64, device="cuda")
+    with pytest.raises(ValueError):
+        _h().hash_tokens(flat[:1024], 16, token_offsets=off)
+    sync()
