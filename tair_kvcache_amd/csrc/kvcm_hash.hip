@@ -8,9 +8,8 @@
 // Design (gfx950, wave64): a workgroup owns 64 requests and is role-split.
 //   wave 0      "chain wave": lane = request. Keeps the state in VGPRs and does nothing but the recurrence,
 //               reading pre-added terms a = v + C from LDS (one ds_read_b128 per 2 steps, prefetched a whole
-//               tile ahead into a second register set). A lone wave issues a dependent VALU instruction 3.5-4 ns
-//               after its producer and independent ones 1.75 ns apart (measured), so the step is written for
-//               depth: three dependent levels, 5 instructions (see chain_step).
+//               tile ahead into a second register set). A wave issues one instruction every 4 clocks, so the step is
+//               written for their number: 5 instructions (see chain_step).
 //   waves 1..3  "loader waves": stream the 64 requests' tokens from HBM in [64 requests x 64 tokens] tiles with
 //               16-byte buffer loads (512-byte row segments), add C, and write them transposed into a 2-slot LDS
 //               ring. Each loader wave owns every third tile and keeps its loads in flight for about three
@@ -20,7 +19,7 @@
 //               With 4-byte tokens such launches use tiles of 128 RAW tokens (512-byte row segments here too): the
 //               loaders store what they loaded and the chain wave converts, one step ahead of its use.
 // Roofline: HBM for many requests (8*block_size + 8 bytes per key); for few requests the bound is the
-// dependent-instruction latency of the chain wave, which no amount of bandwidth removes.
+// instruction issue of the chain wave, which no amount of bandwidth removes.
 #include "kvcm_internal.h"
 
 #include <sched.h>
@@ -36,9 +35,6 @@ namespace {
 #endif
 #ifndef KVCM_HASH_RAW_AHEAD
 #define KVCM_HASH_RAW_AHEAD 1
-#endif
-#ifndef KVCM_HASH_DRAIN_POLICY
-#define KVCM_HASH_DRAIN_POLICY 0
 #endif
 #ifndef KVCM_HASH_TILE_TOKENS
 #define KVCM_HASH_TILE_TOKENS 64
@@ -82,12 +78,12 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // One step of the recurrence with the token term pre-added (a = v + C): h ^= a + (h << 12) + sar(h, 32).
-// The wave that sets the pace is bound by the LATENCY of dependent VALU instructions (3.5-4 ns each, whatever the
-// instruction; measured on a lone wave), so what counts is the depth of the dependence chain, not the instruction
-// count. sar(h, 32) is the sign-extended upper half, and v_mad_i64_i32 (hi * 1 + a) adds it to `a` in ONE
-// instruction that needs only the upper half of h; the shift runs beside it, and the step is three levels deep:
-// {v_mad_i64_i32 | v_lshlrev_b64} -> v_lshl_add_u64 -> 2 x v_xor_b32 (10.9 ns per step against 12.4 ns for the
-// four-level form shift -> add -> add -> xor).
+// The wave that sets the pace issues one vector instruction every 4 clocks, dependent on its predecessor or not (64 steps in
+// a row take 20.9 clocks each, 8.7 ns), so what counts is the number of instructions: these five, and everything else that
+// takes an issue slot of this wave -- LDS reads, key stores, waits, loop control. sar(h, 32) is the sign-extended upper
+// half, and v_mad_i64_i32 (hi * 1 + a) adds it to `a` in ONE instruction; v_lshlrev_b64, v_lshl_add_u64 and two v_xor_b32
+// are the rest (forms with v_mad_u64_u32 for the shift, or in 32-bit halves with carries, take as many or more: 37 to 46
+// clocks measured step by step where this one took 25).
 __device__ __forceinline__ uint64_t chain_step(uint64_t h, uint64_t a) {
     uint64_t a_plus_sar, carry_out;
     asm("v_mad_i64_i32 %0, %1, %2, 1, %3"
@@ -256,13 +252,36 @@ struct GlobalLoader {
 // which the chain wave pulled into registers an iteration ago). A loader issues the loads of its next tile right
 // AFTER the barrier that published its previous one, so they stay in flight for kLoaders - 1 tile periods while the
 // data waits in the loader's registers, not in LDS: more loaders = more bytes in flight per CU at no LDS cost.
+// A request's place among the keys, as the loaders that write staged keys need it.
+struct KeyRow {
+    int64_t first;   // index of its first key
+    int64_t count;   // keys it has; 0 for a row without a request
+};
+
 // What a loader wave needs to write out a group of staged keys (KS kernels only).
 struct KeyDrain {
-    const uint64_t *s_keys;   // LDS: [2][request][kKeyRow] keys of the group being filled and of the one before
-    const int64_t *s_keypos;                                    // LDS: index of each request's first key, -1 = no request
+    const uint64_t *s_keys;      // LDS: [2][request][kKeyRow] keys of the group being filled and of the one before
+    const KeyRow *s_keyrow;      // LDS: where each request's keys go, and how many it has
     int64_t *keys;
-    int32_t full_tiles;  // tiles in which no request has run out of tokens and whose keys may be staged
 };
+
+// Sixteen bytes of staged keys -> global. The chain wave fills rows to the end of the group whether the request still has
+// tokens or not; what lies behind a request's last key stays here. POLICY: 0 written through at system scope, 1 non-temporal.
+template <int POLICY>
+__device__ __forceinline__ void store_keys(const KeyDrain &kd, const KeyRow &row, int32_t group, uint32_t piece, const u32x4 &v) {
+    const int64_t at = static_cast<int64_t>(group) * kKeysPerGroup + piece * 2;
+    int64_t *dst = kd.keys + row.first + at;
+    if (at + 2 <= row.count) {
+        if (POLICY == 0) {
+            asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" : : "v"(dst), "v"(v) : "memory");
+        } else {
+            typedef u32x4 u32x4_a8 __attribute__((aligned(8)));
+            __builtin_nontemporal_store(v, reinterpret_cast<u32x4_a8 *>(dst));
+        }
+    } else if (at < row.count) {
+        *dst = static_cast<int64_t>((static_cast<uint64_t>(v.y) << 32) | v.x);
+    }
+}
 
 // One group of staged keys, LDS -> global: every store instruction writes two requests' rows of 512 bytes, whole cache
 // lines, non-temporal. Written as 8-byte stores from the chain wave (one line per lane, a sixteenth of it at a time)
@@ -280,25 +299,22 @@ __device__ __forceinline__ void drain_keys(const KeyDrain &kd, int32_t group, in
     for (int j = 0; j < kDrainPerStep; ++j) {
         const uint32_t c = static_cast<uint32_t>(step * kDrainPerStep + j) * 64u + lane;  // 16-byte piece of the group's keys
         const uint32_t row = c / (kKeysPerGroup / 2), piece = c % (kKeysPerGroup / 2);
-        const int64_t first = kd.s_keypos[row];
         const u32x4 v = *reinterpret_cast<const u32x4 *>(kd.s_keys + (buf * kReqs + row) * kKeyRow + piece * 2);
-        if (first >= 0) {
-            typedef u32x4 u32x4_a8 __attribute__((aligned(8)));
-            __builtin_nontemporal_store(
-                v, reinterpret_cast<u32x4_a8 *>(kd.keys + first + static_cast<int64_t>(group) * kKeysPerGroup + piece * 2));
-        }
+        store_keys<1>(kd, kd.s_keyrow[row], group, piece, v);
     }
 }
 
 // Half of a closed group (`part` = 0 or 1: every other store instruction), in bursts of eight row pieces: all LDS reads
 // of a burst are under way before its first store goes out, so the loader is back at its loads after about 0.2 us.
+// Written through at system scope: 97-99 us for 16 384 x 4096 tokens where the same stores take 101-105 us non-temporal, 104
+// plain, 100-101 with sc1 alone (65 536 x 4096: 385-388 against 399-403 us).
 __device__ __forceinline__ void drain_half(const KeyDrain &kd, int32_t group, int32_t part, uint32_t lane) {
     const uint32_t buf = static_cast<uint32_t>(group) & 1u;
     constexpr int kBurst = 8;
     static_assert((kDrainSteps * kDrainPerStep / 2) % kBurst == 0, "whole bursts");
 #pragma unroll 1
     for (int32_t base = 0; base < kDrainSteps * kDrainPerStep / 2; base += kBurst) {
-        int64_t first[kBurst];
+        KeyRow to[kBurst];
         u32x4 v[kBurst];
         uint32_t piece[kBurst];
 #pragma unroll
@@ -306,27 +322,12 @@ __device__ __forceinline__ void drain_half(const KeyDrain &kd, int32_t group, in
             const uint32_t c = static_cast<uint32_t>((base + i) * 2 + part) * 64u + lane;
             const uint32_t row = c / (kKeysPerGroup / 2);
             piece[i] = c % (kKeysPerGroup / 2);
-            first[i] = kd.s_keypos[row];
+            to[i] = kd.s_keyrow[row];
             v[i] = *reinterpret_cast<const u32x4 *>(kd.s_keys + (buf * kReqs + row) * kKeyRow + piece[i] * 2);
         }
 #pragma unroll
         for (int i = 0; i < kBurst; ++i) {
-            if (first[i] >= 0) {
-                // written through at system scope: 97-99 us for 16 384 x 4096 tokens where the same stores take
-                // 101-105 us non-temporal, 104 plain, 100-101 with sc1 alone (65 536 x 4096: 385-388 against 399-403 us)
-                int64_t *dst = kd.keys + first[i] + static_cast<int64_t>(group) * kKeysPerGroup + piece[i] * 2;
-#if KVCM_HASH_DRAIN_POLICY == 0
-                asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" : : "v"(dst), "v"(v[i]) : "memory");
-#elif KVCM_HASH_DRAIN_POLICY == 1
-                asm volatile("global_store_dwordx4 %0, %1, off nt" : : "v"(dst), "v"(v[i]) : "memory");
-#elif KVCM_HASH_DRAIN_POLICY == 2
-                asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(dst), "v"(v[i]) : "memory");
-#elif KVCM_HASH_DRAIN_POLICY == 3
-                asm volatile("global_store_dwordx4 %0, %1, off sc1 nt" : : "v"(dst), "v"(v[i]) : "memory");
-#else
-                asm volatile("global_store_dwordx4 %0, %1, off" : : "v"(dst), "v"(v[i]) : "memory");
-#endif
-            }
+            store_keys<0>(kd, to[i], group, piece[i], v[i]);
         }
     }
 }
@@ -348,36 +349,31 @@ __device__ __forceinline__ void drain_tail(const KeyDrain &kd, int32_t group, in
     const uint32_t buf = static_cast<uint32_t>(group) & 1u;
     constexpr int kMaxSteps = (kDrainSteps + kLoaders - 1) / kLoaders;
     constexpr int kN = kMaxSteps * kDrainPerStep;
-    typedef u32x4 u32x4_a8 __attribute__((aligned(8)));
     const int32_t s0 = first_step + (me - first_step % kLoaders + kLoaders) % kLoaders;
-    int64_t first[kN];
+    KeyRow to[kN];
     u32x4 v[kN];
     uint32_t piece[kN];
 #pragma unroll
     for (int i = 0; i < kN; ++i) {
         const int32_t step = s0 + (i / kDrainPerStep) * kLoaders;
-        first[i] = -1;
+        to[i].count = 0;
         if (step < kDrainSteps) {
             const uint32_t c = static_cast<uint32_t>(step * kDrainPerStep + i % kDrainPerStep) * 64u + lane;
             const uint32_t row = c / (kKeysPerGroup / 2);
             piece[i] = c % (kKeysPerGroup / 2);
-            first[i] = kd.s_keypos[row];
+            to[i] = kd.s_keyrow[row];
             v[i] = *reinterpret_cast<const u32x4 *>(kd.s_keys + (buf * kReqs + row) * kKeyRow + piece[i] * 2);
         }
     }
 #pragma unroll
     for (int i = 0; i < kN; ++i) {
-        if (first[i] >= 0) {
-            __builtin_nontemporal_store(
-                v[i], reinterpret_cast<u32x4_a8 *>(kd.keys + first[i] + static_cast<int64_t>(group) * kKeysPerGroup +
-                                                  piece[i] * 2));
-        }
+        store_keys<1>(kd, to[i], group, piece[i], v[i]);
     }
 }
 
 template <typename Loader, typename TokT, int KS, int G, int TOK>
 __device__ __forceinline__ void run_loader(const LoaderCtx<TokT> &ctx, uint64_t (*s_tile)[kReqs][kTT + kPad],
-                                           int64_t lw, int64_t ntiles, uint32_t lane, const KeyDrain &kd) {
+                                           int64_t lw, int64_t ntiles, uint32_t lane, const KeyDrain &kd, bool staged) {
     static_assert(kRing == 2 && kLoaders >= 3, "two ring slots: prefetched from, written to");
     // the burst drain splits a closed group between the kLoaders - 1 loaders whose tile is not due, as halves
     static_assert(KS != kKeysBurst || kLoaders == 3, "drain_half deals a group out to exactly two loaders");
@@ -409,7 +405,7 @@ __device__ __forceinline__ void run_loader(const LoaderCtx<TokT> &ctx, uint64_t 
         if (mine) {
             ld.store(s_tile[slot]);
         }
-        if (KS == kKeysSpread && k >= kKeyGroupTiles && (k / kKeyGroupTiles) * kKeyGroupTiles <= kd.full_tiles &&
+        if (KS == kKeysSpread && staged && k >= kKeyGroupTiles &&
             (turn == 0 ? kLoaders - 1 : turn - 1) == me) {
             // The group of staged keys before the one this tile belongs to was closed by an earlier barrier, and its
             // buffer is not written again before the barrier that ends this group: a sixteenth of it leaves per tile,
@@ -441,21 +437,37 @@ __device__ __forceinline__ void run_loader(const LoaderCtx<TokT> &ctx, uint64_t 
             }
         }
         was_mine = mine;
-        if (KS == kKeysBurst && (k & (G - 1)) == G - 1 && k < kd.full_tiles && turn != me) {
-            // The barrier above closed a group of G tiles. The loader whose tile is due next leaves it alone (its next
-            // wait for memory would wait for these stores as well); the other two write half of it each.
+        if (KS == kKeysBurst && ((k & (G - 1)) == G - 1 || k == nt - 1) && turn != me) {
+            // The barrier above closed a group of G tiles, or what there is of the last one. The loader whose tile is due
+            // next leaves it alone (its next wait for memory would wait for these stores as well); the other two write half
+            // of it each.
             drain_half(kd, k / G, (me - turn + kLoaders) % kLoaders - 1, lane);
         }
     }
-    if (KS == kKeysSpread) {
-        // What the loop did not reach of the last staged group (all of it when the request ends with the group), the
-        // steps dealt out to the loaders; no barrier follows, and nobody writes the buffers any more.
-        const int32_t last = kd.full_tiles / kKeyGroupTiles - 1;
-        if (last >= 0) {
-            const int32_t done = nt - (last + 1) * kKeyGroupTiles;  // steps the loop has taken for this group
-            drain_tail(kd, last, done < 0 ? 0 : done, me, lane);
+    if (KS == kKeysSpread && staged) {
+        // What the loop did not reach: the rest of the last group but one, and all of the last group, the steps dealt out
+        // to the loaders; no barrier follows, and nobody writes the buffers any more.
+        const int32_t last = (nt - 1) / kKeyGroupTiles;
+        if (last >= 1) {
+            drain_tail(kd, last - 1, nt - last * kKeyGroupTiles, me, lane);
         }
+        drain_tail(kd, last, 0, me, lane);
     }
+}
+
+// One group of a lane's row of a tile, LDS -> registers. The scheduler keeps the group where it stands: a lone wave issues a
+// 16-byte read every 6 clocks in groups of 8, every 8.4 in groups of 32 (no more than 15 can be outstanding) and every 12
+// when they stand alone between the steps. Two groups per tile against one, the whole kernel: 160 requests of up to 8192
+// 4-byte tokens 103.9 / 109.3 us, 64 x 4096 8-byte tokens 52.1 / 52.1; four groups 103.3 and 52.9.
+constexpr int kReadGroups = 2;
+template <int N>
+__device__ __forceinline__ void read_row_part(ulonglong2 (&a)[kRowVecs], const uint64_t *row_ptr, int group) {
+    const ulonglong2 *row = reinterpret_cast<const ulonglong2 *>(row_ptr) + group * N;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        a[group * N + i] = row[i];
+    }
+    __builtin_amdgcn_sched_barrier(0);
 }
 
 // The chain wave's work on one tile: kTT steps from the lane's pre-added terms `a`, a key at every block
@@ -469,7 +481,8 @@ __device__ __forceinline__ void run_loader(const LoaderCtx<TokT> &ctx, uint64_t 
 // STAGED (unmasked tiles, block size a compile-time constant up to a tile): the tile's keys go to the lane's row of the LDS key buffer, `staged_row`
 // pointing at the tile's first key there; a loader wave writes the rows out (drain_keys).
 template <int CHUNK, bool MASKED, int BS, bool STAGED = false, bool RAW = false>
-__device__ __forceinline__ void run_tile(const ulonglong2 (&a)[kRowVecs], uint64_t &h, int64_t t0, int64_t my_ntok,
+__device__ __forceinline__ void run_tile(const ulonglong2 (&a)[kRowVecs], ulonglong2 (&next)[kRowVecs],
+                                         const uint64_t *next_row, uint64_t &h, int64_t t0, int64_t my_ntok,
                                          int32_t &since_key, int32_t block_size, int64_t *__restrict__ keys,
                                          int64_t &key_pos, uint64_t *staged_row = nullptr) {
     constexpr int TOK = tile_tokens(RAW);  // steps per tile
@@ -493,8 +506,12 @@ __device__ __forceinline__ void run_tile(const ulonglong2 (&a)[kRowVecs], uint64
             pre[i] = pre_add_i32(raw_token(i));
         }
     }
+    uint64_t held = 0;
 #pragma unroll
     for (int c = 0; c < TOK; c += CHUNK) {
+        if (c % (TOK / kReadGroups) == 0) {
+            read_row_part<kRowVecs / kReadGroups>(next, next_row, c / (TOK / kReadGroups));
+        }
 #pragma unroll
         for (int s = c; s < c + CHUNK; ++s) {
             if (RAW && kAhead > 0) {
@@ -522,21 +539,26 @@ __device__ __forceinline__ void run_tile(const ulonglong2 (&a)[kRowVecs], uint64
             key_due = c + CHUNK == TOK && (t0 + TOK) % BS == 0;
         }
         if (key_due) {
-            if (STAGED) {
-                staged_row[BS > TOK ? 0 : (c + CHUNK) / (BS > 0 ? BS : 1) - 1] = h;
+            // Where a tile holds an even number of keys they leave two at a time, 16 bytes per lane: every lane's key lies
+            // in a cache line of its own, and it is the lines that a store takes its time for, not the bytes (a store of
+            // 64 lanes into 64 lines costs the chain 35 clocks; 64 requests of 4096 tokens 54.5 -> 52.2 us).
+            constexpr bool kPaired = !MASKED && BS >= 1 && TOK % (2 * (BS > 0 ? BS : 1)) == 0;
+            const int key_in_tile = BS > TOK ? 0 : (c + CHUNK) / (BS > 0 ? BS : 1) - 1;
+            if (kPaired && key_in_tile % 2 == 0) {
+                held = h;
+            } else if (kPaired && STAGED) {
+                *reinterpret_cast<ulonglong2 *>(staged_row + key_in_tile - 1) = make_ulonglong2(held, h);
+            } else if (kPaired) {
+                typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+                typedef u64x2 u64x2_a8 __attribute__((aligned(8)));  // one store: wide accesses need dword alignment only
+                *reinterpret_cast<u64x2_a8 *>(keys + key_pos - 1) = u64x2{held, h};
+            } else if (STAGED) {
+                staged_row[key_in_tile] = h;
             } else if (!MASKED || c + CHUNK <= left) {
                 keys[key_pos] = static_cast<int64_t>(h);
             }
             key_pos += 1;
         }
-    }
-}
-
-__device__ __forceinline__ void read_row(ulonglong2 (&a)[kRowVecs], const uint64_t *row_ptr) {
-    const ulonglong2 *row = reinterpret_cast<const ulonglong2 *>(row_ptr);
-#pragma unroll
-    for (int i = 0; i < kRowVecs; ++i) {
-        a[i] = row[i];
     }
 }
 
@@ -553,9 +575,9 @@ struct Uniform {
 // CHUNK = steps between two looks at the block boundary: 8 when block_size % 8 == 0 (a lane is then
 // active for whole chunks or not at all), otherwise 1. BS = block size when it is 1, 8, 16, 32, 64 or 128, otherwise 0.
 // KS != kKeysDirect ("keys staged", block sizes 1 to 64; chosen by the host for batches of many requests, where the launch
-// is bound by memory and not by the chain): the chain wave writes its keys into an LDS buffer instead of to memory, and
-// after every group of tiles in which every request is whole the loader waves write the group out as rows of 512
-// bytes, spread over the next group's tiles (block size 16) or at once.
+// is bound by memory and not by the chain): the chain wave writes its keys into an LDS buffer instead of to memory, whether
+// a request still has tokens or not, and after every group of tiles the loader waves write out what there is of it as rows
+// of up to 512 bytes, spread over the next group's tiles (block size 16) or at once.
 template <typename TokT, int CHUNK, int BS, int KS = kKeysDirect, bool RAW = false>
 __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__restrict__ tokens,
                                                               const int64_t *__restrict__ token_offsets, int32_t R,
@@ -573,7 +595,7 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
     static_assert(!KS || G >= 1, "a group of staged keys is at least one tile");
     constexpr int kDiv = BS > 0 ? BS : 1;  // the first key of tile t of a group lies at position t * TOK / BS of the row
     __shared__ __attribute__((aligned(16))) uint64_t s_keys[KS ? 2 * kReqs * kKeyRow : 2];
-    __shared__ int64_t s_keypos[KS ? kReqs : 1];
+    __shared__ __attribute__((aligned(16))) KeyRow s_keyrow[KS ? kReqs : 1];
 
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -608,7 +630,7 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
         s_start[lane] = start;
         s_ntok[lane] = my_ntok;
         if (KS) {
-            s_keypos[lane] = r < R ? key_pos : -1;
+            s_keyrow[lane] = KeyRow{key_pos, my_ntok / kDiv};  // no tokens, no keys: rows past R among them
         }
     } else {
         ctx.tokens = tokens;
@@ -645,15 +667,19 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
     }
     // tiles [0, n_full) are those in which no request has run out of tokens
     const int32_t n_full = static_cast<int32_t>(full_u < ntiles_u ? full_u : ntiles_u);
-    // ... and of those, the ones whose keys may be staged (whole groups of them are)
-    const int32_t n_stageable = KS == kKeysSpread && ntiles_u < static_cast<uint32_t>(kSpreadFromTiles) ? 0 : n_full;
+    // whether this workgroup's keys are staged
+    const bool staged = KS == kKeysBurst || (KS == kKeysSpread && ntiles_u >= static_cast<uint32_t>(kSpreadFromTiles));
     if (wave != 0) {
         // ---------------------------------------------------------------- loader waves
-        const KeyDrain kd{s_keys, s_keypos, keys, n_stageable};
+        const KeyDrain kd{s_keys, s_keyrow, keys};
         if (buffer_loads) {
-            run_loader<BufferLoader<TokT, RAW>, TokT, KS, G, TOK>(ctx, s_tile, wave - 1, ntiles, lane, kd);
+            run_loader<BufferLoader<TokT, RAW>, TokT, KS, G, TOK>(ctx, s_tile, wave - 1, ntiles, lane, kd, staged);
         } else {
-            run_loader<GlobalLoader<TokT, RAW>, TokT, KS, G, TOK>(ctx, s_tile, wave - 1, ntiles, lane, kd);
+            run_loader<GlobalLoader<TokT, RAW>, TokT, KS, G, TOK>(ctx, s_tile, wave - 1, ntiles, lane, kd, staged);
+            // vmcnt(0), for the compiler's books: it lays this path out in front of the other one and would otherwise take
+            // the registers of these loads for pending there, and wait for ALL outstanding loads -- the next tile's -- in
+            // front of every group of keys that is written out (prefix chain, 64 x 4096: 113 us with that wait, 86 without)
+            __builtin_amdgcn_s_waitcnt(0x0F70);
         }
         return;
     }
@@ -669,53 +695,44 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
         return;
     }
     ulonglong2 cur[kRowVecs], nxt[kRowVecs];
-    read_row(cur, &s_tile[0][lane][0]);
+    read_row_part<kRowVecs>(cur, &s_tile[0][lane][0], 0);
     lds_barrier();  // tile 0 is in registers: its slot may take tile 2
     // Loop control in 32-bit scalars (there are no ordered 64-bit scalar compares, and every vector compare is an issue
     // slot of this wave). A request of 2^37 tokens does not fit the memory of the device, so the tile count fits 32 bits.
     const int32_t nt = static_cast<int32_t>(ntiles);
+    const auto staged_row = [&](int32_t k) -> uint64_t * {
+        return KS ? s_keys + ((k / G & 1) * kReqs + lane) * kKeyRow + (k & (G - 1)) * TOK / kDiv : nullptr;
+    };
     int ring = 0;
     for (int32_t k = 0; k < nt; k += 2) {
         // even tile: compute on `cur`, prefetch the odd tile into `nxt`; then the other way round
         int ring1 = ring + 1 == kRing ? 0 : ring + 1;
-        if (k + 1 < nt) {
-            read_row(nxt, &s_tile[ring1][lane][0]);
-        }
-        // a group of G tiles is staged when all of its tiles are whole for every request
-        const int32_t group = k / G;
-        const bool staged = KS && (group + 1) * G <= n_stageable;
-        uint64_t *staged_row = KS ? s_keys + ((group & 1) * kReqs + lane) * kKeyRow + (k & (G - 1)) * TOK / kDiv : nullptr;
+        const uint64_t *const row1 = &s_tile[ring1][lane][0];  // behind the last tile: read and not used
         if (KS && staged) {
-            run_tile<CHUNK, false, BS, KS != kKeysDirect, RAW>(cur, h, static_cast<int64_t>(k) * TOK, my_ntok, since_key, block_size, keys,
-                                           key_pos, staged_row);
+            run_tile<CHUNK, false, BS, KS != kKeysDirect, RAW>(cur, nxt, row1, h, static_cast<int64_t>(k) * TOK, my_ntok,
+                                                               since_key, block_size, keys, key_pos, staged_row(k));
         } else if (k < n_full) {
-            run_tile<CHUNK, false, BS, false, RAW>(cur, h, static_cast<int64_t>(k) * TOK, my_ntok, since_key, block_size, keys,
-                                       key_pos);
+            run_tile<CHUNK, false, BS, false, RAW>(cur, nxt, row1, h, static_cast<int64_t>(k) * TOK, my_ntok, since_key,
+                                                   block_size, keys, key_pos);
         } else {
-            run_tile<CHUNK, true, BS, false, RAW>(cur, h, static_cast<int64_t>(k) * TOK, my_ntok, since_key, block_size, keys,
-                                      key_pos);
+            run_tile<CHUNK, true, BS, false, RAW>(cur, nxt, row1, h, static_cast<int64_t>(k) * TOK, my_ntok, since_key,
+                                                  block_size, keys, key_pos);
         }
         lds_barrier();
         if (k + 1 >= nt) {
             break;
         }
         ring = ring1 + 1 == kRing ? 0 : ring1 + 1;
-        if (k + 2 < nt) {
-            read_row(cur, &s_tile[ring][lane][0]);
-        }
-        const int32_t group1 = (k + 1) / G;  // the same group unless a group is one tile
-        const bool staged1 = KS && (group1 + 1) * G <= n_stageable;
-        uint64_t *staged_row1 =
-            KS ? s_keys + ((group1 & 1) * kReqs + lane) * kKeyRow + ((k + 1) & (G - 1)) * TOK / kDiv : nullptr;
-        if (KS && staged1) {
-            run_tile<CHUNK, false, BS, KS != kKeysDirect, RAW>(nxt, h, static_cast<int64_t>(k + 1) * TOK, my_ntok, since_key, block_size,
-                                           keys, key_pos, staged_row1);
+        const uint64_t *const row2 = &s_tile[ring][lane][0];
+        if (KS && staged) {
+            run_tile<CHUNK, false, BS, KS != kKeysDirect, RAW>(nxt, cur, row2, h, static_cast<int64_t>(k + 1) * TOK, my_ntok,
+                                                               since_key, block_size, keys, key_pos, staged_row(k + 1));
         } else if (k + 1 < n_full) {
-            run_tile<CHUNK, false, BS, false, RAW>(nxt, h, static_cast<int64_t>(k + 1) * TOK, my_ntok, since_key, block_size, keys,
-                                       key_pos);
+            run_tile<CHUNK, false, BS, false, RAW>(nxt, cur, row2, h, static_cast<int64_t>(k + 1) * TOK, my_ntok, since_key,
+                                                   block_size, keys, key_pos);
         } else {
-            run_tile<CHUNK, true, BS, false, RAW>(nxt, h, static_cast<int64_t>(k + 1) * TOK, my_ntok, since_key, block_size, keys,
-                                      key_pos);
+            run_tile<CHUNK, true, BS, false, RAW>(nxt, cur, row2, h, static_cast<int64_t>(k + 1) * TOK, my_ntok, since_key,
+                                                  block_size, keys, key_pos);
         }
         lds_barrier();
     }
@@ -933,41 +950,37 @@ __global__ __launch_bounds__(256) void iov_crc32_kernel(const kvcm_iov_device *_
 constexpr int32_t kForceGeneralLoader = KVCM_TEST_FORCE_GENERAL_LOADER;
 
 // How keys reach memory, by block size, token width and number of requests in the launch (hash_tokens_kernel<.., KS>).
-// Chosen from timings on tokens that are not in the memory-side cache. 16-token blocks, us for requests of 4096 tokens,
-// direct / spread / burst:
-//   8-byte tokens   64: 61 / 58 / 60      1024: 61 / 59 / 63     4096: 65 / 60 / 64      8192: 76 / 64 / 70
-//                   10 240: 83 / 76 / 73  12 288: 92 / 85 / 83   16 384: 112 / 111 / 107   32 768: 227 / 219 / 209
-//   4-byte tokens   4096: 56 / 58 / 63    8192: 58 / 58 / 64     10 240: 64 / 62 / 66    12 288: 72 / 66 / 67
-//                   16 384: 85 / 81 / 78  32 768: 159 / 151 / 151
-// 8-byte tokens: direct below 2048 requests (there the spread form gains 2 to 4 % on tokens from HBM and loses as much
-// on resident ones, and costs requests of 1024 tokens 6 %), spread from 2048, burst from 10 240.
-// 4-byte tokens: direct below 12 288, burst from there -- and the burst form of 4-byte tokens is the one with raw tiles
-// (RAW = true; the 4-byte figures of these tables are those of the 64-token tiles of pre-added terms it replaced:
-// 16 384 requests 78 -> 62-66 us) (the spread form would gain 3 % between 10 240 and 16 384
-// requests: not worth one more kernel).
+// Chosen from timings on tokens that are not in the memory-side cache, us, requests of 4096 tokens each / of 500 to 4096
+// (a request that has run out makes the direct form compare per key; the staged forms leave that to the loaders).
+//   16-token blocks, 8-byte tokens: direct 64: 56 / 64  1024: 57 / -   2048: 58 / 66  4096: 61 / 69  8192: 73 / 77  10 240: 79 / 86
+//                                   spread                             2048: 59 / 60  4096: 60 / 60  8192: 65 / 70  10 240:  - / -
+//                                   burst  64: 58 / 60  1024: 58 / -   2048: 59 / 60  4096: 60 / 61  8192: 64 / 67  10 240: 68 / 72
+//   spread beats burst by 4 % on 2048 requests of 1024 tokens: direct below 2048, spread from there, burst from 8192.
+//   16-token blocks, 4-byte tokens: direct 4096: 55 / -   8192: 58 / 60  12 288: 70 / -
+//                                   burst  4096: 58 / -   8192: 58 / 61  12 288: 60 / -      (raw tiles, see below)
 // Other block sizes, direct / burst:
-//   block size 1, 8-byte tokens   64: 146 / 129   2048: 158 / 136   8192: 241 / 161   16 384: 300 / 202   32 768: 641 / 415
-//                 4-byte tokens   512: 115 / 119  1024: 119 / 120 (resident: 116 / 92)   8192: 184 / 141   16 384: 249 / 175
-//   block size 8, 8-byte tokens   1024: 72 / 69 (resident: 61 / 64)   2048: 74 / 70   8192: 98 / 77   16 384: 137 / 112
-//                 4-byte tokens   8192: 69 / 71   12 288: 82 / 75   16 384: 100 / 83
-//   block size 32, 8-byte tokens  4096: 60 / 61   8192: 69 / 65   12 288: 93 / 76   16 384: 115 / 99
-//                  4-byte tokens  8192: 57 / 57   12 288: 69 / 62   16 384: 84 / 70
-//   block size 64, 8-byte tokens  4096: 58 / 60   8192: 67 / 63   12 288: 85 / 75   16 384: 109 / 93
-//                  4-byte tokens  8192: 55 / 57   12 288: 64 / 60   16 384: 77 / 72
-//   block size 128 (requests of 16 384 tokens: a group is 8192), 8-byte tokens  4096: 210 / 208   8192: 242 / 222
-//                  16 384: 419 / 356;  4-byte tokens  8192: 198 / 197   16 384: 264 / 204
+//   block size 1, 8-byte tokens   16: 76 / 101 and 149 / 105   32: 87 / 97 and 151 / 105   64: 143 / 89 and 156 / 105   8192: 246 / 115
+//                 4-byte tokens   32: 75 / -   64: 107 / 82 and 146 / 93   1024: 113 / 83   8192: 174 / 96
+//   block size 8, 8-byte tokens   1024: 66 / 62 (of 512 tokens: 14.7 / 15.6)   2048: 68 / 63   8192: 89 / 69   12 288: 104 / 88
+//                 4-byte tokens   8192: 66 / 61 (of 1024 tokens: 20.6 / 23.2)  12 288: 80 / 62
+//   block size 32, 8-byte tokens  4096: 59 / 58 (of 1024 tokens: 21.6 / 22.0)  8192: 66 / 61   12 288: 87 / 76
+//                  4-byte tokens  8192: 56 / 58   12 288: 67 / 60
+//   block size 64, 8-byte tokens  4096: 58 / 57 (of 1024 tokens: 21.6 / 22.0)  8192: 65 / 59   12 288: 79 / 73
+//                  4-byte tokens  8192: 55 / 58   12 288: 67 / 60
+//   block size 128, 8-byte tokens 2048: 56 / 54 (of 1024 tokens: 20.9 / 21.2)  4096: 58 / 55 (21.4 / 21.5)   8192: 64 / 58
+//                   4-byte tokens 8192: 55 / 58   12 288: 65 / 59
 #ifndef KVCM_HASH_SPREAD_FROM_8
 #define KVCM_HASH_SPREAD_FROM_8 2048
 #endif
 // requests from which a launch takes the burst form; INT32_MAX = never
 constexpr int32_t burst_from(int32_t block_size, bool tokens_8_byte) {
     switch (block_size) {
-        case 1: return tokens_8_byte ? 1 : 1024;
+        case 1: return tokens_8_byte ? 32 : 64;
         case 8: return tokens_8_byte ? 2048 : 12288;
-        case 16: return tokens_8_byte ? 10240 : 12288;
+        case 16: return tokens_8_byte ? 8192 : 12288;
         case 32: return tokens_8_byte ? 8192 : 12288;
         case 64: return tokens_8_byte ? 8192 : 12288;
-        case 128: return tokens_8_byte ? 8192 : 12288;
+        case 128: return tokens_8_byte ? 4096 : 12288;
         default: return INT32_MAX;
     }
 }

@@ -272,6 +272,31 @@ def test_staged_keys_at_other_block_sizes(oracle, bs, dtype):
     assert (got[len(want):] == -7).all()
 
 
+@pytest.mark.parametrize("dtype,R,bs", [(np.int64, 31, 1), (np.int64, 32, 1), (np.int64, 100, 1), (np.int32, 63, 1),
+                                        (np.int32, 64, 1), (np.int64, 2048, 16), (np.int64, 8192, 16), (np.int64, 4096, 128),
+                                        (np.int64, 2048, 8), (np.int64, 64, 16), (np.int64, 64, 32), (np.int64, 64, 64)])
+def test_requests_that_end_inside_a_group_of_staged_keys(oracle, dtype, R, bs):
+    """Staged keys leave as rows of pairs: requests with an odd number of keys, with none, with one key into a new group and
+    with one key less than a group, beside requests that go on, so that every kind of row end meets every step of the
+    drain; and on both sides of the request counts at which keys are staged. Spare key slots stay untouched."""
+    rng = np.random.default_rng(1000 * bs + R)
+    ends = np.array([0, 1, 2, 3, 31, 32, 33, 62, 63, 64, 65, 66, 127, 128, 129, 131])    # in keys
+    nkeys = ends[rng.integers(0, len(ends), size=R)]
+    nkeys[::64] = 131                                          # a long one in every workgroup
+    if R > 2000:
+        nkeys[64:128] = rng.integers(0, 20, size=64)           # one workgroup of short requests only
+    lens = nkeys * bs + rng.integers(0, bs, size=R)
+    toff = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    flat = rng.integers(-2**31, 2**31, size=max(int(toff[-1]), 1), dtype=np.int64).astype(dtype)
+    want, woff = oracle.hash_tokens(flat, bs, token_offsets=toff, seed=5, threads=8)
+    keys = torch.full((len(want) + 64,), -7, dtype=torch.int64, device="cuda")
+    got, _ = _h().hash_tokens(dev(flat), bs, token_offsets=dev(toff), seed=5, keys=keys, key_offsets=dev(woff))
+    sync()
+    got = host(got, np.int64)
+    assert (got[:len(want)] == want).all()
+    assert (got[len(want):] == -7).all()
+
+
 @pytest.mark.parametrize("general_loader", [False, True])
 @pytest.mark.parametrize("bs", [8, 16, 32, 64, 128])
 def test_raw_tiles_of_4_byte_tokens(oracle, force_general_hash_loader, bs, general_loader):
