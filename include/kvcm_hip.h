@@ -307,6 +307,16 @@ int32_t kvcm_hip_mask_to_indices(const uint8_t *d_mask, const uint8_t *d_mask2, 
                                  int64_t workspace_bytes, int32_t *d_indices, int32_t *d_count,
                                  kvcm_stream_t stream);
 
+/*
+ * The two above in one call: the ascending list of the positions whose key occurs for the first time and whose byte in
+ * d_saved (or NULL: nothing is saved) is 0. 1 <= n <= kvcm_hip_select_save_max_keys(); d_indices holds n entries,
+ * d_workspace at least kvcm_hip_select_save_workspace_bytes(n) bytes, 8-byte aligned.
+ */
+int64_t kvcm_hip_select_save_max_keys(void);
+int64_t kvcm_hip_select_save_workspace_bytes(int64_t n);
+int32_t kvcm_hip_select_save(const int64_t *d_keys, const uint8_t *d_saved, int64_t n, void *d_workspace,
+                             int64_t workspace_bytes, int32_t *d_indices, int32_t *d_count, kvcm_stream_t stream);
+
 /* ------------------------------------------------------------------------------------------------
  * Buffer check (debug aid of the transfer client)
  * ------------------------------------------------------------------------------------------------ */

@@ -74,6 +74,9 @@ SIGNATURES = {
     "kvcm_hip_first_occurrence_static": (i32, [vp, i64, vp, vp, vp]),
     "kvcm_hip_mask_to_indices_workspace_bytes": (i64, [i64]),
     "kvcm_hip_mask_to_indices": (i32, [vp, vp, i64, vp, i64, vp, vp, vp]),
+    "kvcm_hip_select_save_max_keys": (i64, []),
+    "kvcm_hip_select_save_workspace_bytes": (i64, [i64]),
+    "kvcm_hip_select_save": (i32, [vp, vp, i64, vp, i64, vp, vp, vp]),
     "kvcm_hip_iov_crc32": (i32, [vp, i32, vp, sz, vp]),
     "kvcm_blocks_hash_from_crcs": (i32, [vp, i64, i32, vp]),
     "kvcm_file_store_create": (i32, [i64, i64, i32, i32, C.POINTER(vp)]),

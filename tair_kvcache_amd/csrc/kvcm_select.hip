@@ -93,7 +93,9 @@ __global__ __launch_bounds__(256) void insert_kernel(const int64_t *__restrict__
             }
         }
         if (keys[o] == k) {
-            atomicMin(table + s, i);
+            if (o > i) {  // what a slot holds only ever falls: a smaller index that is there already stays or gives way to a
+                atomicMin(table + s, i);  // yet smaller one, and needs no atomic from the 30 requests that share a prefix
+            }
             break;
         }
         s = (s + 1) & mask;
@@ -193,7 +195,83 @@ __global__ __launch_bounds__(kSelThreads) void write_kernel(const uint8_t *__res
     }
 }
 
+// The list of a whole batch in four launches (fill, insert, choose, list) where first occurrences and mask compaction in a row
+// take six. Bound by latency: every launch is a chain of two or three trips to memory, and what counts is how many follow
+// each other. 256 keys per workgroup, so that 32 768 keys make 128 workgroups.
+constexpr int kListThreads = 256;
+constexpr int kListWaves = kListThreads / 64;
+// Keys up to which a workgroup adds up the counts of all workgroups in front of it itself (16 per thread at most) instead of
+// waiting for a scan of its own.
+constexpr int64_t kListMaxKeys = int64_t{1} << 20;
+
+// One bit per key: first occurrence and not saved yet. The bits of a wave go out as one word, a workgroup's total beside them.
+__global__ __launch_bounds__(kListThreads) void choose_kernel(const int32_t *__restrict__ slot_of, const int32_t *__restrict__ table,
+                                                              const uint8_t *__restrict__ saved, int32_t n,
+                                                              uint64_t *__restrict__ words, int32_t *__restrict__ group_count) {
+    __shared__ int32_t wave_totals[kListWaves];
+    const int32_t i = blockIdx.x * kListThreads + threadIdx.x;
+    bool flag = false;
+    if (i < n) {
+        const int32_t slot = slot_of[i];
+        flag = !(saved && saved[i]) && table[slot] == i;
+    }
+    const uint64_t ballot = __ballot(flag);
+    const int wave = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+        words[blockIdx.x * kListWaves + wave] = ballot;
+        wave_totals[wave] = __popcll(ballot);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int32_t all = 0;
+        for (int w = 0; w < kListWaves; ++w) {
+            all += wave_totals[w];
+        }
+        group_count[blockIdx.x] = all;
+    }
+}
+
+__global__ __launch_bounds__(kListThreads) void list_kernel(const uint64_t *__restrict__ words, const int32_t *__restrict__ group_count,
+                                                            int32_t *__restrict__ indices, int32_t *__restrict__ d_count) {
+    __shared__ int32_t wave_sums[kListWaves];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int32_t group = blockIdx.x;
+    uint64_t word[kListWaves];
+#pragma unroll
+    for (int w = 0; w < kListWaves; ++w) {
+        word[w] = words[group * kListWaves + w];
+    }
+    int32_t sum = 0;
+#pragma unroll 4
+    for (int32_t g = threadIdx.x; g < group; g += kListThreads) {
+        sum += group_count[g];
+    }
+    for (int d = 1; d < 64; d <<= 1) {
+        sum += __shfl_xor(sum, d, 64);
+    }
+    if (lane == 0) {
+        wave_sums[wave] = sum;
+    }
+    __syncthreads();
+    int32_t before = 0, own = 0;
+    uint64_t mine = 0;
+#pragma unroll
+    for (int w = 0; w < kListWaves; ++w) {
+        before += wave_sums[w] + (w < wave ? __popcll(word[w]) : 0);
+        own += w >= wave ? __popcll(word[w]) : 0;
+        mine = w == wave ? word[w] : mine;
+    }
+    if (mine >> lane & 1) {
+        indices[before + __popcll(mine & ((1ull << lane) - 1))] = group * kListThreads + static_cast<int32_t>(threadIdx.x);
+    }
+    if (group == static_cast<int32_t>(gridDim.x) - 1 && threadIdx.x == 0) {
+        *d_count = before + own;  // thread 0: nothing of its own group lies before it
+    }
+}
+
 constexpr int64_t kMaxKeys = int64_t{1} << 30;
+
+int64_t list_groups(int64_t n) { return (n + kListThreads - 1) / kListThreads; }
 
 int64_t table_capacity(int64_t n) {
     int64_t cap = 1024;
@@ -203,19 +281,23 @@ int64_t table_capacity(int64_t n) {
     return cap;
 }
 
-// fill / insert / resolve on a table of `cap` slots (a power of two, >= 2 n); the fill is a kernel, so the
-// sequence may be recorded into a graph.
-int32_t launch_first_occurrence(const int64_t *d_keys, int64_t n, int32_t *table, int64_t cap, int32_t *d_first_idx,
-                                uint8_t *d_is_repeat, hipStream_t s) {
+// An empty table of `cap` slots (a power of two, >= 2 n) and the keys into it; the fill is a kernel, so the sequence may be
+// recorded into a graph.
+void launch_insert(const int64_t *d_keys, int32_t n, int32_t *table, int64_t cap, int32_t *slot_of, hipStream_t s) {
     int log2cap = 0;
     while ((int64_t{1} << log2cap) < cap) {
         log2cap++;
     }
-    const int32_t n32 = static_cast<int32_t>(n);
-    const unsigned groups = static_cast<unsigned>((n + 255) / 256);
     fill_i32_kernel<<<static_cast<unsigned>(cap / 256), 256, 0, s>>>(table, cap, -1);
-    insert_kernel<<<groups, 256, 0, s>>>(d_keys, n32, table, static_cast<uint32_t>(cap - 1), 64 - log2cap, d_first_idx);
-    resolve_kernel<<<groups, 256, 0, s>>>(d_first_idx, table, n32, d_is_repeat);
+    insert_kernel<<<(static_cast<unsigned>(n) + 255) / 256, 256, 0, s>>>(d_keys, n, table, static_cast<uint32_t>(cap - 1), 64 - log2cap,
+                                                                       slot_of);
+}
+
+int32_t launch_first_occurrence(const int64_t *d_keys, int64_t n, int32_t *table, int64_t cap, int32_t *d_first_idx,
+                                uint8_t *d_is_repeat, hipStream_t s) {
+    const int32_t n32 = static_cast<int32_t>(n);
+    launch_insert(d_keys, n32, table, cap, d_first_idx, s);
+    resolve_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, s>>>(d_first_idx, table, n32, d_is_repeat);
     return launch_status();
 }
 
@@ -319,6 +401,43 @@ int32_t kvcm_hip_mask_to_indices(const uint8_t *d_mask, const uint8_t *d_mask2, 
     kvcm::count_kernel<<<G32, kvcm::kSelThreads, 0, s>>>(d_mask, d_mask2, n32, counts);
     kvcm::scan_kernel<<<1, kvcm::kSelThreads, 0, s>>>(counts, G32, d_count);
     kvcm::write_kernel<<<G32, kvcm::kSelThreads, 0, s>>>(d_mask, d_mask2, n32, counts, d_indices);
+    return kvcm::launch_status();
+}
+
+int64_t kvcm_hip_select_save_max_keys(void) { return kvcm::kListMaxKeys; }
+
+int64_t kvcm_hip_select_save_workspace_bytes(int64_t n) {
+    if (n < 0 || n > kvcm::kListMaxKeys) {
+        return KVCM_ERR_TOO_LARGE;
+    }
+    // words first (8-byte aligned), then table, slots and counts
+    return kvcm::list_groups(n) * (kvcm::kListWaves * 8 + 4) + (kvcm::table_capacity(n) + n) * 4;
+}
+
+int32_t kvcm_hip_select_save(const int64_t *d_keys, const uint8_t *d_saved, int64_t n, void *d_workspace,
+                             int64_t workspace_bytes, int32_t *d_indices, int32_t *d_count, kvcm_stream_t stream) {
+    if (n <= 0 || !d_keys || !d_workspace || !d_indices || !d_count) {
+        return KVCM_ERR_INVALID_ARG;
+    }
+    if (n > kvcm::kListMaxKeys) {
+        return KVCM_ERR_TOO_LARGE;
+    }
+    if (workspace_bytes < kvcm_hip_select_save_workspace_bytes(n)) {
+        return KVCM_ERR_INVALID_ARG;
+    }
+    if (reinterpret_cast<uintptr_t>(d_workspace) % 8 != 0) {
+        return KVCM_ERR_ALIGNMENT;
+    }
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    const int64_t groups = kvcm::list_groups(n), cap = kvcm::table_capacity(n);
+    uint64_t *words = static_cast<uint64_t *>(d_workspace);
+    int32_t *table = reinterpret_cast<int32_t *>(words + groups * kvcm::kListWaves);
+    int32_t *slot_of = table + cap, *counts = slot_of + n;
+    const int32_t n32 = static_cast<int32_t>(n);
+    const unsigned grid = static_cast<unsigned>(groups);
+    kvcm::launch_insert(d_keys, n32, table, cap, slot_of, s);
+    kvcm::choose_kernel<<<grid, kvcm::kListThreads, 0, s>>>(slot_of, table, d_saved, n32, words, counts);
+    kvcm::list_kernel<<<grid, kvcm::kListThreads, 0, s>>>(words, counts, d_indices, d_count);
     return kvcm::launch_status();
 }
 

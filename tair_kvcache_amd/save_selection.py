@@ -83,6 +83,24 @@ def parse_block_mask_to_save_indices(response: dict, target_save_num: int, devic
 def select_save_indices(keys: torch.Tensor, saved_mask: Optional[torch.Tensor] = None) -> Tuple[torch.Tensor, torch.Tensor]:
     """Positions in a batch's flat key list that have to be saved: the first occurrence of every key that the
     manager's mask (true = already stored) does not cover. Returns (indices, count) as mask_to_indices."""
+    L = lib()
+    n = keys.numel() if isinstance(keys, torch.Tensor) else 0
+    # Four launches and three buffers in one call, up to the number of keys that the list kernel adds up by itself: 32 768 keys
+    # and the wait for the count 42.6 us, with the two operators in a row 49.3.
+    if 0 < n <= L.kvcm_hip_select_save_max_keys() and keys.is_cuda and keys.dtype == torch.int64 and keys.dim() == 1:
+        saved = None if saved_mask is None else _as_mask(saved_mask, "mask")
+        if saved is not None and saved.numel() != n:
+            raise ValueError("mask and mask2 differ in length")
+        if saved is None or saved.device == keys.device:
+            keys = keys.contiguous()
+            ws_bytes = L.kvcm_hip_select_save_workspace_bytes(n)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=keys.device)
+            indices = torch.empty(n, dtype=torch.int32, device=keys.device)
+            count = torch.empty(1, dtype=torch.int32, device=keys.device)
+            rc = L.kvcm_hip_select_save(ptr(keys), ptr(saved), n, ptr(ws), ws_bytes, ptr(indices), ptr(count),
+                                        stream_handle(keys.device))
+            _lib.check(rc, "kvcm_hip_select_save")
+            return indices, count
     _, rep = first_occurrence(keys)
     if saved_mask is None:
         return mask_to_indices(rep)

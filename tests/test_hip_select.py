@@ -148,3 +148,29 @@ def test_config5_zipf_shared_prefixes_hash_dedup_gather(oracle):
     sync()
     for p in range(P):
         assert torch.equal(staging[:, p].reshape(n * 16, D), pool[p][tidx.reshape(-1).long()]), p
+
+
+@pytest.mark.parametrize("n,distinct", [(1, 1), (64, 3), (255, 255), (256, 100), (257, 257), (511, 20), (65537, 65537), (100001, 7),
+                                        (1 << 20, 1 << 19), ((1 << 20) + 1, 1 << 19)])
+@pytest.mark.parametrize("masked", [0.0, 0.4, 1.0, None])
+def test_save_list_of_a_batch_is_that_of_the_two_operators(oracle, n, distinct, masked):
+    """The list in one call, around a workgroup's 256 keys and on both sides of the number of keys it is used for, against
+    the oracle; keys with a stride, masks as bool, bytes, with a stride, or none."""
+    from tair_kvcache_amd import save_selection
+    rng = np.random.default_rng(n + distinct)
+    keys = _keys_with_repeats(rng, n, distinct)
+    mask = None if masked is None else rng.random(n) < masked
+    rep = oracle.first_occurrence(keys)[1].astype(bool)
+    want = np.flatnonzero(~rep if mask is None else ~(rep | mask))
+    d_keys = torch.from_numpy(np.repeat(keys, 2)).cuda()[::2] if n % 2 else torch.from_numpy(keys).cuda()
+    d_mask = None if mask is None else torch.from_numpy(np.repeat(mask, 3)).cuda()[::3] if n % 3 else torch.from_numpy(
+        mask.astype(np.uint8) * 5).cuda()
+    print(f"save list n={n} distinct={distinct} masked={masked}", flush=True)
+    for _ in range(2):
+        idx, count = save_selection.select_save_indices(d_keys, d_mask)
+        sync()
+        assert idx.shape == (n,) and int(count.item()) == len(want)
+        assert (idx[:len(want)].cpu().numpy() == want).all()
+    if d_mask is not None and n > 1:
+        with pytest.raises(ValueError):
+            save_selection.select_save_indices(d_keys, d_mask[1:])
