@@ -61,10 +61,6 @@ int32_t static_scratch(int32_t **out) {
 constexpr int kSelThreads = 1024;  // 16 waves: one workgroup scans 1024 flags or counts per pass
 constexpr int kSelWaves = kSelThreads / 64;
 
-__device__ inline int32_t table_load(const int32_t *p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
 __global__ __launch_bounds__(256) void fill_i32_kernel(int32_t *__restrict__ p, int64_t n, int32_t v) {
     int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (i < n) {
@@ -85,12 +81,10 @@ __global__ __launch_bounds__(256) void insert_kernel(const int64_t *__restrict__
     const int64_t k = keys[i];
     uint32_t s = static_cast<uint32_t>((static_cast<uint64_t>(k) * kGolden) >> shift) & mask;
     for (;;) {
-        int32_t o = table_load(table + s);
+        // claimed or looked at in one trip to memory; a look before the claim is a trip of its own
+        const int32_t o = atomicCAS(table + s, -1, i);
         if (o < 0) {
-            o = atomicCAS(table + s, -1, i);
-            if (o < 0) {
-                break;  // claimed
-            }
+            break;  // claimed
         }
         if (keys[o] == k) {
             if (o > i) {  // what a slot holds only ever falls: a smaller index that is there already stays or gives way to a
@@ -281,6 +275,10 @@ int64_t table_capacity(int64_t n) {
     return cap;
 }
 
+// Slots of the table of one list: four to eight per key. Every probe is two trips to memory one after the other, and the launch
+// lasts as long as its unluckiest key.
+int64_t list_capacity(int64_t n) { return 2 * table_capacity(n); }
+
 // An empty table of `cap` slots (a power of two, >= 2 n) and the keys into it; the fill is a kernel, so the sequence may be
 // recorded into a graph.
 void launch_insert(const int64_t *d_keys, int32_t n, int32_t *table, int64_t cap, int32_t *slot_of, hipStream_t s) {
@@ -411,7 +409,7 @@ int64_t kvcm_hip_select_save_workspace_bytes(int64_t n) {
         return KVCM_ERR_TOO_LARGE;
     }
     // words first (8-byte aligned), then table, slots and counts
-    return kvcm::list_groups(n) * (kvcm::kListWaves * 8 + 4) + (kvcm::table_capacity(n) + n) * 4;
+    return kvcm::list_groups(n) * (kvcm::kListWaves * 8 + 4) + (kvcm::list_capacity(n) + n) * 4;
 }
 
 int32_t kvcm_hip_select_save(const int64_t *d_keys, const uint8_t *d_saved, int64_t n, void *d_workspace,
@@ -429,7 +427,7 @@ int32_t kvcm_hip_select_save(const int64_t *d_keys, const uint8_t *d_saved, int6
         return KVCM_ERR_ALIGNMENT;
     }
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    const int64_t groups = kvcm::list_groups(n), cap = kvcm::table_capacity(n);
+    const int64_t groups = kvcm::list_groups(n), cap = kvcm::list_capacity(n);
     uint64_t *words = static_cast<uint64_t *>(d_workspace);
     int32_t *table = reinterpret_cast<int32_t *>(words + groups * kvcm::kListWaves);
     int32_t *slot_of = table + cap, *counts = slot_of + n;
