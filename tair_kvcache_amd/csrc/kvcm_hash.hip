@@ -891,11 +891,19 @@ __global__ __launch_bounds__(64) void sha256_first8_kernel(const uint8_t *__rest
     uint32_t st[8] = {0x6a09e667, 0xbb67ae85, 0x3c6ef372, 0xa54ff53a, 0x510e527f, 0x9b05688c, 0x1f83d9ab, 0x5be0cd19};
     for (int64_t base = 0; base < padded_len; base += 64) {
         uint32_t w[16];
+        if (base + 64 <= len) {  // nothing but message: words instead of bytes, a quarter of the loads and no compare per byte
+            __builtin_memcpy(w, msg + base, 64);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int64_t p = base + 4 * j;
-            w[j] = (padded_byte(msg, len, padded_len, p) << 24) | (padded_byte(msg, len, padded_len, p + 1) << 16) |
-                   (padded_byte(msg, len, padded_len, p + 2) << 8) | padded_byte(msg, len, padded_len, p + 3);
+            for (int j = 0; j < 16; ++j) {
+                w[j] = __builtin_bswap32(w[j]);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const int64_t p = base + 4 * j;
+                w[j] = (padded_byte(msg, len, padded_len, p) << 24) | (padded_byte(msg, len, padded_len, p + 1) << 16) |
+                       (padded_byte(msg, len, padded_len, p + 2) << 8) | padded_byte(msg, len, padded_len, p + 3);
+            }
         }
         sha256_compress(st, w);
     }

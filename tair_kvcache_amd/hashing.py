@@ -9,12 +9,19 @@
 A connector that computes keys here can send `block_keys` instead of `token_ids`; the manager prefers them
 (kv_cache_manager/manager/cache_manager.cc:306-318) and the keys are bit-identical to the ones it would compute.
 """
+from array import array
+from itertools import accumulate
 from typing import List, Optional, Sequence, Tuple
 
 import torch
 
 from . import _lib
 from ._torch_util import lib, ptr, require_cuda, stream_handle
+
+try:  # one C loop over a list of strings; absent only when the package was not built with its build.py
+    from ._kvcm_pylist import pack_strings as _pack_strings
+except ImportError:  # host-side convenience only: the strings then go through Python
+    _pack_strings = None
 
 
 # Requests up to which one launch computes the key offsets: it re-reads what lies in front of every 8192 requests, torch's
@@ -154,18 +161,18 @@ def apply_prefix_hash(hash_ids: torch.Tensor, offsets: Optional[torch.Tensor] = 
 
 def sha256_to_int64(data: Sequence[str], device="cuda") -> torch.Tensor:
     """int.from_bytes(sha256(s.encode('utf-8')).digest()[:8], 'big', signed=True) for every string, on the GPU."""
-    enc = [s.encode("utf-8") if isinstance(s, str) else bytes(s) for s in data]
-    n = len(enc)
-    if n == 0:
-        return torch.empty(0, dtype=torch.int64, device=device)
-    lens = torch.tensor([len(e) for e in enc], dtype=torch.int64)
-    off = torch.zeros(n + 1, dtype=torch.int64)
-    torch.cumsum(lens, 0, out=off[1:])
-    blob = torch.frombuffer(bytearray(b"".join(enc) + b"\0"), dtype=torch.uint8)
-    d_blob = blob.to(device)
-    d_off = off.to(device)
+    packed = _pack_strings(data) if _pack_strings is not None and isinstance(data, (list, tuple)) and len(data) else None
+    if packed is None:  # anything but a list of plain strings
+        enc = [s.encode("utf-8") if isinstance(s, str) else bytes(s) for s in data]
+        n = len(enc)
+        if n == 0:
+            return torch.empty(0, dtype=torch.int64, device=device)
+        packed = bytearray(array("q", accumulate((len(e) for e in enc), initial=0)).tobytes() + b"".join(enc) + b"\0")
+    else:
+        n = len(data)
+    d_packed = torch.frombuffer(packed, dtype=torch.uint8).to(device)  # offsets and bytes in one copy
     out = torch.empty(n, dtype=torch.int64, device=device)
-    rc = lib().kvcm_hip_sha256_first8_be(ptr(d_blob), ptr(d_off), n, ptr(out), stream_handle(out.device))
+    rc = lib().kvcm_hip_sha256_first8_be(ptr(d_packed) + 8 * (n + 1), ptr(d_packed), n, ptr(out), stream_handle(out.device))
     _lib.check(rc, "kvcm_hip_sha256_first8_be")
     return out
 

@@ -136,6 +136,23 @@ def test_sha256_keys(oracle):
     assert _h().prepare_block_keys([], None) == ([], 0, 0)
 
 
+@pytest.mark.parametrize("helper", [True, False])
+def test_sha256_of_every_kind_of_sequence(monkeypatch, helper):
+    """Lists, tuples, generators; str, bytes and bytearray, also mixed; lengths around one and two 64-byte chunks, so that
+    whole chunks start at every alignment; with the C packing loop and without."""
+    if not helper:
+        monkeypatch.setattr(_h(), "_pack_strings", None)
+    strs = ["a" * k for k in list(range(0, 70)) + list(range(117, 131)) + [191, 192, 193, 700]]
+    want = [int.from_bytes(hashlib.sha256(s.encode()).digest()[:8], "big", signed=True) for s in strs]
+    forms = [strs, tuple(strs), (s for s in strs), [s.encode() for s in strs], [bytearray(s.encode()) for s in strs],
+             [s if i % 2 else s.encode() for i, s in enumerate(strs)]]
+    for form in forms:
+        assert _h().sha256_to_int64(form).tolist() == want
+    assert _h().sha256_to_int64([]).tolist() == [] and _h().sha256_to_int64(iter([])).tolist() == []
+    with pytest.raises(UnicodeEncodeError):
+        _h().sha256_to_int64(["\ud800"])
+
+
 def test_bad_buffers_are_refused_on_the_host():
     """Short key buffers, offsets of the wrong type, length or device would be out-of-bounds device accesses: ValueError."""
     h = _h()

@@ -407,3 +407,20 @@ def test_generate_blocks_idx_host_equals_the_reference_loop(oracle):
     with pytest.raises(ValueError):
         connector.generate_blocks_idx_host([0], [2 ** 30], 16, 16)  # the slot itself does not fit 32 bits
     assert len(connector.generate_blocks_idx_host([], [1, 2], 16, 16)) == 0
+
+
+def test_packed_strings_are_offsets_then_bytes():
+    """pack_strings: int64 offsets, then the bytes, then one spare byte; None for items that are not plain str or bytes."""
+    import numpy as np
+    from tair_kvcache_amd._kvcm_pylist import pack_strings
+    items = ["abc", "", "\u00e9\u6f22", b"\x00\xff", "x" * 1000]
+    enc = [s.encode() if isinstance(s, str) else s for s in items]
+    offsets = np.concatenate([[0], np.cumsum([len(e) for e in enc])]).astype(np.int64)
+    for form in (items, tuple(items)):
+        assert bytes(pack_strings(form)) == offsets.tobytes() + b"".join(enc) + b"\0"
+    assert bytes(pack_strings([])) == bytes(9)
+    assert pack_strings([1]) is None and pack_strings(["a", bytearray(b"b")]) is None
+    with pytest.raises(UnicodeEncodeError):
+        pack_strings(["\ud800"])
+    with pytest.raises(TypeError):
+        pack_strings("abc")
