@@ -81,6 +81,15 @@ int32_t kvcm_hip_hash_tokens_i32(const int32_t *d_tokens, const int64_t *d_token
                                  const int64_t *d_key_offsets, kvcm_stream_t stream);
 
 /*
+ * The same for offsets that are not known to be sound: d_tokens holds n_tokens entries of token_bytes (4 or 8) and d_keys
+ * n_keys. A request whose blocks reach beyond the tokens, or whose keys beyond the keys, is left out, and nothing outside
+ * either array is read or written. kvcm_hip_prefix_chain is block_size 1, seed 0 and the same array of offsets twice.
+ */
+int32_t kvcm_hip_hash_tokens_checked(const void *d_tokens, int32_t token_bytes, int64_t n_tokens,
+                                     const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t seed,
+                                     int64_t *d_keys, int64_t n_keys, const int64_t *d_key_offsets, kvcm_stream_t stream);
+
+/*
  * The same for R requests of one length, laid out one behind the other ([R][tokens_per_request], token_bytes = 4 or 8):
  * no offset arrays are read. d_key_offsets may be NULL (request r's keys start at r * (tokens_per_request / block_size));
  * d_key_offsets_out, when not NULL, receives those R + 1 offsets. tokens_per_request must be at least block_size.
@@ -98,6 +107,17 @@ int32_t kvcm_hip_hash_tokens_2d(const void *d_tokens, int32_t token_bytes, int32
 #define KVCM_PENDING (-INT64_C(0x4000000000000000))
 int32_t kvcm_hip_key_offsets(const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t limit,
                              int64_t *d_key_offsets, int64_t *h_total, kvcm_stream_t stream);
+
+/*
+ * The same against the number of tokens as well: a request whose blocks reach beyond n_tokens gets the offset -1, and
+ * h_total becomes -1 when there is one (d_key_offsets[R] stays the sum of all requests). With d_workspace (at least
+ * kvcm_hip_key_offsets_workspace_bytes(R) bytes, 8-byte aligned, or NULL) the time stays linear in R; up to 32768 requests
+ * nothing is needed there.
+ */
+int64_t kvcm_hip_key_offsets_workspace_bytes(int32_t R);
+int32_t kvcm_hip_key_offsets_checked(const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t n_tokens,
+                                     int64_t n_keys, void *d_workspace, int64_t workspace_bytes, int64_t *d_key_offsets,
+                                     int64_t *h_total, kvcm_stream_t stream);
 
 /*
  * Blocks the calling thread until *h_value (pinned host memory that work on `stream` writes) is no longer KVCM_PENDING.

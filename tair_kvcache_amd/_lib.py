@@ -55,6 +55,9 @@ SIGNATURES = {
     "kvcm_hip_hash_tokens": (i32, [vp, vp, i32, i32, i64, vp, vp, vp]),
     "kvcm_hip_hash_tokens_i32": (i32, [vp, vp, i32, i32, i64, vp, vp, vp]),
     "kvcm_hip_hash_tokens_2d": (i32, [vp, i32, i32, i64, i32, i64, vp, vp, vp, vp]),
+    "kvcm_hip_hash_tokens_checked": (i32, [vp, i32, i64, vp, i32, i32, i64, vp, i64, vp, vp]),
+    "kvcm_hip_key_offsets_workspace_bytes": (i64, [i32]),
+    "kvcm_hip_key_offsets_checked": (i32, [vp, i32, i32, i64, i64, vp, i64, vp, vp, vp]),
     "kvcm_hip_key_offsets": (i32, [vp, i32, i32, i64, vp, vp, vp]),
     "kvcm_wait_value": (i32, [vp, vp]),
     "kvcm_hip_prefix_chain": (i32, [vp, vp, i32, vp, vp]),

@@ -572,6 +572,21 @@ struct Uniform {
     int64_t *key_offsets_out;  // [R + 1], or NULL
 };
 
+// What the arrays hold, for launches with offsets: a request that names tokens or key slots beyond it is left out, and no
+// load leaves the tokens, whatever the offsets say.
+struct Extent {
+    int64_t tokens;
+    int64_t keys;
+};
+constexpr int64_t kUnknown = INT64_MAX;  // the caller did not say: token offsets are taken as they are
+
+__device__ __forceinline__ int64_t distance(int64_t from, int64_t to) {  // offsets may be anything: no signed overflow
+    return static_cast<int64_t>(static_cast<uint64_t>(to) - static_cast<uint64_t>(from));
+}
+
+// whether [at, at + n) is a non-empty part of [0, size)
+__device__ __forceinline__ bool inside(int64_t at, int64_t n, int64_t size) { return at >= 0 && n > 0 && n <= size - at; }
+
 // CHUNK = steps between two looks at the block boundary: 8 when block_size % 8 == 0 (a lane is then
 // active for whole chunks or not at all), otherwise 1. BS = block size when it is 1, 8, 16, 32, 64 or 128, otherwise 0.
 // KS != kKeysDirect ("keys staged", block sizes 1 to 64; chosen by the host for batches of many requests, where the launch
@@ -584,7 +599,8 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
                                                               int32_t block_size, uint64_t seed,
                                                               int64_t *__restrict__ keys,
                                                               const int64_t *__restrict__ key_offsets,
-                                                              const Uniform uni, int32_t force_global_loads) {
+                                                              const Uniform uni, const Extent have,
+                                                              int32_t force_global_loads) {
     __shared__ __attribute__((aligned(16))) uint64_t s_tile[kRing][kReqs][kTT + kPad];
     __shared__ int64_t s_start[kReqs];
     __shared__ int64_t s_ntok[kReqs];
@@ -610,14 +626,18 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
     if (wave == 0) {
         int64_t start;
         if (token_offsets) {
-            start = token_offsets[r_first];  // rows past R idle at the first row
+            start = token_offsets[r_first];  // rows past R and requests without keys idle at the first row
+            start = start < 0 && have.tokens != kUnknown ? 0 : start;
             if (r < R) {
-                start = token_offsets[r];
-                const int64_t n = token_offsets[r + 1] - start;
-                my_ntok = (n / block_size) * block_size;  // a trailing partial block yields no key
-                key_pos = key_offsets ? key_offsets[r] : r * ((token_offsets[1] - token_offsets[0]) / block_size);
+                const int64_t at = token_offsets[r], n = distance(at, token_offsets[r + 1]);
+                const int64_t nkeys = n / block_size;  // a trailing partial block yields no key
+                key_pos = key_offsets ? key_offsets[r] : r * (distance(token_offsets[0], token_offsets[1]) / block_size);
+                if (inside(key_pos, nkeys, have.keys) &&
+                    (have.tokens == kUnknown || inside(at, nkeys * block_size, have.tokens))) {
+                    start = at;
+                    my_ntok = nkeys * block_size;
+                }
             }
-            my_ntok = key_pos < 0 ? 0 : my_ntok;
         } else {
             start = r_first * uni.tokens;
             if (r < R) {
@@ -636,13 +656,17 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
         ctx.tokens = tokens;
         ctx.s_start = s_start;
         const int64_t r_end = r_first + kReqs < R ? r_first + kReqs : R;
-        const int64_t total = token_offsets ? token_offsets[R] : R * uni.tokens;
+        const bool known = token_offsets && have.tokens != kUnknown;
+        const int64_t total = !token_offsets ? R * uni.tokens : known ? have.tokens : token_offsets[R];
         const int64_t end_token = token_offsets ? token_offsets[r_end] : r_end * uni.tokens;
         ctx.last_token = total - 1;  // >= 0 whenever a tile is loaded: some request has a full block then
         ctx.wg_first_token = token_offsets ? token_offsets[r_first] : r_first * uni.tokens;
+        if (known && (ctx.wg_first_token < 0 || ctx.wg_first_token > total)) {
+            ctx.wg_first_token = ctx.wg_first_token < 0 ? 0 : total;
+        }
         const uint64_t to_end = static_cast<uint64_t>(total - ctx.wg_first_token) * sizeof(TokT);
         ctx.wg_bytes = to_end > 0xFFFFFFFFull ? 0xFFFFFFFFu : static_cast<uint32_t>(to_end);
-        const uint64_t wg_span = static_cast<uint64_t>(end_token - ctx.wg_first_token) * sizeof(TokT);
+        const uint64_t wg_span = static_cast<uint64_t>(distance(ctx.wg_first_token, end_token)) * sizeof(TokT);
         buffer_loads = !force_global_loads && wg_span < 0xFFF00000ull;
         if (uni.key_offsets_out && wave == kLoaders) {  // the last loader: its first tile is the one needed last
             if (r < R) {
@@ -746,9 +770,12 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
 // together), and adds up everything in front of its range itself instead of waiting for a pass of partial sums: one launch,
 // no workspace. 160 requests 3.2 us against 7.5 us on the device (and 3.6 against 22 on the host) for five launches of a
 // general prefix sum; 8192 requests 8.5 against 12.5, 16 384 10.1 against 12.8, then the re-reading shows: 65 536 20 / 13.
+// From kOffsetsRereadUpTo requests on a launch in front leaves the sum of every workgroup's range (`sums`).
 constexpr int kOffsetsThreads = 1024;
 constexpr int kOffsetsPerThread = 8;
 constexpr int64_t kOffsetsPerWg = kOffsetsThreads * kOffsetsPerThread;
+constexpr int32_t kOffsetsRereadUpTo = 32768;
+int64_t offsets_groups(int32_t R) { return (R + kOffsetsPerWg - 1) / kOffsetsPerWg; }
 
 __device__ __forceinline__ int64_t keys_of(int64_t len, int32_t block_size) {
     if (static_cast<uint64_t>(len) >> 32 == 0) {  // 32-bit division: a fifth of the instructions
@@ -757,15 +784,67 @@ __device__ __forceinline__ int64_t keys_of(int64_t len, int32_t block_size) {
     return len > 0 ? len / block_size : 0;
 }
 
+// Keys of one request; `bad` is set when the tokens they are made of are not all there.
+__device__ __forceinline__ int64_t keys_of_request(int64_t at, int64_t next, int32_t block_size, int64_t n_tokens, bool &bad) {
+    const int64_t count = keys_of(distance(at, next), block_size);
+    bad |= n_tokens != kUnknown && count > 0 && !inside(at, count * block_size, n_tokens);
+    return count;
+}
+
+// sums[g] = keys of the requests of workgroup g of key_offsets_kernel, as its complement if one of them is bad
+__global__ __launch_bounds__(kOffsetsThreads) void key_sums_kernel(const int64_t *__restrict__ token_offsets, int32_t R,
+                                                                   int32_t block_size, int64_t n_tokens,
+                                                                   int64_t *__restrict__ sums) {
+    __shared__ int64_t s_sum[kOffsetsThreads / 64];
+    __shared__ int32_t s_bad[kOffsetsThreads / 64];
+    const int64_t base = blockIdx.x * kOffsetsPerWg;
+    const int64_t end = base + kOffsetsPerWg < R ? base + kOffsetsPerWg : R;
+    int64_t sum = 0;
+    bool bad = false;
+#pragma unroll 8
+    for (int64_t i = base + threadIdx.x; i < end; i += kOffsetsThreads) {
+        sum += keys_of_request(token_offsets[i], token_offsets[i + 1], block_size, n_tokens, bad);
+    }
+    for (int d = 1; d < 64; d <<= 1) {
+        sum += __shfl_xor(sum, d, 64);
+    }
+    const bool any = __ballot(bad) != 0;
+    if ((threadIdx.x & 63) == 0) {
+        s_sum[threadIdx.x >> 6] = sum;
+        s_bad[threadIdx.x >> 6] = any;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int64_t all = 0;
+        bool some = false;
+        for (int w = 0; w < kOffsetsThreads / 64; ++w) {
+            all += s_sum[w];
+            some |= s_bad[w] != 0;
+        }
+        sums[blockIdx.x] = some ? ~all : all;
+    }
+}
+
 __global__ __launch_bounds__(kOffsetsThreads) void key_offsets_kernel(const int64_t *__restrict__ token_offsets, int32_t R,
-                                                                      int32_t block_size, int64_t limit,
+                                                                      int32_t block_size, int64_t n_tokens, int64_t limit,
+                                                                      const int64_t *__restrict__ sums,
                                                                       int64_t *__restrict__ key_offsets, int64_t *h_total) {
     __shared__ int64_t s_wave[2][kOffsetsThreads / 64];
+    __shared__ int32_t s_bad[kOffsetsThreads / 64];
     const int32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const int64_t base = blockIdx.x * kOffsetsPerWg;
     int64_t before = 0;
-    for (int64_t i = threadIdx.x; i < base; i += blockDim.x) {
-        before += keys_of(token_offsets[i + 1] - token_offsets[i], block_size);
+    bool bad = false;
+    if (sums) {
+        for (int64_t g = threadIdx.x; g < static_cast<int64_t>(blockIdx.x); g += blockDim.x) {
+            const int64_t v = sums[g];
+            bad |= v < 0;
+            before += v < 0 ? ~v : v;
+        }
+    } else {
+        for (int64_t i = threadIdx.x; i < base; i += blockDim.x) {
+            before += keys_of_request(token_offsets[i], token_offsets[i + 1], block_size, n_tokens, bad);
+        }
     }
     const int64_t first = base + static_cast<int64_t>(threadIdx.x) * kOffsetsPerThread;
     int64_t off[kOffsetsPerThread + 1];
@@ -774,37 +853,45 @@ __global__ __launch_bounds__(kOffsetsThreads) void key_offsets_kernel(const int6
         off[j] = token_offsets[first + j < R ? first + j : R];
     }
     int64_t count[kOffsetsPerThread], sum = 0;
+    uint32_t left_out = 0;
 #pragma unroll
     for (int j = 0; j < kOffsetsPerThread; ++j) {
-        count[j] = keys_of(off[j + 1] - off[j], block_size);
+        bool mine = false;
+        count[j] = keys_of_request(off[j], off[j + 1], block_size, n_tokens, mine);
+        left_out |= mine ? 1u << j : 0u;
         sum += count[j];
     }
+    bad |= left_out != 0;
     int64_t incl = sum;
     for (int d = 1; d < 64; d <<= 1) {
         const int64_t up = __shfl_up(incl, d, 64);
         incl += lane >= d ? up : 0;
         before += __shfl_xor(before, d, 64);
     }
+    const bool any = __ballot(bad) != 0;
     if (lane == 63) {
         s_wave[0][wave] = incl;
         s_wave[1][wave] = before;
+        s_bad[wave] = any;
     }
     __syncthreads();
     int64_t pos = incl - sum;
+    bool some = false;
     for (int w = 0; w < waves; ++w) {
         pos += (w < wave ? s_wave[0][w] : 0) + s_wave[1][w];
+        some |= s_bad[w] != 0;
     }
 #pragma unroll
     for (int j = 0; j < kOffsetsPerThread; ++j) {
         if (first + j < R) {
             const int64_t end = pos + count[j];
-            // beyond the room the caller has: marked, and the hash kernel leaves the request out
-            key_offsets[first + j] = end <= limit ? pos : -1;
+            // without its tokens, or beyond the room the caller has: marked, and the hash kernel leaves the request out
+            key_offsets[first + j] = end <= limit && !(left_out >> j & 1) ? pos : -1;
             pos = end;
             if (first + j == R - 1) {
                 key_offsets[R] = pos;
-                if (h_total) {
-                    __hip_atomic_store(h_total, pos, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+                if (h_total) {  // the last workgroup has seen every request
+                    __hip_atomic_store(h_total, some ? -1 : pos, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
                 }
             }
         }
@@ -999,7 +1086,7 @@ constexpr int32_t burst_from(int32_t block_size, bool tokens_8_byte) {
 template <typename TokT>
 int32_t launch_hash(const TokT *d_tokens, const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t seed,
                     int64_t *d_keys, const int64_t *d_key_offsets, hipStream_t stream,
-                    const Uniform &uni = Uniform{0, 0, nullptr}) {
+                    const Uniform &uni = Uniform{0, 0, nullptr}, const Extent &have = Extent{kUnknown, kUnknown}) {
     if (R < 0 || block_size <= 0) {
         return KVCM_ERR_INVALID_ARG;
     }
@@ -1013,13 +1100,15 @@ int32_t launch_hash(const TokT *d_tokens, const int64_t *d_token_offsets, int32_
     const int32_t force_global = kForceGeneralLoader;
 #define KVCM_LAUNCH_HASH(CHUNK, BS)                                                                                  \
     hipLaunchKernelGGL((hash_tokens_kernel<TokT, CHUNK, BS>), grid, dim3(kThreads), 0, stream, d_tokens,            \
-                       d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, force_global)
+                       d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, have, \
+                       force_global)
     constexpr bool k8 = sizeof(TokT) == 8;
     const bool burst = R >= static_cast<int64_t>(burst_from(block_size, k8)) * KVCM_HASH_BURST_SCALE;
     const bool spread = block_size == 16 && k8 && !burst && R >= KVCM_HASH_SPREAD_FROM_8;
 #define KVCM_LAUNCH_HASH_STAGED(CHUNK, BS, KS)                                                                       \
     hipLaunchKernelGGL((hash_tokens_kernel<TokT, CHUNK, BS, KS>), grid, dim3(kThreads), 0, stream, d_tokens,        \
-                       d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, force_global)
+                       d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, have, \
+                       force_global)
     // 4-byte tokens from as many requests as take the burst form: tiles of 128 raw tokens (512-byte pieces of the
     // token stream per request and load instruction instead of 256-byte ones). Cold timings, 16-token blocks, requests
     // of 4096 tokens, 64-token tiles of pre-added terms / raw tiles: 64 requests 56.8 / 57.3 us, 8192 58.1 / 60.2,
@@ -1028,7 +1117,8 @@ int32_t launch_hash(const TokT *d_tokens, const int64_t *d_token_offsets, int32_
                                       block_size == 128);
 #define KVCM_LAUNCH_HASH_RAW(BS)                                                                                      \
     hipLaunchKernelGGL((hash_tokens_kernel<TokT, 8, BS, kKeysBurst, true>), grid, dim3(kThreads), 0, stream, d_tokens, \
-                       d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, force_global)
+                       d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, have, \
+                       force_global)
     if (raw) {
         if constexpr (!k8) {
             switch (block_size) {
@@ -1164,19 +1254,58 @@ int32_t kvcm_wait_value(const int64_t *h_value, kvcm_stream_t stream) {
     }
 }
 
-int32_t kvcm_hip_key_offsets(const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t limit,
-                             int64_t *d_key_offsets, int64_t *h_total, kvcm_stream_t stream) {
-    if (R <= 0 || block_size <= 0 || !d_token_offsets || !d_key_offsets) {
+int32_t kvcm_hip_hash_tokens_checked(const void *d_tokens, int32_t token_bytes, int64_t n_tokens,
+                                     const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t seed,
+                                     int64_t *d_keys, int64_t n_keys, const int64_t *d_key_offsets, kvcm_stream_t stream) {
+    if ((token_bytes != 4 && token_bytes != 8) || n_tokens < 0 || n_keys < 0) {
         return KVCM_ERR_INVALID_ARG;
+    }
+    const kvcm::Uniform no{0, 0, nullptr};
+    const kvcm::Extent have{n_tokens, n_keys};
+    if (token_bytes == 8) {
+        return kvcm::launch_hash<int64_t>(static_cast<const int64_t *>(d_tokens), d_token_offsets, R, block_size, seed, d_keys,
+                                          d_key_offsets, static_cast<hipStream_t>(stream), no, have);
+    }
+    return kvcm::launch_hash<int32_t>(static_cast<const int32_t *>(d_tokens), d_token_offsets, R, block_size, seed, d_keys,
+                                      d_key_offsets, static_cast<hipStream_t>(stream), no, have);
+}
+
+int64_t kvcm_hip_key_offsets_workspace_bytes(int32_t R) {
+    return R <= kvcm::kOffsetsRereadUpTo ? 0 : kvcm::offsets_groups(R) * 8;
+}
+
+int32_t kvcm_hip_key_offsets_checked(const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t n_tokens,
+                                     int64_t n_keys, void *d_workspace, int64_t workspace_bytes, int64_t *d_key_offsets,
+                                     int64_t *h_total, kvcm_stream_t stream) {
+    if (R <= 0 || block_size <= 0 || n_tokens < 0 || !d_token_offsets || !d_key_offsets) {
+        return KVCM_ERR_INVALID_ARG;
+    }
+    const int64_t groups = kvcm::offsets_groups(R);
+    if (d_workspace && workspace_bytes < kvcm_hip_key_offsets_workspace_bytes(R)) {
+        return KVCM_ERR_INVALID_ARG;
+    }
+    if (reinterpret_cast<uintptr_t>(d_workspace) % 8 != 0) {
+        return KVCM_ERR_ALIGNMENT;
     }
     if (h_total) {
         *h_total = KVCM_PENDING;
     }
-    const int64_t groups = (R + kvcm::kOffsetsPerWg - 1) / kvcm::kOffsetsPerWg;
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    int64_t *sums = R > kvcm::kOffsetsRereadUpTo ? static_cast<int64_t *>(d_workspace) : nullptr;
+    if (sums) {
+        hipLaunchKernelGGL(kvcm::key_sums_kernel, dim3(static_cast<uint32_t>(groups)), dim3(kvcm::kOffsetsThreads), 0, s,
+                           d_token_offsets, R, block_size, n_tokens, sums);
+    }
     const int64_t threads = groups > 1 ? kvcm::kOffsetsThreads : ((R + kvcm::kOffsetsPerThread - 1) / kvcm::kOffsetsPerThread + 63) / 64 * 64;
-    hipLaunchKernelGGL(kvcm::key_offsets_kernel, dim3(static_cast<uint32_t>(groups)), dim3(static_cast<uint32_t>(threads)), 0,
-                       static_cast<hipStream_t>(stream), d_token_offsets, R, block_size, limit, d_key_offsets, h_total);
+    hipLaunchKernelGGL(kvcm::key_offsets_kernel, dim3(static_cast<uint32_t>(groups)), dim3(static_cast<uint32_t>(threads)), 0, s,
+                       d_token_offsets, R, block_size, n_tokens, n_keys, sums, d_key_offsets, h_total);
     return kvcm::launch_status();
+}
+
+int32_t kvcm_hip_key_offsets(const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t limit,
+                             int64_t *d_key_offsets, int64_t *h_total, kvcm_stream_t stream) {
+    return kvcm_hip_key_offsets_checked(d_token_offsets, R, block_size, kvcm::kUnknown, limit, nullptr, 0, d_key_offsets, h_total,
+                                        stream);
 }
 
 int32_t kvcm_hip_prefix_chain(const int64_t *d_digests, const int64_t *d_offsets, int32_t R, int64_t *d_keys,

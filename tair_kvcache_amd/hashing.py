@@ -24,13 +24,6 @@ except ImportError:  # host-side convenience only: the strings then go through P
     _pack_strings = None
 
 
-# Requests up to which one launch computes the key offsets: it re-reads what lies in front of every 8192 requests, torch's
-# five launches do not. Microseconds on the device, one launch / torch: 160 requests 3.2 / 7.5, 8192 8.5 / 12.5, 16 384
-# 10.1 / 12.8, 65 536 20 / 13, 131 072 33 / 13 (and 25 of host time for torch's, always).
-_NATIVE_OFFSETS_UP_TO = 32768
-_NO_LIMIT = 2**62
-
-
 def _require_offsets(t, name, device, entries=None):
     """Offsets are read by the kernel as they are: int64, 1-D, on the tokens' device, R+1 entries."""
     require_cuda(t, name)
@@ -49,7 +42,9 @@ def hash_tokens(tokens: torch.Tensor, block_size: int, token_offsets: Optional[t
 
     tokens: int64 or int32 device tensor, [R, L] (uniform lengths) or flat with token_offsets [R+1].
     Returns (keys, key_offsets): request r owns keys[key_offsets[r]:key_offsets[r+1]], len_r // block_size of
-    them (a trailing partial block yields no key, cache_manager.cc:78). Asynchronous on the current stream when
+    them (a trailing partial block yields no key, cache_manager.cc:78). Offsets that reach beyond `tokens`, or keys beyond
+    `keys`, are never followed: such a request is left out, and where the call waits for the number of keys it raises
+    ValueError. Asynchronous on the current stream when
     `keys` and `key_offsets` are passed in (or the batch is a 2-D tensor); otherwise the call returns once the number of
     keys is known on the host, which does not wait for the keys themselves.
     """
@@ -91,38 +86,35 @@ def hash_tokens(tokens: torch.Tensor, block_size: int, token_offsets: Optional[t
                                            ptr(keys), ptr(key_offsets), ptr(new_offsets), stream_handle(tokens.device))
         _lib.check(rc, "kvcm_hip_hash_tokens_2d")
         return keys, (new_offsets if key_offsets is None else key_offsets)
-    stream = stream_handle(tokens.device)
-    pending = None
+    L, stream, pending = lib(), stream_handle(tokens.device), None
+    if key_offsets is None and R == 0:
+        key_offsets = torch.zeros(1, dtype=torch.int64, device=tokens.device)
     if key_offsets is None:
-        if R == 0 or R > _NATIVE_OFFSETS_UP_TO:
-            counts = (off[1:] - off[:-1]) // block_size
-            key_offsets = torch.zeros(R + 1, dtype=torch.int64, device=tokens.device)
-            torch.cumsum(counts, 0, out=key_offsets[1:])
-        else:
-            # The total is on its way to the host while the keys are being computed into a buffer of the size that the
-            # token count bounds: nobody waits for the hash kernel, and the hash kernel waits for nobody.
-            key_offsets = torch.empty(R + 1, dtype=torch.int64, device=tokens.device)
-            most = _NO_LIMIT
-            if keys is None:
-                most = tokens.numel() // block_size
-                keys = torch.empty(most, dtype=torch.int64, device=tokens.device)
-                pending = torch.empty(1, dtype=torch.int64, pin_memory=True)
-            rc = lib().kvcm_hip_key_offsets(ptr(off), R, block_size, most, ptr(key_offsets), ptr(pending), stream)
-            _lib.check(rc, "kvcm_hip_key_offsets")
+        # The total is on its way to the host while the keys are being computed into a buffer of the size that the
+        # token count bounds: nobody waits for the hash kernel, and the hash kernel waits for nobody.
+        key_offsets = torch.empty(R + 1, dtype=torch.int64, device=tokens.device)
+        if keys is None:
+            keys = torch.empty(tokens.numel() // block_size, dtype=torch.int64, device=tokens.device)
+            pending = torch.empty(1, dtype=torch.int64, pin_memory=True)
+        ws_bytes = L.kvcm_hip_key_offsets_workspace_bytes(R)
+        ws = torch.empty(ws_bytes // 8, dtype=torch.int64, device=tokens.device) if ws_bytes else None
+        rc = L.kvcm_hip_key_offsets_checked(ptr(off), R, block_size, tokens.numel(), keys.numel(), ptr(ws), ws_bytes,
+                                            ptr(key_offsets), ptr(pending), stream)
+        _lib.check(rc, "kvcm_hip_key_offsets_checked")
     if keys is None:
         total = int(key_offsets[-1].item())
         keys = torch.empty(total, dtype=torch.int64, device=tokens.device)
         if total == 0:
             return keys, key_offsets
     if keys.numel() or pending is None:
-        fn = lib().kvcm_hip_hash_tokens if tokens.dtype == torch.int64 else lib().kvcm_hip_hash_tokens_i32
-        rc = fn(ptr(tokens), ptr(off), R, block_size, int(seed), ptr(keys), ptr(key_offsets), stream)
-        _lib.check(rc, "kvcm_hip_hash_tokens")
+        rc = L.kvcm_hip_hash_tokens_checked(ptr(tokens), tokens.element_size(), tokens.numel(), ptr(off), R, block_size,
+                                            int(seed), ptr(keys), keys.numel(), ptr(key_offsets), stream)
+        _lib.check(rc, "kvcm_hip_hash_tokens_checked")
     if pending is not None:
-        _lib.check(lib().kvcm_wait_value(ptr(pending), stream), "kvcm_wait_value")
+        _lib.check(L.kvcm_wait_value(ptr(pending), stream), "kvcm_wait_value")
         total = pending.item()
-        if total > keys.numel():
-            raise ValueError(f"token_offsets name {total} blocks of {block_size} tokens, tokens holds {tokens.numel()}")
+        if not 0 <= total <= keys.numel():
+            raise ValueError(f"token_offsets name blocks of {block_size} tokens beyond the {tokens.numel()} that tokens holds")
         keys = keys[:total]
     return keys, key_offsets
 
@@ -153,9 +145,9 @@ def apply_prefix_hash(hash_ids: torch.Tensor, offsets: Optional[torch.Tensor] = 
         _require_offsets(offsets, "offsets", ids.device)
         offsets = offsets.contiguous()
     keys = torch.empty_like(ids)
-    rc = lib().kvcm_hip_prefix_chain(ptr(ids), ptr(offsets), offsets.numel() - 1, ptr(keys),
-                                     stream_handle(ids.device))
-    _lib.check(rc, "kvcm_hip_prefix_chain")
+    rc = lib().kvcm_hip_hash_tokens_checked(ptr(ids), 8, ids.numel(), ptr(offsets), offsets.numel() - 1, 1, 0, ptr(keys),
+                                            keys.numel(), ptr(offsets), stream_handle(ids.device))
+    _lib.check(rc, "kvcm_hip_hash_tokens_checked")
     return keys.reshape(hash_ids.shape)
 
 

@@ -42,10 +42,11 @@ def golden():
 
 
 class _GeneralLoaderLib:
-    """The shipped library with its three block-key entry points replaced by those of
+    """The shipped library with its block-key entry points replaced by those of
     tests/libkvcm_hash_general_loader.so: the same source built with KVCM_TEST_FORCE_GENERAL_LOADER=1, in which every
     launch takes the loader form of a workgroup whose requests span 4 GiB or more."""
-    _SWAPPED = ("kvcm_hip_hash_tokens", "kvcm_hip_hash_tokens_i32", "kvcm_hip_prefix_chain")
+    _SWAPPED = ("kvcm_hip_hash_tokens", "kvcm_hip_hash_tokens_i32", "kvcm_hip_hash_tokens_checked",
+                "kvcm_hip_hash_tokens_2d", "kvcm_hip_prefix_chain")
 
     def __init__(self):
         import ctypes

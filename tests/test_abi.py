@@ -65,6 +65,19 @@ def test_argument_validation_needs_no_device():
     assert L.kvcm_hip_hash_tokens(p, p, 0, 16, 0, p, None, None) == _lib.OK
     assert L.kvcm_hip_hash_tokens(p, p, 1, 0, 0, p, None, None) == _lib.ERR_INVALID_ARG
     assert L.kvcm_hip_hash_tokens(None, p, 1, 16, 0, p, None, None) == _lib.ERR_INVALID_ARG
+    checked = L.kvcm_hip_hash_tokens_checked
+    assert checked(p, 8, 1, p, 0, 16, 0, p, 1, None, None) == _lib.OK
+    assert checked(p, 2, 1, p, 1, 16, 0, p, 1, None, None) == _lib.ERR_INVALID_ARG
+    assert checked(p, 8, -1, p, 1, 16, 0, p, 1, None, None) == _lib.ERR_INVALID_ARG
+    assert checked(p, 8, 1, p, 1, 16, 0, p, -1, None, None) == _lib.ERR_INVALID_ARG
+    assert checked(p, 4, 1, None, 1, 16, 0, p, 1, None, None) == _lib.ERR_INVALID_ARG
+    offsets = L.kvcm_hip_key_offsets_checked
+    assert offsets(p, 0, 16, 1, 1, None, 0, p, None, None) == _lib.ERR_INVALID_ARG
+    assert offsets(p, 1, 0, 1, 1, None, 0, p, None, None) == _lib.ERR_INVALID_ARG
+    assert offsets(p, 1, 16, -1, 1, None, 0, p, None, None) == _lib.ERR_INVALID_ARG
+    assert offsets(p, 32769, 16, 1, 1, p, 39, p, None, None) == _lib.ERR_INVALID_ARG  # workspace too small
+    assert offsets(p, 1, 16, 1, 1, p + 4, 8, p, None, None) == _lib.ERR_ALIGNMENT
+    assert L.kvcm_hip_key_offsets_workspace_bytes(32768) == 0 and L.kvcm_hip_key_offsets_workspace_bytes(32769) == 5 * 8
     assert L.kvcm_hip_sha256_first8_be(None, None, 0, None, None) == _lib.OK
     assert L.kvcm_hip_iov_crc32(None, 1, None, 4, None) == _lib.ERR_INVALID_ARG
     assert L.kvcm_hip_generate_blocks_idx(p, 1, p, 1, 0, 16, p, None, None) == _lib.ERR_INVALID_ARG

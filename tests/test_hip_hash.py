@@ -390,3 +390,63 @@ def test_offsets_beyond_the_tokens_are_refused():
     with pytest.raises(ValueError):
         _h().hash_tokens(flat[:1024], 16, token_offsets=off)
     sync()
+
+
+@pytest.mark.parametrize("general_loader", [False, True])
+@pytest.mark.parametrize("dtype", [np.int64, np.int32])
+@pytest.mark.parametrize("R", [17, 40001])   # the last request is whole blocks up to the end of the tokens
+def test_offsets_are_not_followed_beyond_the_tokens(oracle, force_general_hash_loader, general_loader, dtype, R):
+    """Offsets that reach beyond `tokens` although the number of blocks would fit, because most requests are shorter than a
+    block: ValueError, as one launch counts the blocks and as two do. An overrun inside a trailing partial block costs no
+    key and changes none. (All arrays are the front of larger ones, whose rest must not matter and must not change.)"""
+    force_general_hash_loader(general_loader)
+    rng = np.random.default_rng(R)
+    n = 16 * R
+    big = rng.integers(-2**31, 2**31, size=2 * n + 4096, dtype=np.int64).astype(dtype)
+    tok = dev(big)[:n]
+    toff = np.minimum(np.arange(R + 1) * 15, n).astype(np.int64)                 # no request holds a block ...
+    for last, ok in ((n, True), (n + 3, True), (n + 16, False), (n + 2000, False)):
+        toff[-1] = last                                                          # ... but the last one
+        d_off = dev(toff)
+        if not ok:
+            with pytest.raises(ValueError):
+                _h().hash_tokens(tok, 16, token_offsets=d_off)
+            continue
+        keys, off = _h().hash_tokens(tok, 16, token_offsets=d_off)
+        sync()
+        want, woff = oracle.hash_tokens(big, 16, token_offsets=toff, threads=8)
+        assert (host(keys, np.int64) == want).all() and (host(off, np.int64) == woff).all(), last
+    # what is asked to go into the caller's own buffer is left out, and marked where the offsets are this call's
+    toff[-1] = n + 16
+    room = torch.full((2 * R + 64,), -7, dtype=torch.int64, device="cuda")
+    _, off = _h().hash_tokens(tok, 16, token_offsets=dev(toff), keys=room[:R])
+    _h().hash_tokens(tok, 16, token_offsets=dev(toff), keys=room[:R], key_offsets=dev(np.zeros(R + 1, dtype=np.int64)))
+    sync()
+    assert (host(room, np.int64) == -7).all() and host(off, np.int64)[R - 1] == -1
+
+
+@pytest.mark.parametrize("general_loader", [False, True])
+def test_keys_beyond_the_callers_buffer_are_left_out(oracle, force_general_hash_loader, general_loader):
+    """A key buffer that holds the keys of some requests only: those are written, the slots behind the buffer are not; the
+    same for a chain whose offsets name more digests than there are."""
+    force_general_hash_loader(general_loader)
+    rng = np.random.default_rng(3)
+    lens = np.array([33, 0, 160, 15, 64, 700, 16])
+    toff = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    flat = rng.integers(0, 152064, size=int(toff[-1]), dtype=np.int64)
+    want, woff = oracle.hash_tokens(flat, 16, token_offsets=toff)
+    for short in (1, 2, 44, 45, 46):
+        room = torch.full((len(want) + 64,), -7, dtype=torch.int64, device="cuda")
+        for koff in (None, dev(woff)):
+            room.fill_(-7)
+            _h().hash_tokens(dev(flat), 16, token_offsets=dev(toff), keys=room[:len(want) - short], key_offsets=koff)
+            sync()
+            got = host(room, np.int64)
+            for r in range(len(lens)):
+                fits = woff[r + 1] <= len(want) - short
+                assert (got[woff[r]:woff[r + 1]] == (want[woff[r]:woff[r + 1]] if fits else -7)).all(), (short, r)
+            assert (got[len(want):] == -7).all()
+    chain, _ = oracle.hash_tokens(flat, 1, token_offsets=toff)
+    got = _h().apply_prefix_hash(dev(flat)[:300], dev(toff))                     # requests 5 and 6 end beyond digest 300
+    sync()
+    assert got.shape == (300,) and (host(got, np.int64)[:272] == chain[:272]).all()
