@@ -86,37 +86,70 @@ def hash_tokens(tokens: torch.Tensor, block_size: int, token_offsets: Optional[t
                                            ptr(keys), ptr(key_offsets), ptr(new_offsets), stream_handle(tokens.device))
         _lib.check(rc, "kvcm_hip_hash_tokens_2d")
         return keys, (new_offsets if key_offsets is None else key_offsets)
-    L, stream, pending = lib(), stream_handle(tokens.device), None
+    stream = stream_handle(tokens.device)
     if key_offsets is None and R == 0:
         key_offsets = torch.zeros(1, dtype=torch.int64, device=tokens.device)
+    if keys is None and key_offsets is None:
+        return _hash_and_count(tokens, off, R, block_size, seed, stream)
     if key_offsets is None:
-        # The total is on its way to the host while the keys are being computed into a buffer of the size that the
-        # token count bounds: nobody waits for the hash kernel, and the hash kernel waits for nobody.
         key_offsets = torch.empty(R + 1, dtype=torch.int64, device=tokens.device)
-        if keys is None:
-            keys = torch.empty(tokens.numel() // block_size, dtype=torch.int64, device=tokens.device)
-            pending = torch.empty(1, dtype=torch.int64, pin_memory=True)
-        ws_bytes = L.kvcm_hip_key_offsets_workspace_bytes(R)
-        ws = torch.empty(ws_bytes // 8, dtype=torch.int64, device=tokens.device) if ws_bytes else None
-        rc = L.kvcm_hip_key_offsets_checked(ptr(off), R, block_size, tokens.numel(), keys.numel(), ptr(ws), ws_bytes,
-                                            ptr(key_offsets), ptr(pending), stream)
-        _lib.check(rc, "kvcm_hip_key_offsets_checked")
+        _launch_offsets(tokens, off, R, block_size, keys, key_offsets, None, stream)
     if keys is None:
         total = int(key_offsets[-1].item())
         keys = torch.empty(total, dtype=torch.int64, device=tokens.device)
         if total == 0:
             return keys, key_offsets
-    if keys.numel() or pending is None:
-        rc = L.kvcm_hip_hash_tokens_checked(ptr(tokens), tokens.element_size(), tokens.numel(), ptr(off), R, block_size,
-                                            int(seed), ptr(keys), keys.numel(), ptr(key_offsets), stream)
-        _lib.check(rc, "kvcm_hip_hash_tokens_checked")
-    if pending is not None:
-        _lib.check(L.kvcm_wait_value(ptr(pending), stream), "kvcm_wait_value")
-        total = pending.item()
-        if not 0 <= total <= keys.numel():
-            raise ValueError(f"token_offsets name blocks of {block_size} tokens beyond the {tokens.numel()} that tokens holds")
-        keys = keys[:total]
+    _launch_keys(tokens, off, R, block_size, seed, keys, key_offsets, stream)
     return keys, key_offsets
+
+
+def _launch_offsets(tokens, off, R, block_size, keys, key_offsets, pending, stream):
+    ws_bytes = lib().kvcm_hip_key_offsets_workspace_bytes(R)
+    ws = torch.empty(ws_bytes // 8, dtype=torch.int64, device=tokens.device) if ws_bytes else None
+    rc = lib().kvcm_hip_key_offsets_checked(ptr(off), R, block_size, tokens.numel(), keys.numel(), ptr(ws), ws_bytes,
+                                            ptr(key_offsets), ptr(pending), stream)
+    _lib.check(rc, "kvcm_hip_key_offsets_checked")
+
+
+def _launch_keys(tokens, off, R, block_size, seed, keys, key_offsets, stream):
+    rc = lib().kvcm_hip_hash_tokens_checked(ptr(tokens), tokens.element_size(), tokens.numel(), ptr(off), R, block_size,
+                                            int(seed), ptr(keys), keys.numel(), ptr(key_offsets), stream)
+    _lib.check(rc, "kvcm_hip_hash_tokens_checked")
+
+
+# Pinned words that a launched kernel has yet to write and nobody waits for any more. torch's pinned-memory pool knows
+# nothing of that kernel, so a word is dropped only once its stream has run dry, and never if the stream cannot say so.
+_owed = {}
+
+
+def _settle(word, device):
+    _owed[id(word)] = word
+    try:
+        torch.cuda.current_stream(device).synchronize()
+    except Exception:
+        return
+    del _owed[id(word)]
+
+
+def _hash_and_count(tokens, off, R, block_size, seed, stream):
+    """(keys, key_offsets) of R > 0 requests when the caller brings neither. The total is on its way to the host while the
+    keys are being computed into a buffer of the size that the token count bounds: nobody waits for the hash kernel, and the
+    hash kernel waits for nobody."""
+    key_offsets = torch.empty(R + 1, dtype=torch.int64, device=tokens.device)
+    keys = torch.empty(tokens.numel() // block_size, dtype=torch.int64, device=tokens.device)
+    pending = torch.empty(1, dtype=torch.int64, pin_memory=True)
+    try:
+        _launch_offsets(tokens, off, R, block_size, keys, key_offsets, pending, stream)
+        if keys.numel():
+            _launch_keys(tokens, off, R, block_size, seed, keys, key_offsets, stream)
+        _lib.check(lib().kvcm_wait_value(ptr(pending), stream), "kvcm_wait_value")
+    except BaseException:  # an interrupt as much as an error: the kernel may still be to come
+        _settle(pending, tokens.device)
+        raise
+    total = pending.item()
+    if not 0 <= total <= keys.numel():
+        raise ValueError(f"token_offsets name blocks of {block_size} tokens beyond the {tokens.numel()} that tokens holds")
+    return keys[:total], key_offsets
 
 
 def gen_key_vector(tokens, block_size: int, device=None) -> List[int]:

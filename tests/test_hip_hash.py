@@ -450,3 +450,33 @@ def test_keys_beyond_the_callers_buffer_are_left_out(oracle, force_general_hash_
     got = _h().apply_prefix_hash(dev(flat)[:300], dev(toff))                     # requests 5 and 6 end beyond digest 300
     sync()
     assert got.shape == (300,) and (host(got, np.int64)[:272] == chain[:272]).all()
+
+
+@pytest.mark.parametrize("fails", ["kvcm_hip_hash_tokens_checked", "kvcm_wait_value"])
+def test_the_word_a_kernel_has_yet_to_write_outlives_an_error(monkeypatch, fails):
+    """A call that ends with an error, or is interrupted, between the launch that writes the number of keys into pinned memory
+    and the wait for it: the stream has run dry before that memory can go to anybody else."""
+    from tair_kvcache_amd import _lib, _torch_util
+    h = _h()
+
+    class Failing:
+        def __getattr__(self, name):
+            if name != fails:
+                return getattr(_torch_util.lib(), name)
+
+            def entry(*args):
+                if name == "kvcm_wait_value":
+                    raise KeyboardInterrupt
+                return _lib.ERR_INVALID_ARG
+            return entry
+
+    off = torch.arange(0, 8193, 64, dtype=torch.int64, device="cuda")
+    tok = torch.zeros(8192, dtype=torch.int64, device="cuda")
+    queued = torch.empty(1 << 28, dtype=torch.int8, device="cuda")
+    monkeypatch.setattr(h, "lib", Failing)
+    sync()
+    for _ in range(64):                                       # some milliseconds of work in front of the kernel
+        queued.zero_()
+    with pytest.raises((_lib.KvcmError, KeyboardInterrupt)):
+        h.hash_tokens(tok, 16, token_offsets=off)
+    assert torch.cuda.current_stream().query() and not h._owed

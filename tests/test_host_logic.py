@@ -424,3 +424,26 @@ def test_packed_strings_are_offsets_then_bytes():
         pack_strings(["\ud800"])
     with pytest.raises(TypeError):
         pack_strings("abc")
+
+
+def test_a_pinned_word_is_kept_when_its_stream_cannot_be_waited_for(monkeypatch):
+    """The device has failed, so whether the kernel that writes the word still comes cannot be known: it stays referenced."""
+    from tair_kvcache_amd import hashing
+
+    class Stream:
+        fails = True
+
+        def synchronize(self):
+            assert hashing._owed                              # held before the wait begins: the wait itself may be interrupted
+            if self.fails:
+                raise RuntimeError("device error")
+
+    monkeypatch.setattr(hashing, "_owed", {})
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: Stream())
+    word = torch.empty(1, dtype=torch.int64)
+    hashing._settle(word, "cuda")
+    assert [w is word for w in hashing._owed.values()] == [True]
+    hashing._owed.clear()
+    Stream.fails = False
+    hashing._settle(word, "cuda")
+    assert not hashing._owed
