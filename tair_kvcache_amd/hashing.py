@@ -93,7 +93,7 @@ def hash_tokens(tokens: torch.Tensor, block_size: int, token_offsets: Optional[t
         return _hash_and_count(tokens, off, R, block_size, seed, stream)
     if key_offsets is None:
         key_offsets = torch.empty(R + 1, dtype=torch.int64, device=tokens.device)
-        _launch_offsets(tokens, off, R, block_size, keys, key_offsets, None, stream)
+        _launch_offsets(tokens, off, R, block_size, keys.numel(), key_offsets, None, stream)
     if keys is None:
         total = int(key_offsets[-1].item())
         keys = torch.empty(total, dtype=torch.int64, device=tokens.device)
@@ -103,10 +103,10 @@ def hash_tokens(tokens: torch.Tensor, block_size: int, token_offsets: Optional[t
     return keys, key_offsets
 
 
-def _launch_offsets(tokens, off, R, block_size, keys, key_offsets, pending, stream):
+def _launch_offsets(tokens, off, R, block_size, n_keys, key_offsets, pending, stream):
     ws_bytes = lib().kvcm_hip_key_offsets_workspace_bytes(R)
     ws = torch.empty(ws_bytes // 8, dtype=torch.int64, device=tokens.device) if ws_bytes else None
-    rc = lib().kvcm_hip_key_offsets_checked(ptr(off), R, block_size, tokens.numel(), keys.numel(), ptr(ws), ws_bytes,
+    rc = lib().kvcm_hip_key_offsets_checked(ptr(off), R, block_size, tokens.numel(), n_keys, ptr(ws), ws_bytes,
                                             ptr(key_offsets), ptr(pending), stream)
     _lib.check(rc, "kvcm_hip_key_offsets_checked")
 
@@ -131,25 +131,38 @@ def _settle(word, device):
     del _owed[id(word)]
 
 
+# Keys up to which the buffer is allocated by what the token count bounds, before the number of keys is known: 256 MiB, a
+# thousandth of the device's memory, which the call needs for itself even if the offsets name few of the tokens. Waiting for
+# the number first costs 8 to 30 us: 2^22 keys of 16-token blocks 116 / 124 us, 2^23 218 / 227, 2^24 405 / 440.
+_KEYS_AHEAD = 1 << 25
+
+
 def _hash_and_count(tokens, off, R, block_size, seed, stream):
     """(keys, key_offsets) of R > 0 requests when the caller brings neither. The total is on its way to the host while the
     keys are being computed into a buffer of the size that the token count bounds: nobody waits for the hash kernel, and the
-    hash kernel waits for nobody."""
+    hash kernel waits for nobody. The keys returned own their bytes, and at most one key per request more (as many trailing
+    partial blocks as there are requests), however much of `tokens` the offsets leave out."""
     key_offsets = torch.empty(R + 1, dtype=torch.int64, device=tokens.device)
-    keys = torch.empty(tokens.numel() // block_size, dtype=torch.int64, device=tokens.device)
+    most = tokens.numel() // block_size
+    keys = torch.empty(most, dtype=torch.int64, device=tokens.device) if most <= _KEYS_AHEAD else None
     pending = torch.empty(1, dtype=torch.int64, pin_memory=True)
     try:
-        _launch_offsets(tokens, off, R, block_size, keys, key_offsets, pending, stream)
-        if keys.numel():
+        _launch_offsets(tokens, off, R, block_size, most, key_offsets, pending, stream)
+        if keys is not None and most:
             _launch_keys(tokens, off, R, block_size, seed, keys, key_offsets, stream)
         _lib.check(lib().kvcm_wait_value(ptr(pending), stream), "kvcm_wait_value")
     except BaseException:  # an interrupt as much as an error: the kernel may still be to come
         _settle(pending, tokens.device)
         raise
     total = pending.item()
-    if not 0 <= total <= keys.numel():
+    if not 0 <= total <= most:
         raise ValueError(f"token_offsets name blocks of {block_size} tokens beyond the {tokens.numel()} that tokens holds")
-    return keys[:total], key_offsets
+    if keys is None:
+        keys = torch.empty(total, dtype=torch.int64, device=tokens.device)
+        if total:
+            _launch_keys(tokens, off, R, block_size, seed, keys, key_offsets, stream)
+        return keys, key_offsets
+    return keys[:total] if most - total <= R else keys[:total].clone(), key_offsets
 
 
 def gen_key_vector(tokens, block_size: int, device=None) -> List[int]:

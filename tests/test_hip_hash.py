@@ -480,3 +480,23 @@ def test_the_word_a_kernel_has_yet_to_write_outlives_an_error(monkeypatch, fails
     with pytest.raises((_lib.KvcmError, KeyboardInterrupt)):
         h.hash_tokens(tok, 16, token_offsets=off)
     assert torch.cuda.current_stream().query() and not h._owed
+
+
+@pytest.mark.parametrize("spare,bs", [(0, 16), (15, 16), (100_000, 16), (100_000, 1), (1 << 24, 1), ((1 << 25) + 64, 1)])
+def test_keys_own_no_more_than_their_bytes(oracle, spare, bs):
+    """The key buffer does not grow with tokens that the offsets leave out, be they fewer or more than what is allocated for
+    before the number of keys is known."""
+    rng = np.random.default_rng(spare)
+    lens = rng.integers(0, 200, size=64)
+    toff = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    flat = rng.integers(0, 152064, size=int(toff[-1]), dtype=np.int64)
+    want, woff = oracle.hash_tokens(flat, bs, token_offsets=toff)
+    tok = torch.zeros(len(flat) + spare, dtype=torch.int64, device="cuda")
+    tok[:len(flat)] = dev(flat)
+    torch.cuda.synchronize()
+    keys, off = _h().hash_tokens(tok, bs, token_offsets=dev(toff))
+    sync()
+    assert (host(keys, np.int64) == want).all() and (host(off, np.int64) == woff).all()
+    assert keys.untyped_storage().nbytes() <= 8 * (len(want) + len(lens))
+    none, _ = _h().hash_tokens(tok, bs, token_offsets=torch.zeros(3, dtype=torch.int64, device="cuda"))
+    assert none.numel() == 0 and none.untyped_storage().nbytes() <= 16
