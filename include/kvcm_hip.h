@@ -121,7 +121,8 @@ int32_t kvcm_hip_key_offsets_checked(const int64_t *d_token_offsets, int32_t R, 
 
 /*
  * Blocks the calling thread until *h_value (pinned host memory that work on `stream` writes) is no longer KVCM_PENDING.
- * Ends with an error instead when the stream has failed, or has drained without writing it.
+ * Ends with an error instead when the stream has failed, or has drained without writing it, or is being captured into a
+ * graph (as kvcm_hip_key_offsets with h_total does there, before it launches anything).
  */
 int32_t kvcm_wait_value(const int64_t *h_value, kvcm_stream_t stream);
 

@@ -22,9 +22,6 @@
 // instruction issue of the chain wave, which no amount of bandwidth removes.
 #include "kvcm_internal.h"
 
-#include <sched.h>
-#include <time.h>
-
 #include <climits>
 
 namespace kvcm {
@@ -1223,37 +1220,6 @@ int32_t kvcm_hip_hash_tokens_2d(const void *d_tokens, int32_t token_bytes, int32
                                       d_key_offsets, static_cast<hipStream_t>(stream), uni);
 }
 
-// The value arrives a few microseconds after the kernel that writes it has started, so the thread looks for it without
-// sleeping at first (sleeping and being woken costs more than the wait), gives its core away between looks after a
-// while, and only then starts to ask the stream whether anything will still come.
-int32_t kvcm_wait_value(const int64_t *h_value, kvcm_stream_t stream) {
-    if (!h_value) {
-        return KVCM_ERR_INVALID_ARG;
-    }
-    const auto arrived = [h_value] { return __atomic_load_n(h_value, __ATOMIC_ACQUIRE) != KVCM_PENDING; };
-    for (int i = 0; i < 4096; ++i) {
-        if (arrived()) {
-            return KVCM_OK;
-        }
-        if (i >= 1024) {
-            sched_yield();
-        } else {
-            __builtin_ia32_pause();
-        }
-    }
-    for (;;) {
-        const hipError_t e = hipStreamQuery(static_cast<hipStream_t>(stream));
-        if (arrived()) {
-            return KVCM_OK;
-        }
-        if (e != hipErrorNotReady) {
-            return e == hipSuccess ? static_cast<int32_t>(hipErrorUnknown) : static_cast<int32_t>(e);
-        }
-        const struct timespec nap = {0, 20000};
-        nanosleep(&nap, nullptr);
-    }
-}
-
 int32_t kvcm_hip_hash_tokens_checked(const void *d_tokens, int32_t token_bytes, int64_t n_tokens,
                                      const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t seed,
                                      int64_t *d_keys, int64_t n_keys, const int64_t *d_key_offsets, kvcm_stream_t stream) {
@@ -1287,10 +1253,14 @@ int32_t kvcm_hip_key_offsets_checked(const int64_t *d_token_offsets, int32_t R, 
     if (reinterpret_cast<uintptr_t>(d_workspace) % 8 != 0) {
         return KVCM_ERR_ALIGNMENT;
     }
+    const hipStream_t s = static_cast<hipStream_t>(stream);
     if (h_total) {
+        // recorded into a graph the launch would write h_total at every replay, long after the caller has given it back
+        if (kvcm::is_capturing(s)) {
+            return static_cast<int32_t>(hipErrorStreamCaptureUnsupported);
+        }
         *h_total = KVCM_PENDING;
     }
-    const hipStream_t s = static_cast<hipStream_t>(stream);
     int64_t *sums = R > kvcm::kOffsetsRereadUpTo ? static_cast<int64_t *>(d_workspace) : nullptr;
     if (sums) {
         hipLaunchKernelGGL(kvcm::key_sums_kernel, dim3(static_cast<uint32_t>(groups)), dim3(kvcm::kOffsetsThreads), 0, s,

@@ -1,7 +1,10 @@
-// kvcm_host.hip -- the entry points of libkvcm_hip.so that are host code and nothing else: version, error text and the
-// per-block hash over iov CRCs. Kept apart from the kernels so that a plain host compiler can build this file (and
+// kvcm_host.hip -- the entry points of libkvcm_hip.so that are host code and nothing else: version, error text, the wait for
+// a value that a kernel writes into host memory, and the per-block hash over iov CRCs. Kept apart from the kernels so that a plain host compiler can build this file (and
 // kvcm_file.hip, kvcm_host_idx.h) for the sanitizer runs of tests/cpp/sanitize.
 #include "kvcm_internal.h"
+
+#include <sched.h>
+#include <time.h>
 
 extern "C" {
 
@@ -23,6 +26,40 @@ const char *kvcm_hip_error_string(int32_t code) {
             return "index out of range";
         default:
             return code > 0 ? hipGetErrorString(static_cast<hipError_t>(code)) : "unknown kvcm error";
+    }
+}
+
+// The value arrives a few microseconds after the kernel that writes it has started, so the thread looks for it without
+// sleeping at first (sleeping and being woken costs more than the wait), gives its core away between looks after a
+// while, and only then starts to ask the stream whether anything will still come.
+int32_t kvcm_wait_value(const int64_t *h_value, kvcm_stream_t stream) {
+    if (!h_value) {
+        return KVCM_ERR_INVALID_ARG;
+    }
+    const auto arrived = [h_value] { return __atomic_load_n(h_value, __ATOMIC_ACQUIRE) != KVCM_PENDING; };
+    for (int i = 0; i < 4096; ++i) {
+        if (arrived()) {
+            return KVCM_OK;
+        }
+        if (i == 0 && kvcm::is_capturing(static_cast<hipStream_t>(stream))) {  // nothing runs before the graph does
+            return static_cast<int32_t>(hipErrorStreamCaptureUnsupported);
+        }
+        if (i >= 1024) {
+            sched_yield();
+        } else {
+            __builtin_ia32_pause();
+        }
+    }
+    for (;;) {
+        const hipError_t e = hipStreamQuery(static_cast<hipStream_t>(stream));
+        if (arrived()) {
+            return KVCM_OK;
+        }
+        if (e != hipErrorNotReady) {
+            return e == hipSuccess ? static_cast<int32_t>(hipErrorUnknown) : static_cast<int32_t>(e);
+        }
+        const struct timespec nap = {0, 20000};
+        nanosleep(&nap, nullptr);
     }
 }
 

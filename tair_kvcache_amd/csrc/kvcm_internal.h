@@ -15,6 +15,13 @@ inline int32_t launch_status() {
     return e == hipSuccess ? KVCM_OK : static_cast<int32_t>(e);
 }
 
+// Whether work on `s` is being recorded into a graph. The null stream never is, and must not be asked: the question alone is
+// an error while another stream is being captured.
+inline bool is_capturing(hipStream_t s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return s && (hipStreamIsCapturing(s, &status) != hipSuccess || status != hipStreamCaptureStatusNone);
+}
+
 // One hashInt64Func step (kv_cache_manager/manager/hash_util.h:8-12) with the token term pre-added:
 // a = value + 0x9e3779b97f4a7c15. Unsigned arithmetic wraps mod 2^64; the right shift is arithmetic.
 __host__ __device__ inline uint64_t hash_step_preadded(uint64_t h, uint64_t a) {

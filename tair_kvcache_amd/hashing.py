@@ -142,6 +142,9 @@ def _hash_and_count(tokens, off, R, block_size, seed, stream):
     keys are being computed into a buffer of the size that the token count bounds: nobody waits for the hash kernel, and the
     hash kernel waits for nobody. The keys returned own their bytes, and at most one key per request more (as many trailing
     partial blocks as there are requests), however much of `tokens` the offsets leave out."""
+    if stream and torch.cuda.is_current_stream_capturing():
+        raise RuntimeError("hash_tokens with token_offsets waits for the number of keys, which a graph cannot: pass keys and "
+                           "key_offsets to capture it")
     key_offsets = torch.empty(R + 1, dtype=torch.int64, device=tokens.device)
     most = tokens.numel() // block_size
     keys = torch.empty(most, dtype=torch.int64, device=tokens.device) if most <= _KEYS_AHEAD else None

@@ -85,6 +85,8 @@ FakeStream *as_stream(hipStream_t s) { return s ? reinterpret_cast<FakeStream *>
 std::atomic<int> g_devices{1};
 std::atomic<long> g_live_allocs{0};
 thread_local int t_device = 0;
+std::atomic<int> g_query_result{hipErrorNotReady};
+std::atomic<bool> g_capturing{false};
 std::mutex g_hook_mu;
 std::function<void()> g_on_get_device;
 
@@ -96,6 +98,9 @@ void fake_hip_on_get_device(std::function<void()> fn) {
     std::lock_guard<std::mutex> lock(g_hook_mu);
     g_on_get_device = std::move(fn);
 }
+
+void fake_hip_set_query_result(int error) { g_query_result = error; }
+void fake_hip_set_capturing(bool on) { g_capturing = on; }
 
 void fake_hip_enqueue(void *stream, std::function<void()> job) {
     as_stream(static_cast<hipStream_t>(stream))->push(std::move(job));
@@ -162,6 +167,18 @@ hipError_t hipStreamDestroy(hipStream_t stream) {
 }
 hipError_t hipStreamSynchronize(hipStream_t stream) {
     as_stream(stream)->drain();
+    return hipSuccess;
+}
+hipError_t hipStreamQuery(hipStream_t stream) {
+    if (g_capturing.load()) {
+        std::abort();
+    }
+    FakeStream *s = as_stream(stream);
+    std::lock_guard<std::mutex> lock(s->mu);
+    return s->jobs.empty() && !s->busy ? hipSuccess : static_cast<hipError_t>(g_query_result.load());
+}
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *status) {
+    *status = g_capturing.load() ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
     return hipSuccess;
 }
 

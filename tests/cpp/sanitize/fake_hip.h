@@ -13,3 +13,8 @@ void fake_hip_on_get_device(std::function<void()> fn);
 // Queues `job` on a stream of the stand-in, behind whatever was queued before: how the stand-ins of the library's
 // kernel entry points (sanitize_host.cpp) do their work "on the device", in stream order.
 void fake_hip_enqueue(void *stream, std::function<void()> job);
+// What hipStreamQuery says of a stream that has something queued (default hipErrorNotReady), as an int; and whether
+// hipStreamIsCapturing says that a stream is being captured. hipStreamQuery on such a stream ends the process: on the real
+// runtime the question invalidates the capture.
+void fake_hip_set_query_result(int error);
+void fake_hip_set_capturing(bool on);

@@ -379,6 +379,44 @@ void buffer_check_pool_blocks_and_wakes() {
     std::puts("ok buffer-check pool: 8 threads on 2 cells; GenKeyVectors");
 }
 
+// kvcm_wait_value: the value at once, late (past the spinning), never, from a stream that has failed, and under capture.
+void wait_for_a_value() {
+    hipStream_t s = nullptr;
+    CHECK(hipStreamCreateWithFlags(&s, hipStreamNonBlocking) == hipSuccess);
+    int64_t value = 7;
+    CHECK(kvcm_wait_value(nullptr, s) == KVCM_ERR_INVALID_ARG);
+    CHECK(kvcm_wait_value(&value, s) == KVCM_OK);
+    for (int ms : {0, 1, 20}) {
+        value = KVCM_PENDING;
+        fake_hip_enqueue(s, [&value, ms] {
+            std::this_thread::sleep_for(std::chrono::milliseconds(ms));
+            __atomic_store_n(&value, int64_t{42}, __ATOMIC_RELEASE);
+        });
+        CHECK(kvcm_wait_value(&value, s) == KVCM_OK && value == 42);
+        CHECK(hipStreamSynchronize(s) == hipSuccess);
+    }
+    value = KVCM_PENDING;
+    CHECK(kvcm_wait_value(&value, s) == hipErrorUnknown);  // nothing queued that could write it
+    std::atomic<bool> release{false};
+    fake_hip_set_query_result(hipErrorIllegalAddress);
+    fake_hip_enqueue(s, [&release] {
+        while (!release.load()) {
+            std::this_thread::sleep_for(std::chrono::milliseconds(1));
+        }
+    });
+    CHECK(kvcm_wait_value(&value, s) == hipErrorIllegalAddress);
+    release = true;
+    fake_hip_set_query_result(hipErrorNotReady);
+    CHECK(hipStreamSynchronize(s) == hipSuccess);
+    fake_hip_set_capturing(true);
+    CHECK(kvcm_wait_value(&value, s) == hipErrorStreamCaptureUnsupported);
+    value = 3;
+    CHECK(kvcm_wait_value(&value, s) == KVCM_OK);  // there already: nothing to ask
+    fake_hip_set_capturing(false);
+    CHECK(hipStreamDestroy(s) == hipSuccess);
+    std::puts("ok waiting for a value: late, never, failed stream, captured stream");
+}
+
 }  // namespace
 
 int main() {
@@ -393,6 +431,7 @@ int main() {
     destroy_while_a_transfer_runs();
     copy_iovs_mixed();
     buffer_check_pool_blocks_and_wakes();
+    wait_for_a_value();
     CHECK(fake_hip_live_allocations() == 0);
     const std::string rm = "rm -rf " + g_dir;
     CHECK(std::system(rm.c_str()) == 0);

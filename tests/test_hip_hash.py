@@ -500,3 +500,34 @@ def test_keys_own_no_more_than_their_bytes(oracle, spare, bs):
     assert keys.untyped_storage().nbytes() <= 8 * (len(want) + len(lens))
     none, _ = _h().hash_tokens(tok, bs, token_offsets=torch.zeros(3, dtype=torch.int64, device="cuda"))
     assert none.numel() == 0 and none.untyped_storage().nbytes() <= 16
+
+
+def test_a_call_that_waits_is_refused_under_capture_before_it_launches_anything(oracle):
+    """Ragged offsets and no key buffer: the call would wait for a number that no graph delivers. It says so without spoiling
+    the capture; with keys and offsets of the caller's it is captured, and every replay hashes the tokens of the day."""
+    from tair_kvcache_amd import _lib
+    rng = np.random.default_rng(8)
+    lens = rng.integers(0, 300, size=70)
+    toff = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    tok, off = torch.zeros(int(toff[-1]), dtype=torch.int64, device="cuda"), dev(toff)
+    keys = torch.empty(len(tok) // 16, dtype=torch.int64, device="cuda")
+    word = torch.full((1,), 5, dtype=torch.int64, pin_memory=True)
+    _h().hash_tokens(tok, 16, token_offsets=off)
+    sync()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        with pytest.raises(RuntimeError, match="key_offsets"):
+            _h().hash_tokens(tok, 16, token_offsets=off)
+        stream = torch.cuda.current_stream().cuda_stream
+        rc = _lib.lib().kvcm_hip_key_offsets(off.data_ptr(), 70, 16, 1 << 40, keys.data_ptr(), word.data_ptr(), stream)
+        assert rc > 0 and word.item() == 5
+        word.fill_(-2**62)                                       # KVCM_PENDING
+        assert _lib.lib().kvcm_wait_value(word.data_ptr(), stream) > 0
+        _, koff = _h().hash_tokens(tok, 16, token_offsets=off, keys=keys)
+    for _ in range(3):
+        flat = rng.integers(0, 152064, size=len(tok), dtype=np.int64)
+        tok.copy_(dev(flat))
+        graph.replay()
+        sync()
+        want, woff = oracle.hash_tokens(flat, 16, token_offsets=toff)
+        assert (host(koff, np.int64) == woff).all() and (host(keys, np.int64)[:len(want)] == want).all()
