@@ -8,6 +8,7 @@
 // waiting for has finished is a data race that ThreadSanitizer sees, and a use after free that AddressSanitizer sees --
 // which is the point.
 #include <hip/hip_runtime_api.h>
+#include <sys/prctl.h>
 
 #include <atomic>
 #include <condition_variable>
@@ -87,6 +88,7 @@ std::atomic<long> g_live_allocs{0};
 thread_local int t_device = 0;
 std::atomic<int> g_query_result{hipErrorNotReady};
 std::atomic<bool> g_capturing{false};
+std::atomic<int> g_query_slack{-1};
 std::mutex g_hook_mu;
 std::function<void()> g_on_get_device;
 
@@ -101,6 +103,7 @@ void fake_hip_on_get_device(std::function<void()> fn) {
 
 void fake_hip_set_query_result(int error) { g_query_result = error; }
 void fake_hip_set_capturing(bool on) { g_capturing = on; }
+int fake_hip_timer_slack_of_last_query() { return g_query_slack.load(); }
 
 void fake_hip_enqueue(void *stream, std::function<void()> job) {
     as_stream(static_cast<hipStream_t>(stream))->push(std::move(job));
@@ -173,6 +176,7 @@ hipError_t hipStreamQuery(hipStream_t stream) {
     if (g_capturing.load()) {
         std::abort();
     }
+    g_query_slack = prctl(PR_GET_TIMERSLACK, 0, 0, 0, 0);
     FakeStream *s = as_stream(stream);
     std::lock_guard<std::mutex> lock(s->mu);
     return s->jobs.empty() && !s->busy ? hipSuccess : static_cast<hipError_t>(g_query_result.load());

@@ -18,3 +18,5 @@ void fake_hip_enqueue(void *stream, std::function<void()> job);
 // runtime the question invalidates the capture.
 void fake_hip_set_query_result(int error);
 void fake_hip_set_capturing(bool on);
+// The timer slack (ns) of the thread that called hipStreamQuery last.
+int fake_hip_timer_slack_of_last_query();

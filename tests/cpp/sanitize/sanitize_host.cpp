@@ -10,6 +10,7 @@
 // Scenarios: the oracle's threaded forms; the index-list walk against brute force; block files with host iovs and
 // with device iovs from 16 concurrent callers; a big get shared among helper threads; a store destroyed while a get
 // or a put is still inside it; the blocking cell pool of the buffer check with more threads than cells.
+#include <sys/prctl.h>
 #include <unistd.h>
 
 #include <atomic>
@@ -395,6 +396,17 @@ void wait_for_a_value() {
         CHECK(kvcm_wait_value(&value, s) == KVCM_OK && value == 42);
         CHECK(hipStreamSynchronize(s) == hipSuccess);
     }
+    // a nap lasts what it says, not that and the thread's timer slack; the slack is the thread's own again afterwards
+    CHECK(prctl(PR_SET_TIMERSLACK, 70000, 0, 0, 0) == 0);
+    value = KVCM_PENDING;
+    fake_hip_enqueue(s, [&value] {
+        std::this_thread::sleep_for(std::chrono::milliseconds(50));
+        __atomic_store_n(&value, int64_t{42}, __ATOMIC_RELEASE);
+    });
+    CHECK(kvcm_wait_value(&value, s) == KVCM_OK && value == 42);
+    CHECK(fake_hip_timer_slack_of_last_query() == 1 && prctl(PR_GET_TIMERSLACK, 0, 0, 0, 0) == 70000);
+    CHECK(prctl(PR_SET_TIMERSLACK, 0, 0, 0, 0) == 0);  // the default again
+    CHECK(hipStreamSynchronize(s) == hipSuccess);
     value = KVCM_PENDING;
     CHECK(kvcm_wait_value(&value, s) == hipErrorUnknown);  // nothing queued that could write it
     std::atomic<bool> release{false};
