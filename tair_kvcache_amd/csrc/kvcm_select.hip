@@ -72,10 +72,18 @@ __device__ inline int32_t table_load(const int32_t *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Keys from which a probe looks at its slot before it tries to claim it. First occurrences, claim at once / look first, us:
-// all keys different 65 536: 22.7 / 23.4  262 144: 41.2 / 42.6  2^20: 117.7 / 105.7; every key eight times 65 536: 11.3 / 13.6
-// 262 144: 22.1 / 24.6  2^20: 61.8 / 41.9. The save list of 262 144: 39.1 / 47.6, of 2^20: 101.3 / 97.1.
-constexpr int32_t kLookFirstFrom = 1 << 18;
+// Keys beyond which a probe looks at its slot before it tries to claim it. Claim at once / look first, us:
+//                            2^16         2^18         5 * 2^16     3 * 2^17     2^19         2^20
+// first, all different   26.4 / 25.1  44.5 / 44.0  42.0 / 50.3  46.9 / 47.2  71.9 / 65.6  117.0 / 105.2
+// first, each 8 times    11.8 / 13.7  21.2 / 23.7  26.3 / 29.8  28.9 / 32.1  35.3 / 31.7   62.4 / 42.2
+// list, all different    18.4 / 18.7  36.0 / 45.1  43.8 / 54.5  52.6 / 49.4  64.1 / 58.8  100.2 / 98.3
+// list, each 8 times     14.1 / 15.1  24.5 / 26.7  28.3 / 32.0  31.9 / 35.5  38.8 / 34.8   70.5 / 49.3
+// The columns of 2^16 and 2^18 keys are at two slots per key for first occurrences, four for the list. In a table that full
+// (less than 2.5 slots per key) claims that fail cost more than looks from 2^17 keys on where keys are different: 2^18 of them
+// 42.5 to 49.8 / 41.6 to 46, by their values.
+constexpr int64_t kLookFirstBeyond = 3 << 17;
+constexpr int64_t kLookFirstBeyondFull = 1 << 17;
+bool look_first(int64_t n, int64_t slots) { return n > (2 * slots < 5 * n ? kLookFirstBeyondFull : kLookFirstBeyond); }
 
 // Open addressing, linear probing, one int32 per slot: -1 = empty, otherwise an index whose key owns the slot.
 // A slot claimed for key K is only ever lowered (atomicMin) by indices that hold the same K, so whatever index a
@@ -288,9 +296,13 @@ int64_t table_capacity(int64_t n) {
     return cap;
 }
 
-// Slots of the table of one list: four to eight per key. Every probe is two trips to memory one after the other, and the launch
-// lasts as long as its unluckiest key.
-int64_t list_capacity(int64_t n) { return 2 * table_capacity(n); }
+// Slots of the table of one list. Up to 2^18 keys four to eight per key: every probe is two trips to memory one after the
+// other, and the launch lasts as long as its unluckiest key. Beyond, 2.5 to 5 per key: the table no longer lies in the caches,
+// and clearing it counts as well (three / six slots per key: 327 680 keys 43.8 / 50, 655 360 70.8 / 71.5 us).
+int64_t list_capacity(int64_t n) {
+    const int64_t cap = table_capacity(n);
+    return n <= int64_t{1} << 18 || 2 * cap < 5 * n ? 2 * cap : cap;
+}
 
 // An empty table of `cap` slots (a power of two, >= 2 n) and the keys into it; the fill is a kernel, so the sequence may be
 // recorded into a graph.
@@ -301,7 +313,7 @@ void launch_insert(const int64_t *d_keys, int32_t n, int32_t *table, int64_t cap
     }
     fill_i32_kernel<<<static_cast<unsigned>(cap / 256), 256, 0, s>>>(table, cap, -1);
     insert_kernel<<<(static_cast<unsigned>(n) + 255) / 256, 256, 0, s>>>(d_keys, n, table, static_cast<uint32_t>(cap - 1), 64 - log2cap,
-                                                                       slot_of, n > kLookFirstFrom);
+                                                                       slot_of, look_first(n, cap));
 }
 
 int32_t launch_first_occurrence(const int64_t *d_keys, int64_t n, int32_t *table, int64_t cap, int32_t *d_first_idx,

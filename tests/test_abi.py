@@ -78,6 +78,16 @@ def test_argument_validation_needs_no_device():
     assert offsets(p, 32769, 16, 1, 1, p, 39, p, None, None) == _lib.ERR_INVALID_ARG  # workspace too small
     assert offsets(p, 1, 16, 1, 1, p + 4, 8, p, None, None) == _lib.ERR_ALIGNMENT
     assert L.kvcm_hip_key_offsets_workspace_bytes(32768) == 0 and L.kvcm_hip_key_offsets_workspace_bytes(32769) == 5 * 8
+    # the table of a save list: a power of two, two slots per key at least (a probe must meet an empty one), eight at most
+    for n in [1, 512, 513, 1 << 18, (1 << 18) + 1, 3 << 17, 419430, 419431, 1 << 19, (1 << 19) + 1, 838861, 1 << 20]:
+        slots = (L.kvcm_hip_select_save_workspace_bytes(n) - (n + 255) // 256 * 36) // 4 - n
+        assert slots & (slots - 1) == 0 and 2 * n <= slots and (slots <= 8 * n or slots == 2048), (n, slots)
+    assert L.kvcm_hip_select_save_workspace_bytes((1 << 20) + 1) == _lib.ERR_TOO_LARGE
+    save = L.kvcm_hip_select_save
+    assert save(p, None, 0, p, 1 << 20, p, p, None) == _lib.ERR_INVALID_ARG
+    assert save(p, None, 1, p, 8, p, p, None) == _lib.ERR_INVALID_ARG  # workspace too small
+    assert save(p, None, 1, p + 4, 1 << 20, p, p, None) == _lib.ERR_ALIGNMENT
+    assert save(p, None, (1 << 20) + 1, p, 1 << 40, p, p, None) == _lib.ERR_TOO_LARGE
     assert L.kvcm_hip_sha256_first8_be(None, None, 0, None, None) == _lib.OK
     assert L.kvcm_hip_iov_crc32(None, 1, None, 4, None) == _lib.ERR_INVALID_ARG
     assert L.kvcm_hip_generate_blocks_idx(p, 1, p, 1, 0, 16, p, None, None) == _lib.ERR_INVALID_ARG

@@ -174,3 +174,20 @@ def test_save_list_of_a_batch_is_that_of_the_two_operators(oracle, n, distinct, 
     if d_mask is not None and n > 1:
         with pytest.raises(ValueError):
             save_selection.select_save_indices(d_keys, d_mask[1:])
+
+
+@pytest.mark.parametrize("n", [1 << 17, (1 << 17) + 1, 209715, 209716, 1 << 18, (1 << 18) + 1, 3 << 17, (3 << 17) + 1, 419430, 419431])
+@pytest.mark.parametrize("each", [1, 8])
+def test_first_occurrences_where_table_and_probes_change(oracle, n, each):
+    """The numbers of keys at which the table of a list changes its size and probes begin to look before they claim."""
+    from tair_kvcache_amd import save_selection
+    keys = _keys_with_repeats(np.random.default_rng(n + each), n, n // each)
+    first, rep = oracle.first_occurrence(keys)
+    d_keys = torch.from_numpy(keys).cuda()
+    print(f"first occurrences n={n} each={each}", flush=True)
+    got_first, got_rep = save_selection.first_occurrence(d_keys)
+    idx, count = save_selection.select_save_indices(d_keys)
+    sync()
+    assert (got_first.cpu().numpy() == first).all() and (got_rep.cpu().numpy() == rep.astype(bool)).all()
+    want = np.flatnonzero(rep == 0)
+    assert int(count.item()) == len(want) and (idx[:len(want)].cpu().numpy() == want).all()
