@@ -627,12 +627,13 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
             start = start < 0 && have.tokens != kUnknown ? 0 : start;
             if (r < R) {
                 const int64_t at = token_offsets[r], n = distance(at, token_offsets[r + 1]);
-                const int64_t nkeys = n / block_size;  // a trailing partial block yields no key
-                key_pos = key_offsets ? key_offsets[r] : r * (distance(token_offsets[0], token_offsets[1]) / block_size);
-                if (inside(key_pos, nkeys, have.keys) &&
-                    (have.tokens == kUnknown || inside(at, nkeys * block_size, have.tokens))) {
+                // a division by a constant where there is one: by a variable it takes longer than the loads in front of it
+                const int32_t bs = BS > 0 ? BS : block_size;
+                const int64_t nkeys = n / bs;  // a trailing partial block yields no key
+                key_pos = key_offsets ? key_offsets[r] : r * (distance(token_offsets[0], token_offsets[1]) / bs);
+                if (inside(key_pos, nkeys, have.keys) && (have.tokens == kUnknown || inside(at, nkeys * bs, have.tokens))) {
                     start = at;
-                    my_ntok = nkeys * block_size;
+                    my_ntok = nkeys * bs;
                 }
             }
         } else {
