@@ -1077,6 +1077,44 @@ constexpr int32_t burst_from(int32_t block_size, bool tokens_8_byte) {
         default: return INT32_MAX;
     }
 }
+// Tokens per request from which such a launch does: the last group leaves after the last token, so staging costs about 1 us
+// more than direct stores and has to earn that first. Lengths are known for [R, L] batches, their mean where the caller has
+// said how many tokens there are; otherwise requests are taken for long. us, staged / direct, at 8192 requests (2048 for 8-token
+// blocks, 4096 for 128; 4-byte tokens 12 288):
+//   equally long        64       256        512        768        1024       1536       2048       4096
+//   bs 8,   8 bytes  5.5/4.5   9.2/8.2   12.6/11.7  16.4/16.7  19.4/19.9  26.5/30.4  33.0/34.5  60.2/64.7
+//   bs 16,  8 bytes  5.4/4.4   9.5/8.6   13.5/13.1  16.5/17.1  19.2/20.2  27.9/30.8  32.4/35.9  60.0/69.3
+//   bs 32,  8 bytes  5.6/4.6   9.5/8.6   13.6/13.0  16.3/16.2  19.4/19.8  26.3/28.3  31.3/34.2  57.9/64.8
+//   bs 64,  8 bytes  6.1/5.0   9.5/8.4   13.5/12.8  16.3/16.1  19.2/19.6  26.3/28.0  31.2/33.7  55.8/61.5
+//   bs 128, 8 bytes  3.5/3.6   9.0/8.1   12.5/11.9  15.5/15.1  18.5/18.3  24.0/25.0  29.5/30.1  52.1/54.9
+//   bs 8,   4 bytes  6.1/4.2   9.1/7.7   12.8/11.4  17.1/15.4  20.9/19.8  27.1/27.1  34.1/35.6  59.3/73.5
+//   bs 16,  4 bytes  6.2/4.3   9.0/7.5   12.8/10.9  16.8/14.0  20.1/18.4  26.2/24.6  33.1/33.3  56.8/65.7
+//   bs 32,  4 bytes  6.4/4.4   8.9/7.4   12.8/10.8  16.8/13.8  20.4/17.7  26.0/22.9  32.8/32.1  56.4/65.3
+//   bs 64,  4 bytes  6.5/4.4   8.9/7.3   12.7/10.6  16.8/13.6  20.4/17.0  26.1/22.5  32.9/31.3  56.0/63.2
+//   bs 128, 4 bytes  3.3/3.3   8.9/7.4   12.7/10.5  16.8/13.5  20.2/16.9  25.8/22.3  32.7/30.7  56.1/61.1
+//   ragged            16..64   64..512   64..768    64..1024   256..1024  64..2048   512..1536  64..4096   1024..2048 500..4096
+//   (mean)              35       215       283        346        554        573        932        969        1477       1710
+//   bs 8,   8 bytes  6.6/4.4  12.9/12.4  16.7/16.3  19.7/19.7  20.3/21.4  34.0/35.3  27.6/31.7  61.3/66.1  34.9/41.9  62.0/73.2
+//   bs 16,  8 bytes  7.9/4.5  14.3/13.0  17.5/17.2  20.6/21.0  20.8/22.7  33.8/36.7  29.2/32.3  61.2/68.1  36.0/42.3  64.9/76.3
+//   bs 32,  8 bytes  5.6/4.4  14.5/12.8  17.4/16.4  20.3/19.9  20.6/21.0  31.8/34.2  27.4/29.3  58.6/63.4  34.5/37.7  62.4/68.3
+//   bs 64,  8 bytes  5.4/4.3  14.7/12.2  17.9/15.8  20.2/19.1  20.3/19.8  32.0/33.1  26.8/27.5  57.4/61.8  33.8/35.7  60.6/64.8
+//   bs 128, 8 bytes  3.5/3.6  12.7/11.1  15.7/14.4  18.6/17.8  18.8/18.5  29.7/29.9  24.8/25.5  51.8/56.2  30.6/32.3  53.5/58.9
+//   bs 8,   4 bytes  8.6/4.2  14.1/11.8  16.8/15.6  20.6/19.3  21.7/20.2  34.0/33.5  28.3/28.7  59.3/62.0  35.4/37.9  60.2/67.6
+//   bs 16,  4 bytes  9.1/4.2  13.9/11.3  17.4/14.6  20.8/17.7  21.5/18.1  33.0/30.6  27.4/25.7  57.2/56.0  33.3/33.7  58.6/60.3
+//   bs 32,  4 bytes  6.3/4.4  14.1/11.0  17.7/14.2  20.9/17.3  21.2/17.6  32.3/29.8  27.8/24.3  57.7/54.1  34.0/31.7  58.4/56.7
+//   bs 64,  4 bytes  6.1/4.1  15.0/10.6  18.3/13.4  21.0/16.4  21.5/16.8  32.3/28.0  27.5/22.9  55.6/51.6  33.5/29.0  56.5/52.8
+//   bs 128, 4 bytes  3.3/3.3  14.2/10.3  17.6/13.0  20.2/16.2  20.7/16.8  32.0/27.5  26.5/22.7  54.7/50.5  32.2/28.6  55.2/51.6
+//   Four times as many requests move the lines little (4-byte tokens, 32 768 requests of 2000 to 8192: bs 64 215/248, 128 208/222).
+constexpr int64_t burst_from_tokens(int32_t block_size, bool tokens_8_byte, bool equally_long) {
+    switch (block_size) {
+        case 8: return tokens_8_byte ? (equally_long ? 512 : 320) : equally_long ? 1280 : 640;
+        case 16: return tokens_8_byte ? (equally_long ? 640 : 320) : equally_long ? 1792 : 1024;
+        case 32: return tokens_8_byte ? (equally_long ? 896 : 560) : equally_long ? 1792 : 1600;
+        case 64: return tokens_8_byte ? 896 : 2304;
+        case 128: return tokens_8_byte ? 960 : 2560;
+        default: return 0;
+    }
+}
 #ifndef KVCM_HASH_BURST_SCALE  // for experiments: 0 = burst wherever it exists, a large number = never
 #define KVCM_HASH_BURST_SCALE 1
 #endif
@@ -1101,8 +1139,13 @@ int32_t launch_hash(const TokT *d_tokens, const int64_t *d_token_offsets, int32_
                        d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, have, \
                        force_global)
     constexpr bool k8 = sizeof(TokT) == 8;
-    const bool burst = R >= static_cast<int64_t>(burst_from(block_size, k8)) * KVCM_HASH_BURST_SCALE;
-    const bool spread = block_size == 16 && k8 && !burst && R >= KVCM_HASH_SPREAD_FROM_8;
+    const bool many = R >= static_cast<int64_t>(burst_from(block_size, k8)) * KVCM_HASH_BURST_SCALE;
+    const int64_t tokens_per_request = !d_token_offsets ? uni.tokens : have.tokens == kUnknown ? kUnknown : have.tokens / R;
+    // Block size 1, 4-byte tokens, staged / direct: 64 requests of 64 tokens 4.9 / 4.3 us, of 128: 6.2 / 5.3, of 16 to 64: 5.4 / 5.2,
+    // of 64 to 512: 14.6 / 19.4; 2048 of 128: 6.5 / 5.9; 16 384 of 128: 7.1 / 10.8.
+    const bool burst = many && (block_size == 1 ? k8 || R > 2048 || tokens_per_request > 128
+                                                : tokens_per_request >= burst_from_tokens(block_size, k8, !d_token_offsets));
+    const bool spread = block_size == 16 && k8 && !many && R >= KVCM_HASH_SPREAD_FROM_8;
 #define KVCM_LAUNCH_HASH_STAGED(CHUNK, BS, KS)                                                                       \
     hipLaunchKernelGGL((hash_tokens_kernel<TokT, CHUNK, BS, KS>), grid, dim3(kThreads), 0, stream, d_tokens,        \
                        d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, have, \

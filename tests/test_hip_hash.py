@@ -531,3 +531,35 @@ def test_a_call_that_waits_is_refused_under_capture_before_it_launches_anything(
         sync()
         want, woff = oracle.hash_tokens(flat, 16, token_offsets=toff)
         assert (host(koff, np.int64) == woff).all() and (host(keys, np.int64)[:len(want)] == want).all()
+
+
+@pytest.mark.parametrize("dtype,bs,R,mean", [
+    (np.int64, 8, 2048, 320), (np.int64, 16, 8192, 320), (np.int64, 32, 8192, 560), (np.int64, 64, 8192, 896),
+    (np.int64, 128, 4096, 960), (np.int32, 8, 12288, 640), (np.int32, 16, 12288, 1024), (np.int32, 32, 12288, 1600),
+    (np.int32, 64, 12288, 2304), (np.int32, 128, 12288, 2560), (np.int32, 1, 64, 129), (np.int32, 1, 2049, 129)])
+def test_mean_lengths_on_both_sides_of_the_staging_rule(oracle, dtype, bs, R, mean):
+    """Thousands of requests are staged from a mean length on: one token less, and exactly that many, from requests that are
+    empty, shorter than a block, around a tile and several tiles long, in whatever workgroup. Spare key slots stay untouched."""
+    rng = np.random.default_rng(bs + R)
+    R += 9                                                     # the last workgroup is partial
+    for n_tokens in (mean * R - 1, mean * R):
+        menu = np.array([0, 1, bs - 1, bs, 63, 64, 65, 127, 128, 129, mean, 2 * mean, 3 * mean + 5])
+        lens = menu[rng.integers(0, len(menu), size=R)].astype(np.int64)
+        lens[:64] = 0                                          # a workgroup without a block
+        short = n_tokens - int(lens.sum())                     # brought to the wanted sum a little at a time
+        step = np.sign(short) * rng.integers(0, 2 * mean, size=R)
+        step[:64] = 0
+        done = np.cumsum(np.abs(np.maximum(step, -lens)))
+        lens += np.where(done <= abs(short), np.maximum(step, -lens), 0)
+        lens[-1] += max(0, n_tokens - int(lens.sum()))
+        lens[np.argmax(lens)] += n_tokens - int(lens.sum())
+        assert lens.sum() == n_tokens and lens.min() >= 0
+        toff = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+        flat = rng.integers(-2**31, 2**31, size=n_tokens, dtype=np.int64).astype(dtype)
+        want, woff = oracle.hash_tokens(flat, bs, token_offsets=toff, seed=7, threads=8)
+        print(f"staging rule: bs={bs} {np.dtype(dtype).name} {R} requests, {n_tokens} tokens", flush=True)
+        keys = torch.full((len(want) + 64,), -7, dtype=torch.int64, device="cuda")
+        _h().hash_tokens(dev(flat), bs, token_offsets=dev(toff), seed=7, keys=keys, key_offsets=dev(woff))
+        sync()
+        got = host(keys, np.int64)
+        assert (got[:len(want)] == want).all() and (got[len(want):] == -7).all()
