@@ -338,6 +338,15 @@ constexpr int kKeysDirect = 0, kKeysSpread = 1, kKeysBurst = 2;
 // A workgroup of a spread kernel whose requests are shorter than this many tiles stores its keys directly: what the last
 // group costs after the loop (about 1.5 us) is more than staging saves on 2048 tokens.
 constexpr int kSpreadFromTiles = 32;
+// Block size 1, 8-byte elements (the prefix chain): a workgroup of few or short equally long requests stores its keys directly
+// too, because a store takes the longer the more lanes it has, and a small launch leaves the memory to it. Direct / staged, us:
+// 4096 digests each, 31 requests 78 / 97, 32: 80 / 93, 48: 106 / 89, 64: 146 / 86; 64 requests of 64 digests 4.4 / 5.4, of 256:
+// 7.9 / 9.2, 512: 13.7 / 14.2, 1024: 24.0 / 24.0; 2048 requests of 256: 10.4 / 10.4, of 512: 19.2 / 16.1. Where requests end at
+// different places staging pays from two of them on: 4 requests of 64 to 512 digests 21.8 / 16.2, of 64 to 4096 155 / 100 --
+// unless nobody fills a tile: 32 of 4 to 64 digests 5.5 / 5.9, 1000 of them 5.8 / 6.2.
+__device__ __forceinline__ bool chain_stays_direct(uint32_t requests, uint32_t workgroups, uint32_t ntiles, uint32_t whole) {
+    return whole + 1 >= ntiles ? requests <= 32 || (ntiles <= 8 && workgroups <= 16) || whole == 0 : false;
+}
 
 // The steps [first_step, kDrainSteps) of a group that belong to loader `me` (step % kLoaders == me), all LDS reads
 // under way before the first store: nothing else is left to do when this runs, so round trips would add up.
@@ -434,7 +443,7 @@ __device__ __forceinline__ void run_loader(const LoaderCtx<TokT> &ctx, uint64_t 
             }
         }
         was_mine = mine;
-        if (KS == kKeysBurst && ((k & (G - 1)) == G - 1 || k == nt - 1) && turn != me) {
+        if (KS == kKeysBurst && staged && ((k & (G - 1)) == G - 1 || k == nt - 1) && turn != me) {
             // The barrier above closed a group of G tiles, or what there is of the last one. The loader whose tile is due
             // next leaves it alone (its next wait for memory would wait for these stores as well); the other two write half
             // of it each.
@@ -690,7 +699,12 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
     // tiles [0, n_full) are those in which no request has run out of tokens
     const int32_t n_full = static_cast<int32_t>(full_u < ntiles_u ? full_u : ntiles_u);
     // whether this workgroup's keys are staged
-    const bool staged = KS == kKeysBurst || (KS == kKeysSpread && ntiles_u >= static_cast<uint32_t>(kSpreadFromTiles));
+    const bool staged =
+        KS == kKeysSpread  ? ntiles_u >= static_cast<uint32_t>(kSpreadFromTiles)
+        : KS != kKeysBurst ? false
+        : BS == 1 && sizeof(TokT) == 8
+            ? !chain_stays_direct(static_cast<uint32_t>(R - r_first < kReqs ? R - r_first : kReqs), gridDim.x, ntiles_u, full_u)
+            : true;
     if (wave != 0) {
         // ---------------------------------------------------------------- loader waves
         const KeyDrain kd{s_keys, s_keyrow, keys};
@@ -1053,6 +1067,7 @@ constexpr int32_t kForceGeneralLoader = KVCM_TEST_FORCE_GENERAL_LOADER;
 //                                   burst  4096: 58 / -   8192: 58 / 61  12 288: 60 / -      (raw tiles, see below)
 // Other block sizes, direct / burst:
 //   block size 1, 8-byte tokens   16: 76 / 101 and 149 / 105   32: 87 / 97 and 151 / 105   64: 143 / 89 and 156 / 105   8192: 246 / 115
+//                                 (one kernel for all, which chooses by workgroup: chain_stays_direct)
 //                 4-byte tokens   32: 75 / -   64: 107 / 82 and 146 / 93   1024: 113 / 83   8192: 174 / 96
 //   block size 8, 8-byte tokens   1024: 66 / 62 (of 512 tokens: 14.7 / 15.6)   2048: 68 / 63   8192: 89 / 69   12 288: 104 / 88
 //                 4-byte tokens   8192: 66 / 61 (of 1024 tokens: 20.6 / 23.2)  12 288: 80 / 62
@@ -1068,7 +1083,7 @@ constexpr int32_t kForceGeneralLoader = KVCM_TEST_FORCE_GENERAL_LOADER;
 // requests from which a launch takes the burst form; INT32_MAX = never
 constexpr int32_t burst_from(int32_t block_size, bool tokens_8_byte) {
     switch (block_size) {
-        case 1: return tokens_8_byte ? 32 : 64;
+        case 1: return tokens_8_byte ? 1 : 64;
         case 8: return tokens_8_byte ? 2048 : 12288;
         case 16: return tokens_8_byte ? 8192 : 12288;
         case 32: return tokens_8_byte ? 8192 : 12288;
@@ -1215,7 +1230,9 @@ int32_t launch_hash(const TokT *d_tokens, const int64_t *d_token_offsets, int32_
             KVCM_LAUNCH_HASH(8, 128);
         }
     } else if (block_size == 1) {  // the prefix chain over digests: a key after every step
-        if (burst) {
+        if constexpr (k8) {
+            KVCM_LAUNCH_HASH_STAGED(1, 1, kKeysBurst);
+        } else if (burst) {
             KVCM_LAUNCH_HASH_STAGED(1, 1, kKeysBurst);
         } else {
             KVCM_LAUNCH_HASH(1, 1);

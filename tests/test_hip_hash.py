@@ -563,3 +563,22 @@ def test_mean_lengths_on_both_sides_of_the_staging_rule(oracle, dtype, bs, R, me
         sync()
         got = host(keys, np.int64)
         assert (got[:len(want)] == want).all() and (got[len(want):] == -7).all()
+
+
+@pytest.mark.parametrize("dtype", [np.int64, np.int32])
+@pytest.mark.parametrize("R", [1, 2, 31, 32, 33, 63, 64, 65, 1024, 1025])
+def test_block_size_1_equally_long_and_ragged(oracle, dtype, R):
+    """A key per token: few or short equally long requests are stored by the chain wave itself, others staged; around 32
+    requests of a workgroup, 16 workgroups and 8 tiles, with lengths that end inside a tile."""
+    rng = np.random.default_rng(R)
+    for length in (1, 63, 64, 65, 448, 511, 512, 513, 576, 600):
+        for spread in (0, 1, 70, length):
+            lens = np.maximum(0, length - rng.integers(0, spread + 1, size=R)).astype(np.int64)
+            toff = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+            flat = rng.integers(-2**31, 2**31, size=max(int(toff[-1]), 1), dtype=np.int64).astype(dtype)
+            want, woff = oracle.hash_tokens(flat, 1, token_offsets=toff, seed=7, threads=8)
+            keys = torch.full((len(want) + 64,), -7, dtype=torch.int64, device="cuda")
+            _h().hash_tokens(dev(flat), 1, token_offsets=dev(toff), seed=7, keys=keys, key_offsets=dev(woff))
+            sync()
+            got = host(keys, np.int64)
+            assert (got[:len(want)] == want).all() and (got[len(want):] == -7).all(), (length, spread)
