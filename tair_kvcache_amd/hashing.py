@@ -27,12 +27,14 @@ except ImportError:  # host-side convenience only: the strings then go through P
 def _require_offsets(t, name, device, entries=None):
     """Offsets are read by the kernel as they are: int64, 1-D, on the tokens' device, R+1 entries."""
     require_cuda(t, name)
-    if t.dtype != torch.int64 or t.dim() != 1 or t.numel() < 1:
+    n = t.numel()
+    if t.dtype != torch.int64 or t.dim() != 1 or n < 1:
         raise ValueError(f"{name} must be a 1-D int64 tensor of R+1 entries")
     if t.device != device:
         raise ValueError(f"{name} is on {t.device}, the tokens on {device}")
-    if entries is not None and t.numel() != entries:
-        raise ValueError(f"{name} has {t.numel()} entries, expected {entries}")
+    if entries is not None and n != entries:
+        raise ValueError(f"{name} has {n} entries, expected {entries}")
+    return n
 
 
 def hash_tokens(tokens: torch.Tensor, block_size: int, token_offsets: Optional[torch.Tensor] = None,
@@ -61,9 +63,8 @@ def hash_tokens(tokens: torch.Tensor, block_size: int, token_offsets: Optional[t
         R = tokens.shape[0]
         total = R * (tokens.shape[1] // block_size)
     else:
-        _require_offsets(token_offsets, "token_offsets", tokens.device)
+        R, total = _require_offsets(token_offsets, "token_offsets", tokens.device) - 1, None
         off = token_offsets.contiguous()
-        R, total = off.numel() - 1, None
     if key_offsets is not None:
         _require_offsets(key_offsets, "key_offsets", tokens.device, R + 1)
         key_offsets = key_offsets.contiguous()
@@ -104,17 +105,21 @@ def hash_tokens(tokens: torch.Tensor, block_size: int, token_offsets: Optional[t
 
 
 def _launch_offsets(tokens, off, R, block_size, n_keys, key_offsets, pending, stream):
-    ws_bytes = lib().kvcm_hip_key_offsets_workspace_bytes(R)
-    ws = torch.empty(ws_bytes // 8, dtype=torch.int64, device=tokens.device) if ws_bytes else None
-    rc = lib().kvcm_hip_key_offsets_checked(ptr(off), R, block_size, tokens.numel(), n_keys, ptr(ws), ws_bytes,
-                                            ptr(key_offsets), ptr(pending), stream)
-    _lib.check(rc, "kvcm_hip_key_offsets_checked")
+    ws, ws_bytes = None, 0
+    if R > 32768:  # fewer need no workspace
+        ws_bytes = lib().kvcm_hip_key_offsets_workspace_bytes(R)
+        ws = torch.empty(ws_bytes // 8, dtype=torch.int64, device=tokens.device)
+    rc = lib().kvcm_hip_key_offsets_checked(off.data_ptr(), R, block_size, tokens.numel(), n_keys, ptr(ws), ws_bytes,
+                                            key_offsets.data_ptr(), ptr(pending), stream)
+    if rc:
+        _lib.check(rc, "kvcm_hip_key_offsets_checked")
 
 
 def _launch_keys(tokens, off, R, block_size, seed, keys, key_offsets, stream):
-    rc = lib().kvcm_hip_hash_tokens_checked(ptr(tokens), tokens.element_size(), tokens.numel(), ptr(off), R, block_size,
-                                            int(seed), ptr(keys), keys.numel(), ptr(key_offsets), stream)
-    _lib.check(rc, "kvcm_hip_hash_tokens_checked")
+    rc = lib().kvcm_hip_hash_tokens_checked(tokens.data_ptr(), tokens.element_size(), tokens.numel(), off.data_ptr(), R,
+                                            block_size, int(seed), keys.data_ptr(), keys.numel(), key_offsets.data_ptr(), stream)
+    if rc:
+        _lib.check(rc, "kvcm_hip_hash_tokens_checked")
 
 
 # Pinned words that a launched kernel has yet to write and nobody waits for any more. torch's pinned-memory pool knows
@@ -153,7 +158,9 @@ def _hash_and_count(tokens, off, R, block_size, seed, stream):
         _launch_offsets(tokens, off, R, block_size, most, key_offsets, pending, stream)
         if keys is not None and most:
             _launch_keys(tokens, off, R, block_size, seed, keys, key_offsets, stream)
-        _lib.check(lib().kvcm_wait_value(ptr(pending), stream), "kvcm_wait_value")
+        rc = lib().kvcm_wait_value(pending.data_ptr(), stream)
+        if rc:
+            _lib.check(rc, "kvcm_wait_value")
     except BaseException:  # an interrupt as much as an error: the kernel may still be to come
         _settle(pending, tokens.device)
         raise
@@ -187,17 +194,19 @@ def apply_prefix_hash(hash_ids: torch.Tensor, offsets: Optional[torch.Tensor] = 
     require_cuda(hash_ids, "hash_ids")
     if hash_ids.dtype != torch.int64:
         raise ValueError("hash_ids must be int64")
-    ids = hash_ids.contiguous().reshape(-1)
+    ids, device = hash_ids.contiguous(), hash_ids.device
+    n, R = ids.numel(), 1
     if offsets is None:
-        offsets = torch.tensor([0, ids.numel()], dtype=torch.int64, device=ids.device)
+        offsets = torch.tensor([0, n], dtype=torch.int64, device=device)
     else:
-        _require_offsets(offsets, "offsets", ids.device)
+        R = _require_offsets(offsets, "offsets", device) - 1
         offsets = offsets.contiguous()
-    keys = torch.empty_like(ids)
-    rc = lib().kvcm_hip_hash_tokens_checked(ptr(ids), 8, ids.numel(), ptr(offsets), offsets.numel() - 1, 1, 0, ptr(keys),
-                                            keys.numel(), ptr(offsets), stream_handle(ids.device))
-    _lib.check(rc, "kvcm_hip_hash_tokens_checked")
-    return keys.reshape(hash_ids.shape)
+    keys = torch.empty(ids.shape, dtype=torch.int64, device=device)
+    at = offsets.data_ptr()
+    rc = lib().kvcm_hip_hash_tokens_checked(ids.data_ptr(), 8, n, at, R, 1, 0, keys.data_ptr(), n, at, stream_handle(device))
+    if rc:
+        _lib.check(rc, "kvcm_hip_hash_tokens_checked")
+    return keys
 
 
 def sha256_to_int64(data: Sequence[str], device="cuda") -> torch.Tensor:
