@@ -78,6 +78,17 @@ def test_argument_validation_needs_no_device():
     assert offsets(p, 32769, 16, 1, 1, p, 39, p, None, None) == _lib.ERR_INVALID_ARG  # workspace too small
     assert offsets(p, 1, 16, 1, 1, p + 4, 8, p, None, None) == _lib.ERR_ALIGNMENT
     assert L.kvcm_hip_key_offsets_workspace_bytes(32768) == 0 and L.kvcm_hip_key_offsets_workspace_bytes(32769) == 5 * 8
+    two_d = L.kvcm_hip_hash_tokens_2d
+    assert two_d(p, 8, 0, 16, 16, 0, p, None, None, None) == _lib.OK
+    assert two_d(p, 2, 1, 16, 16, 0, p, None, None, None) == _lib.ERR_INVALID_ARG
+    assert two_d(p, 8, -1, 16, 16, 0, p, None, None, None) == _lib.ERR_INVALID_ARG
+    assert two_d(p, 8, 1, 15, 16, 0, p, None, None, None) == _lib.ERR_INVALID_ARG  # no whole block
+    assert two_d(None, 8, 1, 16, 16, 0, p, None, None, None) == _lib.ERR_INVALID_ARG
+    assert two_d(p, 8, 1, 16, 16, 0, None, None, None, None) == _lib.ERR_INVALID_ARG
+    assert L.kvcm_hip_key_offsets(None, 1, 16, 1, p, None, None) == _lib.ERR_INVALID_ARG
+    assert L.kvcm_hip_key_offsets(p, 1, 16, 1, None, None, None) == _lib.ERR_INVALID_ARG
+    assert L.kvcm_wait_value(None, None) == _lib.ERR_INVALID_ARG
+    assert L.kvcm_wait_value(p, None) == _lib.OK  # there already: the stream is not asked
     # the table of a save list: a power of two, two slots per key at least (a probe must meet an empty one), eight at most
     for n in [1, 512, 513, 1 << 18, (1 << 18) + 1, 3 << 17, 419430, 419431, 1 << 19, (1 << 19) + 1, 838861, 1 << 20]:
         slots = (L.kvcm_hip_select_save_workspace_bytes(n) - (n + 255) // 256 * 36) // 4 - n

@@ -582,3 +582,36 @@ def test_block_size_1_equally_long_and_ragged(oracle, dtype, R):
             sync()
             got = host(keys, np.int64)
             assert (got[:len(want)] == want).all() and (got[len(want):] == -7).all(), (length, spread)
+
+
+@pytest.mark.parametrize("general_loader", [False, True])
+@pytest.mark.parametrize("dtype,bs,R,lengths", [
+    (np.int64, 16, 2048 + 9, (1024, 2048 + 70)),                      # spread: short workgroups direct, long ones staged
+    (np.int64, 16, 8192 + 9, (639, 640, 1040)),                       # direct and burst
+    (np.int64, 8, 2048 + 9, (511, 512)), (np.int64, 32, 8192 + 9, (895, 900)), (np.int64, 64, 8192 + 9, (895, 897)),
+    (np.int64, 128, 4096 + 9, (959, 961)), (np.int64, 1, 33, (63, 200, 513, 1000)), (np.int64, 1, 1100, (512, 513)),
+    (np.int32, 8, 12288 + 9, (1279, 1280)), (np.int32, 16, 12288 + 9, (1791, 1800)), (np.int32, 32, 12288 + 9, (1791, 1792)),
+    (np.int32, 64, 12288 + 9, (2303, 2304)), (np.int32, 128, 12288 + 9, (2559, 2560)), (np.int32, 1, 64 + 9, (128, 129))])
+def test_equally_long_requests_in_every_form_of_the_kernel(oracle, force_general_hash_loader, general_loader, dtype, bs, R, lengths):
+    """[R, L] batches on both sides of every line of the launch rule, so that the direct, spread, burst and raw-tile forms all
+    read no offset arrays: key offsets written by the launch, or the caller's with gaps between the requests. The last workgroup
+    is partial."""
+    force_general_hash_loader(general_loader)
+    rng = np.random.default_rng(bs + R)
+    for L in lengths:
+        tok = rng.integers(-2**31, 2**31, size=(R, L), dtype=np.int64).astype(dtype)
+        want, woff = oracle.hash_tokens(tok, bs, seed=9, threads=8)
+        per = L // bs
+        print(f"equally long: {R} x {L} {np.dtype(dtype).name}, block size {bs}", flush=True)
+        d_tok = dev(tok)
+        keys, off = _h().hash_tokens(d_tok, bs, seed=9)
+        sync()
+        assert (host(keys, np.int64) == want).all() and (host(off, np.int64) == woff).all(), L
+        gaps = np.arange(R + 1, dtype=np.int64) * (per + 1) + 1
+        spread = torch.full((R * (per + 1) + 1,), -7, dtype=torch.int64, device="cuda")
+        _, same = _h().hash_tokens(d_tok, bs, seed=9, keys=spread, key_offsets=dev(gaps))
+        sync()
+        got = host(spread, np.int64)
+        assert got[0] == -7 and (host(same, np.int64) == gaps).all()
+        got = got[1:].reshape(R, per + 1)
+        assert (got[:, :per] == want.reshape(R, per)).all() and (got[:, per] == -7).all(), L
