@@ -379,7 +379,8 @@ __device__ __forceinline__ void drain_tail(const KeyDrain &kd, int32_t group, in
 
 template <typename Loader, typename TokT, int KS, int G, int TOK>
 __device__ __forceinline__ void run_loader(const LoaderCtx<TokT> &ctx, uint64_t (*s_tile)[kReqs][kTT + kPad],
-                                           int64_t lw, int64_t ntiles, uint32_t lane, const KeyDrain &kd, bool staged) {
+                                           int64_t lw, int64_t ntiles, uint32_t lane, const KeyDrain &kd, bool staged,
+                                           bool apart) {
     static_assert(kRing == 2 && kLoaders >= 3, "two ring slots: prefetched from, written to");
     // the burst drain splits a closed group between the kLoaders - 1 loaders whose tile is not due, as halves
     static_assert(KS != kKeysBurst || kLoaders == 3, "drain_half deals a group out to exactly two loaders");
@@ -447,6 +448,9 @@ __device__ __forceinline__ void run_loader(const LoaderCtx<TokT> &ctx, uint64_t 
             // The barrier above closed a group of G tiles, or what there is of the last one. The loader whose tile is due
             // next leaves it alone (its next wait for memory would wait for these stores as well); the other two write half
             // of it each.
+            if (G == 1 && apart) {
+                __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): keys leave when the next tile's tokens are in
+            }
             drain_half(kd, k / G, (me - turn + kLoaders) % kLoaders - 1, lane);
         }
     }
@@ -593,6 +597,14 @@ __device__ __forceinline__ int64_t distance(int64_t from, int64_t to) {  // offs
 // whether [at, at + n) is a non-empty part of [0, size)
 __device__ __forceinline__ bool inside(int64_t at, int64_t n, int64_t size) { return at >= 0 && n > 0 && n <= size - at; }
 
+// Block size 1 writes as much as it reads. Where every request of a workgroup starts at the same place of a 32 KiB period, their
+// pieces meet in the same channels of memory, and with a workgroup on every CU reads and writes are better kept apart: a loader
+// waits for its tokens before it writes keys. us with / without that wait: 16 384 sequences of 4096 digests 220 / 231, of 8192:
+// 427 / 489, 65 536 of 4096: 799 / 858, 16 384 of 8192 4-byte tokens 352 / 410; but of 2048 (16 KiB apart) 128 / 121, of 6144
+// (48 KiB) 339 / 330, of 4000 to 4160: 330 / 320, and 8192 sequences of 4096, half the CUs, 154 / 122.
+constexpr uint32_t kApartPeriod = 32768;
+constexpr uint32_t kApartFromWorkgroups = 240;
+
 // CHUNK = steps between two looks at the block boundary: 8 when block_size % 8 == 0 (a lane is then
 // active for whole chunks or not at all), otherwise 1. BS = block size when it is 1, 8, 16, 32, 64 or 128, otherwise 0.
 // KS != kKeysDirect ("keys staged", block sizes 1 to 64; chosen by the host for batches of many requests, where the launch
@@ -708,10 +720,12 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
     if (wave != 0) {
         // ---------------------------------------------------------------- loader waves
         const KeyDrain kd{s_keys, s_keyrow, keys};
+        const bool apart = BS == 1 && KS == kKeysBurst && gridDim.x >= kApartFromWorkgroups &&
+                           __all((static_cast<uint32_t>(s_start[lane] - ctx.wg_first_token) * sizeof(TokT)) % kApartPeriod == 0);
         if (buffer_loads) {
-            run_loader<BufferLoader<TokT, RAW>, TokT, KS, G, TOK>(ctx, s_tile, wave - 1, ntiles, lane, kd, staged);
+            run_loader<BufferLoader<TokT, RAW>, TokT, KS, G, TOK>(ctx, s_tile, wave - 1, ntiles, lane, kd, staged, apart);
         } else {
-            run_loader<GlobalLoader<TokT, RAW>, TokT, KS, G, TOK>(ctx, s_tile, wave - 1, ntiles, lane, kd, staged);
+            run_loader<GlobalLoader<TokT, RAW>, TokT, KS, G, TOK>(ctx, s_tile, wave - 1, ntiles, lane, kd, staged, apart);
             // vmcnt(0), for the compiler's books: it lays this path out in front of the other one and would otherwise take
             // the registers of these loads for pending there, and wait for ALL outstanding loads -- the next tile's -- in
             // front of every group of keys that is written out (prefix chain, 64 x 4096: 113 us with that wait, 86 without)

@@ -615,3 +615,25 @@ def test_equally_long_requests_in_every_form_of_the_kernel(oracle, force_general
         assert got[0] == -7 and (host(same, np.int64) == gaps).all()
         got = got[1:].reshape(R, per + 1)
         assert (got[:, :per] == want.reshape(R, per)).all() and (got[:, per] == -7).all(), L
+
+
+@pytest.mark.parametrize("dtype,length", [(np.int64, 4096), (np.int64, 8192), (np.int32, 8192)])
+@pytest.mark.parametrize("R", [240 * 64, 240 * 64 - 64])
+def test_chains_that_start_32_kib_apart(oracle, dtype, length, R):
+    """Block size 1, a workgroup on every CU, requests that start whole multiples of 32 KiB apart: loaders wait for their tokens
+    before they write keys. Workgroups where that holds, where one odd request ends it, and where nothing is to do."""
+    rng = np.random.default_rng(R)
+    lens = np.zeros(R, dtype=np.int64)
+    lens[::16] = length                                     # four to a workgroup, the others empty
+    lens[64 * 100 + 5] = 77                                 # from here on nobody starts at a multiple ...
+    lens[64 * 150 + 5] = length - 77                        # ... and from here on everybody does again
+    lens[64 * 200:64 * 201] = 0
+    toff = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    flat = rng.integers(-2**31, 2**31, size=int(toff[-1]), dtype=np.int64).astype(dtype)
+    want, woff = oracle.hash_tokens(flat, 1, token_offsets=toff, seed=3, threads=8)
+    print(f"chains 32 KiB apart: {R} x {length} {np.dtype(dtype).name}", flush=True)
+    keys = torch.full((len(want) + 64,), -7, dtype=torch.int64, device="cuda")
+    _h().hash_tokens(dev(flat), 1, token_offsets=dev(toff), seed=3, keys=keys, key_offsets=dev(woff))
+    sync()
+    got = host(keys, np.int64)
+    assert (got[:len(want)] == want).all() and (got[len(want):] == -7).all()
