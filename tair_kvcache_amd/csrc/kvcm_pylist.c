@@ -178,6 +178,32 @@ static PyObject *blocks_idx(PyObject *self, PyObject *args) {
     return out;
 }
 
+/* Bytes of a str in UTF-8, written to dst unless that is NULL; -1 with an exception set. ASCII, which is what hash strings are,
+ * is copied as it lies there; anything else is encoded into an object of its own, because PyUnicode_AsUTF8 would leave its
+ * bytes attached to the caller's string for as long as that lives. */
+static Py_ssize_t utf8(PyObject *s, char *dst) {
+    if (PyUnicode_READY(s) < 0) {
+        return -1;
+    }
+    if (PyUnicode_IS_COMPACT_ASCII(s)) {
+        const Py_ssize_t len = PyUnicode_GET_LENGTH(s);
+        if (dst) {
+            memcpy(dst, PyUnicode_DATA(s), (size_t)len);
+        }
+        return len;
+    }
+    PyObject *bytes = PyUnicode_AsUTF8String(s);
+    if (!bytes) {
+        return -1;
+    }
+    const Py_ssize_t len = PyBytes_GET_SIZE(bytes);
+    if (dst) {
+        memcpy(dst, PyBytes_AS_STRING(bytes), (size_t)len);
+    }
+    Py_DECREF(bytes);
+    return len;
+}
+
 /* pack_strings(seq) -> bytearray: int64 offsets [n + 1], then the items' bytes (UTF-8 of a str) back to back, then one spare
  * byte; None when an item is neither exactly str nor exactly bytes (the caller then goes the general way). One buffer, so
  * that strings and offsets reach the device in one copy; 1024 strings of 64 characters take 8 us here, 70 us as a list of
@@ -198,7 +224,8 @@ static PyObject *pack_strings(PyObject *self, PyObject *seq) {
     for (Py_ssize_t i = 0; i < n; ++i) {
         Py_ssize_t len;
         if (PyUnicode_CheckExact(items[i])) {
-            if (!PyUnicode_AsUTF8AndSize(items[i], &len)) {
+            len = utf8(items[i], NULL);
+            if (len < 0) {
                 return NULL;
             }
         } else if (PyBytes_CheckExact(items[i])) {
@@ -221,18 +248,16 @@ static PyObject *pack_strings(PyObject *self, PyObject *seq) {
     memcpy(base, &off, 8);
     for (Py_ssize_t i = 0; i < n; ++i) {
         Py_ssize_t len;
-        const char *src;
         if (PyUnicode_CheckExact(items[i])) {
-            src = PyUnicode_AsUTF8AndSize(items[i], &len); /* kept with the str since the first pass */
+            len = utf8(items[i], dst + off);
+            if (len < 0) {
+                Py_DECREF(out);
+                return NULL;
+            }
         } else {
-            src = PyBytes_AS_STRING(items[i]);
             len = PyBytes_GET_SIZE(items[i]);
+            memcpy(dst + off, PyBytes_AS_STRING(items[i]), (size_t)len);
         }
-        if (!src) {
-            Py_DECREF(out);
-            return NULL;
-        }
-        memcpy(dst + off, src, (size_t)len);
         off += len;
         memcpy(base + 8 * (i + 1), &off, 8);
     }

@@ -211,8 +211,8 @@ def apply_prefix_hash(hash_ids: torch.Tensor, offsets: Optional[torch.Tensor] = 
 
 def sha256_to_int64(data: Sequence[str], device="cuda") -> torch.Tensor:
     """int.from_bytes(sha256(s.encode('utf-8')).digest()[:8], 'big', signed=True) for every string, on the GPU."""
-    packed = _pack_strings(data) if _pack_strings is not None and isinstance(data, (list, tuple)) and len(data) else None
-    if packed is None:  # anything but a list of plain strings
+    packed = _pack_strings(data) if _pack_strings is not None and type(data) in (list, tuple) and data else None
+    if packed is None:  # anything but a list of plain strings; a class of its own may iterate in its own way
         enc = [s.encode("utf-8") if isinstance(s, str) else bytes(s) for s in data]
         n = len(enc)
         if n == 0:

@@ -153,6 +153,17 @@ def test_sha256_of_every_kind_of_sequence(monkeypatch, helper):
         _h().sha256_to_int64(["\ud800"])
 
 
+def test_sha256_of_a_list_that_iterates_in_its_own_way():
+    class Backwards(list):
+        def __iter__(self):
+            return reversed(list.copy(self))
+
+    strs = ["a", "bb", "", "\u00e9\u6f22\U0001f600" * 20]
+    want = [int.from_bytes(hashlib.sha256(s.encode()).digest()[:8], "big", signed=True) for s in reversed(strs)]
+    assert _h().sha256_to_int64(Backwards(strs)).tolist() == want
+    assert _h().sha256_to_int64(strs).tolist() == want[::-1]
+
+
 def test_bad_buffers_are_refused_on_the_host():
     """Short key buffers, offsets of the wrong type, length or device would be out-of-bounds device accesses: ValueError."""
     h = _h()

@@ -1,5 +1,6 @@
 """Host-side mirror of the reference's Python interface: staging-slot pool, result fan-in, argument checks (no GPU)."""
 import inspect
+import sys
 import threading
 import time
 
@@ -422,6 +423,10 @@ def test_packed_strings_are_offsets_then_bytes():
     assert pack_strings([1]) is None and pack_strings(["a", bytearray(b"b")]) is None
     with pytest.raises(UnicodeEncodeError):
         pack_strings(["\ud800"])
+    wide = "".join(["\u00e9\u6f22", "\U0001f600" * 50])      # not the compiler's constant
+    size = sys.getsizeof(wide)
+    assert bytes(pack_strings([wide]))[16:-1] == wide.encode()
+    assert sys.getsizeof(wide) == size                        # nothing stays attached to the caller's string
     with pytest.raises(TypeError):
         pack_strings("abc")
 
