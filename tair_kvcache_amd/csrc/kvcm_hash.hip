@@ -243,12 +243,6 @@ struct GlobalLoader {
     }
 };
 
-// A loader wave's whole life. Loader lw owns tiles lw, lw + kLoaders, ...; tile t lives in ring slot t % kRing.
-// Tiles 0 and 1 are published before the first barrier: the chain wave computes on tile k while its LDS reads of
-// tile k+1 are already in flight, so tile k+2 is what gets written during iteration k (its slot held tile k-1,
-// which the chain wave pulled into registers an iteration ago). A loader issues the loads of its next tile right
-// AFTER the barrier that published its previous one, so they stay in flight for kLoaders - 1 tile periods while the
-// data waits in the loader's registers, not in LDS: more loaders = more bytes in flight per CU at no LDS cost.
 // A request's place among the keys, as the loaders that write staged keys need it.
 struct KeyRow {
     int64_t first;   // index of its first key
@@ -377,6 +371,13 @@ __device__ __forceinline__ void drain_tail(const KeyDrain &kd, int32_t group, in
     }
 }
 
+// A loader wave's whole life. Loader lw owns tiles lw, lw + kLoaders, ...; tile t lives in ring slot t % kRing.
+// Tiles 0 and 1 are published before the first barrier: the chain wave computes on tile k while its LDS reads of
+// tile k+1 are already in flight, so tile k+2 is what gets written during iteration k (its slot held tile k-1,
+// which the chain wave pulled into registers an iteration ago). A loader issues the loads of its next tile right
+// AFTER the barrier that published its previous one, so they stay in flight for kLoaders - 1 tile periods while the
+// data waits in the loader's registers, not in LDS: more loaders = more bytes in flight per CU at no LDS cost.
+// staged: the workgroup's keys pass through LDS and leave through the loaders; apart: reads and writes take turns.
 template <typename Loader, typename TokT, int KS, int G, int TOK>
 __device__ __forceinline__ void run_loader(const LoaderCtx<TokT> &ctx, uint64_t (*s_tile)[kReqs][kTT + kPad],
                                            int64_t lw, int64_t ntiles, uint32_t lane, const KeyDrain &kd, bool staged,
@@ -488,7 +489,7 @@ __device__ __forceinline__ void read_row_part(ulonglong2 (&a)[kRowVecs], const u
 // BS > 0 = the block size is this compile-time constant (a divisor or a multiple of the tile): the places where a key
 // is due are then known when the code is written, and the scalar bookkeeping (add, compare, branch per chunk: one
 // instruction slot in sixteen of the wave that sets the pace) disappears from the loop.
-// STAGED (unmasked tiles, block size a compile-time constant up to a tile): the tile's keys go to the lane's row of the LDS key buffer, `staged_row`
+// STAGED (unmasked tiles, block size a compile-time constant up to two tiles): the tile's keys go to the lane's row of the LDS key buffer, `staged_row`
 // pointing at the tile's first key there; a loader wave writes the rows out (drain_keys).
 template <int CHUNK, bool MASKED, int BS, bool STAGED = false, bool RAW = false>
 __device__ __forceinline__ void run_tile(const ulonglong2 (&a)[kRowVecs], ulonglong2 (&next)[kRowVecs],
@@ -607,8 +608,8 @@ constexpr uint32_t kApartFromWorkgroups = 240;
 
 // CHUNK = steps between two looks at the block boundary: 8 when block_size % 8 == 0 (a lane is then
 // active for whole chunks or not at all), otherwise 1. BS = block size when it is 1, 8, 16, 32, 64 or 128, otherwise 0.
-// KS != kKeysDirect ("keys staged", block sizes 1 to 64; chosen by the host for batches of many requests, where the launch
-// is bound by memory and not by the chain): the chain wave writes its keys into an LDS buffer instead of to memory, whether
+// KS != kKeysDirect ("keys staged", the block sizes with a kernel of their own; chosen by the host where the keys' way to memory
+// bounds the launch: many requests, or a key after every token): the chain wave writes its keys into an LDS buffer instead of to memory, whether
 // a request still has tokens or not, and after every group of tiles the loader waves write out what there is of it as rows
 // of up to 512 bytes, spread over the next group's tiles (block size 16) or at once.
 template <typename TokT, int CHUNK, int BS, int KS = kKeysDirect, bool RAW = false>
@@ -1076,7 +1077,9 @@ constexpr int32_t kForceGeneralLoader = KVCM_TEST_FORCE_GENERAL_LOADER;
 //   16-token blocks, 8-byte tokens: direct 64: 56 / 64  1024: 57 / -   2048: 58 / 66  4096: 61 / 69  8192: 73 / 77  10 240: 79 / 86
 //                                   spread                             2048: 59 / 60  4096: 60 / 60  8192: 65 / 70  10 240:  - / -
 //                                   burst  64: 58 / 60  1024: 58 / -   2048: 59 / 60  4096: 60 / 61  8192: 64 / 67  10 240: 68 / 72
-//   spread beats burst by 4 % on 2048 requests of 1024 tokens: direct below 2048, spread from there, burst from 8192.
+//   spread beats burst by 4 % on 2048 requests of 1024 tokens: direct below 2048, spread from there, burst from 8192. (Of 2048
+//   to 4096 tokens each, 2048 requests take 30.2 to 55.1 direct and 32.1 to 56.4 spread, ragged ones of 500 to 4096 63.7 and 57.0;
+//   below 2048 all stay direct, which costs the ragged ones what the first line says.)
 //   16-token blocks, 4-byte tokens: direct 4096: 55 / -   8192: 58 / 60  12 288: 70 / -
 //                                   burst  4096: 58 / -   8192: 58 / 61  12 288: 60 / -      (raw tiles, see below)
 // Other block sizes, direct / burst:

@@ -194,12 +194,11 @@ def test_bad_buffers_are_refused_on_the_host():
                                    "workgroup_on_every_cu", "every_cu_ragged", "every_cu_two_lengths",
                                    "short_and_long_workgroups"])
 def test_many_requests_take_the_staged_key_path(oracle, dtype, shape):
-    """In launches of thousands of requests the keys of 16-token blocks are collected in LDS and written out as
-    512-byte rows by the loader waves: a sixteenth of a group per tile and the rest after the loop (8-byte tokens, 2048
-    to 10 239 requests; workgroups whose requests are shorter than 32 tiles store directly), or a whole group right
-    after the barrier that closes it (8-byte tokens from 10 240 requests, 4-byte tokens from 12 288). Groups of tiles in
-    which some request has run out, requests past a multiple of 64, and whatever does not fill a group of sixteen tiles
-    go the direct way. Every mixture against the oracle, exact."""
+    """In launches of thousands of requests the keys of 16-token blocks are collected in LDS and written out as rows of up to
+    512 bytes by the loader waves: a sixteenth of a group per tile and the rest after the loop (8-byte tokens, 2048 to 8191
+    requests; workgroups whose requests are shorter than 32 tiles store directly), or a whole group right after the barrier
+    that closes it (8-byte tokens from 8192 requests, 4-byte tokens from 12 288, if they are long enough). Rows end where a
+    request does; requests past a multiple of 64 are in a workgroup of their own. Every mixture against the oracle, exact."""
     rng = np.random.default_rng(5)
     lens = {
         "uniform": np.full(8192, 2048),                                # two whole groups per request
