@@ -84,6 +84,8 @@ int32_t kvcm_hip_hash_tokens_i32(const int32_t *d_tokens, const int64_t *d_token
  * The same for offsets that are not known to be sound: d_tokens holds n_tokens entries of token_bytes (4 or 8) and d_keys
  * n_keys. A request whose blocks reach beyond the tokens, or whose keys beyond the keys, is left out, and nothing outside
  * either array is read or written. kvcm_hip_prefix_chain is block_size 1, seed 0 and the same array of offsets twice.
+ * n_tokens / R also tells the launch how long the requests are: thousands of short ones take another kernel than long ones,
+ * which they are taken for above.
  */
 int32_t kvcm_hip_hash_tokens_checked(const void *d_tokens, int32_t token_bytes, int64_t n_tokens,
                                      const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t seed,
