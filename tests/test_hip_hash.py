@@ -356,6 +356,14 @@ def test_raw_tiles_of_4_byte_tokens(oracle, force_general_hash_loader, bs, gener
     got = host(got, np.int64)
     assert (got[:len(want)] == want).all()
     assert (got[len(want):] == -7).all()
+    # the mean length decides above; through the entry that does not know it, requests count as long and tiles are raw
+    keys.fill_(-7)
+    d_flat, d_toff, d_koff = dev(flat), dev(toff), dev(woff)
+    rc = _h().lib().kvcm_hip_hash_tokens_i32(d_flat.data_ptr(), d_toff.data_ptr(), R, bs, -3, keys.data_ptr(), d_koff.data_ptr(),
+                                             torch.cuda.current_stream().cuda_stream)
+    sync()
+    got = host(keys, np.int64)
+    assert rc == 0 and (got[:len(want)] == want).all() and (got[len(want):] == -7).all()
 
 
 @pytest.mark.parametrize("R,L,bs", [(1, 16, 16), (63, 17, 16), (64, 130, 64), (65, 47, 24), (128, 128, 128), (129, 10, 3)])

@@ -84,3 +84,11 @@ def test_random_launches_of_many_requests(oracle):
         idx = np.repeat(koff[:-1] - woff[:-1], counts) + np.arange(len(want))
         expect[idx] = want
         assert (got == expect).all(), (i, R, bs, seed)
+        # the same through the entry that does not know how long requests are and takes them for long: the staged forms
+        keys.fill_(-7)
+        L, d_flat, d_toff, d_koff = hashing.lib(), dev(flat), dev(toff), dev(koff)
+        entry = L.kvcm_hip_hash_tokens if dtype == np.int64 else L.kvcm_hip_hash_tokens_i32
+        rc = entry(d_flat.data_ptr(), d_toff.data_ptr(), R, bs, seed, keys.data_ptr(), d_koff.data_ptr(),
+                   torch.cuda.current_stream().cuda_stream)
+        sync()
+        assert rc == 0 and (host(keys, np.int64) == expect).all(), (i, R, bs, seed)
