@@ -811,6 +811,436 @@ __device__ __forceinline__ int64_t keys_of(int64_t len, int32_t block_size) {
     return len > 0 ? len / block_size : 0;
 }
 
+// ------------------------------------------------------------------------------------------- few requests per workgroup
+
+// The kernel for launches that leave compute units idle when 64 requests share a workgroup (up to kLeanUpTo requests): 16 requests
+// per workgroup, four waves on the four SIMDs of a compute unit.
+//   wave 0     "chain wave": nothing but the recurrence, 32 steps at a time from terms read 32 steps ahead (two register sets of
+//              64 registers: no accumulation registers), and every 16 steps the state, which is left in LDS two at a time.
+//   waves 1, 2 loaders: 16 x 64 tokens as 16-byte buffer loads, two tiles each under way, C added, rows into an LDS ring.
+//   wave 3     writer: picks the keys out of the states and stores them.
+// Where keys lie between the states (block sizes that 16 does not divide, EVERY), the loader whose turn it is not goes through the
+// tile again: 64 lanes of 16 steps each, from the states in front of them, and leaves the state after every step in the place of
+// its term. So a key costs the chain nothing, whatever the block size, and requests that end early cost nothing either: the chain
+// runs to the end of the longest, and only loaders and writer know where the others end.
+//
+// All 64 lanes of the chain wave stay active, four per request. A wave of which 16 lanes are active issues its instructions at
+// 20.7 to 28.5 clocks per step, depending on the place of its compute unit on the die; with all lanes active it is 20.7 everywhere
+// (five instructions of 4 clocks, measured on all 256 units).
+//
+// Bound: issue slots of the chain wave. Of 25 clocks per step (64 x 16 384 tokens: 10.8 ns) 20.7 are the step, 2.5 the reads of
+// 16 bytes per two steps, 0.8 the state write (26 clocks per 32 steps), 1 the barrier per tile and loop control.
+// us, before / now: 4 x 512 9.6 / 8.1, 64 x 4096 tokens 51.6 / 46.5, 4096 x 4096 55.8 / 49.2, 160 ragged of 48 to 8192 4-byte
+// tokens 102.4 / 89.4, 64 x 4096 of block size 8: 58.7 / 47.3, 24: 64.5 / 47.2, 7: 151 / 48.4, 1: 85.7 / 48.3; prefix chain, 1000
+// sequences of 8 to 1024: 27.5 / 15.6.
+// Tiles of 128 tokens (half as many barriers) take 46.8 and 8.8 where these take 46.5 and 8.2; without the idle loaders' help the
+// writer sets the pace at block size 1 (75).
+constexpr int kLeanRows = 16;    // requests per workgroup
+constexpr int kLeanTok = 64;     // tokens per request and tile
+constexpr int kLeanGroup = 32;   // steps whose terms are read ahead at a time
+constexpr int kLeanStride = 16;  // steps between two states that are left for the writer
+constexpr int kLeanStates = kLeanTok / kLeanStride;
+constexpr int kLeanLoaders = 2;
+constexpr uint32_t kLeanWriter = 1 + kLeanLoaders;
+constexpr int kLeanThreads = 64 * (2 + kLeanLoaders);
+// Offsets from kLeanOutside on lie outside every buffer: a load there fetches nothing.
+constexpr uint32_t kLeanBufferMost = 0xFFFFFF00u, kLeanOutside = 0xFFFFFFF0u;
+
+// One request as every wave of its workgroup sees it: lane i of a wave knows request i % 16.
+struct LeanRow {
+    int64_t start;  // first token
+    int64_t ntok;   // tokens that make up keys
+    int64_t key;    // index of its first key
+};
+
+__device__ __forceinline__ int64_t shfl_i64(int64_t v, int lane) {
+    const int lo = __shfl(static_cast<int>(v), lane, 64), hi = __shfl(static_cast<int>(v >> 32), lane, 64);
+    return static_cast<int64_t>((static_cast<uint64_t>(static_cast<uint32_t>(hi)) << 32) | static_cast<uint32_t>(lo));
+}
+
+// For values that are the same in all lanes where the compiler cannot see it: scalar registers, scalar branches.
+__device__ __forceinline__ int64_t uniform_i64(int64_t v) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(static_cast<uint64_t>(v) >> 32));
+    return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
+// One tile in 16-byte buffer loads. A piece behind its request's last token is not fetched.
+template <typename TokT>
+struct LeanBufferLoader {
+    static constexpr int kEPL = 16 / sizeof(TokT);
+    static constexpr int kLPR = kLeanTok / kEPL;       // lanes per request row
+    static constexpr int kRPW = 64 / kLPR;             // rows per load instruction
+    static constexpr int kNL = kLeanRows / kRPW;       // loads per lane and tile
+    typedef u32x4 Regs[kNL];
+    __amdgpu_buffer_rsrc_t rsrc;
+    uint32_t rel[kNL], lim[kNL];  // byte offset of this lane's piece of tile 0; bytes of the request from that piece on
+    uint32_t sub, piece;
+
+    __device__ __forceinline__ void setup(const TokT *tokens, int64_t first, int64_t total, const LeanRow &row, uint32_t lane) {
+        sub = lane / kLPR;
+        piece = lane % kLPR;
+        const uint64_t bytes = static_cast<uint64_t>(total - first) * sizeof(TokT);
+        rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<TokT *>(tokens + first), 0,
+                                                 bytes > kLeanBufferMost ? kLeanBufferMost : static_cast<uint32_t>(bytes), 0x00020000);
+        const int at = static_cast<int>((row.start - first) * static_cast<int64_t>(sizeof(TokT)));
+        const int len = static_cast<int>(row.ntok * static_cast<int64_t>(sizeof(TokT)));
+#pragma unroll
+        for (int j = 0; j < kNL; ++j) {
+            const int from = j * kRPW + static_cast<int>(sub);
+            const uint32_t bytes_of_row = static_cast<uint32_t>(__shfl(len, from, 64));
+            rel[j] = static_cast<uint32_t>(__shfl(at, from, 64)) + piece * 16u;
+            lim[j] = bytes_of_row > piece * 16u ? bytes_of_row - piece * 16u : 0;
+        }
+    }
+    __device__ __forceinline__ void issue(Regs &regs, int32_t t) const {
+        const uint32_t off = static_cast<uint32_t>(t) * static_cast<uint32_t>(kLeanTok * sizeof(TokT));
+#pragma unroll
+        for (int j = 0; j < kNL; ++j) {
+            regs[j] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off < lim[j] ? rel[j] + off : kLeanOutside, 0, 2);
+        }
+    }
+    __device__ __forceinline__ void store(const Regs &regs, uint64_t (*tile)[kLeanTok + kPad]) const {
+#pragma unroll
+        for (int j = 0; j < kNL; ++j) {
+            const u32x4 v = regs[j];
+            ulonglong2 *dst = reinterpret_cast<ulonglong2 *>(&tile[j * kRPW + sub][piece * kEPL]);
+            if (sizeof(TokT) == 8) {
+                dst[0] = make_ulonglong2(((static_cast<uint64_t>(v.y) << 32) | v.x) + kGolden,
+                                         ((static_cast<uint64_t>(v.w) << 32) | v.z) + kGolden);
+            } else {
+                dst[0] = make_ulonglong2(pre_add_i32(v.x), pre_add_i32(v.y));
+                dst[1] = make_ulonglong2(pre_add_i32(v.z), pre_add_i32(v.w));
+            }
+        }
+    }
+};
+
+// The same with an address per token, for workgroups whose requests span 4 GiB or more.
+template <typename TokT>
+struct LeanGlobalLoader {
+    static_assert(kLeanTok == 64, "a lane per token of a request's row");
+    typedef TokT Regs[kLeanRows];
+    const TokT *tokens;
+    LeanRow row;
+    uint32_t lane;
+    __device__ __forceinline__ void setup(const TokT *tokens_, int64_t, int64_t, const LeanRow &row_, uint32_t lane_) {
+        tokens = tokens_;
+        row = row_;
+        lane = lane_;
+    }
+    __device__ __forceinline__ void issue(Regs &regs, int32_t t) const {
+        const int64_t at = static_cast<int64_t>(t) * kLeanTok + lane;
+#pragma unroll
+        for (int j = 0; j < kLeanRows; ++j) {
+            const int64_t ntok = shfl_i64(row.ntok, j), start = shfl_i64(row.start, j);  // while all lanes are here
+            regs[j] = at < ntok ? tokens[start + at] : 0;
+        }
+    }
+    __device__ __forceinline__ void store(const Regs &regs, uint64_t (*tile)[kLeanTok + kPad]) const {
+#pragma unroll
+        for (int j = 0; j < kLeanRows; ++j) {
+            tile[j][lane] = static_cast<uint64_t>(static_cast<int64_t>(regs[j])) + kGolden;
+        }
+    }
+};
+
+template <bool EVERY>
+struct LeanShared {
+    static constexpr int kRing = EVERY ? 8 : 2;
+    uint64_t tile[kRing][kLeanRows][kLeanTok + kPad];  // terms; EVERY: then the states after every step
+    uint64_t state[4][kLeanRows][kLeanStates + 2];     // states after every 16 steps, of four tiles
+    KeyRow keyrow[kLeanRows];                          // the writer's own
+};
+
+// Who does what when. Barrier b ends interval b; there are nt + 2 of them, EVERY: nt + 3.
+//   loader      stores tile t in interval t (its slot was read for the last time in interval t - 1 or before)
+//   chain wave  reads the rest of tile t and goes through it in intervals t + 1 and t + 2: its barrier stands in front of the
+//               tile's last 32 steps, when the last terms are in registers and those of the next tile are about to be asked for;
+//               the tile's last states are written in interval t + 2
+//   EVERY       loader t % 2 expands tile t in interval t + 3 (tile t + 3 is the other one's)
+//   writer      stores the keys of tile t in interval t + 3, EVERY: t + 4 (tile t + 8 takes its slot, tile t + 4 its states)
+
+// The states after every token of tile t, in place of the tile's terms: 64 lanes go through 16 steps each, from the states
+// that the chain wave left.
+__device__ __forceinline__ void lean_expand(LeanShared<true> &sh, int32_t t, uint64_t seed, uint32_t lane) {
+    using SH = LeanShared<true>;
+    static_assert(kLeanRows * kLeanStates == 64, "a lane per stretch of 16 steps");
+    const uint32_t r = lane % kLeanRows, part = lane / kLeanRows;
+    uint64_t h = part ? sh.state[t & 3][r][part - 1] : t ? sh.state[(t - 1) & 3][r][kLeanStates - 1] : seed;
+    ulonglong2 *const terms = reinterpret_cast<ulonglong2 *>(&sh.tile[t & (SH::kRing - 1)][r][part * kLeanStride]);
+    ulonglong2 a[kLeanStride / 2];
+#pragma unroll
+    for (int i = 0; i < kLeanStride / 2; ++i) {
+        a[i] = terms[i];
+    }
+#pragma unroll
+    for (int i = 0; i < kLeanStride / 2; ++i) {
+        const uint64_t h1 = chain_step(h, a[i].x);
+        h = chain_step(h1, a[i].y);
+        terms[i] = make_ulonglong2(h1, h);
+    }
+}
+
+// A loader wave's whole life: tiles me, me + 2, ..., in two register sets taking turns.
+template <typename Loader, bool EVERY>
+__device__ __forceinline__ void lean_load(LeanShared<EVERY> &sh, const Loader &ld, int32_t me, int32_t nt, uint64_t seed,
+                                          uint32_t lane) {
+    constexpr int32_t kAhead = 2 * kLeanLoaders;
+    typename Loader::Regs even, odd;
+    int32_t barriers = nt + (EVERY ? 3 : 2);
+    const auto barrier = [&] {
+        if (barriers > 0) {
+            lds_barrier();
+            --barriers;
+        }
+    };
+    const auto turn = [&](typename Loader::Regs &regs, int32_t t) {
+        if (t < nt) {
+            ld.store(regs, sh.tile[t & (LeanShared<EVERY>::kRing - 1)]);
+        }
+        // also beyond the last tile, where nothing is fetched: how many loads are under way is then known when the code is
+        // written, and a tile is waited for without the one behind it
+        ld.issue(regs, t + kAhead);
+        barrier();
+        if constexpr (EVERY) {  // the other loader's turn: its tile is t + 1
+            if (t >= 2 && t - 2 < nt) {
+                lean_expand(sh, t - 2, seed, lane);
+            }
+        }
+        barrier();
+    };
+    ld.issue(even, me);
+    ld.issue(odd, me + kLeanLoaders);
+    if (me) {
+        barrier();
+    }
+    for (int32_t t = me; barriers > 0; t += kAhead) {
+        turn(even, t);
+        turn(odd, t + kLeanLoaders);
+    }
+}
+
+// The writer's whole life. Keys lie `per` states apart (of those that are kept: every 16th step's, EVERY: every step's).
+template <bool EVERY>
+__device__ __forceinline__ void lean_write(LeanShared<EVERY> &sh, int32_t nt, const LeanRow &row, int64_t count, int32_t block_size,
+                                           int64_t *__restrict__ keys, uint32_t lane) {
+    constexpr uint32_t kUnit = EVERY ? 1 : kLeanStride, kUnits = kLeanTok / kUnit;  // states per tile
+    const uint32_t per = static_cast<uint32_t>(block_size) / kUnit;
+    const uint32_t q = kUnits / per;
+    const uint32_t most = q * per == kUnits ? q : q + 1;              // keys per tile
+    const uint32_t lg = most > 1 ? 32 - __builtin_clz(most - 1) : 0;  // log2 of the lanes that a request's keys take
+    int64_t before = 0;                                               // keys of the tiles so far
+    uint32_t off = per;                                               // states to the next key
+    if (lane < kLeanRows) {
+        sh.keyrow[lane] = KeyRow{row.key, count};
+    }
+    lds_barrier();
+    lds_barrier();
+    if (EVERY) {
+        lds_barrier();
+    }
+    for (int32_t t = 0; t < nt; ++t) {
+        lds_barrier();
+        uint64_t(*const tile)[kLeanTok + kPad] = sh.tile[t & (LeanShared<EVERY>::kRing - 1)];
+        const uint32_t nk = off > kUnits ? 0 : off + q * per <= kUnits ? q + 1 : q;
+        for (uint32_t e = lane; e < static_cast<uint32_t>(kLeanRows) << lg; e += 64) {
+            const uint32_t r = e >> lg, j = e & ((1u << lg) - 1);
+            const KeyRow to = sh.keyrow[r];
+            if (j < nk && before + j < to.count) {
+                const uint32_t at = off - 1 + j * per;
+                keys[to.first + before + j] = static_cast<int64_t>(EVERY ? tile[r][at] : sh.state[t & 3][r][at]);
+            }
+        }
+        before += nk;
+        off += nk * per - kUnits;
+    }
+}
+
+// The same for block size 1, where every state is a key: 512 bytes of a request at a time, 16 per lane.
+__device__ __forceinline__ void lean_write_all(LeanShared<true> &sh, int32_t nt, const LeanRow &row, int64_t count,
+                                               int64_t *__restrict__ keys, uint32_t lane) {
+    typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+    typedef u64x2 u64x2_a8 __attribute__((aligned(8)));
+    constexpr int kN = kLeanRows / 2;  // two requests' rows per store instruction
+    const uint32_t half = lane / 32, piece = lane % 32;
+    int64_t *dst[kN];
+    int32_t pairs[kN], singles[kN];  // tiles in which both of this lane's keys, or the first, belong to the request
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+        const int64_t left = shfl_i64(count, i * 2 + half) - piece * 2;
+        dst[i] = keys + shfl_i64(row.key, i * 2 + half) + piece * 2;
+        pairs[i] = left >= 2 ? static_cast<int32_t>((left - 2) / kLeanTok + 1) : 0;
+        singles[i] = left >= 1 ? static_cast<int32_t>((left - 1) / kLeanTok + 1) : 0;
+    }
+    // tiles that all 16 requests fill
+    const int32_t full = static_cast<int32_t>(wave_min_u32(static_cast<uint32_t>(count / kLeanTok)));
+    lds_barrier();
+    lds_barrier();
+    lds_barrier();
+    for (int32_t t = 0; t < nt; ++t) {
+        lds_barrier();
+        const uint64_t(*const tile)[kLeanTok + kPad] = sh.tile[t & (LeanShared<true>::kRing - 1)];
+        u64x2 v[kN];
+#pragma unroll
+        for (int i = 0; i < kN; ++i) {
+            v[i] = *reinterpret_cast<const u64x2 *>(&tile[i * 2 + half][piece * 2]);
+        }
+        if (t < full) {
+#pragma unroll
+            for (int i = 0; i < kN; ++i) {
+                *reinterpret_cast<u64x2_a8 *>(dst[i]) = v[i];
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < kN; ++i) {
+                if (t < pairs[i]) {
+                    *reinterpret_cast<u64x2_a8 *>(dst[i]) = v[i];
+                } else if (t < singles[i]) {
+                    *dst[i] = static_cast<int64_t>(v[i].x);
+                }
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < kN; ++i) {
+            dst[i] += kLeanTok;
+        }
+    }
+}
+
+template <typename TokT, bool EVERY>
+__global__ __launch_bounds__(kLeanThreads) void hash_lean_kernel(const TokT *__restrict__ tokens,
+                                                                 const int64_t *__restrict__ token_offsets, int32_t R,
+                                                                 int32_t block_size, uint64_t seed, int64_t *__restrict__ keys,
+                                                                 const int64_t *__restrict__ key_offsets, const Uniform uni,
+                                                                 const Extent have, int32_t force_global_loads) {
+    using SH = LeanShared<EVERY>;
+    __shared__ __attribute__((aligned(16))) SH sh;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t r_first = static_cast<int64_t>(blockIdx.x) * kLeanRows;
+    const int64_t r = r_first + lane % kLeanRows;
+    LeanRow row{0, 0, 0};
+    int64_t count = 0, first = 0, span = 0, total;
+    int32_t nt;  // tiles of the longest request
+    if (token_offsets) {
+        const int64_t r_end = r_first + kLeanRows < R ? r_first + kLeanRows : R;
+        const bool known = have.tokens != kUnknown;
+        first = token_offsets[r_first];
+        total = known ? have.tokens : token_offsets[R];
+        span = distance(first, token_offsets[r_end]);
+        if (known && (first < 0 || first > total)) {
+            first = first < 0 ? 0 : total;
+        }
+        if (r < R) {
+            const int64_t at = token_offsets[r];
+            const int64_t nkeys = keys_of(distance(at, token_offsets[r + 1]), block_size);
+            row.key = key_offsets ? key_offsets[r] : r * keys_of(distance(token_offsets[0], token_offsets[1]), block_size);
+            if (inside(row.key, nkeys, have.keys) && (!known || inside(at, nkeys * block_size, total))) {
+                row.start = at;
+                row.ntok = nkeys * block_size;
+                count = nkeys;
+            }
+        }
+        nt = static_cast<int32_t>(wave_max_u32(static_cast<uint32_t>((row.ntok + kLeanTok - 1) / kLeanTok)));
+    } else {
+        first = r_first * uni.tokens;
+        total = R * uni.tokens;
+        span = kLeanRows * uni.tokens;
+        if (r < R) {
+            row.start = r * uni.tokens;
+            row.key = key_offsets ? key_offsets[r] : r * uni.keys;
+            count = row.key < 0 ? 0 : uni.keys;
+            row.ntok = count * block_size;
+        }
+        nt = static_cast<int32_t>((uni.keys * block_size + kLeanTok - 1) / kLeanTok);
+        if (uni.key_offsets_out && wave == kLeanWriter) {
+            if (lane < kLeanRows && r < R) {
+                uni.key_offsets_out[r] = r * uni.keys;
+            }
+            if (r_first + kLeanRows >= R && lane == 0) {
+                uni.key_offsets_out[R] = R * uni.keys;
+            }
+        }
+    }
+    nt = __builtin_amdgcn_readfirstlane(nt);
+    if (nt == 0) {
+        return;
+    }
+    first = uniform_i64(first);
+    total = uniform_i64(total);
+    span = uniform_i64(span);
+    if (wave == kLeanWriter) {
+        if constexpr (EVERY) {
+            if (block_size == 1) {
+                lean_write_all(sh, nt, row, count, keys, lane);
+                return;
+            }
+        }
+        lean_write<EVERY>(sh, nt, row, count, block_size, keys, lane);
+        return;
+    }
+    if (wave != 0) {
+        if (!force_global_loads && span >= 0 && static_cast<uint64_t>(span) * sizeof(TokT) < 0xFFF00000ull) {
+            LeanBufferLoader<TokT> ld;
+            ld.setup(tokens, first, total, row, lane);
+            lean_load<LeanBufferLoader<TokT>, EVERY>(sh, ld, wave - 1, nt, seed, lane);
+        } else {
+            LeanGlobalLoader<TokT> ld;
+            ld.setup(tokens, first, total, row, lane);
+            lean_load<LeanGlobalLoader<TokT>, EVERY>(sh, ld, wave - 1, nt, seed, lane);
+        }
+        return;
+    }
+    constexpr int kPieces = kLeanGroup / 2, NG = kLeanTok / kLeanGroup;
+    static_assert(NG % 2 == 0 && kLeanGroup == 2 * kLeanStride, "register sets take turns; two states per group, one write");
+    const uint32_t mine = lane % kLeanRows;
+    uint64_t h = seed, held = 0;
+    ulonglong2 a[2][kPieces];
+    const auto read_group = [&](ulonglong2 (&to)[kPieces], const uint64_t *from) {
+#pragma unroll
+        for (int i = 0; i < kPieces; ++i) {
+            to[i] = reinterpret_cast<const ulonglong2 *>(from)[i];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    lds_barrier();
+    read_group(a[0], &sh.tile[0][mine][0]);
+    uint64_t *at = nullptr;  // where the states of the group before go
+    for (int32_t k = 0; k < nt; ++k) {
+        const uint64_t *const row_now = &sh.tile[k & (SH::kRing - 1)][mine][0], *const row_next = &sh.tile[(k + 1) & (SH::kRing - 1)][mine][0];
+        uint64_t *const states = &sh.state[k & 3][mine][0];
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            // This group's terms, asked for 32 steps ago. Waited for before the next are asked for: the counter of LDS operations
+            // ends at 15, so behind 16 newer reads the wait would be for the first of those.
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+            if (g + 1 == NG) {
+                lds_barrier();
+            }
+            if (g > 0 || k > 0) {
+                *reinterpret_cast<ulonglong2 *>(at) = make_ulonglong2(held, h);
+            }
+            at = states + 2 * g;
+            read_group(a[(g + 1) & 1], g + 1 < NG ? row_now + (g + 1) * kLeanGroup : row_next);  // behind the last tile: not used
+#pragma unroll
+            for (int s = 0; s < kLeanGroup; ++s) {
+                const ulonglong2 v = a[g & 1][s / 2];
+                h = chain_step(h, (s & 1) ? v.y : v.x);
+                if (s == kLeanStride - 1) {
+                    held = h;
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    *reinterpret_cast<ulonglong2 *>(at) = make_ulonglong2(held, h);
+    lds_barrier();
+    if (EVERY) {
+        lds_barrier();
+    }
+}
+
 // Keys of one request; `bad` is set when the tokens they are made of are not all there.
 __device__ __forceinline__ int64_t keys_of_request(int64_t at, int64_t next, int32_t block_size, int64_t n_tokens, bool &bad) {
     const int64_t count = keys_of(distance(at, next), block_size);
@@ -1147,6 +1577,10 @@ constexpr int64_t burst_from_tokens(int32_t block_size, bool tokens_8_byte, bool
         default: return 0;
     }
 }
+// Requests up to which a launch takes workgroups of 16 (hash_lean_kernel): as many as give each of the 256 compute units one. A
+// second one on a unit shares its SIMDs, and one of 16 reads 512 bytes of each of 16 requests at a time where the other kernel
+// reads 64. us, 16 per workgroup / 64: 4096 requests of 4096 tokens 49.2 / 55.8, 5120: 59.0 / 56.8, 8192: 71.4 / 59.9.
+constexpr int32_t kLeanUpTo = 256 * kLeanRows;
 #ifndef KVCM_HASH_BURST_SCALE  // for experiments: 0 = burst wherever it exists, a large number = never
 #define KVCM_HASH_BURST_SCALE 1
 #endif
@@ -1166,6 +1600,17 @@ int32_t launch_hash(const TokT *d_tokens, const int64_t *d_token_offsets, int32_
     }
     const dim3 grid(static_cast<uint32_t>((static_cast<int64_t>(R) + kReqs - 1) / kReqs));
     const int32_t force_global = kForceGeneralLoader;
+    if (R <= kLeanUpTo) {
+        const dim3 lean_grid(static_cast<uint32_t>((static_cast<int64_t>(R) + kLeanRows - 1) / kLeanRows));
+        if (block_size % kLeanStride == 0) {
+            hipLaunchKernelGGL((hash_lean_kernel<TokT, false>), lean_grid, dim3(kLeanThreads), 0, stream, d_tokens, d_token_offsets, R,
+                               block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, have, force_global);
+        } else {
+            hipLaunchKernelGGL((hash_lean_kernel<TokT, true>), lean_grid, dim3(kLeanThreads), 0, stream, d_tokens, d_token_offsets, R,
+                               block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, have, force_global);
+        }
+        return launch_status();
+    }
 #define KVCM_LAUNCH_HASH(CHUNK, BS)                                                                                  \
     hipLaunchKernelGGL((hash_tokens_kernel<TokT, CHUNK, BS>), grid, dim3(kThreads), 0, stream, d_tokens,            \
                        d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, have, \

@@ -655,3 +655,36 @@ def test_chains_that_start_32_kib_apart(oracle, dtype, length, R):
     sync()
     got = host(keys, np.int64)
     assert (got[:len(want)] == want).all() and (got[len(want):] == -7).all()
+
+
+@pytest.mark.parametrize("general_loader", [False, True])
+@pytest.mark.parametrize("dtype", [np.int64, np.int32])
+@pytest.mark.parametrize("bs", [1, 2, 7, 8, 16, 24, 48, 63, 64, 65, 80, 128, 208, 1000])
+def test_sixteen_requests_per_workgroup(oracle, force_general_hash_loader, general_loader, dtype, bs):
+    """Launches of up to 4096 requests: lengths on and around a tile of 64 tokens, its halves and the 16 steps between two kept
+    states, blocks shorter and longer than each of them, workgroups in which one request outlasts the others by many tiles,
+    request counts around a workgroup's 16 and around the last count that takes this form; ragged with gaps between the keys of
+    neighbours, and equally long."""
+    force_general_hash_loader(general_loader)
+    rng = np.random.default_rng(bs)
+    menu = np.array([0, 1, 15, 16, 17, 31, 32, 33, 47, 48, 63, 64, 65, 95, 96, 97, 127, 128, 129, 191, 192, 193, 255, 256, 257, 320,
+                     bs - 1, bs, bs + 1, 2 * bs, 3 * bs + 1])
+    for R in (1, 15, 16, 17, 33, 4095, 4096, 4097):
+        lens = menu[rng.integers(0, len(menu), size=R)]
+        lens[-1] = 1100 if R < 100 else 700                                # the last workgroup outlasts the others
+        toff = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+        flat = rng.integers(-2**31, 2**31, size=int(toff[-1]), dtype=np.int64).astype(dtype)
+        want, woff = oracle.hash_tokens(flat, bs, token_offsets=toff, seed=R, threads=8)
+        koff = woff + np.arange(R + 1)                                      # one slot between neighbours that must stay
+        room = torch.full((len(want) + R + 1,), -7, dtype=torch.int64, device="cuda")
+        _h().hash_tokens(dev(flat), bs, token_offsets=dev(toff), seed=R, keys=room, key_offsets=dev(koff))
+        sync()
+        expect = np.full(len(want) + R + 1, -7, dtype=np.int64)
+        expect[np.arange(len(want)) + np.repeat(np.arange(R), np.diff(woff))] = want
+        assert (host(room, np.int64) == expect).all(), (R, bs)
+    for R, L in ((1, 64), (5, 65), (16, 128), (18, 1000), (33, 4096), (4096, 72)):
+        tok = rng.integers(-2**31, 2**31, size=(R, L), dtype=np.int64).astype(dtype)
+        want, woff = oracle.hash_tokens(tok, bs, seed=-1, threads=8)
+        keys, off = _h().hash_tokens(dev(tok), bs, seed=-1)
+        sync()
+        assert (host(keys, np.int64) == want).all() and (host(off, np.int64) == woff).all(), (R, L, bs)
