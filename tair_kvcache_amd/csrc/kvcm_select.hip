@@ -8,6 +8,7 @@
 //
 // Small integer kernels, nowhere near a bandwidth bound: n is the number of block keys of a batch (thousands).
 #include <atomic>
+#include <climits>
 #include <mutex>
 
 #include "kvcm_internal.h"
@@ -210,7 +211,7 @@ __global__ __launch_bounds__(kSelThreads) void write_kernel(const uint8_t *__res
     }
 }
 
-// The list of a whole batch in four launches (fill, insert, choose, list) where first occurrences and mask compaction in a row
+// The list of a batch of more keys than part_kernel takes, in four launches (fill, insert, choose, list) where first occurrences and mask compaction in a row
 // take six. Bound by latency: every launch is a chain of two or three trips to memory, and what counts is how many follow
 // each other. 256 keys per workgroup, so that 32 768 keys make 128 workgroups.
 constexpr int kListThreads = 256;
@@ -281,6 +282,202 @@ __global__ __launch_bounds__(kListThreads) void list_kernel(const uint64_t *__re
     }
     if (group == static_cast<int32_t>(gridDim.x) - 1 && threadIdx.x == 0) {
         *d_count = before + own;  // thread 0: nothing of its own group lies before it
+    }
+}
+
+// The list of up to kPartMaxKeys keys in two launches. Every workgroup reads ALL keys and takes those whose hash value falls into
+// its part, so a part's table fits the LDS: no table in memory to clear, no chain of probes through memory, and nobody waits for
+// anybody. Bound: every compute unit reads every key (64 bytes a clock from its L2) and looks at it, about 70 clocks for 64 keys of
+// a wave; the keys that are taken wait in LDS until 64 of them can be entered at a time, because a branch for the few lanes whose
+// key it is costs a wave as much as 64 of them (32 768 keys 12.4 to 15.0, so 9.2 to 9.7 us). Two launches against four, us, all
+// different / each 8 times: 1000 keys 11.3 / 12.0 -> 6.7 / 6.6, 16 384 14.2 / 11.7 -> 7.8 / 7.7, 32 768 13.9 / 11.8 -> 9.7 / 9.2,
+// 65 536 16.3 / 14.3 -> 13.3 / 12.8; 100 000 keys 20.9 / 17.1 and 17.8 / 17.7, 131 072 23.0 / 18.5 and 21.3 / 21.0, so beyond 65 536
+// the table in memory stays.
+constexpr int kPartThreads = 1024;
+constexpr int64_t kPartMaxKeys = int64_t{1} << 16;
+constexpr uint64_t kNoKey = 0x8000000000000000ull;  // an empty slot; a key of this value is kept apart
+
+struct PartShape {
+    int log2_parts, log2_slots;
+};
+
+// One part per compute unit where there are keys for it, and eight slots per key of an even share.
+PartShape part_shape(int64_t n) {
+    PartShape p{n > 4096 ? 8 : n > 512 ? 6 : 4, 8};
+    while ((int64_t{1} << (p.log2_slots + p.log2_parts)) < 8 * n) {
+        ++p.log2_slots;
+    }
+    return p;
+}
+
+// Both halves times odd constants, modulo 2^32; the upper bits choose the part, the next ones the slot. In 64-bit multiply-adds,
+// which issue at the full rate (a 32-bit multiplication takes four times as long).
+__device__ __forceinline__ uint32_t part_hash(uint64_t k) {
+    uint64_t x, carry;
+    asm("v_mad_u64_u32 %0, %1, %2, %3, 0" : "=v"(x), "=s"(carry) : "v"(static_cast<uint32_t>(k)), "s"(0x9e3779b1u));
+    asm("v_mad_u64_u32 %0, %1, %2, %3, %4" : "=v"(x), "=s"(carry) : "v"(static_cast<uint32_t>(k >> 32)), "s"(0x85ebca77u), "v"(x));
+    return static_cast<uint32_t>(x);
+}
+
+// flags[i] = keys[i] is a first occurrence and not saved yet. Exactly one write per key: whoever learns that an index is not the
+// smallest of its key clears it -- its own, or the one it has just replaced -- and what is left in the table at the end is set.
+__global__ __launch_bounds__(kPartThreads) void part_kernel(const uint64_t *__restrict__ keys, int32_t n, int log2_parts, int log2_slots,
+                                                            const uint8_t *__restrict__ saved, uint8_t *__restrict__ flags) {
+    extern __shared__ __attribute__((aligned(16))) uint64_t s_key[];
+    const uint32_t slots = 1u << log2_slots, mask = slots - 1;
+    int32_t *const s_first = reinterpret_cast<int32_t *>(s_key + slots);  // smallest index of the slot's key
+    __shared__ int32_t s_first_no_key;
+    __shared__ uint64_t s_wait_key[kPartThreads / 64][2 * 64];
+    __shared__ int32_t s_wait_idx[kPartThreads / 64][2 * 64];
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (uint32_t i = threadIdx.x; i < slots; i += kPartThreads) {
+        s_key[i] = kNoKey;
+        s_first[i] = INT32_MAX;
+    }
+    if (threadIdx.x == 0) {
+        s_first_no_key = INT32_MAX;
+    }
+    __syncthreads();
+    const auto put = [&](int32_t *first, int32_t i) {
+        const int32_t was = atomicMin(first, i);
+        if (was != INT32_MAX) {
+            flags[was < i ? i : was] = 0;
+        }
+    };
+    const auto take = [&](uint64_t k, int32_t i) {
+        if (k == kNoKey) {
+            put(&s_first_no_key, i);
+            return;
+        }
+        uint32_t s = (part_hash(k) << log2_parts) >> (32 - log2_slots);
+        for (uint32_t tries = 0; tries < slots; ++tries) {
+            const uint64_t o = atomicCAS(reinterpret_cast<unsigned long long *>(s_key + s), kNoKey, k);
+            if (o == kNoKey || o == k) {
+                put(s_first + s, i);
+                return;
+            }
+            s = (s + 1) & mask;
+        }
+        // More different keys than slots, all of one part: keys made to collide. Looked for one by one.
+        int32_t j = 0;
+        while (j < i && keys[j] != k) {
+            ++j;
+        }
+        flags[i] = j == i && !(saved && saved[i]);
+    };
+    uint64_t *const wait_key = s_wait_key[wave];
+    int32_t *const wait_idx = s_wait_idx[wave];
+    uint32_t waiting = 0;
+    const auto enter = [&](uint32_t count) {  // the last `count` keys that wait
+        __builtin_amdgcn_wave_barrier();
+        waiting -= count;
+        if (lane < count) {
+            take(wait_key[waiting + lane], wait_idx[waiting + lane]);
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
+    const auto look = [&](uint64_t k, int32_t i, bool there) {
+        const bool hit = part_hash(k) >> (32 - log2_parts) == blockIdx.x && there;
+        const uint64_t hits = __ballot(hit);
+        if (hits) {
+            if (hit) {
+                const uint32_t at = waiting + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(hits >> 32),
+                                                                        __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(hits), 0));
+                wait_key[at] = k;
+                wait_idx[at] = i;
+            }
+            waiting += __popcll(hits);
+            if (waiting >= 64) {
+                enter(64);
+            }
+        }
+    };
+    typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+    typedef u64x2 u64x2_a8 __attribute__((aligned(8)));
+    constexpr int kAhead = 4;
+    constexpr int32_t kStep = 2 * kPartThreads;
+    for (int32_t base = 0; base < n; base += kAhead * kStep) {
+        u64x2 k[kAhead];
+        const int32_t first = base + static_cast<int32_t>(threadIdx.x) * 2;
+        if (base + kAhead * kStep <= n) {
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a) {
+                k[a] = *reinterpret_cast<const u64x2_a8 *>(keys + first + a * kStep);
+            }
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a) {
+                look(k[a].x, first + a * kStep, true);
+                look(k[a].y, first + a * kStep + 1, true);
+            }
+        } else {
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a) {
+                const int32_t i = first + a * kStep;
+                k[a] = u64x2{i < n ? keys[i] : 0, i + 1 < n ? keys[i + 1] : 0};
+            }
+#pragma unroll
+            for (int a = 0; a < kAhead; ++a) {
+                if (base + a * kStep < n) {
+                    look(k[a].x, first + a * kStep, first + a * kStep < n);
+                    look(k[a].y, first + a * kStep + 1, first + a * kStep + 1 < n);
+                }
+            }
+        }
+    }
+    enter(waiting);
+    __syncthreads();
+    for (uint32_t s = threadIdx.x; s <= slots; s += kPartThreads) {
+        const int32_t f = s < slots ? s_first[s] : s_first_no_key;
+        if (f != INT32_MAX) {
+            flags[f] = !(saved && saved[f]);
+        }
+    }
+}
+
+// The ascending list of the set flags. A workgroup takes 1024 of them, four per thread, and counts all flags in front of its own.
+constexpr int kPartListThreads = 256;
+__global__ __launch_bounds__(kPartListThreads) void part_list_kernel(const uint32_t *__restrict__ flags4, int32_t n,
+                                                                     int32_t *__restrict__ indices, int32_t *__restrict__ d_count) {
+    __shared__ int32_t s_before[kPartListThreads / 64], s_own[kPartListThreads / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int32_t first = (blockIdx.x * kPartListThreads + threadIdx.x) * 4;
+    uint32_t mine = first < n ? flags4[first / 4] : 0;
+    if (first + 4 > n && first < n) {
+        mine &= (1u << 8 * (n - first)) - 1;
+    }
+    int32_t before = 0;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    typedef u32x4 u32x4_a8 __attribute__((aligned(8)));
+    const u32x4_a8 *const front = reinterpret_cast<const u32x4_a8 *>(flags4);
+#pragma unroll 4
+    for (int32_t i = threadIdx.x; i < static_cast<int32_t>(blockIdx.x) * kPartListThreads / 4; i += kPartListThreads) {
+        const u32x4 f = front[i];
+        before += __popc(f.x) + __popc(f.y) + __popc(f.z) + __popc(f.w);
+    }
+    const int32_t own = __popc(mine);
+    int32_t incl = own;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int32_t up = __shfl_up(incl, d, 64);
+        incl += lane >= d ? up : 0;
+        before += __shfl_xor(before, d, 64);
+    }
+    if (lane == 63) {
+        s_before[wave] = before;
+        s_own[wave] = incl;
+    }
+    __syncthreads();
+    int32_t at = incl - own;
+    for (int w = 0; w < kPartListThreads / 64; ++w) {
+        at += s_before[w] + (w < wave ? s_own[w] : 0);
+    }
+#pragma unroll
+    for (int b = 0; b < 4; ++b) {
+        if (mine >> 8 * b & 1) {
+            indices[at++] = first + b;
+        }
+    }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == kPartListThreads - 1) {
+        *d_count = at;
     }
 }
 
@@ -433,7 +630,7 @@ int64_t kvcm_hip_select_save_workspace_bytes(int64_t n) {
     if (n < 0 || n > kvcm::kListMaxKeys) {
         return KVCM_ERR_TOO_LARGE;
     }
-    // words first (8-byte aligned), then table, slots and counts
+    // words first (8-byte aligned), then table, slots and counts; up to kPartMaxKeys keys the first n bytes are flags instead
     return kvcm::list_groups(n) * (kvcm::kListWaves * 8 + 4) + (kvcm::list_capacity(n) + n) * 4;
 }
 
@@ -452,6 +649,15 @@ int32_t kvcm_hip_select_save(const int64_t *d_keys, const uint8_t *d_saved, int6
         return KVCM_ERR_ALIGNMENT;
     }
     const hipStream_t s = static_cast<hipStream_t>(stream);
+    if (n <= kvcm::kPartMaxKeys) {
+        const kvcm::PartShape p = kvcm::part_shape(n);
+        uint8_t *const flags = static_cast<uint8_t *>(d_workspace);
+        kvcm::part_kernel<<<1u << p.log2_parts, kvcm::kPartThreads, 12u << p.log2_slots, s>>>(
+            reinterpret_cast<const uint64_t *>(d_keys), static_cast<int32_t>(n), p.log2_parts, p.log2_slots, d_saved, flags);
+        kvcm::part_list_kernel<<<static_cast<unsigned>((n + 1023) / 1024), kvcm::kPartListThreads, 0, s>>>(
+            reinterpret_cast<const uint32_t *>(flags), static_cast<int32_t>(n), d_indices, d_count);
+        return kvcm::launch_status();
+    }
     const int64_t groups = kvcm::list_groups(n), cap = kvcm::list_capacity(n);
     uint64_t *words = static_cast<uint64_t *>(d_workspace);
     int32_t *table = reinterpret_cast<int32_t *>(words + groups * kvcm::kListWaves);

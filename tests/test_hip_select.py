@@ -191,3 +191,40 @@ def test_first_occurrences_where_table_and_probes_change(oracle, n, each):
     assert (got_first.cpu().numpy() == first).all() and (got_rep.cpu().numpy() == rep.astype(bool)).all()
     want = np.flatnonzero(rep == 0)
     assert int(count.item()) == len(want) and (idx[:len(want)].cpu().numpy() == want).all()
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 63, 64, 65, 511, 512, 513, 1023, 1024, 1025, 4095, 4096, 4097, 8191, 8192, 8193, 65535, 65536])
+@pytest.mark.parametrize("kind", ["different", "repeated", "one", "marker", "small", "colliding"])
+def test_save_list_from_parts(oracle, n, kind):
+    """Lists that are made from a table per workgroup: sizes around a flag word, a workgroup's 1024 flags, the steps in the number of
+    parts and the last size that takes this form; all keys alike; the value that marks an empty slot among the keys; consecutive
+    small numbers; and more different keys of one part and one slot than the part's table holds, each twice."""
+    from tair_kvcache_amd import save_selection
+    rng = np.random.default_rng(n)
+    if kind == "different":
+        keys = rng.integers(-2**63, 2**63 - 1, size=n, dtype=np.int64)
+    elif kind == "repeated":
+        keys = _keys_with_repeats(rng, n, max(1, n // 9))
+    elif kind == "one":
+        keys = np.full(n, -3, dtype=np.int64)
+    elif kind == "marker":
+        keys = np.where(rng.random(n) < 0.3, np.int64(-2**63), rng.integers(0, max(1, n // 2), size=n))
+    elif kind == "small":
+        keys = rng.permutation(n).astype(np.int64)
+    else:
+        if n > 8193:
+            pytest.skip("thousands of keys that are looked for one by one: enough of them in 8193")
+        # low word * 0x9e3779b1 + high word * 0x85ebca77 (modulo 2^32) below 2^6: one part, one slot
+        high = np.arange((n + 1) // 2, dtype=np.uint64) * 977
+        inverse = pow(0x9E3779B1, -1, 1 << 32)
+        low = ((rng.integers(0, 64, size=len(high)).astype(np.uint64) - high * np.uint64(0x85EBCA77)) & np.uint64(0xFFFFFFFF))
+        low = (low * np.uint64(inverse)) & np.uint64(0xFFFFFFFF)
+        assert ((low * np.uint64(0x9E3779B1) + high * np.uint64(0x85EBCA77)) & np.uint64(0xFFFFFFFF)).max() < 64
+        keys = rng.permutation(np.resize(((high << np.uint64(32)) | low).astype(np.int64), n))
+    mask = rng.random(n) < 0.25
+    rep = oracle.first_occurrence(keys)[1].astype(bool)
+    for m in (None, mask):
+        want = np.flatnonzero(~rep if m is None else ~(rep | m))
+        idx, count = save_selection.select_save_indices(torch.from_numpy(keys).cuda(), None if m is None else torch.from_numpy(m).cuda())
+        sync()
+        assert int(count.item()) == len(want) and (idx[:len(want)].cpu().numpy() == want).all()
