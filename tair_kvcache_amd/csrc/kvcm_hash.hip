@@ -1368,6 +1368,7 @@ __constant__ uint32_t kShaK[64] = {
     0x748f82ee, 0x78a5636f, 0x84c87814, 0x8cc70208, 0x90befffa, 0xa4506ceb, 0xbef9a3f7, 0xc67178f2};
 
 __device__ __forceinline__ uint32_t rotr(uint32_t x, int n) { return __builtin_amdgcn_alignbit(x, x, n); }
+__device__ __forceinline__ uint32_t xor3(uint32_t x, uint32_t y, uint32_t z) { return __builtin_amdgcn_bitop3_b32(x, y, z, 0x96); }
 
 // One FIPS 180-4 compression; w holds the 16 big-endian message words and is used as the rolling schedule.
 __device__ void sha256_compress(uint32_t (&st)[8], uint32_t (&w)[16]) {
@@ -1376,14 +1377,14 @@ __device__ void sha256_compress(uint32_t (&st)[8], uint32_t (&w)[16]) {
     for (int i = 0; i < 64; ++i) {
         if (i >= 16) {
             const uint32_t w15 = w[(i + 1) & 15], w2 = w[(i + 14) & 15];
-            const uint32_t s0 = rotr(w15, 7) ^ rotr(w15, 18) ^ (w15 >> 3);
-            const uint32_t s1 = rotr(w2, 17) ^ rotr(w2, 19) ^ (w2 >> 10);
+            const uint32_t s0 = xor3(rotr(w15, 7), rotr(w15, 18), w15 >> 3);
+            const uint32_t s1 = xor3(rotr(w2, 17), rotr(w2, 19), w2 >> 10);
             w[i & 15] = w[i & 15] + s0 + w[(i + 9) & 15] + s1;
         }
-        const uint32_t S1 = rotr(e, 6) ^ rotr(e, 11) ^ rotr(e, 25);
+        const uint32_t S1 = xor3(rotr(e, 6), rotr(e, 11), rotr(e, 25));
         const uint32_t ch = (e & f) ^ (~e & g);
         const uint32_t t1 = h + S1 + ch + kShaK[i] + w[i & 15];
-        const uint32_t S0 = rotr(a, 2) ^ rotr(a, 13) ^ rotr(a, 22);
+        const uint32_t S0 = xor3(rotr(a, 2), rotr(a, 13), rotr(a, 22));
         const uint32_t mj = (a & b) ^ (a & c) ^ (b & c);
         const uint32_t t2 = S0 + mj;
         h = g;
@@ -1405,53 +1406,59 @@ __device__ void sha256_compress(uint32_t (&st)[8], uint32_t (&w)[16]) {
     st[7] += h;
 }
 
-// Byte i of the padded message of length len: data, 0x80, zeros, 64-bit big-endian bit length.
-__device__ __forceinline__ uint32_t padded_byte(const uint8_t *msg, int64_t len, int64_t padded_len, int64_t i) {
-    if (i < len) {
-        return msg[i];
-    }
-    if (i == len) {
-        return 0x80u;
-    }
-    if (i >= padded_len - 8) {
-        const uint64_t bits = static_cast<uint64_t>(len) * 8u;
-        return static_cast<uint32_t>((bits >> (8 * (padded_len - 1 - i))) & 0xffu);
-    }
-    return 0u;
-}
-
 // One lane per string: key = big-endian signed int64 of SHA-256(bytes)[0:8]
 // (kv_cache_manager/py_connector/sglang/connector.py:397-401).
+// Bound: a compression is 1400 instructions of 4 clocks, one after the other, 2.6 us with what surrounds it, and a string of 64
+// characters takes two. What lies in a block is read as words, only the word that holds the message's end byte by byte, and three
+// operands are xored at a time. us a launch, before / now: 1024 or 16 384 strings of 64 characters 10.4 / 8.0, of 16: 8.0 / 5.4, 1024 of
+// 1 to 200: 32.9 / 20.5. The bytes may lie in pinned host memory: 1024 strings of 64 characters 11.1.
 __global__ __launch_bounds__(64) void sha256_first8_kernel(const uint8_t *__restrict__ bytes,
                                                            const int64_t *__restrict__ offsets, int32_t N,
                                                            int64_t *__restrict__ out) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= N) {
-        return;
-    }
+    // lanes beyond the last string go through it as well: a wave with few active lanes issues more slowly
+    const int64_t lane = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x, i = lane < N ? lane : N - 1;
     const uint8_t *msg = bytes + offsets[i];
     const int64_t len = offsets[i + 1] - offsets[i];
-    const int64_t padded_len = ((len + 8) / 64 + 1) * 64;
     uint32_t st[8] = {0x6a09e667, 0xbb67ae85, 0x3c6ef372, 0xa54ff53a, 0x510e527f, 0x9b05688c, 0x1f83d9ab, 0x5be0cd19};
-    for (int64_t base = 0; base < padded_len; base += 64) {
+    const int64_t blocks = (len + 8) / 64 + 1;
+    for (int64_t k = 0; k < blocks; ++k) {
         uint32_t w[16];
-        if (base + 64 <= len) {  // nothing but message: words instead of bytes, a quarter of the loads and no compare per byte
-            __builtin_memcpy(w, msg + base, 64);
+        const uint8_t *const at = msg + k * 64;
+        if (k * 64 + 64 <= len) {
+            __builtin_memcpy(w, at, 64);
 #pragma unroll
             for (int j = 0; j < 16; ++j) {
                 w[j] = __builtin_bswap32(w[j]);
             }
         } else {
+            const int32_t left = static_cast<int32_t>(len - k * 64);  // message bytes in this block; below 0 in a block behind its end
+            uint32_t end = 0;  // the word behind the whole ones: up to three bytes and the terminating bit
+            if (left >= 0) {
+                const int32_t n = left & 3;
+                const uint8_t *const rest = at + (left - n);
+                end = n > 0 ? static_cast<uint32_t>(rest[0]) << 24 : 0;
+                end |= n > 1 ? static_cast<uint32_t>(rest[1]) << 16 : 0;
+                end |= n > 2 ? static_cast<uint32_t>(rest[2]) << 8 : 0;
+                end |= 0x80000000u >> 8 * n;
+            }
 #pragma unroll
             for (int j = 0; j < 16; ++j) {
-                const int64_t p = base + 4 * j;
-                w[j] = (padded_byte(msg, len, padded_len, p) << 24) | (padded_byte(msg, len, padded_len, p + 1) << 16) |
-                       (padded_byte(msg, len, padded_len, p + 2) << 8) | padded_byte(msg, len, padded_len, p + 3);
+                uint32_t v = 0;
+                if (4 * j + 4 <= left) {
+                    __builtin_memcpy(&v, at + 4 * j, 4);
+                }
+                w[j] = left >= 0 && left >> 2 == j ? end : __builtin_bswap32(v);
+            }
+            if (k + 1 == blocks) {
+                w[14] = static_cast<uint32_t>(static_cast<uint64_t>(len) >> 29);
+                w[15] = static_cast<uint32_t>(len) << 3;
             }
         }
         sha256_compress(st, w);
     }
-    out[i] = static_cast<int64_t>((static_cast<uint64_t>(st[0]) << 32) | st[1]);
+    if (lane < N) {
+        out[i] = static_cast<int64_t>((static_cast<uint64_t>(st[0]) << 32) | st[1]);
+    }
 }
 
 // ------------------------------------------------------------------------------------------- iov CRC-32

@@ -178,16 +178,16 @@ static PyObject *blocks_idx(PyObject *self, PyObject *args) {
     return out;
 }
 
-/* Bytes of a str in UTF-8, written to dst unless that is NULL; -1 with an exception set. ASCII, which is what hash strings are,
+/* Bytes of a str in UTF-8, written to dst unless that is NULL or has no room for them; -1 with an exception set. ASCII, which is what hash strings are,
  * is copied as it lies there; anything else is encoded into an object of its own, because PyUnicode_AsUTF8 would leave its
  * bytes attached to the caller's string for as long as that lives. */
-static Py_ssize_t utf8(PyObject *s, char *dst) {
+static Py_ssize_t utf8(PyObject *s, char *dst, Py_ssize_t room) {
     if (PyUnicode_READY(s) < 0) {
         return -1;
     }
     if (PyUnicode_IS_COMPACT_ASCII(s)) {
         const Py_ssize_t len = PyUnicode_GET_LENGTH(s);
-        if (dst) {
+        if (dst && len <= room) {
             memcpy(dst, PyUnicode_DATA(s), (size_t)len);
         }
         return len;
@@ -197,77 +197,157 @@ static Py_ssize_t utf8(PyObject *s, char *dst) {
         return -1;
     }
     const Py_ssize_t len = PyBytes_GET_SIZE(bytes);
-    if (dst) {
+    if (dst && len <= room) {
         memcpy(dst, PyBytes_AS_STRING(bytes), (size_t)len);
     }
     Py_DECREF(bytes);
     return len;
 }
 
-/* pack_strings(seq) -> bytearray: int64 offsets [n + 1], then the items' bytes (UTF-8 of a str) back to back, then one spare
- * byte; None when an item is neither exactly str nor exactly bytes (the caller then goes the general way). One buffer, so
- * that strings and offsets reach the device in one copy; 1024 strings of 64 characters take 8 us here, 70 us as a list of
- * encoded strings, a tensor of lengths and a join. UnicodeEncodeError for a str that UTF-8 cannot hold, as str.encode. */
+/* Bytes that `seq` takes packed: int64 offsets [n + 1], then the items' bytes (UTF-8 of a str) back to back, then one spare byte.
+ * 0 when an item is neither exactly str nor exactly bytes; -1 with an exception set, UnicodeEncodeError for a str that UTF-8
+ * cannot hold, as str.encode. */
+static Py_ssize_t packed_size(PyObject *seq) {
+    const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
+    PyObject **items = PySequence_Fast_ITEMS(seq);
+    if (n > (PY_SSIZE_T_MAX - 16) / 8) {
+        PyErr_SetString(PyExc_OverflowError, "too many strings");
+        return -1;
+    }
+    Py_ssize_t total = 8 * (n + 1) + 1;
+    for (Py_ssize_t i = 0; i < n; ++i) {
+        Py_ssize_t len;
+        if (PyUnicode_CheckExact(items[i])) {
+            len = utf8(items[i], NULL, 0);
+            if (len < 0) {
+                return -1;
+            }
+        } else if (PyBytes_CheckExact(items[i])) {
+            len = PyBytes_GET_SIZE(items[i]);
+        } else {
+            return 0;
+        }
+        if (len > PY_SSIZE_T_MAX - total) {
+            PyErr_SetString(PyExc_OverflowError, "strings too long");
+            return -1;
+        }
+        total += len;
+    }
+    return total;
+}
+
+/* Packs `seq` into the `size` bytes at `base`: 1, 0 when it does not take exactly that many (any more), -1 with an exception set. */
+static int pack(PyObject *seq, char *base, Py_ssize_t size) {
+    const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
+    PyObject **items = PySequence_Fast_ITEMS(seq);
+    if (n > (size - 9) / 8) {
+        return 0;
+    }
+    char *dst = base + 8 * (n + 1);
+    const Py_ssize_t room = size - 8 * (n + 1) - 1;
+    int64_t off = 0;
+    memcpy(base, &off, 8);
+    for (Py_ssize_t i = 0; i < n; ++i) {
+        Py_ssize_t len;
+        if (PyUnicode_CheckExact(items[i])) {
+            len = utf8(items[i], dst + off, room - off);
+            if (len < 0) {
+                return -1;
+            }
+        } else if (PyBytes_CheckExact(items[i])) {
+            len = PyBytes_GET_SIZE(items[i]);
+            if (len <= room - off) {
+                memcpy(dst + off, PyBytes_AS_STRING(items[i]), (size_t)len);
+            }
+        } else {
+            return 0;
+        }
+        if (len > room - off) {
+            return 0;
+        }
+        off += len;
+        memcpy(base + 8 * (i + 1), &off, 8);
+    }
+    dst[off] = 0;
+    return off == room;
+}
+
+/* strings_size(seq) -> bytes that `seq` takes packed, or None when an item is neither exactly str nor exactly bytes (the caller then
+ * goes the general way). */
+static PyObject *strings_size(PyObject *self, PyObject *seq) {
+    (void)self;
+    if (!is_seq(seq)) {
+        PyErr_SetString(PyExc_TypeError, "strings_size takes a list or tuple");
+        return NULL;
+    }
+    const Py_ssize_t size = packed_size(seq);
+    if (size < 0) {
+        return NULL;
+    }
+    if (size == 0) {
+        Py_RETURN_NONE;
+    }
+    return PyLong_FromSsize_t(size);
+}
+
+/* pack_strings_into(seq, address, size) -> number of strings that now lie there, or None when `seq` does not take exactly `size` bytes
+ * (any more: the list may have changed since it was measured). */
+static PyObject *pack_strings_into(PyObject *self, PyObject *args) {
+    (void)self;
+    PyObject *seq;
+    unsigned long long address;
+    Py_ssize_t size;
+    if (!PyArg_ParseTuple(args, "OKn", &seq, &address, &size)) {
+        return NULL;
+    }
+    if (!is_seq(seq)) {
+        PyErr_SetString(PyExc_TypeError, "pack_strings_into takes a list or tuple");
+        return NULL;
+    }
+    const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
+    const int done = pack(seq, (char *)(uintptr_t)address, size);
+    if (done < 0) {
+        return NULL;
+    }
+    if (!done) {
+        Py_RETURN_NONE;
+    }
+    return PyLong_FromSsize_t(n);
+}
+
+/* pack_strings(seq) -> the same in a bytearray, or None when an item is neither exactly str nor exactly bytes. One buffer, so that
+ * strings and offsets reach the device in one copy; 1024 strings of 64 characters take 8 us here, 70 us as a list of encoded
+ * strings, a tensor of lengths and a join. */
 static PyObject *pack_strings(PyObject *self, PyObject *seq) {
     (void)self;
     if (!is_seq(seq)) {
         PyErr_SetString(PyExc_TypeError, "pack_strings takes a list or tuple");
         return NULL;
     }
-    const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
-    PyObject **items = PySequence_Fast_ITEMS(seq);
-    if (n > (PY_SSIZE_T_MAX - 16) / 8) {
-        PyErr_SetString(PyExc_OverflowError, "too many strings");
+    const Py_ssize_t size = packed_size(seq);
+    if (size < 0) {
         return NULL;
     }
-    Py_ssize_t total = 8 * (n + 1) + 1;
-    for (Py_ssize_t i = 0; i < n; ++i) {
-        Py_ssize_t len;
-        if (PyUnicode_CheckExact(items[i])) {
-            len = utf8(items[i], NULL);
-            if (len < 0) {
-                return NULL;
-            }
-        } else if (PyBytes_CheckExact(items[i])) {
-            len = PyBytes_GET_SIZE(items[i]);
-        } else {
-            Py_RETURN_NONE;
-        }
-        if (len > PY_SSIZE_T_MAX - total) {
-            PyErr_SetString(PyExc_OverflowError, "strings too long");
-            return NULL;
-        }
-        total += len;
+    if (size == 0) {
+        Py_RETURN_NONE;
     }
-    PyObject *out = PyByteArray_FromStringAndSize(NULL, total);
+    PyObject *out = PyByteArray_FromStringAndSize(NULL, size);
     if (!out) {
         return NULL;
     }
-    char *base = PyByteArray_AS_STRING(out), *dst = base + 8 * (n + 1);
-    int64_t off = 0;
-    memcpy(base, &off, 8);
-    for (Py_ssize_t i = 0; i < n; ++i) {
-        Py_ssize_t len;
-        if (PyUnicode_CheckExact(items[i])) {
-            len = utf8(items[i], dst + off);
-            if (len < 0) {
-                Py_DECREF(out);
-                return NULL;
-            }
-        } else {
-            len = PyBytes_GET_SIZE(items[i]);
-            memcpy(dst + off, PyBytes_AS_STRING(items[i]), (size_t)len);
-        }
-        off += len;
-        memcpy(base + 8 * (i + 1), &off, 8);
+    if (pack(seq, PyByteArray_AS_STRING(out), size) < 0) {
+        Py_DECREF(out);
+        return NULL;
     }
-    dst[off] = 0;
     return out;
 }
 
 static PyMethodDef methods[] = {
     {"pack_strings", pack_strings, METH_O,
      "list or tuple of str or bytes -> bytearray of int64 offsets [n + 1], the bytes, and one spare byte, or None"},
+    {"strings_size", strings_size, METH_O, "list or tuple of str or bytes -> bytes that it takes packed, or None"},
+    {"pack_strings_into", pack_strings_into, METH_VARARGS,
+     "(list or tuple of str or bytes, address, size) -> number of strings that now lie there packed, or None if the size is another"},
     {"blocks_idx", blocks_idx, METH_VARARGS,
      "(manager_block_idxes, local_block_ids, manager_block_size, local_block_size) -> bytes of int32 token slots, or None"},
     {"pack_i32", pack_i32, METH_O, "list or tuple of ints (or of lists of ints) -> bytes of native int32"},

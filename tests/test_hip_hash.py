@@ -688,3 +688,38 @@ def test_sixteen_requests_per_workgroup(oracle, force_general_hash_loader, gener
         keys, off = _h().hash_tokens(dev(tok), bs, seed=-1)
         sync()
         assert (host(keys, np.int64) == want).all() and (host(off, np.int64) == woff).all(), (R, L, bs)
+
+
+def test_hash_strings_that_wait_behind_other_work(monkeypatch):
+    """Calls whose strings the kernel has yet to read when the next ones arrive: more of them than are read in place, from two
+    threads, strings of many lengths; then more bytes than are read in place; and nothing stays lent out."""
+    import threading
+    h = _h()
+    monkeypatch.setattr(h, "_LENT_MOST", 8)
+
+    def key(s):
+        return int.from_bytes(hashlib.sha256(s.encode()).digest()[:8], "big", signed=True)
+
+    got = {}
+
+    def many(t):
+        torch.cuda._sleep(2_000_000)
+        for i in range(20):
+            strs = [chr(97 + (i + k) % 26) * ((7 * i + 13 * k + t) % 140) for k in range(1 + 11 * i)]
+            got[t, i] = (strs, h.sha256_to_int64(strs))
+
+    threads = [threading.Thread(target=many, args=(t,)) for t in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    sync()
+    assert len(got) == 40
+    for strs, keys in got.values():
+        assert keys.tolist() == [key(s) for s in strs]
+    monkeypatch.setattr(h, "_PINNED_MOST", 100)
+    assert h.sha256_to_int64(["x" * 200, "y"]).tolist() == [key("x" * 200), key("y")]
+    monkeypatch.undo()
+    h.sha256_to_int64(["z"])
+    sync()
+    assert h._settled_event(torch.device("cuda:0")) is not None and not h._lent

@@ -452,3 +452,25 @@ def test_a_pinned_word_is_kept_when_its_stream_cannot_be_waited_for(monkeypatch)
     Stream.fails = False
     hashing._settle(word, "cuda")
     assert not hashing._owed
+
+
+def test_hash_strings_are_packed_where_the_caller_says():
+    """strings_size / pack_strings_into: what pack_strings gives, at an address, if the list still takes exactly as many bytes; nothing
+    beyond them is written."""
+    import ctypes
+    from tair_kvcache_amd._kvcm_pylist import pack_strings, pack_strings_into, strings_size
+    for form in (["a", "bb", ""], ("x", b"yy", "é漢" * 5), [], [""], [b"q" * 100] * 3):
+        want = bytes(pack_strings(form))
+        assert strings_size(form) == len(want)
+        room = ctypes.create_string_buffer(b"\x55" * (len(want) + 8), len(want) + 8)
+        assert pack_strings_into(form, ctypes.addressof(room), len(want)) == len(form)
+        assert room.raw == want + b"\x55" * 8
+        for size in range(max(0, len(want) - 12), len(want) + 8):
+            if size != len(want):
+                assert pack_strings_into(form, ctypes.addressof(room), size) is None
+                assert room.raw[max(size, len(want)):] == b"\x55" * (len(want) + 8 - max(size, len(want)))
+    assert strings_size([1]) is None and strings_size(["a", bytearray(b"b")]) is None
+    with pytest.raises(UnicodeEncodeError):
+        strings_size(["\ud800"])
+    with pytest.raises(TypeError):
+        strings_size("abc")
