@@ -4,8 +4,14 @@ import torch
 from . import _lib
 
 
+# torch's own short cut to the handle of a device's current stream, without the Stream object around it (2.0 us a call, 0.2 so)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(device):
     """The current torch stream of `device` as the void* the C-ABI takes."""
+    if _raw_stream is not None and device.type == "cuda" and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
