@@ -92,6 +92,18 @@ int32_t kvcm_hip_hash_tokens_checked(const void *d_tokens, int32_t token_bytes, 
                                      int64_t *d_keys, int64_t n_keys, const int64_t *d_key_offsets, kvcm_stream_t stream);
 
 /*
+ * Added to token_bytes above, for 1 to KVCM_COUNT_KEYS_UP_TO requests: the launch makes the key offsets itself, as
+ * kvcm_hip_key_offsets_checked would have in front of it. d_key_offsets is then the address of a kvcm_key_count in HOST memory,
+ * which is read before the call returns; kvcm_wait_value() waits for h_total, which is written while the keys are being computed.
+ */
+#define KVCM_COUNT_KEYS 0x100
+#define KVCM_COUNT_KEYS_UP_TO 4096
+typedef struct kvcm_key_count {
+    int64_t *d_key_offsets; /* receives R + 1 offsets, -1 for a request that is left out */
+    int64_t *h_total;       /* pinned host memory: KVCM_PENDING, then the sum of all requests or -1 */
+} kvcm_key_count;
+
+/*
  * The same for R requests of one length, laid out one behind the other ([R][tokens_per_request], token_bytes = 4 or 8):
  * no offset arrays are read. d_key_offsets may be NULL (request r's keys start at r * (tokens_per_request / block_size));
  * d_key_offsets_out, when not NULL, receives those R + 1 offsets. tokens_per_request must be at least block_size.

@@ -48,6 +48,14 @@ class IovDevice(C.Structure):
     _fields_ = [("base", vp), ("size", sz)]
 
 
+class KeyCount(C.Structure):
+    """struct kvcm_key_count."""
+    _fields_ = [("d_key_offsets", vp), ("h_total", vp)]
+
+
+COUNT_KEYS = 0x100  # KVCM_COUNT_KEYS
+COUNT_KEYS_UP_TO = 4096  # KVCM_COUNT_KEYS_UP_TO
+
 # symbol -> (restype, argtypes); every prototype of include/kvcm_hip.h
 SIGNATURES = {
     "kvcm_hip_version": (i32, []),

@@ -63,25 +63,6 @@ constexpr int kThreads = KVCM_COPY_THREADS;
 constexpr int kCPT = KVCM_COPY_CHUNKS_PER_THREAD;  // chunks per thread per span
 constexpr uint32_t kSpan = static_cast<uint32_t>(kThreads) * kCPT;
 
-// n / d for n < 2^31 as a multiply and a shift: mul = ceil(2^(31+L) / d), L = ceil(log2 d).
-struct FastDiv {
-    uint32_t mul;
-    uint32_t shift;
-};
-
-FastDiv make_fastdiv(uint32_t d) {
-    uint32_t L = 0;
-    while ((uint64_t{1} << L) < d) {
-        ++L;
-    }
-    const uint64_t pow = uint64_t{1} << (31 + L);
-    return FastDiv{static_cast<uint32_t>((pow + d - 1) / d), 31 + L};
-}
-
-__device__ __forceinline__ uint32_t fast_div(uint32_t n, FastDiv f) {
-    return static_cast<uint32_t>((static_cast<uint64_t>(n) * f.mul) >> f.shift);
-}
-
 struct CopyArgs {
     unsigned char *staging;
     int64_t entry_stride;

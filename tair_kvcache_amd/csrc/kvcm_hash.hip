@@ -804,11 +804,25 @@ constexpr int64_t kOffsetsPerWg = kOffsetsThreads * kOffsetsPerThread;
 constexpr int32_t kOffsetsRereadUpTo = 32768;
 int64_t offsets_groups(int32_t R) { return (R + kOffsetsPerWg - 1) / kOffsetsPerWg; }
 
+// For launches that count their keys themselves (hash_lean_kernel): where the offsets and the total go, or NULL twice.
+struct CountOut {
+    int64_t *key_offsets;  // [R + 1]
+    int64_t *h_total;      // pinned
+    FastDiv by_block;      // n / block size for n < 2^31
+};
+
 __device__ __forceinline__ int64_t keys_of(int64_t len, int32_t block_size) {
     if (static_cast<uint64_t>(len) >> 32 == 0) {  // 32-bit division: a fifth of the instructions
         return static_cast<uint32_t>(len) / static_cast<uint32_t>(block_size);
     }
     return len > 0 ? len / block_size : 0;
+}
+
+// Keys of one request; `bad` is set when the tokens they are made of are not all there.
+__device__ __forceinline__ int64_t keys_of_request(int64_t at, int64_t next, int32_t block_size, int64_t n_tokens, bool &bad) {
+    const int64_t count = keys_of(distance(at, next), block_size);
+    bad |= n_tokens != kUnknown && count > 0 && !inside(at, count * block_size, n_tokens);
+    return count;
 }
 
 // ------------------------------------------------------------------------------------------- few requests per workgroup
@@ -1057,6 +1071,94 @@ __device__ __forceinline__ void lean_write(LeanShared<EVERY> &sh, int32_t nt, co
     }
 }
 
+// Keys of the requests [base, base + kAhead * 128) in front of r_first, a pair of requests per lane and load.
+template <int kAhead>
+__device__ __forceinline__ int64_t lean_keys_of(const int64_t *__restrict__ token_offsets, int64_t base, int64_t r_first,
+                                                int32_t block_size, const Extent &have, const FastDiv by_block, uint32_t lane,
+                                                bool &bad) {
+    typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+    typedef u64x2 u64x2_a8 __attribute__((aligned(8)));
+    static_assert(kLeanRows % 2 == 0, "lanes take requests in pairs");
+    u64x2 from[kAhead];
+    uint64_t to[kAhead];
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+        const int64_t i = base + j * 128 + lane * 2;
+        from[j] = u64x2{0, 0};
+        to[j] = 0;
+        if (i < r_first) {
+            from[j] = *reinterpret_cast<const u64x2_a8 *>(token_offsets + i);
+            to[j] = static_cast<uint64_t>(token_offsets[i + 2]);
+        }
+    }
+    bool odd = false;  // beyond the tokens or longer than the short division takes: looked at again, one by one
+    int64_t sum = 0;
+#pragma unroll
+    for (int j = 0; j < kAhead; ++j) {
+        const uint64_t len0 = from[j].y - from[j].x, len1 = to[j] - from[j].y;
+        odd |= to[j] > static_cast<uint64_t>(have.tokens) || from[j].y > to[j] || from[j].x > from[j].y || (len0 | len1) >> 31 != 0;
+        sum += fast_div(static_cast<uint32_t>(len0), by_block) + fast_div(static_cast<uint32_t>(len1), by_block);
+    }
+    if (__ballot(odd) != 0) {
+        sum = 0;
+        for (int j = 0; j < kAhead; ++j) {
+            const int64_t i = base + j * 128 + lane * 2;
+            for (int64_t k = i; k < i + 2 && k < r_first; ++k) {
+                sum += keys_of_request(token_offsets[k], token_offsets[k + 1], block_size, have.tokens, bad);
+            }
+        }
+    }
+    return sum;
+}
+
+// Keys of all requests in front of a workgroup, added up by its writer wave while the loaders wait for their first tokens, so that
+// no launch has to make the offsets first and nobody waits for another workgroup. Bound by trips to the caches, for the offsets and,
+// with few requests, for the instructions: 2048 requests unrolled, whatever their number, cost 1 us more at 30 to 1000 of them.
+// us a call that waits for the total, a launch for the offsets in front / here: 160 requests of 48 to 8192 4-byte tokens 94.2 / 90.9,
+// 4 of 162 to 1296 20.7 / 17.6, 1500 of 700 to 1400 23.2 / 19.8, 4096 of 500 to 4096 in blocks of 24 55.1 / 51.2.
+__device__ __forceinline__ int64_t lean_keys_before(const int64_t *__restrict__ token_offsets, int64_t r_first, int32_t block_size,
+                                                    const Extent &have, const FastDiv by_block, uint32_t lane, bool &bad) {
+    constexpr int kMany = 8, kFew = 2;
+    int64_t before = 0, base = 0;
+    for (; r_first - base > kMany * 64; base += kMany * 128) {
+        before += lean_keys_of<kMany>(token_offsets, base, r_first, block_size, have, by_block, lane, bad);
+    }
+    for (; base < r_first; base += kFew * 128) {
+        before += lean_keys_of<kFew>(token_offsets, base, r_first, block_size, have, by_block, lane, bad);
+    }
+    return before;
+}
+
+// The key offsets of a workgroup's requests, and of the last one the total. before: this lane's share of the keys in front.
+__device__ __forceinline__ void lean_key_offsets(int64_t r_first, int32_t R, int64_t before, int64_t own, bool bad_before, bool bad,
+                                                 const Extent &have, const CountOut &out, uint32_t lane, LeanRow &row, int64_t &count) {
+    const int64_t r = r_first + lane;
+    const bool mine = lane < kLeanRows && r < R;
+    own = mine ? own : 0;
+    int64_t incl = own;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int64_t up = __shfl_up(incl, d, 64);
+        incl += static_cast<int>(lane) >= d ? up : 0;
+        before += __shfl_xor(before, d, 64);
+    }
+    const int64_t key = before + incl - own;
+    const bool any = __ballot(bad_before || (mine && bad)) != 0;
+    // without its tokens, or beyond the room the caller has: marked, and left out
+    const bool fits = !bad && key + own <= have.keys;
+    if (mine) {
+        out.key_offsets[r] = fits ? key : -1;
+        if (r == R - 1) {
+            out.key_offsets[R] = key + own;
+            // relaxed: whoever waits for it reads nothing else by it (a release writes the whole L2 back first)
+            __hip_atomic_store(out.h_total, any ? -1 : key + own, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+    // every lane knows request lane % 16
+    row.key = shfl_i64(key, lane % kLeanRows);
+    const int64_t n = shfl_i64(fits ? own : 0, lane % kLeanRows);
+    count = row.ntok > 0 ? n : 0;
+}
+
 // The same for block size 1, where every state is a key: 512 bytes of a request at a time, 16 per lane.
 __device__ __forceinline__ void lean_write_all(LeanShared<true> &sh, int32_t nt, const LeanRow &row, int64_t count,
                                                int64_t *__restrict__ keys, uint32_t lane) {
@@ -1113,7 +1215,7 @@ __global__ __launch_bounds__(kLeanThreads) void hash_lean_kernel(const TokT *__r
                                                                  const int64_t *__restrict__ token_offsets, int32_t R,
                                                                  int32_t block_size, uint64_t seed, int64_t *__restrict__ keys,
                                                                  const int64_t *__restrict__ key_offsets, const Uniform uni,
-                                                                 const Extent have, int32_t force_global_loads) {
+                                                                 const Extent have, const CountOut out, int32_t force_global_loads) {
     using SH = LeanShared<EVERY>;
     __shared__ __attribute__((aligned(16))) SH sh;
     const uint32_t lane = threadIdx.x & 63u;
@@ -1132,17 +1234,27 @@ __global__ __launch_bounds__(kLeanThreads) void hash_lean_kernel(const TokT *__r
         if (known && (first < 0 || first > total)) {
             first = first < 0 ? 0 : total;
         }
-        if (r < R) {
-            const int64_t at = token_offsets[r];
-            const int64_t nkeys = keys_of(distance(at, token_offsets[r + 1]), block_size);
-            row.key = key_offsets ? key_offsets[r] : r * keys_of(distance(token_offsets[0], token_offsets[1]), block_size);
-            if (inside(row.key, nkeys, have.keys) && (!known || inside(at, nkeys * block_size, total))) {
-                row.start = at;
-                row.ntok = nkeys * block_size;
-                count = nkeys;
-            }
+        const int64_t at = token_offsets[r < R ? r : R], next = token_offsets[r < R ? r + 1 : R];
+        const bool counts = out.key_offsets && wave == kLeanWriter;
+        int64_t before = 0;
+        bool bad_before = false;
+        if (counts) {
+            before = lean_keys_before(token_offsets, r_first, block_size, have, out.by_block, lane, bad_before);
+        }
+        const int64_t nkeys = keys_of(distance(at, next), block_size);
+        const bool there = !known || inside(at, nkeys * block_size, total);
+        // where the keys go is the writer's business alone if this launch counts them
+        row.key = out.key_offsets ? 0 : key_offsets ? key_offsets[r < R ? r : 0]
+                                                    : r * keys_of(distance(token_offsets[0], token_offsets[1]), block_size);
+        if (r < R && (out.key_offsets || inside(row.key, nkeys, have.keys)) && there) {
+            row.start = at;
+            row.ntok = nkeys * block_size;
+            count = nkeys;
         }
         nt = static_cast<int32_t>(wave_max_u32(static_cast<uint32_t>((row.ntok + kLeanTok - 1) / kLeanTok)));
+        if (counts) {
+            lean_key_offsets(r_first, R, before, nkeys, bad_before, nkeys > 0 && !there, have, out, lane, row, count);
+        }
     } else {
         first = r_first * uni.tokens;
         total = R * uni.tokens;
@@ -1239,13 +1351,6 @@ __global__ __launch_bounds__(kLeanThreads) void hash_lean_kernel(const TokT *__r
     if (EVERY) {
         lds_barrier();
     }
-}
-
-// Keys of one request; `bad` is set when the tokens they are made of are not all there.
-__device__ __forceinline__ int64_t keys_of_request(int64_t at, int64_t next, int32_t block_size, int64_t n_tokens, bool &bad) {
-    const int64_t count = keys_of(distance(at, next), block_size);
-    bad |= n_tokens != kUnknown && count > 0 && !inside(at, count * block_size, n_tokens);
-    return count;
 }
 
 // sums[g] = keys of the requests of workgroup g of key_offsets_kernel, as its complement if one of them is bad
@@ -1348,7 +1453,7 @@ __global__ __launch_bounds__(kOffsetsThreads) void key_offsets_kernel(const int6
             if (first + j == R - 1) {
                 key_offsets[R] = pos;
                 if (h_total) {  // the last workgroup has seen every request
-                    __hip_atomic_store(h_total, some ? -1 : pos, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+                    __hip_atomic_store(h_total, some ? -1 : pos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
                 }
             }
         }
@@ -1588,6 +1693,7 @@ constexpr int64_t burst_from_tokens(int32_t block_size, bool tokens_8_byte, bool
 // second one on a unit shares its SIMDs, and one of 16 reads 512 bytes of each of 16 requests at a time where the other kernel
 // reads 64. us, 16 per workgroup / 64: 4096 requests of 4096 tokens 49.2 / 55.8, 5120: 59.0 / 56.8, 8192: 71.4 / 59.9.
 constexpr int32_t kLeanUpTo = 256 * kLeanRows;
+static_assert(KVCM_COUNT_KEYS_UP_TO == kLeanUpTo, "only hash_lean_kernel counts keys");
 #ifndef KVCM_HASH_BURST_SCALE  // for experiments: 0 = burst wherever it exists, a large number = never
 #define KVCM_HASH_BURST_SCALE 1
 #endif
@@ -1595,7 +1701,8 @@ constexpr int32_t kLeanUpTo = 256 * kLeanRows;
 template <typename TokT>
 int32_t launch_hash(const TokT *d_tokens, const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t seed,
                     int64_t *d_keys, const int64_t *d_key_offsets, hipStream_t stream,
-                    const Uniform &uni = Uniform{0, 0, nullptr}, const Extent &have = Extent{kUnknown, kUnknown}) {
+                    const Uniform &uni = Uniform{0, 0, nullptr}, const Extent &have = Extent{kUnknown, kUnknown},
+                    const CountOut &out = CountOut{nullptr, nullptr, {0, 0}}) {
     if (R < 0 || block_size <= 0) {
         return KVCM_ERR_INVALID_ARG;
     }
@@ -1611,10 +1718,10 @@ int32_t launch_hash(const TokT *d_tokens, const int64_t *d_token_offsets, int32_
         const dim3 lean_grid(static_cast<uint32_t>((static_cast<int64_t>(R) + kLeanRows - 1) / kLeanRows));
         if (block_size % kLeanStride == 0) {
             hipLaunchKernelGGL((hash_lean_kernel<TokT, false>), lean_grid, dim3(kLeanThreads), 0, stream, d_tokens, d_token_offsets, R,
-                               block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, have, force_global);
+                               block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, have, out, force_global);
         } else {
             hipLaunchKernelGGL((hash_lean_kernel<TokT, true>), lean_grid, dim3(kLeanThreads), 0, stream, d_tokens, d_token_offsets, R,
-                               block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, have, force_global);
+                               block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, have, out, force_global);
         }
         return launch_status();
     }
@@ -1753,17 +1860,36 @@ int32_t kvcm_hip_hash_tokens_2d(const void *d_tokens, int32_t token_bytes, int32
 int32_t kvcm_hip_hash_tokens_checked(const void *d_tokens, int32_t token_bytes, int64_t n_tokens,
                                      const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t seed,
                                      int64_t *d_keys, int64_t n_keys, const int64_t *d_key_offsets, kvcm_stream_t stream) {
+    const bool counts = (token_bytes & KVCM_COUNT_KEYS) != 0;
+    token_bytes &= ~KVCM_COUNT_KEYS;
     if ((token_bytes != 4 && token_bytes != 8) || n_tokens < 0 || n_keys < 0) {
         return KVCM_ERR_INVALID_ARG;
+    }
+    kvcm::CountOut out{nullptr, nullptr, {0, 0}};
+    if (counts) {
+        const kvcm_key_count *const to = reinterpret_cast<const kvcm_key_count *>(d_key_offsets);
+        if (R <= 0 || block_size <= 0 || !d_tokens || !d_token_offsets || !d_keys || !to || !to->d_key_offsets || !to->h_total) {
+            return KVCM_ERR_INVALID_ARG;
+        }
+        if (R > KVCM_COUNT_KEYS_UP_TO) {
+            return KVCM_ERR_TOO_LARGE;
+        }
+        // recorded into a graph the launch would write h_total at every replay, long after the caller has given it back
+        if (kvcm::is_capturing(static_cast<hipStream_t>(stream))) {
+            return static_cast<int32_t>(hipErrorStreamCaptureUnsupported);
+        }
+        *to->h_total = KVCM_PENDING;
+        out = kvcm::CountOut{to->d_key_offsets, to->h_total, kvcm::make_fastdiv(static_cast<uint32_t>(block_size))};
+        d_key_offsets = nullptr;
     }
     const kvcm::Uniform no{0, 0, nullptr};
     const kvcm::Extent have{n_tokens, n_keys};
     if (token_bytes == 8) {
         return kvcm::launch_hash<int64_t>(static_cast<const int64_t *>(d_tokens), d_token_offsets, R, block_size, seed, d_keys,
-                                          d_key_offsets, static_cast<hipStream_t>(stream), no, have);
+                                          d_key_offsets, static_cast<hipStream_t>(stream), no, have, out);
     }
     return kvcm::launch_hash<int32_t>(static_cast<const int32_t *>(d_tokens), d_token_offsets, R, block_size, seed, d_keys,
-                                      d_key_offsets, static_cast<hipStream_t>(stream), no, have);
+                                      d_key_offsets, static_cast<hipStream_t>(stream), no, have, out);
 }
 
 int64_t kvcm_hip_key_offsets_workspace_bytes(int32_t R) {

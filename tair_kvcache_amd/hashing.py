@@ -9,6 +9,7 @@
 A connector that computes keys here can send `block_keys` instead of `token_ids`; the manager prefers them
 (kv_cache_manager/manager/cache_manager.cc:306-318) and the keys are bit-identical to the ones it would compute.
 """
+import ctypes
 import threading
 from array import array
 from collections import deque
@@ -117,9 +118,14 @@ def _launch_offsets(tokens, off, R, block_size, n_keys, key_offsets, pending, st
         _lib.check(rc, "kvcm_hip_key_offsets_checked")
 
 
-def _launch_keys(tokens, off, R, block_size, seed, keys, key_offsets, stream):
-    rc = lib().kvcm_hip_hash_tokens_checked(tokens.data_ptr(), tokens.element_size(), tokens.numel(), off.data_ptr(), R,
-                                            block_size, int(seed), keys.data_ptr(), keys.numel(), key_offsets.data_ptr(), stream)
+def _launch_keys(tokens, off, R, block_size, seed, keys, key_offsets, stream, pending=None):
+    """With `pending` the launch writes key_offsets, and their last into that pinned word, itself."""
+    token_bytes, at = tokens.element_size(), key_offsets.data_ptr()
+    if pending is not None:
+        token_bytes |= _lib.COUNT_KEYS
+        at = ctypes.byref(_lib.KeyCount(at, pending.data_ptr()))
+    rc = lib().kvcm_hip_hash_tokens_checked(tokens.data_ptr(), token_bytes, tokens.numel(), off.data_ptr(), R,
+                                            block_size, int(seed), keys.data_ptr(), keys.numel(), at, stream)
     if rc:
         _lib.check(rc, "kvcm_hip_hash_tokens_checked")
 
@@ -144,6 +150,14 @@ def _settle(word, device):
 _KEYS_AHEAD = 1 << 25
 
 
+def _counted_by_the_hash(R, n_tokens):
+    """Whether the hash launch makes the key offsets itself. That saves a launch, but the total comes later out of the larger
+    kernel, the more so the more requests there are, and where a call waits longer for it than for the keys nothing is saved. us a
+    call, two launches / one: 600 requests of 50 to 100 tokens 16.8 / 16.5, 1000: 16.5 / 16.9, 2500: 16.9 / 18.3; 1500 of 350 to 700
+    17.1 / 17.2, of 450 to 900 18.1 / 17.4; 2500 of 350 to 700 17.9 / 18.3, of 450 to 900 18.5 / 18.1."""
+    return R <= 640 or (R <= _lib.COUNT_KEYS_UP_TO and n_tokens >= 576 * R)
+
+
 def _hash_and_count(tokens, off, R, block_size, seed, stream):
     """(keys, key_offsets) of R > 0 requests when the caller brings neither. The total is on its way to the host while the
     keys are being computed into a buffer of the size that the token count bounds: nobody waits for the hash kernel, and the
@@ -157,9 +171,12 @@ def _hash_and_count(tokens, off, R, block_size, seed, stream):
     keys = torch.empty(most, dtype=torch.int64, device=tokens.device) if most <= _KEYS_AHEAD else None
     pending = torch.empty(1, dtype=torch.int64, pin_memory=True)
     try:
-        _launch_offsets(tokens, off, R, block_size, most, key_offsets, pending, stream)
-        if keys is not None and most:
-            _launch_keys(tokens, off, R, block_size, seed, keys, key_offsets, stream)
+        if keys is not None and most and _counted_by_the_hash(R, tokens.numel()):
+            _launch_keys(tokens, off, R, block_size, seed, keys, key_offsets, stream, pending)
+        else:
+            _launch_offsets(tokens, off, R, block_size, most, key_offsets, pending, stream)
+            if keys is not None and most:
+                _launch_keys(tokens, off, R, block_size, seed, keys, key_offsets, stream)
         rc = lib().kvcm_wait_value(pending.data_ptr(), stream)
         if rc:
             _lib.check(rc, "kvcm_wait_value")

@@ -71,6 +71,12 @@ def test_argument_validation_needs_no_device():
     assert checked(p, 8, -1, p, 1, 16, 0, p, 1, None, None) == _lib.ERR_INVALID_ARG
     assert checked(p, 8, 1, p, 1, 16, 0, p, -1, None, None) == _lib.ERR_INVALID_ARG
     assert checked(p, 4, 1, None, 1, 16, 0, p, 1, None, None) == _lib.ERR_INVALID_ARG
+    count = ctypes.byref(_lib.KeyCount(p, p))
+    assert checked(p, 8 | _lib.COUNT_KEYS, 1, p, 0, 16, 0, p, 1, count, None) == _lib.ERR_INVALID_ARG
+    assert checked(p, 8 | _lib.COUNT_KEYS, 1, p, 1, 16, 0, p, 1, None, None) == _lib.ERR_INVALID_ARG
+    assert checked(p, 8 | _lib.COUNT_KEYS, 1, p, 1, 16, 0, p, 1, ctypes.byref(_lib.KeyCount(p, None)), None) == _lib.ERR_INVALID_ARG
+    assert checked(p, 2 | _lib.COUNT_KEYS, 1, p, 1, 16, 0, p, 1, count, None) == _lib.ERR_INVALID_ARG
+    assert checked(p, 8 | _lib.COUNT_KEYS, 1, p, _lib.COUNT_KEYS_UP_TO + 1, 16, 0, p, 1, count, None) == _lib.ERR_TOO_LARGE
     offsets = L.kvcm_hip_key_offsets_checked
     assert offsets(p, 0, 16, 1, 1, None, 0, p, None, None) == _lib.ERR_INVALID_ARG
     assert offsets(p, 1, 0, 1, 1, None, 0, p, None, None) == _lib.ERR_INVALID_ARG

@@ -443,6 +443,31 @@ def test_offsets_are_not_followed_beyond_the_tokens(oracle, force_general_hash_l
     assert (host(room, np.int64) == -7).all() and host(off, np.int64)[R - 1] == -1
 
 
+@pytest.mark.parametrize("one_launch", [True, False])
+@pytest.mark.parametrize("dtype,bs", [(np.int64, 16), (np.int32, 1), (np.int32, 7), (np.int64, 7)])
+@pytest.mark.parametrize("R", [1, 16, 17, 271, 272, 273, 529, 1040, 1041, 1552, 1553, 4096, 4097])
+def test_one_launch_counts_and_hashes(oracle, monkeypatch, one_launch, dtype, bs, R):
+    """Ragged batches whose offsets the launch itself makes, at the edges of its workgroups (16 requests), of the offsets that a
+    wave adds up at a time (256, and 1024 while more than 512 are left) and of the most it takes: keys, offsets, and requests that
+    are not all there, any one of which, in front of a workgroup or its own, is found. The same as two launches."""
+    monkeypatch.setattr(_h(), "_counted_by_the_hash", lambda R, n: one_launch and R <= 4096)
+    rng = np.random.default_rng(R * bs)
+    lens = rng.integers(0, 100, size=R)
+    lens[R // 2] += 3 * bs
+    toff = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    flat = rng.integers(-2**31, 2**31, size=int(toff[-1]) + 40, dtype=np.int64).astype(dtype)
+    want, woff = oracle.hash_tokens(flat, bs, token_offsets=toff, threads=8)
+    keys, off = _h().hash_tokens(dev(flat), bs, token_offsets=dev(toff))
+    sync()
+    assert (host(off, np.int64) == woff).all() and (host(keys, np.int64) == want).all()
+    for r in {0, R // 2, R - 1}:
+        far = toff.copy()
+        far[r + 1] = len(flat) + bs                          # and whoever comes next begins there
+        with pytest.raises(ValueError):
+            _h().hash_tokens(dev(flat), bs, token_offsets=dev(far))
+    sync()
+
+
 @pytest.mark.parametrize("general_loader", [False, True])
 def test_keys_beyond_the_callers_buffer_are_left_out(oracle, force_general_hash_loader, general_loader):
     """A key buffer that holds the keys of some requests only: those are written, the slots behind the buffer are not; the
