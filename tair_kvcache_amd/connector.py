@@ -438,14 +438,17 @@ class DataTransferManager:
                 pool_token_slots=self._kvcache_info.local_token_num, stream=stream)
             done = self._thread_event()
             done.record(stream)
-            done.synchronize()
+            try:
+                buffers = self._slot_buffers(slots)  # while the copy runs: 5 us for 128 blocks
+            finally:  # not before the copy has ended may the slots go to anybody else
+                done.synchronize()
             if isinstance(block_token_indices, torch.Tensor) and block_token_indices.is_cuda and \
                     blocks_idx_error(block_token_indices.device):
                 # indices built on the device named a block beyond the request's block list: those rows were skipped
                 # by the gather, so the staged bytes are not the request's KV cache and must not be saved
                 result = (self._cm.ClientErrorCode.ER_INVALID_PARAMS, [])
             else:
-                result = self._transfer_client.SaveKvCaches(remote_uris, self._slot_buffers(slots))
+                result = self._transfer_client.SaveKvCaches(remote_uris, buffers)
         finally:
             if slots is not None:
                 self._copy_buffer_allocator.free_buffer(slots)

@@ -134,9 +134,8 @@ class CopyBufferAllocator:
         if not buffers:
             return
         with self._cond:
-            for idx in buffers:
-                if idx >= self.max_count or idx < 0:
-                    raise ValueError(f"Buffer idx {idx} wrong")
+            if min(buffers) < 0 or max(buffers) >= self.max_count:
+                raise ValueError(f"Buffer idx {next(i for i in buffers if i >= self.max_count or i < 0)} wrong")
             n = len(buffers)
             if self._inuse_count < n:
                 raise RuntimeError(f"Trying to free {n} buffers, but only {self._inuse_count} are in use")

@@ -409,6 +409,41 @@ class DeviceStagingClient:
         return ClientErrorCode.ER_OK
 
 
+@pytest.mark.parametrize("when", ["none", "never recorded", "happened", "to come"])
+def test_a_save_takes_the_cache_as_the_event_leaves_it(when):
+    """The blocks saved are those of the cache at the event, be that still to come (milliseconds of work in front of it), past or
+    not there at all; and slots whose buffers cannot be made come back only when nothing writes them any more."""
+    from tair_kvcache_amd import connector
+    from tair_kvcache_amd.kernel.gather_scatter_helper import CopyBufferAllocator
+    kv = {"l": torch.zeros(2, 64, 16, 8, 32, dtype=torch.int16, device="cuda")}
+    info = connector.register_kv_caches(kv, manager_block_size=16, local_block_size=16)
+    alloc = CopyBufferAllocator(torch.device("cuda"), torch.int16, list(info.per_manager_block_shape), 12)
+    client = DeviceStagingClient(alloc)
+    mgr = connector.DataTransferManager(info, 16, alloc, client, max_workers=1)
+    uris, idx = [f"mem://b{i}" for i in range(12)], [[16 * (5 * b) + t for t in range(16)] for b in range(12)]
+    want = torch.arange(kv["l"].numel(), device="cuda").to(torch.int16).view_as(kv["l"])
+    queued = torch.empty(1 << 28, dtype=torch.int8, device="cuda")
+    sync()
+    event = None if when == "none" else torch.cuda.Event()
+    for _ in range(64 if when == "to come" else 0):
+        queued.zero_()
+    kv["l"].copy_(want)
+    if when in ("happened", "to come"):
+        event.record()
+    if when != "to come":
+        sync()
+    out = []
+    mgr.save_task(connector.MultiResult(1, out.extend), 0, uris, idx, event)
+    assert [int(c) for c in out[0]] == [0] * 12
+    for b, uri in enumerate(uris):
+        assert torch.equal(client.store[uri].reshape(2, 16, 8, 32), want[:, 5 * b].cpu())
+    mgr._slot_buffers = lambda slots: 1 // 0
+    with pytest.raises(ZeroDivisionError):
+        mgr.save_task(connector.MultiResult(1, out.extend), 0, uris, idx, event)
+    assert mgr._save_stream.query() and alloc._inuse_count == 0
+    mgr.shutdown()
+
+
 def test_transfer_manager_with_staging_in_hbm(oracle):
     """The same save/load choreography with the staging pool on the GPU: slots are handed over as GPU iovs."""
     from tair_kvcache_amd import connector
