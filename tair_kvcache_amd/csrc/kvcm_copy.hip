@@ -26,9 +26,8 @@
 //   registers; nothing is reshaped in memory. When a span lies inside one tile (and one run) the tile number,
 //   pool pointer and slot are workgroup-uniform: scalar arithmetic and scalar loads, and a thread's own work is
 //   two address adds. Otherwise chunk -> (tile, run, offset) is two multiply-shift divisions per thread.
-//   Every byte is touched once: loads carry the non-temporal hint (+4 % gather against plain accesses), and so
-//   do stores, except where whole tiles move (block-table form): there the staging side of a gather is written
-//   through at system scope and the pool side of a scatter carries both bits (see the store site below).
+//   Every byte is touched once: loads carry the non-temporal hint (+4 % gather against plain accesses); stores carry it, are
+//   written through at system scope, or both, by size and shape of the launch (store_policy).
 //
 // Roofline: HBM. Algorithmic bytes per tile = 2 * T * row_bytes (+ trailer), index bytes are negligible.
 #include "kvcm_internal.h"
@@ -48,12 +47,6 @@ namespace {
 #endif
 #ifndef KVCM_COPY_NT_LOAD
 #define KVCM_COPY_NT_LOAD 1
-#endif
-#ifndef KVCM_COPY_GATHER_STORE_POLICY
-#define KVCM_COPY_GATHER_STORE_POLICY 1
-#endif
-#ifndef KVCM_COPY_SCATTER_STORE_POLICY
-#define KVCM_COPY_SCATTER_STORE_POLICY 2
 #endif
 #ifndef KVCM_COPY_NT_STORE
 #define KVCM_COPY_NT_STORE 1
@@ -84,7 +77,7 @@ struct CopyArgs {
     FastDiv div_entry;
     FastDiv div_units;
     int32_t xcd_remap;
-    int32_t staging_on_line_grid;  // staging base, block stride and tile stride are multiples of 128
+    int32_t store_policy;
 };
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -135,16 +128,14 @@ __device__ __forceinline__ void store_chunk(unsigned char *p, typename Chunk<CS>
 #endif
 }
 
-// 16-byte chunks, the form every engine layout takes. POLICY 0: non-temporal; 1: written through at system scope
-// (sc1); 2: both; 3: sc0 sc1.
-template <int POLICY>
-__device__ __forceinline__ void store_chunk16(unsigned char *p, u32x4 v) {
-    if (POLICY == 1) {
+// How a store of 16 bytes goes to memory, chosen per launch (store_policy below).
+enum StorePolicy { kStoreNt = 0, kStoreThrough = 1, kStoreThroughNt = 2 };  // nt, sc1 (written through at system scope), both
+
+__device__ __forceinline__ void store_chunk16(unsigned char *p, u32x4 v, int32_t policy) {
+    if (policy == kStoreThrough) {
         asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
-    } else if (POLICY == 2) {
+    } else if (policy == kStoreThroughNt) {
         asm volatile("global_store_dwordx4 %0, %1, off sc1 nt" : : "v"(p), "v"(v) : "memory");
-    } else if (POLICY == 3) {
-        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" : : "v"(p), "v"(v) : "memory");
     } else {
         store_chunk<16>(p, v);
     }
@@ -154,15 +145,20 @@ __device__ __forceinline__ void store_chunk16(unsigned char *p, u32x4 v) {
 // row size. Pool base pointers live in device memory; a pool row that is not dword-aligned (CS > 1) is moved
 // byte by byte by the one thread that owns the chunk.
 //
-// UNI_TILE: every span lies inside one tile (chunks_per_tile is a multiple of the span), so the tile number, the
-// pool base pointer and the staging tile address are workgroup-uniform: scalar arithmetic and scalar loads.
-// RUN = how widely a run of consecutive slots is shared (needs UNI_TILE):
+// TILE = how widely a tile is shared:
+//   kTilePerGroup  every span lies inside one tile (chunks_per_tile is a multiple of the span): the tile number, the pool base
+//                  pointer and the staging tile address are workgroup-uniform, scalar arithmetic and scalar loads;
+//   kTilePerWave   a tile and a run are whole numbers of wavefronts' worth of chunks (latent attention's 1152-byte rows in blocks
+//                  of 16: 1152 chunks): the same per wave;
+//   kTilePerThread anything else: divisions and table reads per thread.
+// RUN = how widely a run of consecutive slots is shared (no more widely than the tile):
 //   kRunPerGroup  every span lies inside one run (block-table fast path, or rows of 4 KiB and more): the run's
 //                 first slot is one scalar load per workgroup and a thread's own work is two address adds;
 //   kRunPerWave   a run is a whole number of wavefronts' worth of chunks (rows of 1 KiB and more): the slot is a
 //                 scalar load per wave;
 //   kRunPerThread anything else: the run number is a multiply-shift division per thread and the slot a vector load.
 enum RunMode { kRunPerThread = 0, kRunPerWave = 1, kRunPerGroup = 2 };
+enum TileMode { kTilePerThread = 0, kTilePerWave = 1, kTilePerGroup = 2 };
 
 // Where a launch finds its index tables. PtrIdx: two arrays in device memory (every entry point that takes d_ pointers).
 // KernargIdx: the tables travel INSIDE the kernel's argument block, run starts first, staging slots behind them -- the
@@ -183,11 +179,12 @@ struct KernargIdx {
     __device__ __forceinline__ int64_t slot(uint32_t b) const { return e.v[staging_first + b]; }
 };
 
-template <int CS, bool SCATTER, bool UNI_TILE, int RUN, typename Idx>
+template <int CS, bool SCATTER, int TILE, int RUN, typename Idx>
 __device__ __forceinline__ void copy_span_body(const CopyArgs &a, const void *const *__restrict__ ptr_table,
                                                const void *const *__restrict__ trailer_table, const Idx &idx,
                                                const int32_t *__restrict__ trailer_idx) {
     using V = typename Chunk<CS>::V;
+    constexpr bool kUniTile = TILE != kTilePerThread;
 
     // Consecutive workgroup ids land on consecutive XCDs (8 per device, one L2 each). With the remap every XCD
     // walks one contiguous eighth of the unit range instead of every eighth unit.
@@ -203,8 +200,12 @@ __device__ __forceinline__ void copy_span_body(const CopyArgs &a, const void *co
         const uint32_t b = fast_div(unit, a.div_units);
         const uint32_t span = unit - b * a.units_per_block;
         const int64_t runs_b = static_cast<int64_t>(b) * a.runs;  // index of the block's first run
-        // workgroup-uniform part: the three table reads below are independent scalar loads in the UNI_* forms
-        const uint32_t g_first = span * kSpan;
+        // workgroup- or wave-uniform part: the three table reads below are independent scalar loads in the UNI_* forms
+        static_assert(TILE != kTilePerWave || (kCPT == 1 && RUN == kRunPerWave), "one chunk per thread, a slot per wave");
+        const uint32_t g_first = span * kSpan + (TILE == kTilePerWave ? __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u) : 0);
+        if (TILE == kTilePerWave && g_first >= a.chunks_per_block) {
+            continue;  // the last span of a block may have fewer waves
+        }
         const uint32_t p_first = fast_div(g_first, a.div_tile);
         const uint32_t cc_first = g_first - p_first * a.chunks_per_tile;
         const uint32_t r_first = fast_div(cc_first, a.div_run);
@@ -215,14 +216,15 @@ __device__ __forceinline__ void copy_span_body(const CopyArgs &a, const void *co
             slot_shared = idx.run(runs_b + r_first);
         } else if (RUN == kRunPerWave) {
             // one chunk per thread: a wave's 64 chunks start at a multiple of 64 and lie inside one run
-            r_shared = __builtin_amdgcn_readfirstlane(fast_div(cc_first + (threadIdx.x & ~63u), a.div_run));
+            r_shared = TILE == kTilePerWave ? r_first
+                                            : __builtin_amdgcn_readfirstlane(fast_div(cc_first + (threadIdx.x & ~63u), a.div_run));
             slot_shared = idx.run(runs_b + r_shared);
         }
-        const void *pool_first = UNI_TILE ? ptr_table[entry_first] : nullptr;
+        const void *pool_first = kUniTile ? ptr_table[entry_first] : nullptr;
         // the span that starts a tile also moves the tile's trailer: its table entries are workgroup-uniform too
         int32_t trailer_idx_first = -1;
         const void *trailer_base_first = nullptr;
-        if (UNI_TILE && a.trailer_bytes > 0 && cc_first == 0) {
+        if (kUniTile && a.trailer_bytes > 0 && cc_first == 0) {
             trailer_idx_first = trailer_idx[b];
             trailer_base_first = trailer_table[p_first];
         }
@@ -239,31 +241,31 @@ __device__ __forceinline__ void copy_span_body(const CopyArgs &a, const void *co
         unsigned char *tr_dst = nullptr;
 #pragma unroll
         for (int u = 0; u < kCPT; ++u) {
-            const uint32_t in_span = threadIdx.x + static_cast<uint32_t>(u) * kThreads;
+            const uint32_t in_span = (TILE == kTilePerWave ? threadIdx.x & 63u : threadIdx.x) + static_cast<uint32_t>(u) * kThreads;
             const uint32_t g = g_first + in_span;
             pp[u] = nullptr;
             sp[u] = nullptr;
             if (g < a.chunks_per_block) {
-                const uint32_t p = UNI_TILE ? p_first : fast_div(g, a.div_tile);
-                const uint32_t cc = UNI_TILE ? cc_first + in_span : g - p * a.chunks_per_tile;
+                const uint32_t p = kUniTile ? p_first : fast_div(g, a.div_tile);
+                const uint32_t cc = kUniTile ? cc_first + in_span : g - p * a.chunks_per_tile;
                 const uint32_t r = RUN != kRunPerThread ? r_shared : fast_div(cc, a.div_run);
                 const uint32_t off = cc - r * a.chunks_per_run;
                 const int64_t slot = RUN != kRunPerThread ? slot_shared : static_cast<int64_t>(idx.run(runs_b + r));
                 unsigned char *tile = block + static_cast<int64_t>(p) * a.tile_stride;
                 if (slot >= 0 && slot < limit) {
-                    const uint32_t entry = UNI_TILE ? entry_first : fast_div(p, a.div_entry);
+                    const uint32_t entry = kUniTile ? entry_first : fast_div(p, a.div_entry);
                     const uint32_t inner = p - entry * a.ptrs_per_entry;
-                    const void *base = UNI_TILE ? pool_first : ptr_table[entry];
+                    const void *base = kUniTile ? pool_first : ptr_table[entry];
                     unsigned char *pool = static_cast<unsigned char *>(const_cast<void *>(base)) +
                                           static_cast<int64_t>(inner) * a.entry_stride;
                     pp[u] = pool + slot * a.row_bytes + static_cast<int64_t>(off) * CS;
                     sp[u] = tile + static_cast<int64_t>(cc) * CS;
                 }
-                if (a.trailer_bytes > 0 && cc == 0 && (UNI_TILE ? trailer_idx_first : trailer_idx[b]) >= 0) {
+                if (a.trailer_bytes > 0 && cc == 0 && (kUniTile ? trailer_idx_first : trailer_idx[b]) >= 0) {
                     // the thread that owns a tile's first chunk also moves the tile's trailer (a negative trailer
                     // index means "no trailer for this block": nothing is read or written)
-                    const int64_t t_idx = UNI_TILE ? trailer_idx_first : trailer_idx[b];
-                    const void *t_base = UNI_TILE ? trailer_base_first : trailer_table[p];
+                    const int64_t t_idx = kUniTile ? trailer_idx_first : trailer_idx[b];
+                    const void *t_base = kUniTile ? trailer_base_first : trailer_table[p];
                     unsigned char *tr = static_cast<unsigned char *>(const_cast<void *>(t_base)) + t_idx * a.trailer_bytes;
                     unsigned char *st = tile + a.tile_payload;
                     if (a.trailer_bytes == 4 && ((reinterpret_cast<uintptr_t>(tr) | reinterpret_cast<uintptr_t>(st)) & 3u) == 0) {
@@ -300,20 +302,7 @@ __device__ __forceinline__ void copy_span_body(const CopyArgs &a, const void *co
 #pragma unroll
             for (int u = 0; u < kCPT; ++u) {
                 if constexpr (CS == 16) {
-                    // Block-table form (whole tiles move): the staging side of a gather is written through at system
-                    // scope (sc1), measured +1.5 to +4.6 % over non-temporal stores at the benchmark layouts and +1.6 %
-                    // for 128-block tasks; the pool side of a scatter carries sc1 and nt together (+1.3 to +2.5 %, and a
-                    // 24 MiB launch that fits the caches finishes 45 % sooner). With token-granular indices either bit
-                    // costs 0.5 to 2.5 %: those stores stay non-temporal. Where staging tiles do not start on cache-line
-                    // boundaries (a 4-byte scale behind every tile) a wave's kilobyte begins and ends inside a line, and
-                    // writing partial lines through costs 15 % (5.2 against 6.0 TB/s): non-temporal there as well.
-                    constexpr int kPolicy = RUN != kRunPerGroup ? 0
-                                            : (SCATTER ? KVCM_COPY_SCATTER_STORE_POLICY : KVCM_COPY_GATHER_STORE_POLICY);
-                    if (kPolicy != 0 && !SCATTER && !a.staging_on_line_grid) {
-                        store_chunk16<0>(sp[u], v[u]);
-                    } else {
-                        store_chunk16<kPolicy>(SCATTER ? pp[u] : sp[u], v[u]);
-                    }
+                    store_chunk16(SCATTER ? pp[u] : sp[u], v[u], RUN == kRunPerThread ? kStoreNt : a.store_policy);
                 } else {
                     store_chunk<CS>(SCATTER ? pp[u] : sp[u], v[u]);
                 }
@@ -345,7 +334,7 @@ __device__ __forceinline__ void copy_span_body(const CopyArgs &a, const void *co
     }
 }
 
-template <int CS, bool SCATTER, bool UNI_TILE, int RUN>
+template <int CS, bool SCATTER, int TILE, int RUN>
 __global__ __launch_bounds__(kThreads) void copy_span_kernel(const CopyArgs a,
                                                              // read-only tables, never written by this kernel:
                                                              // __restrict__ lets uniform reads become scalar loads
@@ -354,17 +343,17 @@ __global__ __launch_bounds__(kThreads) void copy_span_kernel(const CopyArgs a,
                                                              const int32_t *__restrict__ run_start,
                                                              const int32_t *__restrict__ staging_idx,
                                                              const int32_t *__restrict__ trailer_idx) {
-    copy_span_body<CS, SCATTER, UNI_TILE, RUN>(a, ptr_table, trailer_table, PtrIdx{run_start, staging_idx}, trailer_idx);
+    copy_span_body<CS, SCATTER, TILE, RUN>(a, ptr_table, trailer_table, PtrIdx{run_start, staging_idx}, trailer_idx);
 }
 
 // The same kernel with its index tables in the argument block (host index lists).
-template <int CS, bool SCATTER, bool UNI_TILE, int RUN>
+template <int CS, bool SCATTER, int TILE, int RUN>
 __global__ __launch_bounds__(kThreads) void copy_span_kernarg_kernel(const EmbeddedIdx emb, const CopyArgs a,
                                                                      uint32_t staging_first,
                                                                      const void *const *__restrict__ ptr_table,
                                                                      const void *const *__restrict__ trailer_table,
                                                                      const int32_t *__restrict__ trailer_idx) {
-    copy_span_body<CS, SCATTER, UNI_TILE, RUN>(a, ptr_table, trailer_table, KernargIdx{emb, staging_first}, trailer_idx);
+    copy_span_body<CS, SCATTER, TILE, RUN>(a, ptr_table, trailer_table, KernargIdx{emb, staging_first}, trailer_idx);
 }
 
 // out[b][i] = block_ids[(m_b*T_mgr + i) / T_eng] * T_eng + (m_b*T_mgr + i) % T_eng
@@ -404,24 +393,61 @@ int32_t align_class(uint64_t bits) {
     return 1;
 }
 
+// Stores of launches whose waves each move a kilobyte of one run (smaller pieces stay non-temporal: written through they cost up to
+// 25 %). Written through (sc1) the data stays in the 256 MiB memory-side cache, which is right for what a gather leaves in staging, and
+// wrong for what a scatter leaves in the pool while staging could stay there: a scatter that fits the cache carries nt. GB/s, nt / sc1 / both:
+//   scatter, whole tiles of 2^k bytes  128 KiB 5866 / 6504 / 6149 (4 GiB), 64 KiB - / 6306 / 6107, 32 KiB - / 5714 / 5592 (1.5 GiB);
+//                                      16 KiB, 115 MiB, again and again: - / 5400 / 5850
+//   scatter, other tiles               9 KiB 5519 / 5599 / 5512, 18 KiB 5532 / 5615 / 5537, 20 KiB - / 5621 / 5415,
+//                                      36 KiB - / 5668 / 5823, 72 KiB - / 5721 / 6132 (1.5 GiB)
+//   scatter, a slot per token          1 KiB, 1.8 GiB: 5510 / 5460 / -
+//   gather, whole tiles of 2^k         - / 6245 / 6249 (4 GiB), - / 6681 / 5860 (180 MiB)
+//   gather, other tiles                18 KiB 5828 / 5630 / 5951, 36 KiB - / 5944 / 6142 (1.5 GiB), - / 5974 / 6002 (600 MiB),
+//                                      - / 5949 / 5911 (400 MiB), - / 6639 / 5914 (180 MiB)
+//   gather, a slot per token           1 KiB 5732 / 5666 / 5859, 2 KiB 5814 / 5855 / 5936 (1.8 GiB)
+// Staging tiles that do not start on cache lines (a 4-byte scale behind every tile) make a wave's kilobyte begin and end inside one,
+// and partial lines written through cost a gather 15 % (5.2 against 6.0 TB/s).
+int32_t store_policy(const CopyArgs &a, bool scatter, int64_t run_bytes, int64_t launch_bytes, bool group_tiles) {
+    const bool power_of_two = (run_bytes & (run_bytes - 1)) == 0;
+    const bool group_runs = group_tiles && a.chunks_per_run % kSpan == 0;
+    if (scatter) {
+        if (group_tiles && !group_runs) {
+            return kStoreNt;  // a slot per token
+        }
+        if (!group_runs) {  // us, a tile per thread and nt / a tile per wave and this: 18 KiB, 1.7 GiB 703 / 655, 115 MiB 45.1 / 42.1
+            return launch_bytes < (int64_t{1536} << 20) ? kStoreNt : kStoreThrough;
+        }
+        // us, both / sc1, again and again on the same blocks: 32 KiB, 900 MiB 335 / 338, 1.7 GiB 632 / 635, 64 KiB 567 / 570, 8 KiB
+        // 638 / 644; 128 KiB, 4 GiB 1363 / 1298
+        return launch_bytes >= (int64_t{3} << 30) && (power_of_two || run_bytes < (32 << 10)) ? kStoreThrough : kStoreThroughNt;
+    }
+    if (((reinterpret_cast<uint64_t>(a.staging) | static_cast<uint64_t>(a.block_stride) | static_cast<uint64_t>(a.tile_stride)) & 127u) != 0) {
+        return kStoreNt;
+    }
+    if (group_tiles && !group_runs) {  // a slot per token; 2 KiB, 300 MiB, again and again: nt 101 us, sc1 103
+        return launch_bytes < (int64_t{768} << 20) ? kStoreNt : kStoreThroughNt;
+    }
+    return launch_bytes < (int64_t{400} << 20) || (power_of_two && group_runs) ? kStoreThrough : kStoreThroughNt;
+}
+
 // emb != nullptr: the index tables are *emb (copied into the kernel's argument block by the launch), run starts from
 // entry 0, staging slots from entry `staging_first`; the descriptor's d_run_start / d_staging_idx are not looked at.
-template <int CS, bool UNI_TILE, int RUN>
+template <int CS, int TILE, int RUN>
 void launch_span(const CopyArgs &a, const kvcm_copy_desc *d, bool scatter, uint32_t grid, hipStream_t stream,
                  const EmbeddedIdx *emb, uint32_t staging_first) {
     if (emb) {
         if (scatter) {
-            hipLaunchKernelGGL((copy_span_kernarg_kernel<CS, true, UNI_TILE, RUN>), dim3(grid), dim3(kThreads), 0,
+            hipLaunchKernelGGL((copy_span_kernarg_kernel<CS, true, TILE, RUN>), dim3(grid), dim3(kThreads), 0,
                                stream, *emb, a, staging_first, d->d_ptr_table, d->d_trailer_ptr_table, d->d_trailer_idx);
         } else {
-            hipLaunchKernelGGL((copy_span_kernarg_kernel<CS, false, UNI_TILE, RUN>), dim3(grid), dim3(kThreads), 0,
+            hipLaunchKernelGGL((copy_span_kernarg_kernel<CS, false, TILE, RUN>), dim3(grid), dim3(kThreads), 0,
                                stream, *emb, a, staging_first, d->d_ptr_table, d->d_trailer_ptr_table, d->d_trailer_idx);
         }
     } else if (scatter) {
-        hipLaunchKernelGGL((copy_span_kernel<CS, true, UNI_TILE, RUN>), dim3(grid), dim3(kThreads), 0, stream, a,
+        hipLaunchKernelGGL((copy_span_kernel<CS, true, TILE, RUN>), dim3(grid), dim3(kThreads), 0, stream, a,
                            d->d_ptr_table, d->d_trailer_ptr_table, d->d_run_start, d->d_staging_idx, d->d_trailer_idx);
     } else {
-        hipLaunchKernelGGL((copy_span_kernel<CS, false, UNI_TILE, RUN>), dim3(grid), dim3(kThreads), 0, stream, a,
+        hipLaunchKernelGGL((copy_span_kernel<CS, false, TILE, RUN>), dim3(grid), dim3(kThreads), 0, stream, a,
                            d->d_ptr_table, d->d_trailer_ptr_table, d->d_run_start, d->d_staging_idx, d->d_trailer_idx);
     }
 }
@@ -496,20 +522,23 @@ int32_t launch_copy(const kvcm_copy_desc *d, bool scatter, hipStream_t stream, c
     }
     const bool uni_tile = a.chunks_per_tile % kSpan == 0;
     const uint32_t g32 = static_cast<uint32_t>(grid);
-    a.staging_on_line_grid = ((reinterpret_cast<uint64_t>(d->d_staging) | static_cast<uint64_t>(a.block_stride) |
-                               static_cast<uint64_t>(a.tile_stride)) & 127u) == 0;
+    a.store_policy = store_policy(a, scatter, run_bytes, payload * d->P * d->B, uni_tile);
     if (cs == 16 && uni_tile && a.chunks_per_run % kSpan == 0) {
-        launch_span<16, true, kRunPerGroup>(a, d, scatter, g32, stream, emb, staging_first);
+        launch_span<16, kTilePerGroup, kRunPerGroup>(a, d, scatter, g32, stream, emb, staging_first);
     } else if (cs == 16 && uni_tile && kCPT == 1 && a.chunks_per_run % 64 == 0) {
-        launch_span<16, true, kRunPerWave>(a, d, scatter, g32, stream, emb, staging_first);
+        launch_span<16, kTilePerGroup, kRunPerWave>(a, d, scatter, g32, stream, emb, staging_first);
     } else if (cs == 16 && uni_tile) {
-        launch_span<16, true, kRunPerThread>(a, d, scatter, g32, stream, emb, staging_first);
+        launch_span<16, kTilePerGroup, kRunPerThread>(a, d, scatter, g32, stream, emb, staging_first);
+    } else if (cs == 16 && kCPT == 1 && a.chunks_per_run % 64 == 0) {
+        // GB/s, per thread / per wave, 1.5 GiB: 1152-byte rows in tiles of 16, runs of 16 gather 5366 / 5951, scatter 5245 / 5615,
+        // runs of 8 5332 / 5895, 5246 / 5599; 576-byte rows in tiles of 32 5373 / 5950, 5252 / 5613; 320 in 16 5273 / 5803, 5210 / 5560
+        launch_span<16, kTilePerWave, kRunPerWave>(a, d, scatter, g32, stream, emb, staging_first);
     } else if (cs == 16) {
-        launch_span<16, false, kRunPerThread>(a, d, scatter, g32, stream, emb, staging_first);
+        launch_span<16, kTilePerThread, kRunPerThread>(a, d, scatter, g32, stream, emb, staging_first);
     } else if (cs == 4) {
-        launch_span<4, false, kRunPerThread>(a, d, scatter, g32, stream, emb, staging_first);
+        launch_span<4, kTilePerThread, kRunPerThread>(a, d, scatter, g32, stream, emb, staging_first);
     } else {
-        launch_span<1, false, kRunPerThread>(a, d, scatter, g32, stream, emb, staging_first);
+        launch_span<1, kTilePerThread, kRunPerThread>(a, d, scatter, g32, stream, emb, staging_first);
     }
     return launch_status();
 }

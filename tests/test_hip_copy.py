@@ -358,3 +358,38 @@ def test_block_major_pools_are_the_one_array_case(oracle):
     g = host(fresh, np.uint16)
     rest = np.setdiff1d(np.arange(nblk), ids)
     assert (g[ids] == pool[ids]).all() and not g[rest].any()
+
+
+@pytest.mark.parametrize("row,T,run,P,B", [
+    (1152, 16, 16, 5, 7), (1152, 16, 8, 5, 7), (576, 32, 16, 3, 6), (576, 16, 16, 3, 5), (320, 16, 16, 2, 3),
+    (1024, 1, 1, 3, 5), (1024, 3, 1, 1, 9), (1024, 5, 1, 7, 3), (3072, 7, 1, 3, 4),          # tiles of whole waves
+    (1152, 16, 16, 61, 360), (1152, 16, 16, 61, 730), (1152, 16, 16, 61, 1450),             # 386 and 783 MiB, 1.5 GiB
+    (1152, 32, 32, 61, 180), (1152, 32, 32, 61, 190), (1152, 32, 32, 61, 350), (1152, 32, 32, 61, 370),
+    (1024, 16, 1, 56, 450), (1024, 16, 1, 56, 920), (2048, 16, 16, 64, 220), (2048, 16, 16, 64, 1560)])
+def test_waves_tiles_and_store_policies(row, T, run, P, B):
+    """Tiles that are whole waves' worth of chunks but not whole spans (the last span of a block with one to four waves), and launches
+    on both sides of every line of the rule that chooses how stores go to memory: both directions against torch's own indexing,
+    nothing else written."""
+    bgs = _ops()
+    rng = np.random.default_rng(row * T + B)
+    slots = B * T // run + 3
+    pool = torch.randint(0, 256, (P, slots, run * row), dtype=torch.uint8, device="cuda")
+    runs = torch.from_numpy(rng.permutation(slots)[:B * (T // run)].astype(np.int32)).cuda()
+    order = torch.from_numpy(rng.permutation(B).astype(np.int32)).cuda()
+    staging = torch.zeros(B + 1, P, T // run, run * row, dtype=torch.uint8, device="cuda")
+    bgs.paged_gather_kv_caches(ptr_table(list(pool)), staging[:B], runs * run, order, T, row, run)
+    want = pool[:, runs.long()].view(P, B, T // run, run * row)
+    for p in range(P):
+        assert torch.equal(staging[order.long(), p], want[p]), p
+    assert not staging[B].any()
+    fresh = torch.zeros_like(pool)
+    bgs.paged_scatter_kv_caches(ptr_table(list(fresh)), staging[:B], runs * run, order, T, row, run)
+    rest = torch.ones(slots, dtype=torch.bool, device="cuda")
+    rest[runs.long()] = False
+    for p in range(P):
+        assert torch.equal(fresh[p, runs.long()], pool[p, runs.long()]) and not fresh[p, rest].any(), p
+    if run == T:  # the same from a list: the tables in the argument block
+        again = torch.zeros_like(staging)
+        tokens = (runs.view(B, 1) * run + torch.arange(T, dtype=torch.int32, device="cuda")).reshape(-1).tolist()
+        bgs.batch_gather_kv_caches(ptr_table(list(pool)), again[:B], tokens, order.tolist(), T, row)
+        assert torch.equal(again, staging)
