@@ -21,6 +21,7 @@
 // Roofline: HBM for many requests (8*block_size + 8 bytes per key); for few requests the bound is the
 // instruction issue of the chain wave, which no amount of bandwidth removes.
 #include "kvcm_internal.h"
+#include "kvcm_key_count.h"
 
 #include <climits>
 
@@ -589,14 +590,6 @@ struct Extent {
     int64_t tokens;
     int64_t keys;
 };
-constexpr int64_t kUnknown = INT64_MAX;  // the caller did not say: token offsets are taken as they are
-
-__device__ __forceinline__ int64_t distance(int64_t from, int64_t to) {  // offsets may be anything: no signed overflow
-    return static_cast<int64_t>(static_cast<uint64_t>(to) - static_cast<uint64_t>(from));
-}
-
-// whether [at, at + n) is a non-empty part of [0, size)
-__device__ __forceinline__ bool inside(int64_t at, int64_t n, int64_t size) { return at >= 0 && n > 0 && n <= size - at; }
 
 // Block size 1 writes as much as it reads. Where every request of a workgroup starts at the same place of a 32 KiB period, their
 // pieces meet in the same channels of memory, and with a workgroup on every CU reads and writes are better kept apart: a loader
@@ -810,20 +803,6 @@ struct CountOut {
     int64_t *h_total;      // pinned
     FastDiv by_block;      // n / block size for n < 2^31
 };
-
-__device__ __forceinline__ int64_t keys_of(int64_t len, int32_t block_size) {
-    if (static_cast<uint64_t>(len) >> 32 == 0) {  // 32-bit division: a fifth of the instructions
-        return static_cast<uint32_t>(len) / static_cast<uint32_t>(block_size);
-    }
-    return len > 0 ? len / block_size : 0;
-}
-
-// Keys of one request; `bad` is set when the tokens they are made of are not all there.
-__device__ __forceinline__ int64_t keys_of_request(int64_t at, int64_t next, int32_t block_size, int64_t n_tokens, bool &bad) {
-    const int64_t count = keys_of(distance(at, next), block_size);
-    bad |= n_tokens != kUnknown && count > 0 && !inside(at, count * block_size, n_tokens);
-    return count;
-}
 
 // ------------------------------------------------------------------------------------------- few requests per workgroup
 
@@ -1104,7 +1083,7 @@ __device__ __forceinline__ int64_t lean_keys_of(const int64_t *__restrict__ toke
         for (int j = 0; j < kAhead; ++j) {
             const int64_t i = base + j * 128 + lane * 2;
             for (int64_t k = i; k < i + 2 && k < r_first; ++k) {
-                sum += keys_of_request(token_offsets[k], token_offsets[k + 1], block_size, have.tokens, bad);
+                sum = add_keys(sum, keys_of_request(token_offsets[k], token_offsets[k + 1], block_size, have.tokens, bad));
             }
         }
     }
@@ -1121,10 +1100,10 @@ __device__ __forceinline__ int64_t lean_keys_before(const int64_t *__restrict__ 
     constexpr int kMany = 8, kFew = 2;
     int64_t before = 0, base = 0;
     for (; r_first - base > kMany * 64; base += kMany * 128) {
-        before += lean_keys_of<kMany>(token_offsets, base, r_first, block_size, have, by_block, lane, bad);
+        before = add_keys(before, lean_keys_of<kMany>(token_offsets, base, r_first, block_size, have, by_block, lane, bad));
     }
     for (; base < r_first; base += kFew * 128) {
-        before += lean_keys_of<kFew>(token_offsets, base, r_first, block_size, have, by_block, lane, bad);
+        before = add_keys(before, lean_keys_of<kFew>(token_offsets, base, r_first, block_size, have, by_block, lane, bad));
     }
     return before;
 }
@@ -1138,19 +1117,20 @@ __device__ __forceinline__ void lean_key_offsets(int64_t r_first, int32_t R, int
     int64_t incl = own;
     for (int d = 1; d < 64; d <<= 1) {
         const int64_t up = __shfl_up(incl, d, 64);
-        incl += static_cast<int>(lane) >= d ? up : 0;
-        before += __shfl_xor(before, d, 64);
+        incl = add_keys(incl, static_cast<int>(lane) >= d ? up : 0);
+        before = add_keys(before, __shfl_xor(before, d, 64));
     }
-    const int64_t key = before + incl - own;
+    const int64_t in_front = __shfl_up(incl, 1, 64);
+    const int64_t key = add_keys(before, lane > 0 ? in_front : 0), end = add_keys(key, own);
     const bool any = __ballot(bad_before || (mine && bad)) != 0;
     // without its tokens, or beyond the room the caller has: marked, and left out
-    const bool fits = !bad && key + own <= have.keys;
+    const bool fits = !bad && keys_fit(key, own, have.keys);
     if (mine) {
         out.key_offsets[r] = fits ? key : -1;
         if (r == R - 1) {
-            out.key_offsets[R] = key + own;
+            out.key_offsets[R] = end;
             // relaxed: whoever waits for it reads nothing else by it (a release writes the whole L2 back first)
-            __hip_atomic_store(out.h_total, any ? -1 : key + own, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(out.h_total, any ? -1 : end, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
     // every lane knows request lane % 16
@@ -1365,10 +1345,10 @@ __global__ __launch_bounds__(kOffsetsThreads) void key_sums_kernel(const int64_t
     bool bad = false;
 #pragma unroll 8
     for (int64_t i = base + threadIdx.x; i < end; i += kOffsetsThreads) {
-        sum += keys_of_request(token_offsets[i], token_offsets[i + 1], block_size, n_tokens, bad);
+        sum = add_keys(sum, keys_of_request(token_offsets[i], token_offsets[i + 1], block_size, n_tokens, bad));
     }
     for (int d = 1; d < 64; d <<= 1) {
-        sum += __shfl_xor(sum, d, 64);
+        sum = add_keys(sum, __shfl_xor(sum, d, 64));
     }
     const bool any = __ballot(bad) != 0;
     if ((threadIdx.x & 63) == 0) {
@@ -1380,7 +1360,7 @@ __global__ __launch_bounds__(kOffsetsThreads) void key_sums_kernel(const int64_t
         int64_t all = 0;
         bool some = false;
         for (int w = 0; w < kOffsetsThreads / 64; ++w) {
-            all += s_sum[w];
+            all = add_keys(all, s_sum[w]);
             some |= s_bad[w] != 0;
         }
         sums[blockIdx.x] = some ? ~all : all;
@@ -1401,11 +1381,11 @@ __global__ __launch_bounds__(kOffsetsThreads) void key_offsets_kernel(const int6
         for (int64_t g = threadIdx.x; g < static_cast<int64_t>(blockIdx.x); g += blockDim.x) {
             const int64_t v = sums[g];
             bad |= v < 0;
-            before += v < 0 ? ~v : v;
+            before = add_keys(before, v < 0 ? ~v : v);
         }
     } else {
         for (int64_t i = threadIdx.x; i < base; i += blockDim.x) {
-            before += keys_of_request(token_offsets[i], token_offsets[i + 1], block_size, n_tokens, bad);
+            before = add_keys(before, keys_of_request(token_offsets[i], token_offsets[i + 1], block_size, n_tokens, bad));
         }
     }
     const int64_t first = base + static_cast<int64_t>(threadIdx.x) * kOffsetsPerThread;
@@ -1421,15 +1401,16 @@ __global__ __launch_bounds__(kOffsetsThreads) void key_offsets_kernel(const int6
         bool mine = false;
         count[j] = keys_of_request(off[j], off[j + 1], block_size, n_tokens, mine);
         left_out |= mine ? 1u << j : 0u;
-        sum += count[j];
+        sum = add_keys(sum, count[j]);
     }
     bad |= left_out != 0;
     int64_t incl = sum;
     for (int d = 1; d < 64; d <<= 1) {
         const int64_t up = __shfl_up(incl, d, 64);
-        incl += lane >= d ? up : 0;
-        before += __shfl_xor(before, d, 64);
+        incl = add_keys(incl, lane >= d ? up : 0);
+        before = add_keys(before, __shfl_xor(before, d, 64));
     }
+    const int64_t in_front = __shfl_up(incl, 1, 64);
     const bool any = __ballot(bad) != 0;
     if (lane == 63) {
         s_wave[0][wave] = incl;
@@ -1437,19 +1418,18 @@ __global__ __launch_bounds__(kOffsetsThreads) void key_offsets_kernel(const int6
         s_bad[wave] = any;
     }
     __syncthreads();
-    int64_t pos = incl - sum;
+    int64_t pos = lane > 0 ? in_front : 0;
     bool some = false;
     for (int w = 0; w < waves; ++w) {
-        pos += (w < wave ? s_wave[0][w] : 0) + s_wave[1][w];
+        pos = add_keys(add_keys(pos, w < wave ? s_wave[0][w] : 0), s_wave[1][w]);
         some |= s_bad[w] != 0;
     }
 #pragma unroll
     for (int j = 0; j < kOffsetsPerThread; ++j) {
         if (first + j < R) {
-            const int64_t end = pos + count[j];
             // without its tokens, or beyond the room the caller has: marked, and the hash kernel leaves the request out
-            key_offsets[first + j] = end <= limit && !(left_out >> j & 1) ? pos : -1;
-            pos = end;
+            key_offsets[first + j] = keys_fit(pos, count[j], limit) && !(left_out >> j & 1) ? pos : -1;
+            pos = add_keys(pos, count[j]);
             if (first + j == R - 1) {
                 key_offsets[R] = pos;
                 if (h_total) {  // the last workgroup has seen every request

@@ -3,11 +3,12 @@
 //
 // What is compiled in, with a plain host compiler: oracle/kvcm_oracle.c (the checker itself), the library's host-only
 // translation units tair_kvcache_amd/csrc/kvcm_file.hip and kvcm_host.hip, the host walk over index lists
-// (kvcm_host_idx.h) and the C++ layer include/kvcm_hip.hpp. The HIP runtime underneath is fake_hip.cpp: malloc'd
+// (kvcm_host_idx.h), the arithmetic of key offsets (kvcm_key_count.h) and the C++ layer include/kvcm_hip.hpp. The HIP runtime underneath is fake_hip.cpp: malloc'd
 // "device" memory and streams that really are asynchronous. The three kernel entry points the C++ layer calls are
 // stand-ins that do the oracle's work in stream order.
 //
-// Scenarios: the oracle's threaded forms; the index-list walk against brute force; block files with host iovs and
+// Scenarios: the oracle's threaded forms; the index-list walk against brute force; key offsets of requests whose token
+// offsets may hold anything, against 128-bit sums; block files with host iovs and
 // with device iovs from 16 concurrent callers; a big get shared among helper threads; a store destroyed while a get
 // or a put is still inside it; the blocking cell pool of the buffer check with more threads than cells.
 #include <sys/prctl.h>
@@ -27,6 +28,7 @@
 #include "fake_hip.h"
 #include "kvcm_hip.hpp"
 #include "kvcm_host_idx.h"
+#include "kvcm_key_count.h"
 #include "kvcm_oracle.h"
 
 #define CHECK(cond)                                                                  \
@@ -429,6 +431,70 @@ void wait_for_a_value() {
     std::puts("ok waiting for a value: late, never, failed stream, captured stream");
 }
 
+__extension__ typedef __int128 Wide;
+
+// Key offsets as the launches make them, request by request and as sums of halves, for any token offsets: a request gets a place
+// only if its tokens are all there and its keys end inside the room, places never overlap, and they are the exact sums.
+void key_offsets_of(const std::vector<int64_t> &off, int32_t block_size, int64_t n_tokens, int64_t n_keys) {
+    const size_t R = off.size() - 1;
+    std::vector<int64_t> count(R), level;
+    std::vector<Wide> exact(R + 1, 0);
+    int64_t before = 0, written_to = 0;
+    for (size_t r = 0; r < R; ++r) {
+        bool bad = false;
+        count[r] = kvcm::keys_of_request(off[r], off[r + 1], block_size, n_tokens, bad);
+        CHECK(count[r] >= 0 && (count[r] == 0 || bad || kvcm::inside(off[r], count[r] * block_size, n_tokens)));
+        exact[r + 1] = exact[r] + count[r];
+        const bool fits = !bad && kvcm::keys_fit(before, count[r], n_keys);
+        CHECK(fits == (!bad && exact[r + 1] <= n_keys));
+        if (fits) {
+            CHECK(before == exact[r] && before >= written_to && before + count[r] <= n_keys);
+            written_to = before + count[r];
+        }
+        before = kvcm::add_keys(before, count[r]);
+        CHECK(before == (exact[r + 1] < kvcm::kMostKeys ? static_cast<int64_t>(exact[r + 1]) : kvcm::kMostKeys));
+    }
+    for (level = count; level.size() > 1;) {  // lanes and waves add up in another order
+        std::vector<int64_t> next;
+        for (size_t i = 0; i < level.size(); i += 2) {
+            next.push_back(kvcm::add_keys(i + 1 < level.size() ? level[i + 1] : 0, level[i]));
+        }
+        level = next;
+    }
+    CHECK(kvcm::add_keys(level[0], 0) == before);
+}
+
+void key_offsets_of_any_token_offsets() {
+    const int64_t far = (int64_t{1} << 62) + (int64_t{1} << 40);
+    key_offsets_of({0, far, 0, far, 0, 5}, 1, 4096, 4096);  // sums that wrap to below zero and, doubled, past it
+    key_offsets_of({0, far, 0, far, 0, far, 0, far, 0, 5, 4000}, 1, 4096, 4096);
+    key_offsets_of({0, INT64_MAX, 0, 64}, 1, 64, 64);
+    std::vector<int64_t> pairs;
+    for (int i = 0; i < 40; ++i) {
+        pairs.insert(pairs.end(), {0, far});
+        key_offsets_of(pairs, 16, 4096, 256);
+        std::vector<int64_t> then = pairs;
+        then.insert(then.end(), {0, 16, 64, 4096});
+        key_offsets_of(then, 16, 4096, 256);
+    }
+    std::mt19937_64 rng(11);
+    const int64_t menu[] = {INT64_MIN, INT64_MIN + 1, -far, -1, 0, 1, 15, 16, 17, 4096, far, INT64_MAX - 1, INT64_MAX};
+    for (int it = 0; it < 20000; ++it) {
+        std::vector<int64_t> off(2 + rng() % 70);
+        for (auto &o : off) {
+            const uint64_t kind = rng() % 8;
+            o = kind < 3 ? static_cast<int64_t>(rng() % 5000) : kind < 7 ? menu[rng() % 13] : static_cast<int64_t>(rng());
+        }
+        key_offsets_of(off, std::vector<int32_t>{1, 7, 16, INT32_MAX}[rng() % 4], 4096, static_cast<int64_t>(rng() % 5000));
+    }
+    std::vector<int64_t> sound(2000, 0);  // nothing is left out where nothing is wrong
+    for (size_t r = 1; r < sound.size(); ++r) {
+        sound[r] = sound[r - 1] + static_cast<int64_t>(rng() % 100);
+    }
+    key_offsets_of(sound, 16, sound.back(), sound.back() / 16);
+    std::puts("ok key offsets of any token offsets");
+}
+
 }  // namespace
 
 int main() {
@@ -437,6 +503,7 @@ int main() {
     g_dir = tmpl;
     oracle_threaded_forms();
     index_list_walk();
+    key_offsets_of_any_token_offsets();
     blocks_hash();
     file_store_concurrent_callers();
     big_get_shared_among_helpers();

@@ -468,6 +468,53 @@ def test_one_launch_counts_and_hashes(oracle, monkeypatch, one_launch, dtype, bs
     sync()
 
 
+@pytest.mark.parametrize("one_launch", [True, False])
+@pytest.mark.parametrize("dtype", [np.int64, np.int32])
+@pytest.mark.parametrize("bs,bad", [(1, 1), (1, 2), (1, 3), (16, 1), (16, 16), (16, 32), (16, 300), (7, 30)])
+def test_offsets_whose_counts_add_up_to_more_than_63_bits(oracle, monkeypatch, one_launch, dtype, bs, bad):
+    """Requests that name tokens far beyond the array, many enough that their counts would wrap to below zero and back, in front of
+    sound ones, in the same workgroup and in later ones: nothing is written but the keys of requests that are all there and fit, at
+    the exact place; everybody else gets the offset -1. (The key buffer is the middle of a larger one that must not change.)"""
+    h = _h()
+    rng = np.random.default_rng(bs + bad)
+    n = 4096
+    far = 2**62 + 2**40
+    toff = [0, 16, 16 + 3 * bs, 0] + [far, 0] * bad + [5, 5 + 2 * bs, 300, 300 + bs, n] + [n] * 20 + [n - bs, n]
+    R = len(toff) - 1
+    flat = rng.integers(-2**31, 2**31, size=n, dtype=np.int64).astype(dtype)
+    tok, off = dev(flat), dev(np.array(toff, dtype=np.int64))
+    room = torch.full((3 * n,), -7, dtype=torch.int64, device="cuda")
+    koff = torch.full((R + 1,), -9, dtype=torch.int64, device="cuda")
+    word = torch.empty(1, dtype=torch.int64, pin_memory=True)
+    stream = torch.cuda.current_stream().cuda_stream
+    sync()
+    if one_launch:
+        h._launch_keys(tok, off, R, bs, 3, room[n:2 * n], koff, stream, word)
+    else:
+        h._launch_offsets(tok, off, R, bs, n, koff, word, stream)
+        h._launch_keys(tok, off, R, bs, 3, room[n:2 * n], koff, stream)
+    sync()
+    want_room, want_koff, at, left_out = np.full(3 * n, -7, dtype=np.int64), [], 0, 0
+    for a, b in zip(toff[:-1], toff[1:]):
+        length = (b - a + 2**63) % 2**64 - 2**63                    # distances are formed in 64 bits
+        count = max(0, length) // bs
+        whole = count == 0 or (0 <= a and a + count * bs <= n)
+        left_out += not whole
+        fits = whole and at + count <= n
+        want_koff.append(at if fits else -1)
+        if fits and count:
+            want_room[n + at:n + at + count], _ = oracle.hash_tokens(flat[a:a + count * bs].astype(np.int64)[None], bs, seed=3)
+        at += count
+    want_koff.append(min(at, 2**62))
+    assert left_out and word.item() == -1
+    assert host(koff, np.int64).tolist() == want_koff
+    assert (host(room, np.int64) == want_room).all()
+    monkeypatch.setattr(h, "_counted_by_the_hash", lambda R, n: one_launch)
+    with pytest.raises(ValueError):
+        h.hash_tokens(tok, bs, token_offsets=off)
+    sync()
+
+
 @pytest.mark.parametrize("general_loader", [False, True])
 def test_keys_beyond_the_callers_buffer_are_left_out(oracle, force_general_hash_loader, general_loader):
     """A key buffer that holds the keys of some requests only: those are written, the slots behind the buffer are not; the

@@ -2,10 +2,10 @@
 reference has the same for its own host code: .bazelrc:108-115 `--config=asan`, kv_cache_manager/client/test/asan_runner.py).
 
 `make -C tests/cpp sanitize` compiles oracle/kvcm_oracle.c, the library's host-only translation units
-(csrc/kvcm_file.hip, csrc/kvcm_host.hip, csrc/kvcm_host_idx.h) and include/kvcm_hip.hpp with a plain host compiler
+(csrc/kvcm_file.hip, csrc/kvcm_host.hip, csrc/kvcm_host_idx.h, csrc/kvcm_key_count.h) and include/kvcm_hip.hpp with a plain host compiler
 over a host stand-in of the HIP runtime (tests/cpp/sanitize/fake_hip.cpp), twice, and runs tests/cpp/sanitize/
 sanitize_host.cpp in both builds: 16 concurrent callers of a file store, a store destroyed while a transfer is inside
-it, the blocking cell pool, the index-list walk, the oracle's threaded forms. No GPU code is involved."""
+it, the blocking cell pool, the index-list walk, the sums of key offsets, the oracle's threaded forms. No GPU code is involved."""
 import os
 import shutil
 import subprocess
