@@ -240,7 +240,7 @@ static Py_ssize_t packed_size(PyObject *seq) {
 static int pack(PyObject *seq, char *base, Py_ssize_t size) {
     const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
     PyObject **items = PySequence_Fast_ITEMS(seq);
-    if (n > (size - 9) / 8) {
+    if (size < 9 || n > (size - 9) / 8) { /* the division rounds towards zero */
         return 0;
     }
     char *dst = base + 8 * (n + 1);

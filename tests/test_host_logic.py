@@ -469,6 +469,12 @@ def test_hash_strings_are_packed_where_the_caller_says():
             if size != len(want):
                 assert pack_strings_into(form, ctypes.addressof(room), size) is None
                 assert room.raw[max(size, len(want)):] == b"\x55" * (len(want) + 8 - max(size, len(want)))
+        for size in range(len(want) + 1):  # any size at all, an overrun past a smaller one included
+            room = ctypes.create_string_buffer(b"\x55" * (len(want) + 8), len(want) + 8)
+            assert pack_strings_into(form, ctypes.addressof(room), size) == (len(form) if size == len(want) else None)
+            assert room.raw[size:] == b"\x55" * (len(want) + 8 - size), (form, size)
+    for size in (0, -1, -8, -2**62):
+        assert pack_strings_into([], ctypes.addressof(room), size) is None
     assert strings_size([1]) is None and strings_size(["a", bytearray(b"b")]) is None
     with pytest.raises(UnicodeEncodeError):
         strings_size(["\ud800"])
