@@ -92,16 +92,16 @@ int32_t kvcm_hip_hash_tokens_checked(const void *d_tokens, int32_t token_bytes, 
                                      int64_t *d_keys, int64_t n_keys, const int64_t *d_key_offsets, kvcm_stream_t stream);
 
 /*
- * Added to token_bytes above, for 1 to KVCM_COUNT_KEYS_UP_TO requests: the launch makes the key offsets itself, as
- * kvcm_hip_key_offsets_checked would have in front of it. d_key_offsets is then the address of a kvcm_key_count in HOST memory,
- * which is read before the call returns; kvcm_wait_value() waits for h_total, which is written while the keys are being computed.
+ * The same for 1 to KVCM_COUNT_KEYS_UP_TO requests with key offsets that the launch makes itself, as kvcm_hip_key_offsets_checked
+ * would have in front of it: d_key_offsets receives R + 1 offsets, -1 for a request that is left out. h_total is PINNED host
+ * memory: the call sets it to KVCM_PENDING, and the launch, while the keys are being computed, to the sum of all requests, or to
+ * -1 where tokens are missing; kvcm_wait_value() waits for that.
  */
-#define KVCM_COUNT_KEYS 0x100
 #define KVCM_COUNT_KEYS_UP_TO 4096
-typedef struct kvcm_key_count {
-    int64_t *d_key_offsets; /* receives R + 1 offsets, -1 for a request that is left out */
-    int64_t *h_total;       /* pinned host memory: KVCM_PENDING, then the sum of all requests or -1 */
-} kvcm_key_count;
+int32_t kvcm_hip_hash_tokens_counted(const void *d_tokens, int32_t token_bytes, int64_t n_tokens,
+                                     const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t seed,
+                                     int64_t *d_keys, int64_t n_keys, int64_t *d_key_offsets, int64_t *h_total,
+                                     kvcm_stream_t stream);
 
 /*
  * The same for R requests of one length, laid out one behind the other ([R][tokens_per_request], token_bytes = 4 or 8):

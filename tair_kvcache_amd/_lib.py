@@ -48,12 +48,6 @@ class IovDevice(C.Structure):
     _fields_ = [("base", vp), ("size", sz)]
 
 
-class KeyCount(C.Structure):
-    """struct kvcm_key_count."""
-    _fields_ = [("d_key_offsets", vp), ("h_total", vp)]
-
-
-COUNT_KEYS = 0x100  # KVCM_COUNT_KEYS
 COUNT_KEYS_UP_TO = 4096  # KVCM_COUNT_KEYS_UP_TO
 
 # symbol -> (restype, argtypes); every prototype of include/kvcm_hip.h
@@ -64,6 +58,7 @@ SIGNATURES = {
     "kvcm_hip_hash_tokens_i32": (i32, [vp, vp, i32, i32, i64, vp, vp, vp]),
     "kvcm_hip_hash_tokens_2d": (i32, [vp, i32, i32, i64, i32, i64, vp, vp, vp, vp]),
     "kvcm_hip_hash_tokens_checked": (i32, [vp, i32, i64, vp, i32, i32, i64, vp, i64, vp, vp]),
+    "kvcm_hip_hash_tokens_counted": (i32, [vp, i32, i64, vp, i32, i32, i64, vp, i64, vp, vp, vp]),
     "kvcm_hip_key_offsets_workspace_bytes": (i64, [i32]),
     "kvcm_hip_key_offsets_checked": (i32, [vp, i32, i32, i64, i64, vp, i64, vp, vp, vp]),
     "kvcm_hip_key_offsets": (i32, [vp, i32, i32, i64, vp, vp, vp]),

@@ -1840,36 +1840,44 @@ int32_t kvcm_hip_hash_tokens_2d(const void *d_tokens, int32_t token_bytes, int32
 int32_t kvcm_hip_hash_tokens_checked(const void *d_tokens, int32_t token_bytes, int64_t n_tokens,
                                      const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t seed,
                                      int64_t *d_keys, int64_t n_keys, const int64_t *d_key_offsets, kvcm_stream_t stream) {
-    const bool counts = (token_bytes & KVCM_COUNT_KEYS) != 0;
-    token_bytes &= ~KVCM_COUNT_KEYS;
     if ((token_bytes != 4 && token_bytes != 8) || n_tokens < 0 || n_keys < 0) {
         return KVCM_ERR_INVALID_ARG;
-    }
-    kvcm::CountOut out{nullptr, nullptr, {0, 0}};
-    if (counts) {
-        const kvcm_key_count *const to = reinterpret_cast<const kvcm_key_count *>(d_key_offsets);
-        if (R <= 0 || block_size <= 0 || !d_tokens || !d_token_offsets || !d_keys || !to || !to->d_key_offsets || !to->h_total) {
-            return KVCM_ERR_INVALID_ARG;
-        }
-        if (R > KVCM_COUNT_KEYS_UP_TO) {
-            return KVCM_ERR_TOO_LARGE;
-        }
-        // recorded into a graph the launch would write h_total at every replay, long after the caller has given it back
-        if (kvcm::is_capturing(static_cast<hipStream_t>(stream))) {
-            return static_cast<int32_t>(hipErrorStreamCaptureUnsupported);
-        }
-        *to->h_total = KVCM_PENDING;
-        out = kvcm::CountOut{to->d_key_offsets, to->h_total, kvcm::make_fastdiv(static_cast<uint32_t>(block_size))};
-        d_key_offsets = nullptr;
     }
     const kvcm::Uniform no{0, 0, nullptr};
     const kvcm::Extent have{n_tokens, n_keys};
     if (token_bytes == 8) {
         return kvcm::launch_hash<int64_t>(static_cast<const int64_t *>(d_tokens), d_token_offsets, R, block_size, seed, d_keys,
-                                          d_key_offsets, static_cast<hipStream_t>(stream), no, have, out);
+                                          d_key_offsets, static_cast<hipStream_t>(stream), no, have);
     }
     return kvcm::launch_hash<int32_t>(static_cast<const int32_t *>(d_tokens), d_token_offsets, R, block_size, seed, d_keys,
-                                      d_key_offsets, static_cast<hipStream_t>(stream), no, have, out);
+                                      d_key_offsets, static_cast<hipStream_t>(stream), no, have);
+}
+
+int32_t kvcm_hip_hash_tokens_counted(const void *d_tokens, int32_t token_bytes, int64_t n_tokens,
+                                     const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t seed,
+                                     int64_t *d_keys, int64_t n_keys, int64_t *d_key_offsets, int64_t *h_total,
+                                     kvcm_stream_t stream) {
+    if ((token_bytes != 4 && token_bytes != 8) || n_tokens < 0 || n_keys < 0 || R <= 0 || block_size <= 0 || !d_tokens ||
+        !d_token_offsets || !d_keys || !d_key_offsets || !h_total) {
+        return KVCM_ERR_INVALID_ARG;
+    }
+    if (R > KVCM_COUNT_KEYS_UP_TO) {
+        return KVCM_ERR_TOO_LARGE;
+    }
+    // recorded into a graph the launch would write h_total at every replay, long after the caller has given it back
+    if (kvcm::is_capturing(static_cast<hipStream_t>(stream))) {
+        return static_cast<int32_t>(hipErrorStreamCaptureUnsupported);
+    }
+    *h_total = KVCM_PENDING;
+    const kvcm::Uniform no{0, 0, nullptr};
+    const kvcm::Extent have{n_tokens, n_keys};
+    const kvcm::CountOut out{d_key_offsets, h_total, kvcm::make_fastdiv(static_cast<uint32_t>(block_size))};
+    if (token_bytes == 8) {
+        return kvcm::launch_hash<int64_t>(static_cast<const int64_t *>(d_tokens), d_token_offsets, R, block_size, seed, d_keys,
+                                          nullptr, static_cast<hipStream_t>(stream), no, have, out);
+    }
+    return kvcm::launch_hash<int32_t>(static_cast<const int32_t *>(d_tokens), d_token_offsets, R, block_size, seed, d_keys,
+                                      nullptr, static_cast<hipStream_t>(stream), no, have, out);
 }
 
 int64_t kvcm_hip_key_offsets_workspace_bytes(int32_t R) {

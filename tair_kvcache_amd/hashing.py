@@ -9,7 +9,6 @@
 A connector that computes keys here can send `block_keys` instead of `token_ids`; the manager prefers them
 (kv_cache_manager/manager/cache_manager.cc:306-318) and the keys are bit-identical to the ones it would compute.
 """
-import ctypes
 import threading
 from array import array
 from collections import deque
@@ -120,12 +119,15 @@ def _launch_offsets(tokens, off, R, block_size, n_keys, key_offsets, pending, st
 
 def _launch_keys(tokens, off, R, block_size, seed, keys, key_offsets, stream, pending=None):
     """With `pending` the launch writes key_offsets, and their last into that pinned word, itself."""
-    token_bytes, at = tokens.element_size(), key_offsets.data_ptr()
     if pending is not None:
-        token_bytes |= _lib.COUNT_KEYS
-        at = ctypes.byref(_lib.KeyCount(at, pending.data_ptr()))
-    rc = lib().kvcm_hip_hash_tokens_checked(tokens.data_ptr(), token_bytes, tokens.numel(), off.data_ptr(), R,
-                                            block_size, int(seed), keys.data_ptr(), keys.numel(), at, stream)
+        rc = lib().kvcm_hip_hash_tokens_counted(tokens.data_ptr(), tokens.element_size(), tokens.numel(), off.data_ptr(), R,
+                                                block_size, int(seed), keys.data_ptr(), keys.numel(), key_offsets.data_ptr(),
+                                                pending.data_ptr(), stream)
+        if rc:
+            _lib.check(rc, "kvcm_hip_hash_tokens_counted")
+        return
+    rc = lib().kvcm_hip_hash_tokens_checked(tokens.data_ptr(), tokens.element_size(), tokens.numel(), off.data_ptr(), R,
+                                            block_size, int(seed), keys.data_ptr(), keys.numel(), key_offsets.data_ptr(), stream)
     if rc:
         _lib.check(rc, "kvcm_hip_hash_tokens_checked")
 

@@ -46,7 +46,7 @@ class _GeneralLoaderLib:
     tests/libkvcm_hash_general_loader.so: the same source built with KVCM_TEST_FORCE_GENERAL_LOADER=1, in which every
     launch takes the loader form of a workgroup whose requests span 4 GiB or more."""
     _SWAPPED = ("kvcm_hip_hash_tokens", "kvcm_hip_hash_tokens_i32", "kvcm_hip_hash_tokens_checked",
-                "kvcm_hip_hash_tokens_2d", "kvcm_hip_prefix_chain")
+                "kvcm_hip_hash_tokens_counted", "kvcm_hip_hash_tokens_2d", "kvcm_hip_prefix_chain")
 
     def __init__(self):
         import ctypes

@@ -71,12 +71,19 @@ def test_argument_validation_needs_no_device():
     assert checked(p, 8, -1, p, 1, 16, 0, p, 1, None, None) == _lib.ERR_INVALID_ARG
     assert checked(p, 8, 1, p, 1, 16, 0, p, -1, None, None) == _lib.ERR_INVALID_ARG
     assert checked(p, 4, 1, None, 1, 16, 0, p, 1, None, None) == _lib.ERR_INVALID_ARG
-    count = ctypes.byref(_lib.KeyCount(p, p))
-    assert checked(p, 8 | _lib.COUNT_KEYS, 1, p, 0, 16, 0, p, 1, count, None) == _lib.ERR_INVALID_ARG
-    assert checked(p, 8 | _lib.COUNT_KEYS, 1, p, 1, 16, 0, p, 1, None, None) == _lib.ERR_INVALID_ARG
-    assert checked(p, 8 | _lib.COUNT_KEYS, 1, p, 1, 16, 0, p, 1, ctypes.byref(_lib.KeyCount(p, None)), None) == _lib.ERR_INVALID_ARG
-    assert checked(p, 2 | _lib.COUNT_KEYS, 1, p, 1, 16, 0, p, 1, count, None) == _lib.ERR_INVALID_ARG
-    assert checked(p, 8 | _lib.COUNT_KEYS, 1, p, _lib.COUNT_KEYS_UP_TO + 1, 16, 0, p, 1, count, None) == _lib.ERR_TOO_LARGE
+    # four or eight, and nothing else: the offsets are never looked at on the host, whatever they point at
+    for odd in (0x100, 4 | 0x100, 8 | 0x100, 12, 16, -8):
+        assert checked(p, odd, 1, p, 1, 16, 0, p, 1, 8, None) == _lib.ERR_INVALID_ARG
+    counted = L.kvcm_hip_hash_tokens_counted
+    assert counted(p, 8, 1, p, 0, 16, 0, p, 1, p, p, None) == _lib.ERR_INVALID_ARG
+    assert counted(p, 8, 1, p, 1, 16, 0, p, 1, None, p, None) == _lib.ERR_INVALID_ARG
+    assert counted(p, 8, 1, p, 1, 16, 0, p, 1, p, None, None) == _lib.ERR_INVALID_ARG
+    assert counted(p, 2, 1, p, 1, 16, 0, p, 1, p, p, None) == _lib.ERR_INVALID_ARG
+    assert counted(p, 8, -1, p, 1, 16, 0, p, 1, p, p, None) == _lib.ERR_INVALID_ARG
+    assert counted(p, 8, 1, p, 1, 0, 0, p, 1, p, p, None) == _lib.ERR_INVALID_ARG
+    assert counted(p, 8, 1, None, 1, 16, 0, p, 1, p, p, None) == _lib.ERR_INVALID_ARG
+    assert counted(p, 8, 1, p, _lib.COUNT_KEYS_UP_TO + 1, 16, 0, p, 1, p, p, None) == _lib.ERR_TOO_LARGE
+    assert one.value == 0  # refused before the total is marked as pending
     offsets = L.kvcm_hip_key_offsets_checked
     assert offsets(p, 0, 16, 1, 1, None, 0, p, None, None) == _lib.ERR_INVALID_ARG
     assert offsets(p, 1, 0, 1, 1, None, 0, p, None, None) == _lib.ERR_INVALID_ARG
