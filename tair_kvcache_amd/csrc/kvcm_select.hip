@@ -319,6 +319,14 @@ __device__ __forceinline__ uint32_t part_hash(uint64_t k) {
     return static_cast<uint32_t>(x);
 }
 
+// All bits of a key into all bits of the result (the finalizer of MurmurHash3): whatever pattern brings keys into one part, this
+// one spreads them.
+__device__ __forceinline__ uint64_t mix_key(uint64_t k) {
+    k = (k ^ (k >> 33)) * 0xff51afd7ed558ccdull;
+    k = (k ^ (k >> 33)) * 0xc4ceb9fe1a85ec53ull;
+    return k ^ (k >> 33);
+}
+
 // flags[i] = keys[i] is a first occurrence and not saved yet. Exactly one write per key: whoever learns that an index is not the
 // smallest of its key clears it -- its own, or the one it has just replaced -- and what is left in the table at the end is set.
 __global__ __launch_bounds__(kPartThreads) void part_kernel(const uint64_t *__restrict__ keys, int32_t n, int log2_parts, int log2_slots,
@@ -326,16 +334,28 @@ __global__ __launch_bounds__(kPartThreads) void part_kernel(const uint64_t *__re
     extern __shared__ __attribute__((aligned(16))) uint64_t s_key[];
     const uint32_t slots = 1u << log2_slots, mask = slots - 1;
     int32_t *const s_first = reinterpret_cast<int32_t *>(s_key + slots);  // smallest index of the slot's key
-    __shared__ int32_t s_first_no_key;
+    __shared__ int32_t s_first_no_key, s_full, s_hits;
     __shared__ uint64_t s_wait_key[kPartThreads / 64][2 * 64];
     __shared__ int32_t s_wait_idx[kPartThreads / 64][2 * 64];
     const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    for (uint32_t i = threadIdx.x; i < slots; i += kPartThreads) {
-        s_key[i] = kNoKey;
-        s_first[i] = INT32_MAX;
-    }
+    const auto clear = [&] {
+        for (uint32_t i = threadIdx.x; i < slots; i += kPartThreads) {
+            s_key[i] = kNoKey;
+            s_first[i] = INT32_MAX;
+        }
+    };
+    const auto write_out = [&] {
+        for (uint32_t s = threadIdx.x; s <= slots; s += kPartThreads) {
+            const int32_t f = s < slots ? s_first[s] : s_first_no_key;
+            if (f != INT32_MAX) {
+                flags[f] = !(saved && saved[f]);
+            }
+        }
+    };
+    clear();
     if (threadIdx.x == 0) {
         s_first_no_key = INT32_MAX;
+        s_full = s_hits = 0;
     }
     __syncthreads();
     const auto put = [&](int32_t *first, int32_t i) {
@@ -344,26 +364,24 @@ __global__ __launch_bounds__(kPartThreads) void part_kernel(const uint64_t *__re
             flags[was < i ? i : was] = 0;
         }
     };
-    const auto take = [&](uint64_t k, int32_t i) {
-        if (k == kNoKey) {
-            put(&s_first_no_key, i);
-            return;
-        }
-        uint32_t s = (part_hash(k) << log2_parts) >> (32 - log2_slots);
+    const auto probe = [&](uint64_t k, int32_t i, uint32_t s) {  // false: all slots hold other keys
         for (uint32_t tries = 0; tries < slots; ++tries) {
             const uint64_t o = atomicCAS(reinterpret_cast<unsigned long long *>(s_key + s), kNoKey, k);
             if (o == kNoKey || o == k) {
                 put(s_first + s, i);
-                return;
+                return true;
             }
             s = (s + 1) & mask;
         }
-        // More different keys than slots, all of one part: keys made to collide. Looked for one by one.
-        int32_t j = 0;
-        while (j < i && keys[j] != k) {
-            ++j;
+        return false;
+    };
+    const auto take = [&](uint64_t k, int32_t i) {
+        if (k == kNoKey) {
+            put(&s_first_no_key, i);
+        } else if (__hip_atomic_load(&s_full, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0 &&
+                   !probe(k, i, (part_hash(k) << log2_parts) >> (32 - log2_slots))) {
+            __hip_atomic_store(&s_full, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
-        flags[i] = j == i && !(saved && saved[i]);
     };
     uint64_t *const wait_key = s_wait_key[wave];
     int32_t *const wait_idx = s_wait_idx[wave];
@@ -426,11 +444,41 @@ __global__ __launch_bounds__(kPartThreads) void part_kernel(const uint64_t *__re
     }
     enter(waiting);
     __syncthreads();
-    for (uint32_t s = threadIdx.x; s <= slots; s += kPartThreads) {
-        const int32_t f = s < slots ? s_first[s] : s_first_no_key;
-        if (f != INT32_MAX) {
-            flags[f] = !(saved && saved[f]);
+    if (s_full == 0) {
+        write_out();
+        return;
+    }
+    // More different keys than slots, all of one part: keys with a pattern that the sum of products maps to one place. Their part is
+    // gone through once more, as many times over as bring the number of keys down to half the slots, a share of the mixed keys
+    // at a time. What has been cleared so far stays so (a smaller index of that key is known), everything else is decided again.
+    const auto mine = [&](uint64_t k) { return k != kNoKey && part_hash(k) >> (32 - log2_parts) == blockIdx.x; };
+    int32_t hits = 0;
+#pragma unroll 4
+    for (int32_t i = threadIdx.x; i < n; i += kPartThreads) {
+        hits += mine(keys[i]);
+    }
+    atomicAdd(&s_hits, hits);
+    __syncthreads();
+    int log2_shares = 1;
+    while ((s_hits >> log2_shares) > static_cast<int32_t>(slots / 2)) {
+        ++log2_shares;
+    }
+    for (uint32_t share = 0; share < 1u << log2_shares; ++share) {
+        clear();
+        __syncthreads();
+        for (int32_t i = threadIdx.x; i < n; i += kPartThreads) {
+            const uint64_t k = keys[i], m = mix_key(k);
+            if (static_cast<uint32_t>(m >> 32) >> (32 - log2_shares) == share && mine(k) && !probe(k, i, static_cast<uint32_t>(m) & mask)) {
+                int32_t j = 0;  // made against this function, too: looked for one by one
+                while (j < i && keys[j] != k) {
+                    ++j;
+                }
+                flags[i] = j == i && !(saved && saved[i]);
+            }
         }
+        __syncthreads();
+        write_out();
+        __syncthreads();
     }
 }
 

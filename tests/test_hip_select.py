@@ -193,6 +193,17 @@ def test_first_occurrences_where_table_and_probes_change(oracle, n, each):
     assert int(count.item()) == len(want) and (idx[:len(want)].cpu().numpy() == want).all()
 
 
+def _colliding_keys(rng, n, below):
+    """n keys, each twice, with low word * 0x9e3779b1 + high word * 0x85ebca77 (modulo 2^32) below `below`: one part, and one slot of
+    it for 64."""
+    high = np.arange((n + 1) // 2, dtype=np.uint64) * 977
+    inverse = pow(0x9E3779B1, -1, 1 << 32)
+    low = ((rng.integers(0, below, size=len(high)).astype(np.uint64) - high * np.uint64(0x85EBCA77)) & np.uint64(0xFFFFFFFF))
+    low = (low * np.uint64(inverse)) & np.uint64(0xFFFFFFFF)
+    assert ((low * np.uint64(0x9E3779B1) + high * np.uint64(0x85EBCA77)) & np.uint64(0xFFFFFFFF)).max() < below
+    return rng.permutation(np.resize(((high << np.uint64(32)) | low).astype(np.int64), n))
+
+
 @pytest.mark.parametrize("n", [1, 2, 3, 5, 63, 64, 65, 511, 512, 513, 1023, 1024, 1025, 4095, 4096, 4097, 8191, 8192, 8193, 65535, 65536])
 @pytest.mark.parametrize("kind", ["different", "repeated", "one", "marker", "small", "colliding"])
 def test_save_list_from_parts(oracle, n, kind):
@@ -212,15 +223,7 @@ def test_save_list_from_parts(oracle, n, kind):
     elif kind == "small":
         keys = rng.permutation(n).astype(np.int64)
     else:
-        if n > 8193:
-            pytest.skip("thousands of keys that are looked for one by one: enough of them in 8193")
-        # low word * 0x9e3779b1 + high word * 0x85ebca77 (modulo 2^32) below 2^6: one part, one slot
-        high = np.arange((n + 1) // 2, dtype=np.uint64) * 977
-        inverse = pow(0x9E3779B1, -1, 1 << 32)
-        low = ((rng.integers(0, 64, size=len(high)).astype(np.uint64) - high * np.uint64(0x85EBCA77)) & np.uint64(0xFFFFFFFF))
-        low = (low * np.uint64(inverse)) & np.uint64(0xFFFFFFFF)
-        assert ((low * np.uint64(0x9E3779B1) + high * np.uint64(0x85EBCA77)) & np.uint64(0xFFFFFFFF)).max() < 64
-        keys = rng.permutation(np.resize(((high << np.uint64(32)) | low).astype(np.int64), n))
+        keys = _colliding_keys(rng, n, 64)
     mask = rng.random(n) < 0.25
     rep = oracle.first_occurrence(keys)[1].astype(bool)
     for m in (None, mask):
@@ -228,3 +231,20 @@ def test_save_list_from_parts(oracle, n, kind):
         idx, count = save_selection.select_save_indices(torch.from_numpy(keys).cuda(), None if m is None else torch.from_numpy(m).cuda())
         sync()
         assert int(count.item()) == len(want) and (idx[:len(want)].cpu().numpy() == want).all()
+
+
+@pytest.mark.parametrize("below", [64, 1 << 24])
+def test_keys_of_one_part_are_not_looked_for_one_by_one(below):
+    """65 536 keys that all belong to one of the 256 parts, with one slot to start from or with any: the list takes milliseconds where a
+    search through the keys in front of each, in one workgroup, takes hundreds of them."""
+    from tair_kvcache_amd import save_selection
+    d_keys = torch.from_numpy(_colliding_keys(np.random.default_rng(below), 65536, below)).cuda()
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    sync()
+    start.record()
+    _, count = save_selection.select_save_indices(d_keys)
+    end.record()
+    sync()
+    ms = start.elapsed_time(end)
+    print(f"save list of 65 536 keys of one part: {ms:.2f} ms", flush=True)
+    assert int(count.item()) == 32768 and ms < 20
