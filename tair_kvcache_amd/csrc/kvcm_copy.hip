@@ -200,7 +200,7 @@ __device__ __forceinline__ void copy_span_body(const CopyArgs &a, const void *co
         const uint32_t b = fast_div(unit, a.div_units);
         const uint32_t span = unit - b * a.units_per_block;
         const int64_t runs_b = static_cast<int64_t>(b) * a.runs;  // index of the block's first run
-        // workgroup- or wave-uniform part: the three table reads below are independent scalar loads in the UNI_* forms
+        // workgroup- or wave-uniform part: the three table reads below are independent scalar loads where tile and run are shared
         static_assert(TILE != kTilePerWave || (kCPT == 1 && RUN == kRunPerWave), "one chunk per thread, a slot per wave");
         const uint32_t g_first = span * kSpan + (TILE == kTilePerWave ? __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u) : 0);
         if (TILE == kTilePerWave && g_first >= a.chunks_per_block) {
@@ -394,40 +394,54 @@ int32_t align_class(uint64_t bits) {
 }
 
 // Stores of launches whose waves each move a kilobyte of one run (smaller pieces stay non-temporal: written through they cost up to
-// 25 %). Written through (sc1) the data stays in the 256 MiB memory-side cache, which is right for what a gather leaves in staging, and
-// wrong for what a scatter leaves in the pool while staging could stay there: a scatter that fits the cache carries nt. GB/s, nt / sc1 / both:
-//   scatter, whole tiles of 2^k bytes  128 KiB 5866 / 6504 / 6149 (4 GiB), 64 KiB - / 6306 / 6107, 32 KiB - / 5714 / 5592 (1.5 GiB);
-//                                      16 KiB, 115 MiB, again and again: - / 5400 / 5850
-//   scatter, other tiles               9 KiB 5519 / 5599 / 5512, 18 KiB 5532 / 5615 / 5537, 20 KiB - / 5621 / 5415,
-//                                      36 KiB - / 5668 / 5823, 72 KiB - / 5721 / 6132 (1.5 GiB)
-//   scatter, a slot per token          1 KiB, 1.8 GiB: 5510 / 5460 / -
-//   gather, whole tiles of 2^k         - / 6245 / 6249 (4 GiB), - / 6681 / 5860 (180 MiB)
-//   gather, other tiles                18 KiB 5828 / 5630 / 5951, 36 KiB - / 5944 / 6142 (1.5 GiB), - / 5974 / 6002 (600 MiB),
-//                                      - / 5949 / 5911 (400 MiB), - / 6639 / 5914 (180 MiB)
-//   gather, a slot per token           1 KiB 5732 / 5666 / 5859, 2 KiB 5814 / 5855 / 5936 (1.8 GiB)
+// 25 %). Written through (sc1) the data stays in the 256 MiB memory-side cache. That is right for what a gather leaves in staging,
+// whose slots are handed out again and again, as long as they fit; blocks of the pool change from call to call, so a launch repeated
+// on the same ones says nothing. GB/s, nt / sc1 / both, read and written bytes together, blocks changing from launch to launch (4 GiB
+// and more in turn), mean over nine or ten distances between the arrays of the pool (24 GiB: one):
+//   scatter, whole tiles of       100 MiB              400 MiB              1.2 GiB              4 GiB                24 GiB
+//     4 KiB                       5095 / 5026 / 5047   5394 / 5341 / 5386   5480 / 5440 / 5490   5510 / 5484 / 5527   5520 / 5377 / 5561
+//     32 KiB                      5136 / 5160 / 5118   5476 / 5466 / 5484   5572 / 5578 / 5588   5667 / 5622 / 5702   5441 / 5420 / 5463
+//     64 KiB                      5627 / 5649 / 5695   5989 / 6090 / 6142   6120 / 6221 / 6288   6138 / 6281 / 6328   6056 / 6147 / 6265
+//     128 KiB                     5839 / 5824 / 5854   6178 / 6274 / 6291   6365 / 6416 / 6470   6327 / 6482 / 6474   6233 / 6352 / 6346
+//     512 KiB                                          6287 / 6307 / 6362   6386 / 6449 / 6492   6437 / 6510 / 6547   6406 / 6480 / 6505 (20 GiB)
+//     36 KiB                      5200 / 5090 / 5222   5590 / 5423 / 5657   5665 / 5529 / 5741   5647 / 5574 / 5721   5539 / 5408 / 5625
+//     72 KiB                      5501 / 5166 / 5636   5894 / 5485 / 6072   5979 / 5580 / 6179   6022 / 5630 / 6231   5933 / 5466 / 6119
+//   scatter, 18 KiB, wave tiles   5070 / 5067 / 5052   5421 / 5375 / 5424   5493 / 5477 / 5506   5530 / 5521 / 5548   5416 / 5384 / 5428
+//   scatter, a 1 KiB row a slot   5069 / 5000 / 5032   5378 / 5316 / 5367   5458 / 5436 / 5462   5500 / 5486 / 5517   5367 / 5405 / 5374
+//   gather, whole tiles of
+//     4 KiB                       5331 / 5293 / 5360   5671 / 5655 / 5754   5755 / 5779 / 5869   5784 / 5806 / 5917   6250 / 6181 / 6321
+//     32 KiB                      5404 / 5443 / 5464   5796 / 5850 / 5900   5887 / 5973 / 6005   5959 / 6064 / 6090   6234 / 6278 / 6309
+//     128 KiB                     5841 / 5831 / 5845   6207 / 6242 / 6283   6354 / 6416 / 6449   6355 / 6441 / 6461   6534 / 6553 / 6579
+//     72 KiB                      5653 / 5578 / 5720   6054 / 5988 / 6168   6146 / 6099 / 6272   6187 / 6156 / 6320   6437 / 6425 / 6502
+//   gather, 18 KiB, wave tiles    5300 / 5070 / 5373   5679 / 5417 / 5799   5757 / 5502 / 5890   5793 / 5541 / 5933   6122 / 6029 / 6200
+//   gather, a 1 KiB row a slot    5247 / 5111 / 5256   5580 / 5455 / 5634   5663 / 5587 / 5763   5697 / 5651 / 5836   5971 / 5824 / 6040
+//   the same into the same staging every time          120 MiB              260 MiB              420 MiB
+//     32 KiB                                           5597 / 6476 / 5695   5873 / 6508 / 5953   5959 / 5991 / 6074
+//     72 KiB                                           5848 / 6522 / 5920   6011 / 6817 / 6093   6132 / 6109 / 6254
+//     18 KiB, wave tiles                               5463 / 6292 / 5563   5405 / 6042 / 5502   5773 / 5533 / 5899
+// A scatter of whole spans carries both: from 100 MiB on nothing is more than 1 % ahead of it on the mean. But where the arrays of the pool lie a little
+// more than a power of two apart, stores with nt fall behind (128 KiB tiles, 32.25 or 512.25 MiB apart: 5826 / 6462 / 6138 at 4 GiB,
+// 5855 / 6489 / 6161 at 20 GiB; at other distances 6384 / 6481 / 6519), and launches of 3 GiB and more of such tiles, where sc1 costs 0.1
+// to 1 % otherwise, are written through alone. (The same holds for tiles of 16 to 64 KiB, up to 13 %, but there sc1 costs up to 2 % at
+// other distances. What lies how far apart only the device's pointer table knows.)
 // Staging tiles that do not start on cache lines (a 4-byte scale behind every tile) make a wave's kilobyte begin and end inside one,
 // and partial lines written through cost a gather 15 % (5.2 against 6.0 TB/s).
 int32_t store_policy(const CopyArgs &a, bool scatter, int64_t run_bytes, int64_t launch_bytes, bool group_tiles) {
-    const bool power_of_two = (run_bytes & (run_bytes - 1)) == 0;
     const bool group_runs = group_tiles && a.chunks_per_run % kSpan == 0;
     if (scatter) {
-        if (group_tiles && !group_runs) {
-            return kStoreNt;  // a slot per token
+        if (!group_runs) {
+            return kStoreNt;
         }
-        if (!group_runs) {  // us, a tile per thread and nt / a tile per wave and this: 18 KiB, 1.7 GiB 703 / 655, 115 MiB 45.1 / 42.1
-            return launch_bytes < (int64_t{1536} << 20) ? kStoreNt : kStoreThrough;
-        }
-        // us, both / sc1, again and again on the same blocks: 32 KiB, 900 MiB 335 / 338, 1.7 GiB 632 / 635, 64 KiB 567 / 570, 8 KiB
-        // 638 / 644; 128 KiB, 4 GiB 1363 / 1298
-        return launch_bytes >= (int64_t{3} << 30) && (power_of_two || run_bytes < (32 << 10)) ? kStoreThrough : kStoreThroughNt;
+        const bool large_power_of_two = run_bytes >= (128 << 10) && (run_bytes & (run_bytes - 1)) == 0;
+        return large_power_of_two && launch_bytes >= (int64_t{3} << 30) ? kStoreThrough : kStoreThroughNt;
     }
     if (((reinterpret_cast<uint64_t>(a.staging) | static_cast<uint64_t>(a.block_stride) | static_cast<uint64_t>(a.tile_stride)) & 127u) != 0) {
         return kStoreNt;
     }
-    if (group_tiles && !group_runs) {  // a slot per token; 2 KiB, 300 MiB, again and again: nt 101 us, sc1 103
+    if (group_tiles && !group_runs) {  // a slot per token
         return launch_bytes < (int64_t{768} << 20) ? kStoreNt : kStoreThroughNt;
     }
-    return launch_bytes < (int64_t{400} << 20) || (power_of_two && group_runs) ? kStoreThrough : kStoreThroughNt;
+    return launch_bytes < (int64_t{400} << 20) ? kStoreThrough : kStoreThroughNt;
 }
 
 // emb != nullptr: the index tables are *emb (copied into the kernel's argument block by the launch), run starts from
@@ -530,8 +544,9 @@ int32_t launch_copy(const kvcm_copy_desc *d, bool scatter, hipStream_t stream, c
     } else if (cs == 16 && uni_tile) {
         launch_span<16, kTilePerGroup, kRunPerThread>(a, d, scatter, g32, stream, emb, staging_first);
     } else if (cs == 16 && kCPT == 1 && a.chunks_per_run % 64 == 0) {
-        // GB/s, per thread / per wave, 1.5 GiB: 1152-byte rows in tiles of 16, runs of 16 gather 5366 / 5951, scatter 5245 / 5615,
-        // runs of 8 5332 / 5895, 5246 / 5599; 576-byte rows in tiles of 32 5373 / 5950, 5252 / 5613; 320 in 16 5273 / 5803, 5210 / 5560
+        // GB/s, per thread / per wave, 2 GiB of changing blocks: 1152-byte rows in tiles of 16, runs of 16 gather 5245 / 5824, scatter
+        // 5203 / 5447, runs of 8 5264 / 5864, 5227 / 5492; 576-byte rows in tiles of 32 5317 / 5930, 5273 / 5548; 60 MiB of them
+        // 4579 / 4668, 4540 / 4804
         launch_span<16, kTilePerWave, kRunPerWave>(a, d, scatter, g32, stream, emb, staging_first);
     } else if (cs == 16) {
         launch_span<16, kTilePerThread, kRunPerThread>(a, d, scatter, g32, stream, emb, staging_first);

@@ -365,7 +365,8 @@ def test_block_major_pools_are_the_one_array_case(oracle):
     (1024, 1, 1, 3, 5), (1024, 3, 1, 1, 9), (1024, 5, 1, 7, 3), (3072, 7, 1, 3, 4),          # tiles of whole waves
     (1152, 16, 16, 61, 360), (1152, 16, 16, 61, 730), (1152, 16, 16, 61, 1450),             # 386 and 783 MiB, 1.5 GiB
     (1152, 32, 32, 61, 180), (1152, 32, 32, 61, 190), (1152, 32, 32, 61, 350), (1152, 32, 32, 61, 370),
-    (1024, 16, 1, 56, 450), (1024, 16, 1, 56, 920), (2048, 16, 16, 64, 220), (2048, 16, 16, 64, 1560)])
+    (1024, 16, 1, 56, 450), (1024, 16, 1, 56, 920), (2048, 16, 16, 64, 220), (2048, 16, 16, 64, 1560),
+    (2048, 64, 64, 40, 600), (2048, 64, 64, 40, 620), (2048, 32, 32, 40, 1240)])                # 128 KiB runs, 2.9 and 3.03 GiB; 64 KiB runs
 def test_waves_tiles_and_store_policies(row, T, run, P, B):
     """Tiles that are whole waves' worth of chunks but not whole spans (the last span of a block with one to four waves), and launches
     on both sides of every line of the rule that chooses how stores go to memory: both directions against torch's own indexing,
