@@ -1238,7 +1238,7 @@ __global__ __launch_bounds__(kLeanThreads) void hash_lean_kernel(const TokT *__r
     } else {
         first = r_first * uni.tokens;
         total = R * uni.tokens;
-        span = kLeanRows * uni.tokens;
+        span = (R - r_first < kLeanRows ? R - r_first : kLeanRows) * uni.tokens;  // of the requests that there are
         if (r < R) {
             row.start = r * uni.tokens;
             row.key = key_offsets ? key_offsets[r] : r * uni.keys;
@@ -1246,6 +1246,9 @@ __global__ __launch_bounds__(kLeanThreads) void hash_lean_kernel(const TokT *__r
             row.ntok = count * block_size;
         }
         nt = static_cast<int32_t>((uni.keys * block_size + kLeanTok - 1) / kLeanTok);
+        if (key_offsets && __ballot(count > 0) == 0) {
+            nt = 0;  // the caller wants no keys of any of them
+        }
         if (uni.key_offsets_out && wave == kLeanWriter) {
             if (lane < kLeanRows && r < R) {
                 uni.key_offsets_out[r] = r * uni.keys;

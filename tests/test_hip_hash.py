@@ -764,6 +764,54 @@ def test_sixteen_requests_per_workgroup(oracle, force_general_hash_loader, gener
         assert (host(keys, np.int64) == want).all() and (host(off, np.int64) == woff).all(), (R, L, bs)
 
 
+def _ms(call):
+    """The shortest of five runs, in ms of the GPU."""
+    best = []
+    for _ in range(5):
+        start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        start.record()
+        call()
+        end.record()
+        sync()
+        best.append(start.elapsed_time(end))
+    return min(best)
+
+
+def test_one_request_of_more_than_a_sixteenth_of_4_gib(oracle):
+    """The requests that a workgroup does not have say nothing about how far its tokens reach: one request of 2^28 bytes and more takes
+    the loader that keeps up with the chain, at the pace of a shorter one."""
+    L = (1 << 25) + 64
+    tok = torch.randint(0, 128256, (1, L), dtype=torch.int64, device="cuda")
+    keys = torch.empty(L // 4096, dtype=torch.int64, device="cuda")
+    short = _ms(lambda: _h().hash_tokens(tok[:, :L // 2].contiguous(), 4096, keys=keys))
+    whole = _ms(lambda: _h().hash_tokens(tok, 4096, keys=keys))
+    print(f"2^24 tokens {short:.1f} ms, 2^25 {whole:.1f} ms", flush=True)
+    want, _ = oracle.hash_tokens(tok.cpu().numpy(), 4096)
+    assert (host(keys, np.int64) == want).all()
+    assert whole < 2.4 * short
+
+
+@pytest.mark.parametrize("R", [16, 40])
+def test_a_workgroup_of_requests_that_are_left_out_does_not_run(oracle, R):
+    """[R, L] batches with the caller's own key offsets, negative for requests whose keys nobody wants: where that is all of a
+    workgroup, it takes the time of a launch and not that of the recurrence; the others' keys are where they should be."""
+    L = 1 << 16
+    tok = torch.randint(0, 128256, (R, L), dtype=torch.int64, device="cuda")
+    keys = torch.full((R * (L // 64) + 1,), -7, dtype=torch.int64, device="cuda")
+    want, woff = oracle.hash_tokens(tok.cpu().numpy(), 64, threads=8)
+    none = torch.full((R + 1,), -1, dtype=torch.int64, device="cuda")
+    some = woff.copy()
+    some[[0, 5, R - 1]] = -1
+    some = dev(some)
+    assert _ms(lambda: _h().hash_tokens(tok, 64, keys=keys, key_offsets=none)) < 0.25    # 65 536 steps take 0.7 ms
+    assert (host(keys, np.int64) == -7).all()
+    _h().hash_tokens(tok, 64, keys=keys, key_offsets=some)
+    sync()
+    expect = want.reshape(R, -1).copy()
+    expect[[0, 5, R - 1]] = -7
+    assert (host(keys, np.int64)[:-1] == expect.reshape(-1)).all()
+
+
 def test_hash_strings_that_wait_behind_other_work(monkeypatch):
     """Calls whose strings the kernel has yet to read when the next ones arrive: more of them than are read in place, from two
     threads, strings of many lengths; then more bytes than are read in place; and nothing stays lent out."""
