@@ -124,7 +124,7 @@ int32_t kvcm_hip_key_offsets(const int64_t *d_token_offsets, int32_t R, int32_t 
 
 /*
  * The same against the number of tokens as well: a request whose blocks reach beyond n_tokens gets the offset -1, and
- * h_total becomes -1 when there is one (d_key_offsets[R] stays the sum of all requests, 2^62 where it would be more: a request
+ * h_total becomes -1 when there is one (d_key_offsets[R] stays the sum of all requests, 2^41 where it would be more: a request
  * behind that many keys gets the offset -1 as well). With d_workspace (at least
  * kvcm_hip_key_offsets_workspace_bytes(R) bytes, 8-byte aligned, or NULL) the time stays linear in R; up to 32768 requests
  * nothing is needed there.

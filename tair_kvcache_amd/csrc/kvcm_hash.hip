@@ -1083,7 +1083,7 @@ __device__ __forceinline__ int64_t lean_keys_of(const int64_t *__restrict__ toke
         for (int j = 0; j < kAhead; ++j) {
             const int64_t i = base + j * 128 + lane * 2;
             for (int64_t k = i; k < i + 2 && k < r_first; ++k) {
-                sum = add_keys(sum, keys_of_request(token_offsets[k], token_offsets[k + 1], block_size, have.tokens, bad));
+                sum += keys_of_request(token_offsets[k], token_offsets[k + 1], block_size, have.tokens, bad);
             }
         }
     }
@@ -1100,15 +1100,16 @@ __device__ __forceinline__ int64_t lean_keys_before(const int64_t *__restrict__ 
     constexpr int kMany = 8, kFew = 2;
     int64_t before = 0, base = 0;
     for (; r_first - base > kMany * 64; base += kMany * 128) {
-        before = add_keys(before, lean_keys_of<kMany>(token_offsets, base, r_first, block_size, have, by_block, lane, bad));
+        before += lean_keys_of<kMany>(token_offsets, base, r_first, block_size, have, by_block, lane, bad);
     }
     for (; base < r_first; base += kFew * 128) {
-        before = add_keys(before, lean_keys_of<kFew>(token_offsets, base, r_first, block_size, have, by_block, lane, bad));
+        before += lean_keys_of<kFew>(token_offsets, base, r_first, block_size, have, by_block, lane, bad);
     }
     return before;
 }
 
-// The key offsets of a workgroup's requests, and of the last one the total. before: this lane's share of the keys in front.
+// The key offsets of a workgroup's requests, and of the last one the total. before: this lane's share of the keys in front. (4096
+// requests of kMostKeys at most: no sum needs bringing down before the end.)
 __device__ __forceinline__ void lean_key_offsets(int64_t r_first, int32_t R, int64_t before, int64_t own, bool bad_before, bool bad,
                                                  const Extent &have, const CountOut &out, uint32_t lane, LeanRow &row, int64_t &count) {
     const int64_t r = r_first + lane;
@@ -1117,20 +1118,19 @@ __device__ __forceinline__ void lean_key_offsets(int64_t r_first, int32_t R, int
     int64_t incl = own;
     for (int d = 1; d < 64; d <<= 1) {
         const int64_t up = __shfl_up(incl, d, 64);
-        incl = add_keys(incl, static_cast<int>(lane) >= d ? up : 0);
-        before = add_keys(before, __shfl_xor(before, d, 64));
+        incl += static_cast<int>(lane) >= d ? up : 0;
+        before += __shfl_xor(before, d, 64);
     }
-    const int64_t in_front = __shfl_up(incl, 1, 64);
-    const int64_t key = add_keys(before, lane > 0 ? in_front : 0), end = add_keys(key, own);
+    const int64_t key = before + incl - own, total = at_most_all_keys(key + own);
     const bool any = __ballot(bad_before || (mine && bad)) != 0;
     // without its tokens, or beyond the room the caller has: marked, and left out
     const bool fits = !bad && keys_fit(key, own, have.keys);
     if (mine) {
         out.key_offsets[r] = fits ? key : -1;
         if (r == R - 1) {
-            out.key_offsets[R] = end;
+            out.key_offsets[R] = total;
             // relaxed: whoever waits for it reads nothing else by it (a release writes the whole L2 back first)
-            __hip_atomic_store(out.h_total, any ? -1 : end, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(out.h_total, any ? -1 : total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
     // every lane knows request lane % 16
@@ -1348,10 +1348,10 @@ __global__ __launch_bounds__(kOffsetsThreads) void key_sums_kernel(const int64_t
     bool bad = false;
 #pragma unroll 8
     for (int64_t i = base + threadIdx.x; i < end; i += kOffsetsThreads) {
-        sum = add_keys(sum, keys_of_request(token_offsets[i], token_offsets[i + 1], block_size, n_tokens, bad));
+        sum += keys_of_request(token_offsets[i], token_offsets[i + 1], block_size, n_tokens, bad);
     }
     for (int d = 1; d < 64; d <<= 1) {
-        sum = add_keys(sum, __shfl_xor(sum, d, 64));
+        sum += __shfl_xor(sum, d, 64);
     }
     const bool any = __ballot(bad) != 0;
     if ((threadIdx.x & 63) == 0) {
@@ -1363,9 +1363,10 @@ __global__ __launch_bounds__(kOffsetsThreads) void key_sums_kernel(const int64_t
         int64_t all = 0;
         bool some = false;
         for (int w = 0; w < kOffsetsThreads / 64; ++w) {
-            all = add_keys(all, s_sum[w]);
+            all += s_sum[w];
             some |= s_bad[w] != 0;
         }
+        all = at_most_all_keys(all);
         sums[blockIdx.x] = some ? ~all : all;
     }
 }
@@ -1384,13 +1385,14 @@ __global__ __launch_bounds__(kOffsetsThreads) void key_offsets_kernel(const int6
         for (int64_t g = threadIdx.x; g < static_cast<int64_t>(blockIdx.x); g += blockDim.x) {
             const int64_t v = sums[g];
             bad |= v < 0;
-            before = add_keys(before, v < 0 ? ~v : v);
+            before += v < 0 ? ~v : v;
         }
     } else {
         for (int64_t i = threadIdx.x; i < base; i += blockDim.x) {
-            before = add_keys(before, keys_of_request(token_offsets[i], token_offsets[i + 1], block_size, n_tokens, bad));
+            before += keys_of_request(token_offsets[i], token_offsets[i + 1], block_size, n_tokens, bad);
         }
     }
+    before = at_most_all_keys(before);
     const int64_t first = base + static_cast<int64_t>(threadIdx.x) * kOffsetsPerThread;
     int64_t off[kOffsetsPerThread + 1];
 #pragma unroll
@@ -1404,16 +1406,15 @@ __global__ __launch_bounds__(kOffsetsThreads) void key_offsets_kernel(const int6
         bool mine = false;
         count[j] = keys_of_request(off[j], off[j + 1], block_size, n_tokens, mine);
         left_out |= mine ? 1u << j : 0u;
-        sum = add_keys(sum, count[j]);
+        sum += count[j];
     }
     bad |= left_out != 0;
     int64_t incl = sum;
     for (int d = 1; d < 64; d <<= 1) {
         const int64_t up = __shfl_up(incl, d, 64);
-        incl = add_keys(incl, lane >= d ? up : 0);
-        before = add_keys(before, __shfl_xor(before, d, 64));
+        incl += lane >= d ? up : 0;
+        before += __shfl_xor(before, d, 64);
     }
-    const int64_t in_front = __shfl_up(incl, 1, 64);
     const bool any = __ballot(bad) != 0;
     if (lane == 63) {
         s_wave[0][wave] = incl;
@@ -1421,10 +1422,10 @@ __global__ __launch_bounds__(kOffsetsThreads) void key_offsets_kernel(const int6
         s_bad[wave] = any;
     }
     __syncthreads();
-    int64_t pos = lane > 0 ? in_front : 0;
+    int64_t pos = incl - sum;
     bool some = false;
     for (int w = 0; w < waves; ++w) {
-        pos = add_keys(add_keys(pos, w < wave ? s_wave[0][w] : 0), s_wave[1][w]);
+        pos += (w < wave ? s_wave[0][w] : 0) + s_wave[1][w];
         some |= s_bad[w] != 0;
     }
 #pragma unroll
@@ -1432,8 +1433,9 @@ __global__ __launch_bounds__(kOffsetsThreads) void key_offsets_kernel(const int6
         if (first + j < R) {
             // without its tokens, or beyond the room the caller has: marked, and the hash kernel leaves the request out
             key_offsets[first + j] = keys_fit(pos, count[j], limit) && !(left_out >> j & 1) ? pos : -1;
-            pos = add_keys(pos, count[j]);
+            pos += count[j];
             if (first + j == R - 1) {
+                pos = at_most_all_keys(pos);
                 key_offsets[R] = pos;
                 if (h_total) {  // the last workgroup has seen every request
                     __hip_atomic_store(h_total, some ? -1 : pos, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -1873,7 +1875,7 @@ int32_t kvcm_hip_hash_tokens_counted(const void *d_tokens, int32_t token_bytes, 
     }
     *h_total = KVCM_PENDING;
     const kvcm::Uniform no{0, 0, nullptr};
-    const kvcm::Extent have{n_tokens, n_keys};
+    const kvcm::Extent have{n_tokens, kvcm::room_for_keys(n_keys)};
     const kvcm::CountOut out{d_key_offsets, h_total, kvcm::make_fastdiv(static_cast<uint32_t>(block_size))};
     if (token_bytes == 8) {
         return kvcm::launch_hash<int64_t>(static_cast<const int64_t *>(d_tokens), d_token_offsets, R, block_size, seed, d_keys,
@@ -1915,7 +1917,7 @@ int32_t kvcm_hip_key_offsets_checked(const int64_t *d_token_offsets, int32_t R, 
     }
     const int64_t threads = groups > 1 ? kvcm::kOffsetsThreads : ((R + kvcm::kOffsetsPerThread - 1) / kvcm::kOffsetsPerThread + 63) / 64 * 64;
     hipLaunchKernelGGL(kvcm::key_offsets_kernel, dim3(static_cast<uint32_t>(groups)), dim3(static_cast<uint32_t>(threads)), 0, s,
-                       d_token_offsets, R, block_size, n_tokens, n_keys, sums, d_key_offsets, h_total);
+                       d_token_offsets, R, block_size, n_tokens, kvcm::room_for_keys(n_keys), sums, d_key_offsets, h_total);
     return kvcm::launch_status();
 }
 

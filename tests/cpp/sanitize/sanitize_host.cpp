@@ -433,35 +433,39 @@ void wait_for_a_value() {
 
 __extension__ typedef __int128 Wide;
 
-// Key offsets as the launches make them, request by request and as sums of halves, for any token offsets: a request gets a place
-// only if its tokens are all there and its keys end inside the room, places never overlap, and they are the exact sums.
-void key_offsets_of(const std::vector<int64_t> &off, int32_t block_size, int64_t n_tokens, int64_t n_keys) {
-    const size_t R = off.size() - 1;
-    std::vector<int64_t> count(R), level;
-    std::vector<Wide> exact(R + 1, 0);
-    int64_t before = 0, written_to = 0;
+// Key offsets as the launches make them, for any token offsets: a request gets a place only if its tokens are all there and its keys
+// end inside the room, places never overlap, and they are the exact sums. Counts of a workgroup are added up as they come, here
+// under a sanitizer that sees an overflow; what lies in front of it in shares, each brought down to kMostKeys.
+void key_offsets_of(const std::vector<int64_t> &off, int32_t block_size, int64_t n_tokens, int64_t n_keys, size_t group = 8192) {
+    const size_t R = off.size() - 1, lanes = 1024;
+    std::vector<int64_t> shares(lanes, 0);
+    Wide exact = 0;
+    int64_t before = 0, written_to = 0, pos = 0;
+    const int64_t room = kvcm::room_for_keys(n_keys);
     for (size_t r = 0; r < R; ++r) {
+        if (r % group == 0) {
+            before = 0;
+            for (const int64_t s : shares) {
+                before += kvcm::at_most_all_keys(s);
+            }
+            pos = before;
+        }
         bool bad = false;
-        count[r] = kvcm::keys_of_request(off[r], off[r + 1], block_size, n_tokens, bad);
-        CHECK(count[r] >= 0 && (count[r] == 0 || bad || kvcm::inside(off[r], count[r] * block_size, n_tokens)));
-        exact[r + 1] = exact[r] + count[r];
-        const bool fits = !bad && kvcm::keys_fit(before, count[r], n_keys);
-        CHECK(fits == (!bad && exact[r + 1] <= n_keys));
+        const int64_t count = kvcm::keys_of_request(off[r], off[r + 1], block_size, n_tokens, bad);
+        CHECK(count >= 0 && (count == 0 || bad || kvcm::inside(off[r], count * block_size, n_tokens)));
+        const int64_t len = kvcm::distance(off[r], off[r + 1]);
+        const Wide exact_count = len > 0 ? len / block_size : 0;
+        const bool fits = !bad && kvcm::keys_fit(pos, count, room);
+        CHECK(fits == (!bad && exact + exact_count <= n_keys && exact + exact_count < kvcm::kMostKeys));
         if (fits) {
-            CHECK(before == exact[r] && before >= written_to && before + count[r] <= n_keys);
-            written_to = before + count[r];
+            CHECK(pos == exact && pos >= written_to && pos + count <= n_keys);
+            written_to = pos + count;
         }
-        before = kvcm::add_keys(before, count[r]);
-        CHECK(before == (exact[r + 1] < kvcm::kMostKeys ? static_cast<int64_t>(exact[r + 1]) : kvcm::kMostKeys));
+        exact += exact_count;
+        pos += count;
+        CHECK(kvcm::at_most_all_keys(pos) == (exact < kvcm::kMostKeys ? static_cast<int64_t>(exact) : kvcm::kMostKeys));
+        shares[r % lanes] += count;
     }
-    for (level = count; level.size() > 1;) {  // lanes and waves add up in another order
-        std::vector<int64_t> next;
-        for (size_t i = 0; i < level.size(); i += 2) {
-            next.push_back(kvcm::add_keys(i + 1 < level.size() ? level[i + 1] : 0, level[i]));
-        }
-        level = next;
-    }
-    CHECK(kvcm::add_keys(level[0], 0) == before);
 }
 
 void key_offsets_of_any_token_offsets() {
@@ -487,6 +491,16 @@ void key_offsets_of_any_token_offsets() {
         }
         key_offsets_of(off, std::vector<int32_t>{1, 7, 16, INT32_MAX}[rng() % 4], 4096, static_cast<int64_t>(rng() % 5000));
     }
+    std::vector<int64_t> most;  // two workgroups of as many keys as a request can name
+    for (int i = 0; i < 8192; ++i) {
+        most.insert(most.end(), {0, INT64_MAX});
+    }
+    most.insert(most.end(), {0, 16});
+    for (const size_t group : {64, 4096, 8192}) {
+        key_offsets_of(most, 1, 4096, INT64_MAX, group);
+        key_offsets_of(most, 1, INT64_MAX, INT64_MAX, group);
+    }
+    CHECK(kvcm::kMostKeys <= INT64_MAX >> 21);  // a thread's share of 2^31 requests
     std::vector<int64_t> sound(2000, 0);  // nothing is left out where nothing is wrong
     for (size_t r = 1; r < sound.size(); ++r) {
         sound[r] = sound[r - 1] + static_cast<int64_t>(rng() % 100);

@@ -505,7 +505,7 @@ def test_offsets_whose_counts_add_up_to_more_than_63_bits(oracle, monkeypatch, o
         if fits and count:
             want_room[n + at:n + at + count], _ = oracle.hash_tokens(flat[a:a + count * bs].astype(np.int64)[None], bs, seed=3)
         at += count
-    want_koff.append(min(at, 2**62))
+    want_koff.append(min(at, 2**41))
     assert left_out and word.item() == -1
     assert host(koff, np.int64).tolist() == want_koff
     assert (host(room, np.int64) == want_room).all()
