@@ -235,20 +235,22 @@ def apply_prefix_hash(hash_ids: torch.Tensor, offsets: Optional[torch.Tensor] = 
 # place / copied from pinned memory: 1024 strings of 64 characters 14 / 28, 16 384 of 64: 33 / 46, of 200 (3.4 MB): 88 / 91.
 _PINNED_MOST = 4 << 20
 # Packed strings that launched kernels have yet to read, oldest first, with the event behind each. Calls that find as many as this
-# under way copy instead.
+# under way, or with whose own there would be more bytes than this, copy instead: what finished calls leave here until the next one
+# comes is no more than that either.
 _LENT_MOST = 64
+_LENT_BYTES_MOST = 16 << 20
 _lent = deque()
 _lent_lock = threading.Lock()
 _spare_events = {}  # device -> events whose strings have been given back
 
 
-def _settled_event(device):
-    """An event for the next packed strings, or None if too many are under way; gives back what has been read."""
+def _settled_event(device, size=0):
+    """An event for the next `size` bytes of packed strings, or None if too many are under way; gives back what has been read."""
     with _lent_lock:
         while _lent and _lent[0][1].query():
             was, event, _ = _lent.popleft()
             _spare_events.setdefault(was, []).append(event)
-        if len(_lent) >= _LENT_MOST:
+        if len(_lent) >= _LENT_MOST or size + sum(pinned.numel() for _, _, pinned in _lent) > _LENT_BYTES_MOST:
             return None
         spare = _spare_events.get(device)
         return spare.pop() if spare else torch.cuda.Event()
@@ -266,14 +268,15 @@ def _sha256_in_place(data, device):
         return None
     out = torch.empty(n, dtype=torch.int64, device=device)
     require_cuda(out, "device")
-    event = _settled_event(out.device)
+    event = _settled_event(out.device, size)
     if event is None:
         return None
     stream = torch.cuda.current_stream(out.device)
     try:
         rc = lib().kvcm_hip_sha256_first8_be(at + 8 * (n + 1), at, n, out.data_ptr(), stream.cuda_stream)
         event.record(stream)
-        _lent.append((out.device, event, pinned))
+        with _lent_lock:
+            _lent.append((out.device, event, pinned))
     except BaseException:  # an interrupt as much as an error: the kernel may still be to come
         _settle(pinned, out.device)
         raise

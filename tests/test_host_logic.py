@@ -480,3 +480,31 @@ def test_hash_strings_are_packed_where_the_caller_says():
         strings_size(["\ud800"])
     with pytest.raises(TypeError):
         strings_size("abc")
+
+
+def test_packed_strings_under_way_are_bounded_in_number_and_bytes(monkeypatch):
+    """Calls that would have more strings, or more bytes of them, lent to kernels than the bounds say get no event (and copy
+    instead); what has been read is given back by the next call, oldest first."""
+    from collections import deque
+    from tair_kvcache_amd import hashing
+
+    class Event:
+        done = False
+
+        def query(self):
+            return self.done
+
+    events = [Event() for _ in range(5)]
+    lent = deque(("dev", e, torch.empty(1000, dtype=torch.uint8)) for e in events)
+    spare = {"dev": ["spare"] * 10}
+    monkeypatch.setattr(hashing, "_lent", lent)
+    monkeypatch.setattr(hashing, "_spare_events", spare)
+    monkeypatch.setattr(hashing, "_LENT_BYTES_MOST", 6000)
+    assert hashing._settled_event("dev", 1000) == "spare" and hashing._settled_event("dev", 1001) is None
+    events[1].done = True                                      # not the oldest: it waits for its turn
+    assert hashing._settled_event("dev", 1001) is None and len(lent) == 5
+    events[0].done = True
+    assert hashing._settled_event("dev", 3000) is events[1] and len(lent) == 3 and events[0] in spare["dev"]
+    assert hashing._settled_event("dev", 3001) is None
+    monkeypatch.setattr(hashing, "_LENT_MOST", 3)
+    assert hashing._settled_event("dev", 0) is None
