@@ -5,6 +5,8 @@
 // token, h <- h ^ (v + C + (h << 12) + (h >> 32)), and is emitted at every block boundary. The step mixes
 // + and ^, so a request is a serial chain of len dependent steps; the parallelism is across requests.
 //
+// Two kernels, by number of requests. Up to kLeanUpTo (4096) hash_lean_kernel: 16 requests per workgroup, so that there is one for
+// each compute unit; its design and what bounds it stand above it. Beyond, hash_tokens_kernel:
 // Design (gfx950, wave64): a workgroup owns 64 requests and is role-split.
 //   wave 0      "chain wave": lane = request. Keeps the state in VGPRs and does nothing but the recurrence,
 //               reading pre-added terms a = v + C from LDS (one ds_read_b128 per 2 steps, prefetched a whole
@@ -333,14 +335,12 @@ constexpr int kKeysDirect = 0, kKeysSpread = 1, kKeysBurst = 2;
 // A workgroup of a spread kernel whose requests are shorter than this many tiles stores its keys directly: what the last
 // group costs after the loop (about 1.5 us) is more than staging saves on 2048 tokens.
 constexpr int kSpreadFromTiles = 32;
-// Block size 1, 8-byte elements (the prefix chain): a workgroup of few or short equally long requests stores its keys directly
-// too, because a store takes the longer the more lanes it has, and a small launch leaves the memory to it. Direct / staged, us:
-// 4096 digests each, 31 requests 78 / 97, 32: 80 / 93, 48: 106 / 89, 64: 146 / 86; 64 requests of 64 digests 4.4 / 5.4, of 256:
-// 7.9 / 9.2, 512: 13.7 / 14.2, 1024: 24.0 / 24.0; 2048 requests of 256: 10.4 / 10.4, of 512: 19.2 / 16.1. Where requests end at
-// different places staging pays from two of them on: 4 requests of 64 to 512 digests 21.8 / 16.2, of 64 to 4096 155 / 100 --
-// unless nobody fills a tile: 32 of 4 to 64 digests 5.5 / 5.9, 1000 of them 5.8 / 6.2.
-__device__ __forceinline__ bool chain_stays_direct(uint32_t requests, uint32_t workgroups, uint32_t ntiles, uint32_t whole) {
-    return whole + 1 >= ntiles ? requests <= 32 || (ntiles <= 8 && workgroups <= 16) || whole == 0 : false;
+// Block size 1, 8-byte elements (the prefix chain): a workgroup in which nobody fills a tile stores its keys directly (1000 sequences
+// of 4 to 64 digests 5.8 us, staged 6.2), and so does one of few equally long requests, the last of a launch, because a store takes
+// the longer the more lanes it has (4096 digests each, 31 requests direct / staged 78 / 97, 32: 80 / 93, 48: 106 / 89, 64: 146 / 86).
+// Where requests end at different places staging pays from two of them on: 4 requests of 64 to 4096 digests 155 / 100.
+__device__ __forceinline__ bool chain_stays_direct(uint32_t requests, uint32_t ntiles, uint32_t whole) {
+    return whole + 1 >= ntiles && (requests <= 32 || whole == 0);
 }
 
 // The steps [first_step, kDrainSteps) of a group that belong to loader `me` (step % kLoaders == me), all LDS reads
@@ -709,7 +709,7 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
         KS == kKeysSpread  ? ntiles_u >= static_cast<uint32_t>(kSpreadFromTiles)
         : KS != kKeysBurst ? false
         : BS == 1 && sizeof(TokT) == 8
-            ? !chain_stays_direct(static_cast<uint32_t>(R - r_first < kReqs ? R - r_first : kReqs), gridDim.x, ntiles_u, full_u)
+            ? !chain_stays_direct(static_cast<uint32_t>(R - r_first < kReqs ? R - r_first : kReqs), ntiles_u, full_u)
             : true;
     if (wave != 0) {
         // ---------------------------------------------------------------- loader waves
@@ -1598,54 +1598,62 @@ __global__ __launch_bounds__(256) void iov_crc32_kernel(const kvcm_iov_device *_
 #endif
 constexpr int32_t kForceGeneralLoader = KVCM_TEST_FORCE_GENERAL_LOADER;
 
-// How keys reach memory, by block size, token width and number of requests in the launch (hash_tokens_kernel<.., KS>).
+// Requests up to which a launch takes workgroups of 16 (hash_lean_kernel): as many as give each of the 256 compute units one. A
+// second one on a unit shares its SIMDs, and one of 16 reads 512 bytes of each of 16 requests at a time where the other kernel
+// reads 64. us, 16 per workgroup / 64: 4096 requests of 4096 tokens 49.2 / 55.8, 5120: 59.0 / 56.8, 8192: 71.4 / 59.9. The line
+// holds for either token width, every block size and short requests too, though a launch of those is few tiles long. us on changing
+// tokens, 64 per workgroup (in the form that launch took) / 16:
+//                     4096 x 64   x 256      x 1024      x 4096         0..128     0..512      0..2048     512 x 1024
+//   bs 1,   8 bytes   6.5/4.9     11.2/8.7   29.0/19.0   99.3/58.2      8.9/6.6    19.9/12.2   58.1/30.7   26.6/15.7
+//   bs 16,  8 bytes   5.3/4.3     8.7/7.1    18.6/15.7   56.0/49.3      6.9/5.5    13.8/10.2   37.6/27.1   17.7/14.5
+//   bs 128, 8 bytes   -           8.6/7.1    18.3/15.4   51.9/48.8      -          12.6/9.8    30.8/26.0   17.5/14.5
+//   bs 1,   4 bytes   5.8/4.7     9.8/7.9    24.9/18.3   85.0/52.9      8.1/6.3    17.1/11.7   51.2/30.3   23.8/15.4
+//   bs 16,  4 bytes   4.7/4.0     7.3/6.4    16.2/15.1   50.6/48.7      6.0/5.2    11.2/9.6    30.0/26.4   15.6/14.1
+//   bs 128, 4 bytes   -           7.3/6.4    16.1/14.9   50.6/48.1      -          10.4/9.3    27.9/25.5   15.7/14.1
+constexpr int32_t kLeanUpTo = 256 * kLeanRows;
+static_assert(KVCM_COUNT_KEYS_UP_TO == kLeanUpTo, "only hash_lean_kernel counts keys");
+
+// How keys reach memory in larger launches, by block size, token width and number of requests (hash_tokens_kernel<.., KS>).
 // Chosen from timings on tokens that are not in the memory-side cache, us, requests of 4096 tokens each / of 500 to 4096
 // (a request that has run out makes the direct form compare per key; the staged forms leave that to the loaders).
-//   16-token blocks, 8-byte tokens: direct 64: 56 / 64  1024: 57 / -   2048: 58 / 66  4096: 61 / 69  8192: 73 / 77  10 240: 79 / 86
-//                                   spread                             2048: 59 / 60  4096: 60 / 60  8192: 65 / 70  10 240:  - / -
-//                                   burst  64: 58 / 60  1024: 58 / -   2048: 59 / 60  4096: 60 / 61  8192: 64 / 67  10 240: 68 / 72
-//   spread beats burst by 4 % on 2048 requests of 1024 tokens: direct below 2048, spread from there, burst from 8192. (Of 2048
-//   to 4096 tokens each, 2048 requests take 30.2 to 55.1 direct and 32.1 to 56.4 spread, ragged ones of 500 to 4096 63.7 and 57.0;
-//   below 2048 all stay direct, which costs the ragged ones what the first line says.)
+//   16-token blocks, 8-byte tokens: direct 4096: 61 / 69  8192: 73 / 77  10 240: 79 / 86
+//                                   spread 4096: 60 / 60  8192: 65 / 70
+//                                   burst  4096: 60 / 61  8192: 64 / 67  10 240: 68 / 72
+//   (up to 8191 spread, whose short workgroups store directly: kSpreadFromTiles)
 //   16-token blocks, 4-byte tokens: direct 4096: 55 / -   8192: 58 / 60  12 288: 70 / -
 //                                   burst  4096: 58 / -   8192: 58 / 61  12 288: 60 / -      (raw tiles, see below)
 // Other block sizes, direct / burst:
-//   block size 1, 8-byte tokens   16: 76 / 101 and 149 / 105   32: 87 / 97 and 151 / 105   64: 143 / 89 and 156 / 105   8192: 246 / 115
-//                                 (one kernel for all, which chooses by workgroup: chain_stays_direct)
-//                 4-byte tokens   32: 75 / -   64: 107 / 82 and 146 / 93   1024: 113 / 83   8192: 174 / 96
-//   block size 8, 8-byte tokens   1024: 66 / 62 (of 512 tokens: 14.7 / 15.6)   2048: 68 / 63   8192: 89 / 69   12 288: 104 / 88
+//   block size 1, 8-byte tokens   8192: 246 / 115   (a workgroup may still store directly: chain_stays_direct)
+//                 4-byte tokens   8192: 174 / 96   16 384 of 128 tokens: 10.8 / 7.1
+//   block size 8, 8-byte tokens   4160: 70 / 62   8192: 89 / 69   12 288: 104 / 88
 //                 4-byte tokens   8192: 66 / 61 (of 1024 tokens: 20.6 / 23.2)  12 288: 80 / 62
 //   block size 32, 8-byte tokens  4096: 59 / 58 (of 1024 tokens: 21.6 / 22.0)  8192: 66 / 61   12 288: 87 / 76
 //                  4-byte tokens  8192: 56 / 58   12 288: 67 / 60
 //   block size 64, 8-byte tokens  4096: 58 / 57 (of 1024 tokens: 21.6 / 22.0)  8192: 65 / 59   12 288: 79 / 73
 //                  4-byte tokens  8192: 55 / 58   12 288: 67 / 60
-//   block size 128, 8-byte tokens 2048: 56 / 54 (of 1024 tokens: 20.9 / 21.2)  4096: 58 / 55 (21.4 / 21.5)   8192: 64 / 58
+//   block size 128, 8-byte tokens 4160: 54 / 52 (of 1024 tokens: 18.3 / 18.5)  8192: 64 / 58
 //                   4-byte tokens 8192: 55 / 58   12 288: 65 / 59
-#ifndef KVCM_HASH_SPREAD_FROM_8
-#define KVCM_HASH_SPREAD_FROM_8 2048
-#endif
-// requests from which a launch takes the burst form; INT32_MAX = never
+// Requests from which a launch takes the burst form: all, where it is the better one right behind kLeanUpTo; INT32_MAX = never.
 constexpr int32_t burst_from(int32_t block_size, bool tokens_8_byte) {
     switch (block_size) {
-        case 1: return tokens_8_byte ? 1 : 64;
-        case 8: return tokens_8_byte ? 2048 : 12288;
+        case 1: return 0;
+        case 8: return tokens_8_byte ? 0 : 12288;
         case 16: return tokens_8_byte ? 8192 : 12288;
         case 32: return tokens_8_byte ? 8192 : 12288;
         case 64: return tokens_8_byte ? 8192 : 12288;
-        case 128: return tokens_8_byte ? 4096 : 12288;
+        case 128: return tokens_8_byte ? 0 : 12288;
         default: return INT32_MAX;
     }
 }
 // Tokens per request from which such a launch does: the last group leaves after the last token, so staging costs about 1 us
 // more than direct stores and has to earn that first. Lengths are known for [R, L] batches, their mean where the caller has
-// said how many tokens there are; otherwise requests are taken for long. us, staged / direct, at 8192 requests (2048 for 8-token
-// blocks, 4096 for 128; 4-byte tokens 12 288):
+// said how many tokens there are; otherwise requests are taken for long. us, staged / direct, at 8192 requests (4-byte tokens 12 288):
 //   equally long        64       256        512        768        1024       1536       2048       4096
-//   bs 8,   8 bytes  5.5/4.5   9.2/8.2   12.6/11.7  16.4/16.7  19.4/19.9  26.5/30.4  33.0/34.5  60.2/64.7
+//   bs 8,   8 bytes  6.4/5.4  10.1/9.2   13.9/14.2  17.7/19.5  21.0/23.3  29.9/36.9  35.4/43.1  64.5/80.4
 //   bs 16,  8 bytes  5.4/4.4   9.5/8.6   13.5/13.1  16.5/17.1  19.2/20.2  27.9/30.8  32.4/35.9  60.0/69.3
 //   bs 32,  8 bytes  5.6/4.6   9.5/8.6   13.6/13.0  16.3/16.2  19.4/19.8  26.3/28.3  31.3/34.2  57.9/64.8
 //   bs 64,  8 bytes  6.1/5.0   9.5/8.4   13.5/12.8  16.3/16.1  19.2/19.6  26.3/28.0  31.2/33.7  55.8/61.5
-//   bs 128, 8 bytes  3.5/3.6   9.0/8.1   12.5/11.9  15.5/15.1  18.5/18.3  24.0/25.0  29.5/30.1  52.1/54.9
+//   bs 128, 8 bytes  -         9.8/8.9   13.5/13.0  16.4/16.3  19.2/19.5  26.6/28.2  30.9/33.7  54.0/59.6
 //   bs 8,   4 bytes  6.1/4.2   9.1/7.7   12.8/11.4  17.1/15.4  20.9/19.8  27.1/27.1  34.1/35.6  59.3/73.5
 //   bs 16,  4 bytes  6.2/4.3   9.0/7.5   12.8/10.9  16.8/14.0  20.1/18.4  26.2/24.6  33.1/33.3  56.8/65.7
 //   bs 32,  4 bytes  6.4/4.4   8.9/7.4   12.8/10.8  16.8/13.8  20.4/17.7  26.0/22.9  32.8/32.1  56.4/65.3
@@ -1653,16 +1661,18 @@ constexpr int32_t burst_from(int32_t block_size, bool tokens_8_byte) {
 //   bs 128, 4 bytes  3.3/3.3   8.9/7.4   12.7/10.5  16.8/13.5  20.2/16.9  25.8/22.3  32.7/30.7  56.1/61.1
 //   ragged            16..64   64..512   64..768    64..1024   256..1024  64..2048   512..1536  64..4096   1024..2048 500..4096
 //   (mean)              35       215       283        346        554        573        932        969        1477       1710
-//   bs 8,   8 bytes  6.6/4.4  12.9/12.4  16.7/16.3  19.7/19.7  20.3/21.4  34.0/35.3  27.6/31.7  61.3/66.1  34.9/41.9  62.0/73.2
 //   bs 16,  8 bytes  7.9/4.5  14.3/13.0  17.5/17.2  20.6/21.0  20.8/22.7  33.8/36.7  29.2/32.3  61.2/68.1  36.0/42.3  64.9/76.3
 //   bs 32,  8 bytes  5.6/4.4  14.5/12.8  17.4/16.4  20.3/19.9  20.6/21.0  31.8/34.2  27.4/29.3  58.6/63.4  34.5/37.7  62.4/68.3
 //   bs 64,  8 bytes  5.4/4.3  14.7/12.2  17.9/15.8  20.2/19.1  20.3/19.8  32.0/33.1  26.8/27.5  57.4/61.8  33.8/35.7  60.6/64.8
-//   bs 128, 8 bytes  3.5/3.6  12.7/11.1  15.7/14.4  18.6/17.8  18.8/18.5  29.7/29.9  24.8/25.5  51.8/56.2  30.6/32.3  53.5/58.9
 //   bs 8,   4 bytes  8.6/4.2  14.1/11.8  16.8/15.6  20.6/19.3  21.7/20.2  34.0/33.5  28.3/28.7  59.3/62.0  35.4/37.9  60.2/67.6
 //   bs 16,  4 bytes  9.1/4.2  13.9/11.3  17.4/14.6  20.8/17.7  21.5/18.1  33.0/30.6  27.4/25.7  57.2/56.0  33.3/33.7  58.6/60.3
 //   bs 32,  4 bytes  6.3/4.4  14.1/11.0  17.7/14.2  20.9/17.3  21.2/17.6  32.3/29.8  27.8/24.3  57.7/54.1  34.0/31.7  58.4/56.7
 //   bs 64,  4 bytes  6.1/4.1  15.0/10.6  18.3/13.4  21.0/16.4  21.5/16.8  32.3/28.0  27.5/22.9  55.6/51.6  33.5/29.0  56.5/52.8
 //   bs 128, 4 bytes  3.3/3.3  14.2/10.3  17.6/13.0  20.2/16.2  20.7/16.8  32.0/27.5  26.5/22.7  54.7/50.5  32.2/28.6  55.2/51.6
+//   ragged            0..128   0..512     0..640     0..768     0..1024    0..1280    0..1792    0..2048    0..4096
+//   (mean)              64       256        320        384        512        640        896        1024       2048
+//   bs 8,   8 bytes  9.1/7.1  15.5/15.1  17.0/17.9  18.9/20.7  22.9/26.2  26.9/31.7  34.7/42.7  38.7/49.2  71.4/95.8
+//   bs 128, 8 bytes  -        15.7/13.1  16.8/14.9  17.4/16.4  20.3/20.1  23.3/23.7  30.0/31.0  33.3/34.6  60.2/63.5
 //   Four times as many requests move the lines little (4-byte tokens, 32 768 requests of 2000 to 8192: bs 64 215/248, 128 208/222).
 constexpr int64_t burst_from_tokens(int32_t block_size, bool tokens_8_byte, bool equally_long) {
     switch (block_size) {
@@ -1674,14 +1684,6 @@ constexpr int64_t burst_from_tokens(int32_t block_size, bool tokens_8_byte, bool
         default: return 0;
     }
 }
-// Requests up to which a launch takes workgroups of 16 (hash_lean_kernel): as many as give each of the 256 compute units one. A
-// second one on a unit shares its SIMDs, and one of 16 reads 512 bytes of each of 16 requests at a time where the other kernel
-// reads 64. us, 16 per workgroup / 64: 4096 requests of 4096 tokens 49.2 / 55.8, 5120: 59.0 / 56.8, 8192: 71.4 / 59.9.
-constexpr int32_t kLeanUpTo = 256 * kLeanRows;
-static_assert(KVCM_COUNT_KEYS_UP_TO == kLeanUpTo, "only hash_lean_kernel counts keys");
-#ifndef KVCM_HASH_BURST_SCALE  // for experiments: 0 = burst wherever it exists, a large number = never
-#define KVCM_HASH_BURST_SCALE 1
-#endif
 
 template <typename TokT>
 int32_t launch_hash(const TokT *d_tokens, const int64_t *d_token_offsets, int32_t R, int32_t block_size, int64_t seed,
@@ -1715,20 +1717,17 @@ int32_t launch_hash(const TokT *d_tokens, const int64_t *d_token_offsets, int32_
                        d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, have, \
                        force_global)
     constexpr bool k8 = sizeof(TokT) == 8;
-    const bool many = R >= static_cast<int64_t>(burst_from(block_size, k8)) * KVCM_HASH_BURST_SCALE;
+    const bool many = R >= burst_from(block_size, k8);
     const int64_t tokens_per_request = !d_token_offsets ? uni.tokens : have.tokens == kUnknown ? kUnknown : have.tokens / R;
-    // Block size 1, 4-byte tokens, staged / direct: 64 requests of 64 tokens 4.9 / 4.3 us, of 128: 6.2 / 5.3, of 16 to 64: 5.4 / 5.2,
-    // of 64 to 512: 14.6 / 19.4; 2048 of 128: 6.5 / 5.9; 16 384 of 128: 7.1 / 10.8.
-    const bool burst = many && (block_size == 1 ? k8 || R > 2048 || tokens_per_request > 128
-                                                : tokens_per_request >= burst_from_tokens(block_size, k8, !d_token_offsets));
-    const bool spread = block_size == 16 && k8 && !many && R >= KVCM_HASH_SPREAD_FROM_8;
+    const bool burst = many && tokens_per_request >= burst_from_tokens(block_size, k8, !d_token_offsets);
+    const bool spread = block_size == 16 && k8 && !many;
 #define KVCM_LAUNCH_HASH_STAGED(CHUNK, BS, KS)                                                                       \
     hipLaunchKernelGGL((hash_tokens_kernel<TokT, CHUNK, BS, KS>), grid, dim3(kThreads), 0, stream, d_tokens,        \
                        d_token_offsets, R, block_size, static_cast<uint64_t>(seed), d_keys, d_key_offsets, uni, have, \
                        force_global)
     // 4-byte tokens from as many requests as take the burst form: tiles of 128 raw tokens (512-byte pieces of the
     // token stream per request and load instruction instead of 256-byte ones). Cold timings, 16-token blocks, requests
-    // of 4096 tokens, 64-token tiles of pre-added terms / raw tiles: 64 requests 56.8 / 57.3 us, 8192 58.1 / 60.2,
+    // of 4096 tokens, 64-token tiles of pre-added terms / raw tiles: 8192 requests 58.1 / 60.2 us,
     // 12 288 66.6 / 62.2, 16 384 77.3 / 66.4, 32 768 149 / 127.
     const bool raw = !k8 && burst && (block_size == 8 || block_size == 16 || block_size == 32 || block_size == 64 ||
                                       block_size == 128);
@@ -1791,13 +1790,7 @@ int32_t launch_hash(const TokT *d_tokens, const int64_t *d_token_offsets, int32_
             KVCM_LAUNCH_HASH(8, 128);
         }
     } else if (block_size == 1) {  // the prefix chain over digests: a key after every step
-        if constexpr (k8) {
-            KVCM_LAUNCH_HASH_STAGED(1, 1, kKeysBurst);
-        } else if (burst) {
-            KVCM_LAUNCH_HASH_STAGED(1, 1, kKeysBurst);
-        } else {
-            KVCM_LAUNCH_HASH(1, 1);
-        }
+        KVCM_LAUNCH_HASH_STAGED(1, 1, kKeysBurst);
     } else if (block_size % 8 == 0) {
         KVCM_LAUNCH_HASH(8, 0);
     } else {
