@@ -451,9 +451,10 @@ __global__ __launch_bounds__(kPartThreads) void part_kernel(const uint64_t *__re
     // More different keys than slots, all of one part: keys with a pattern that the sum of products maps to one place. Their part is
     // gone through once more, as many times over as bring the number of keys down to half the slots, a share of the mixed keys
     // at a time. What has been cleared so far stays so (a smaller index of that key is known), everything else is decided again.
+    // 65 536 keys, each twice, all of one part 2.1 ms, with one slot to start from 4.8; 8192 of the latter 0.47 (looked for one by one,
+    // in the keys in front of each, 5.8 and the square of that for more). The look at s_full per key that is entered takes 0.5 %.
     const auto mine = [&](uint64_t k) { return k != kNoKey && part_hash(k) >> (32 - log2_parts) == blockIdx.x; };
     int32_t hits = 0;
-#pragma unroll 4
     for (int32_t i = threadIdx.x; i < n; i += kPartThreads) {
         hits += mine(keys[i]);
     }

@@ -232,7 +232,7 @@ def apply_prefix_hash(hash_ids: torch.Tensor, offsets: Optional[torch.Tensor] = 
 
 # Bytes of packed strings up to which the kernel reads them where they are packed, in pinned host memory: a copy in front of it
 # takes longer than the reads do, and from pageable memory the caller waits for it and for all work in front of it. us per call, in
-# place / copied from pinned memory: 1024 strings of 64 characters 14 / 28, 16 384 of 64: 33 / 46, of 200 (3.4 MB): 88 / 91.
+# place / copied: one string of 64 characters 12.6 / 21.9, 1024: 18.0 / 36.9, 16 384: 89 / 173, of 200 (3.4 MB): 161 / 376.
 _PINNED_MOST = 4 << 20
 # Packed strings that launched kernels have yet to read, oldest first, with the event behind each. Calls that find as many as this
 # under way, or with whose own there would be more bytes than this, copy instead: what finished calls leave here until the next one
