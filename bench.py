@@ -37,9 +37,10 @@ HBM_PEAK_GBPS = 8000.0  # MI355X HBM3E, published peak
 # read from inside this process, so the figures are carried here together with the digest of the kernel sources they
 # were measured on: a run whose sources differ reports traffic null and says why.
 KERNEL_SOURCES = ("tair_kvcache_amd/csrc/kvcm_copy.hip", "tair_kvcache_amd/csrc/kvcm_hash.hip",
-                  "tair_kvcache_amd/csrc/kvcm_internal.h", "tair_kvcache_amd/csrc/kvcm_host_idx.h")
-MEASURED_TRAFFIC = {"sources_sha256": "0ce44f437a73c9fe", "unique_blocks": 12416, "gather": 52076724646,
-                    "scatter": 52076193414, "hash_saturated": 571017961, "hash_saturated_i32": 302656148, "prefix_chain": 1074226605}
+                  "tair_kvcache_amd/csrc/kvcm_internal.h", "tair_kvcache_amd/csrc/kvcm_host_idx.h",
+                  "tair_kvcache_amd/csrc/kvcm_key_count.h")
+MEASURED_TRAFFIC = {"sources_sha256": "0eff9b14e23ffb42", "unique_blocks": 12416, "gather": 52076691187,
+                    "scatter": 52076141055, "hash_saturated": 571000408, "hash_saturated_i32": 302658806, "prefix_chain": 1074243081}
 
 # Llama-3-8B KV layout: the configuration the headline metric is quoted on
 LAYERS, KV_HEADS, HEAD_DIM, ITEMSIZE = 32, 8, 128, 2
