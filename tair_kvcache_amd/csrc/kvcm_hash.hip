@@ -206,8 +206,20 @@ struct BufferLoader {
     }
 };
 
+// Offsets need not ascend: a request may begin in front of its workgroup's first token. So loads count from the first token of
+// all wherever 32 bits reach the last one, and only in larger arrays from the workgroup's first. There a request may be out of reach,
+// in front of it or 4 GiB and more behind it; hash_lean_kernel looks at each, hash_tokens_kernel (where that costs block size 1 up to
+// 2 %) at where the workgroup's last one ends.
+constexpr uint64_t kBufferReach = 0xFFF00000u;
+template <typename TokT>
+__device__ __forceinline__ bool within_reach(int64_t total) { return static_cast<uint64_t>(total) < kBufferReach / sizeof(TokT); }
+template <typename TokT>
+__device__ __forceinline__ bool out_of_reach(int64_t start, int64_t ntok, int64_t first) {
+    return ntok > 0 && (start < first || !within_reach<TokT>(start - first + ntok));
+}
+
 // Loader, general form: one element per load through global addresses, positions clamped to the last token of
-// the batch. Used when the workgroup's requests span 4 GiB or more, which a 32-bit buffer offset cannot address.
+// the batch. Used when a 32-bit buffer offset does not reach one of the workgroup's requests.
 template <typename TokT, bool RAW = false>
 struct GlobalLoader {
     static constexpr int kTok = tile_tokens(RAW);
@@ -634,6 +646,7 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
     int64_t my_ntok = 0, key_pos = 0;
     LoaderCtx<TokT> ctx;
     bool buffer_loads = false;
+    int64_t first_start = 0;
     const int64_t r_first = static_cast<int64_t>(blockIdx.x) * kReqs;
     if (wave == 0) {
         int64_t start;
@@ -671,16 +684,17 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
         const int64_t r_end = r_first + kReqs < R ? r_first + kReqs : R;
         const bool known = token_offsets && have.tokens != kUnknown;
         const int64_t total = !token_offsets ? R * uni.tokens : known ? have.tokens : token_offsets[R];
-        const int64_t end_token = token_offsets ? token_offsets[r_end] : r_end * uni.tokens;
         ctx.last_token = total - 1;  // >= 0 whenever a tile is loaded: some request has a full block then
-        ctx.wg_first_token = token_offsets ? token_offsets[r_first] : r_first * uni.tokens;
+        first_start = token_offsets ? token_offsets[r_first] : r_first * uni.tokens;
+        ctx.wg_first_token = within_reach<TokT>(total) ? 0 : first_start;
         if (known && (ctx.wg_first_token < 0 || ctx.wg_first_token > total)) {
             ctx.wg_first_token = ctx.wg_first_token < 0 ? 0 : total;
         }
         const uint64_t to_end = static_cast<uint64_t>(total - ctx.wg_first_token) * sizeof(TokT);
         ctx.wg_bytes = to_end > 0xFFFFFFFFull ? 0xFFFFFFFFu : static_cast<uint32_t>(to_end);
+        const int64_t end_token = token_offsets ? token_offsets[r_end] : r_end * uni.tokens;
         const uint64_t wg_span = static_cast<uint64_t>(distance(ctx.wg_first_token, end_token)) * sizeof(TokT);
-        buffer_loads = !force_global_loads && wg_span < 0xFFF00000ull;
+        buffer_loads = !force_global_loads && (within_reach<TokT>(total) || wg_span < kBufferReach);
         if (uni.key_offsets_out && wave == kLoaders) {  // the last loader: its first tile is the one needed last
             if (r < R) {
                 uni.key_offsets_out[r] = r * uni.keys;
@@ -715,7 +729,7 @@ __global__ __launch_bounds__(kThreads) void hash_tokens_kernel(const TokT *__res
         // ---------------------------------------------------------------- loader waves
         const KeyDrain kd{s_keys, s_keyrow, keys};
         const bool apart = BS == 1 && KS == kKeysBurst && gridDim.x >= kApartFromWorkgroups &&
-                           __all((static_cast<uint32_t>(s_start[lane] - ctx.wg_first_token) * sizeof(TokT)) % kApartPeriod == 0);
+                           __all((static_cast<uint32_t>(s_start[lane] - first_start) * sizeof(TokT)) % kApartPeriod == 0);
         if (buffer_loads) {
             run_loader<BufferLoader<TokT, RAW>, TokT, KS, G, TOK>(ctx, s_tile, wave - 1, ntiles, lane, kd, staged, apart);
         } else {
@@ -909,7 +923,7 @@ struct LeanBufferLoader {
     }
 };
 
-// The same with an address per token, for workgroups whose requests span 4 GiB or more.
+// The same with an address per token, for workgroups with a request that a buffer offset does not reach.
 template <typename TokT>
 struct LeanGlobalLoader {
     static_assert(kLeanTok == 64, "a lane per token of a request's row");
@@ -1203,16 +1217,16 @@ __global__ __launch_bounds__(kLeanThreads) void hash_lean_kernel(const TokT *__r
     const int64_t r_first = static_cast<int64_t>(blockIdx.x) * kLeanRows;
     const int64_t r = r_first + lane % kLeanRows;
     LeanRow row{0, 0, 0};
-    int64_t count = 0, first = 0, span = 0, total;
+    int64_t count = 0, first = 0, total;
     int32_t nt;  // tiles of the longest request
     if (token_offsets) {
-        const int64_t r_end = r_first + kLeanRows < R ? r_first + kLeanRows : R;
         const bool known = have.tokens != kUnknown;
-        first = token_offsets[r_first];
         total = known ? have.tokens : token_offsets[R];
-        span = distance(first, token_offsets[r_end]);
-        if (known && (first < 0 || first > total)) {
-            first = first < 0 ? 0 : total;
+        if (!within_reach<TokT>(total)) {
+            first = token_offsets[r_first];
+            if (known && (first < 0 || first > total)) {
+                first = first < 0 ? 0 : total;
+            }
         }
         const int64_t at = token_offsets[r < R ? r : R], next = token_offsets[r < R ? r + 1 : R];
         const bool counts = out.key_offsets && wave == kLeanWriter;
@@ -1236,9 +1250,8 @@ __global__ __launch_bounds__(kLeanThreads) void hash_lean_kernel(const TokT *__r
             lean_key_offsets(r_first, R, before, nkeys, bad_before, nkeys > 0 && !there, have, out, lane, row, count);
         }
     } else {
-        first = r_first * uni.tokens;
         total = R * uni.tokens;
-        span = (R - r_first < kLeanRows ? R - r_first : kLeanRows) * uni.tokens;  // of the requests that there are
+        first = within_reach<TokT>(total) ? 0 : r_first * uni.tokens;
         if (r < R) {
             row.start = r * uni.tokens;
             row.key = key_offsets ? key_offsets[r] : r * uni.keys;
@@ -1264,7 +1277,6 @@ __global__ __launch_bounds__(kLeanThreads) void hash_lean_kernel(const TokT *__r
     }
     first = uniform_i64(first);
     total = uniform_i64(total);
-    span = uniform_i64(span);
     if (wave == kLeanWriter) {
         if constexpr (EVERY) {
             if (block_size == 1) {
@@ -1276,7 +1288,8 @@ __global__ __launch_bounds__(kLeanThreads) void hash_lean_kernel(const TokT *__r
         return;
     }
     if (wave != 0) {
-        if (!force_global_loads && span >= 0 && static_cast<uint64_t>(span) * sizeof(TokT) < 0xFFF00000ull) {
+        const bool buffer_loads = within_reach<TokT>(total) || __ballot(out_of_reach<TokT>(row.start, row.ntok, first)) == 0;
+        if (buffer_loads && !force_global_loads) {
             LeanBufferLoader<TokT> ld;
             ld.setup(tokens, first, total, row, lane);
             lean_load<LeanBufferLoader<TokT>, EVERY>(sh, ld, wave - 1, nt, seed, lane);
@@ -1301,6 +1314,10 @@ __global__ __launch_bounds__(kLeanThreads) void hash_lean_kernel(const TokT *__r
     };
     lds_barrier();
     read_group(a[0], &sh.tile[0][mine][0]);
+    // A step is 32 bytes of code, and where the loop begins within 32 bytes decides up to 1 % (64 x 4096 8-byte tokens 47.1 us at byte
+    // 8 or 12, 47.6 at 28). This, in front of the first tile, which the compiler takes out of the loop, puts it at 8, and at 16 where
+    // EVERY state is kept (48.9 to 49.2), whatever the code above takes.
+    asm volatile(".p2align 6\n\ts_nop 0\n\ts_nop 0\n\ts_nop 0");
     uint64_t *at = nullptr;  // where the states of the group before go
     for (int32_t k = 0; k < nt; ++k) {
         const uint64_t *const row_now = &sh.tile[k & (SH::kRing - 1)][mine][0], *const row_next = &sh.tile[(k + 1) & (SH::kRing - 1)][mine][0];

@@ -516,6 +516,37 @@ def test_offsets_whose_counts_add_up_to_more_than_63_bits(oracle, monkeypatch, o
 
 
 @pytest.mark.parametrize("general_loader", [False, True])
+@pytest.mark.parametrize("dtype,bs", [(np.int64, 16), (np.int32, 7), (np.int64, 1), (np.int32, 16)])
+@pytest.mark.parametrize("R", [20, 1000, 4200])
+def test_offsets_that_go_back(oracle, force_general_hash_loader, general_loader, dtype, bs, R):
+    """Token offsets that do not ascend: a request that ends in front of its start has no keys, and the ones behind it, wherever
+    they begin (in front of their workgroup's first offset, behind its last), those of their own tokens."""
+    force_general_hash_loader(general_loader)
+    rng = np.random.default_rng(R * bs)
+    n = 20000
+    flat = rng.integers(-2**31, 2**31, size=n, dtype=np.int64).astype(dtype)
+    toff = [n - 300]
+    for r in range(R):
+        toff.append(toff[-1] + int(rng.integers(0, 300)))
+        if toff[-1] > n or rng.random() < 0.2:
+            toff[-1] = int(rng.integers(0, max(1, min(n - 600, toff[-2]))))
+    counts = [max(0, b - a) // bs for a, b in zip(toff[:-1], toff[1:])]
+    koff = np.concatenate([[0], np.cumsum(counts)]).astype(np.int64)
+    assert any(b < a for a, b in zip(toff[:-1], toff[1:])) and max(toff) <= n
+    want = [oracle.hash_tokens(flat[None, a:a + c * bs].astype(np.int64), bs, seed=9)[0] for a, c in zip(toff, counts) if c]
+    want = np.concatenate(want)
+    tok, off = dev(flat), dev(np.array(toff, dtype=np.int64))
+    keys = torch.full((len(want) + 64,), -7, dtype=torch.int64, device="cuda")
+    _h().hash_tokens(tok, bs, token_offsets=off, seed=9, keys=keys, key_offsets=dev(koff))
+    sync()
+    assert (host(keys, np.int64)[:len(want)] == want).all() and (host(keys, np.int64)[len(want):] == -7).all()
+    if koff[-1] <= n // bs:                                      # counted by the call as well
+        got, goff = _h().hash_tokens(tok, bs, token_offsets=off, seed=9)
+        sync()
+        assert (host(got, np.int64) == want).all() and (host(goff, np.int64) == koff).all()
+
+
+@pytest.mark.parametrize("general_loader", [False, True])
 def test_keys_beyond_the_callers_buffer_are_left_out(oracle, force_general_hash_loader, general_loader):
     """A key buffer that holds the keys of some requests only: those are written, the slots behind the buffer are not; the
     same for a chain whose offsets name more digests than there are."""
